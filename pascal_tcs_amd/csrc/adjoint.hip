@@ -10,7 +10,7 @@
 //     adjoints go to the periodic sources, the mean projection is symmetric);
 //   * cell updates (projection, dPhat history, block corrections, pressure
 //     RHS, pseudo-update): vector-Jacobian products of the cell formulas
-//     (ad.h: each cell's recorded inputs, one dual-number pass per input);
+//     (rev.h: one reverse pass a cell);
 //   * each ADI stage x = A^-1 d: lambda = A^-T xbar by the transposed line
 //     solve (the stage's rows, transposed in place along the line, solved by
 //     the single-rank PaScaL_TDMA kernel), row adjoints abar_i = -lambda_i
@@ -23,6 +23,8 @@
 // The adjoint fields of the state (T, U, V, W, P, dPhat, dP0) and of the
 // temperature wall arrays are kept in the context.
 #define TCS_FORM adj
+#define TCS_REV
+#include "rev.h"
 #include "momentum.hip"
 #include "pressure.hip"
 #include "thermal.hip"
@@ -51,7 +53,6 @@ struct AdjWork {
     double *X[4][3];                // ADI stage solutions (interior layout)
     double *lam, *abar, *bbar, *cbar, *aT, *cT, *rint;  // interior layout
     double *scal;
-    int *flag;
     std::vector<void *> all;
 };
 
@@ -262,11 +263,10 @@ __global__ void k_row_bars(Grid g, int axis, int jlo, int cyc, const double *__r
 
 template <class Cell>
 int cell_vjp(tcs_ctx *c, AdjWork *w, const Cell &cell, int jlo, OutBars ob, InBars<Cell::NF> ib) {
-    // the LDS input sets keep an index in 28 bits: the largest array (a full
-    // field) must be indexed within it
-    if (c->nfull + FIELD_FRONT + 1 > ((size_t)1 << AD_KEY_IBITS)) return TCS_E_ARG;
-    const dim3 blk(64), grd((unsigned)((c->n1m + 63) / 64), (unsigned)(c->n2m - jlo + 1), (unsigned)c->n3m);
-    TCS_LAUNCH(c->stream, "adj_cell_vjp", (k_cell_vjp<Cell>), grd, blk, 0, cell, jlo, c->n2m, ob, ib, w->flag);
+    const int lw = std::min(64, c->n1m), rows = 64 / lw;
+    const dim3 blk(64), grd((unsigned)(c->n1m / lw), (unsigned)((c->n2m - jlo + rows) / rows),
+                            (unsigned)(c->n3m / VJP_KB));
+    TCS_LAUNCH(c->stream, "adj_cell_vjp", (k_cell_vjp<Cell>), grd, blk, 0, cell, jlo, c->n2m, lw, ob, ib);
     return TCS_OK;
 }
 
@@ -345,10 +345,17 @@ __global__ void k_coeffi_adj(Grid g, Phys p, const double *__restrict__ T, const
     bT[q] += mu.d * bMu[g.t2(j, k)] + ir.d * biR[g.t2(j, k)];
 }
 
-// the stale viscosities transposed (one thread; six outputs, few inputs)
-__global__ void k_stale_adj(Grid g, const double *__restrict__ Mu, const double *__restrict__ bstale,
-                            double *__restrict__ bMu) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// the stale viscosities transposed: the copies of their adjoints summed,
+// then, on one thread, six outputs of a few inputs
+__global__ void __launch_bounds__(64) k_stale_adj(Grid g, const double *__restrict__ Mu,
+                                                  const double *__restrict__ bstale, double *__restrict__ bMu) {
+    double b[6];
+    for (int q = 0; q < 6; q++) {
+        double s = 0.0;
+        for (int c = threadIdx.x; c < REV_STALE; c += 64) s += bstale[q + REV_STALE_STRIDE * c];
+        b[q] = lane_sum(s, 64);
+    }
+    if (threadIdx.x != 0) return;
     Rec rec;
     rec.n = 0;
     double v[6];
@@ -357,7 +364,7 @@ __global__ void k_stale_adj(Grid g, const double *__restrict__ Mu, const double 
         Dual o[6];
         stale_values<Dual>(g, SeedPtr{Mu, rec.idx[r]}, o);
         double s = 0.0;
-        for (int q = 0; q < 6; q++) s += o[q].d * bstale[q];
+        for (int q = 0; q < 6; q++) s += o[q].d * b[q];
         bMu[rec.idx[r]] += s;
     }
 }
@@ -625,7 +632,7 @@ static int backward(tcs_ctx *c, AdjWork *w, double dt) {
     // the step's own tables and scalars start from zero next time
     TCS_HIP(hipMemsetAsync(w->bMu, 0, c->ntab * sizeof(double), c->stream));
     TCS_HIP(hipMemsetAsync(w->biR, 0, c->ntab * sizeof(double), c->stream));
-    TCS_HIP(hipMemsetAsync(w->bstale, 0, 6 * sizeof(double), c->stream));
+    TCS_HIP(hipMemsetAsync(w->bstale, 0, REV_STALE * REV_STALE_STRIDE * sizeof(double), c->stream));
     return TCS_OK;
 }
 
@@ -658,19 +665,11 @@ static int adjoint_alloc(tcs_ctx *c) {
                        &w->sU1, &w->sV1, &w->sW1, &w->sdP, &w->tmp[0], &w->tmp[1], &w->tmp[2], &w->tmp[3]})
         rc |= get(p, c->nfull);
     for (double **p : {&w->bMu, &w->biR, &w->sMu, &w->siR}) rc |= get(p, c->ntab);
-    rc |= get(&w->bstale, 6) | get(&w->sstale, 6) | get(&w->scal, 1);
+    rc |= get(&w->bstale, (size_t)REV_STALE * REV_STALE_STRIDE) | get(&w->sstale, 6) | get(&w->scal, 1);
     for (int q = 0; q < TCS_NWALL; q++) rc |= get(&w->bwall[q], c->nwall);
     for (int s = 0; s < 4; s++)
         for (int q = 0; q < 3; q++) rc |= get(&w->X[s][q], c->nint);
     for (double **p : {&w->lam, &w->abar, &w->bbar, &w->cbar, &w->aT, &w->cT, &w->rint}) rc |= get(p, c->nint);
-    {
-        void *q = nullptr;
-        if (hipMalloc(&q, sizeof(int)) != hipSuccess || hipMemset(q, 0, sizeof(int)) != hipSuccess) rc = TCS_E_HIP;
-        else {
-            w->all.push_back(q);
-            w->flag = (int *)q;
-        }
-    }
     if (rc != TCS_OK) {
         adjoint_free(c);
         set_error("tcs_adjoint: device allocation failed");
@@ -754,16 +753,11 @@ extern "C" int tcs_adjoint_step(tcs_ctx *c, double dt) {
         set_error("tcs_adjoint_step: the adjoint differentiates the plain FP64 step (precision 0)");
         return TCS_E_ARG;
     }
+    // the interface's limit on the grid (2^28 values a field)
+    if (c->nfull + FIELD_FRONT + 1 > ((size_t)1 << 28)) return TCS_E_ARG;
     TCS_TRY(adjoint_alloc(c));
     c->cfl_valid = 0;
     TCS_TRY(adj::forward_keep(c, c->adj, dt));
     TCS_TRY(adj::backward(c, c->adj, dt));
-    int flag = 0;
-    TCS_HIP(hipMemcpyAsync(&flag, c->adj->flag, sizeof(int), hipMemcpyDeviceToHost, c->stream));
-    TCS_HIP(hipStreamSynchronize(c->stream));
-    if (flag) {
-        set_error("tcs_adjoint_step: a cell read more distinct inputs than the recorder holds");
-        return TCS_E_STATE;
-    }
     return TCS_OK;
 }

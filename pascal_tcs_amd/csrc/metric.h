@@ -11,7 +11,7 @@
 //
 // sc<S>(x): a constant of the formulas (a literal, a physical constant, dt,
 // a mask) in the arithmetic of S: float for S = float, else the double
-// itself (the double and dual-number instantiations are unchanged).
+// itself (also in the reverse pass).
 template <class S>
 __device__ __forceinline__ constexpr auto sc(double x) {
     if constexpr (std::is_same<S, float>::value) return (float)x;
@@ -30,7 +30,7 @@ __device__ __forceinline__ const double *mtab(const Grid &g) {
     else if constexpr (M == M_DX3) return g.dx3;
     else return g.dmx3;
 }
-#ifdef TCS_RECIP
+#if defined(TCS_RECIP) || defined(TCS_REV)
 template <int M>
 __device__ __forceinline__ const double *rtab(const Grid &g) {
     if constexpr (M == M_DX1) return g.rdx1;
@@ -65,6 +65,16 @@ struct RMetric {
 };
 __device__ __forceinline__ double operator/(double x, MVal m) { return x * m.r; }
 __device__ __forceinline__ double operator/(MVal a, MVal b) { return a.v * b.r; }
+#ifdef TCS_REV  // the adjoint's reverse pass (rev.h) multiplies by the reciprocals as the fast forms do
+template <class A, std::enable_if_t<node_v<A>, int> = 0>
+__device__ __forceinline__ auto operator/(A &&x, MVal m) { return std::forward<A>(x) * m.r; }
+template <class A, std::enable_if_t<node_v<A>, int> = 0>
+__device__ __forceinline__ auto operator*(MVal m, A &&x) { return m.v * std::forward<A>(x); }
+template <int M>
+__device__ __forceinline__ RMetric rmetric(const Grid &g) { return RMetric{mtab<M>(g), rtab<M>(g)}; }
+#endif
+#endif
+#ifdef TCS_RECIP
 struct MValF {
     float v, r;
     __device__ __forceinline__ operator float() const { return v; }
@@ -95,5 +105,12 @@ __device__ __forceinline__ auto metric(const Grid &g) {
 }
 #else
 template <class S, int M, bool D64 = false>
-__device__ __forceinline__ const double *metric(const Grid &g) { return mtab<M>(g); }
+__device__ __forceinline__ auto metric(const Grid &g) {
+#ifdef TCS_REV
+    if constexpr (is_rev<S>()) return rmetric<M>(g);
+    else return mtab<M>(g);
+#else
+    return mtab<M>(g);
+#endif
+}
 #endif

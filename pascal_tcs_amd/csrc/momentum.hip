@@ -120,62 +120,62 @@ __global__ void k_momentum_stale(Grid g, const double *__restrict__ Mu, double *
 // right-hand side; the functor after it carries its arguments.
 
 // ---------------------------------------------------------------- dU -------
-template <class S, int WM, class FP>
+template <class S, int WM, class FP, class I>
 __device__ __forceinline__ void dU_z_row(const Grid &g, const Phys &p, double dt, FP U,
     FP V, FP W, FP P,
     FP T, FP Mu, FP iR,
     FP UBCup, FP UBCbt, FP VBCup,
     FP VBCbt,
-    int i, int j, int k, S &am, S &ac, S &ap, S &rhsout) {
+    I i, I j, I k, S &am, S &ac, S &ap, S &rhsout) {
     ROW_METRICS
-    const int im = i - 1, ip = i + 1, jm = j - 1, jp = j + 1, km = k - 1, kp = k + 1;
+    const auto im = i - 1, ip = i + 1, jm = j - 1, jp = j + 1, km = k - 1, kp = k + 1;
     const int jum = g.jC[jm], jup = g.jC[jp];
-    const S Cmu = sc<S>(p.Cmu);
+    const auto Cmu = as<S>(sc<S>(p.Cmu));
 #define Uf(a, b, c) U[g.ix(a, b, c)]
 #define Vf(a, b, c) V[g.ix(a, b, c)]
 #define Wf(a, b, c) W[g.ix(a, b, c)]
-    const S u1 = sc<S>(0.5) * (Uf(im, j, k) + Uf(i, j, k));
-    const S u2 = sc<S>(0.5) * (Uf(ip, j, k) + Uf(i, j, k));
-    const S v3 = sc<S>(0.5) * (dx1[im] * Vf(i, j, k) + dx1[i] * Vf(im, j, k)) / dmx1[i];
-    const S v4 = sc<S>(0.5) * (dx1[im] * Vf(i, jp, k) + dx1[i] * Vf(im, jp, k)) / dmx1[i];
-    const S w5 = sc<S>(0.5) * (dx1[im] * Wf(i, j, k) + dx1[i] * Wf(im, j, k)) / dmx1[i];
-    const S w6 = sc<S>(0.5) * (dx1[im] * Wf(i, j, kp) + dx1[i] * Wf(im, j, kp)) / dmx1[i];
+    const auto u1 = as<S>(sc<S>(0.5) * (Uf(im, j, k) + Uf(i, j, k)));
+    const auto u2 = as<S>(sc<S>(0.5) * (Uf(ip, j, k) + Uf(i, j, k)));
+    const auto v3 = as<S>(sc<S>(0.5) * (dx1[im] * Vf(i, j, k) + dx1[i] * Vf(im, j, k)) / dmx1[i]);
+    const auto v4 = as<S>(sc<S>(0.5) * (dx1[im] * Vf(i, jp, k) + dx1[i] * Vf(im, jp, k)) / dmx1[i]);
+    const auto w5 = as<S>(sc<S>(0.5) * (dx1[im] * Wf(i, j, k) + dx1[i] * Wf(im, j, k)) / dmx1[i]);
+    const auto w6 = as<S>(sc<S>(0.5) * (dx1[im] * Wf(i, j, kp) + dx1[i] * Wf(im, j, kp)) / dmx1[i]);
 
-    const S dudx1 = (Uf(i, j, k) - Uf(im, j, k)) / dx1[im];
-    const S dudx2 = (Uf(ip, j, k) - Uf(i, j, k)) / dx1[i];
-    const S dudy3 = (Uf(i, j, k) - Uf(i, jm, k)) / dmx2[j];
-    const S dudy4 = (Uf(i, jp, k) - Uf(i, j, k)) / dmx2[jp];
-    const S dudz5 = (Uf(i, j, k) - Uf(i, j, km)) / dmx3[k];
-    const S dudz6 = (Uf(i, j, kp) - Uf(i, j, k)) / dmx3[kp];
-    const S dvdx3 = (Vf(i, j, k) - Vf(im, j, k)) / dmx1[i];
-    const S dvdx4 = (Vf(i, jp, k) - Vf(im, jp, k)) / dmx1[i];
-    const S dwdx5 = (Wf(i, j, k) - Wf(im, j, k)) / dmx1[i];
-    const S dwdx6 = (Wf(i, j, kp) - Wf(im, j, kp)) / dmx1[i];
+    const auto dudx1 = as<S>((Uf(i, j, k) - Uf(im, j, k)) / dx1[im]);
+    const auto dudx2 = as<S>((Uf(ip, j, k) - Uf(i, j, k)) / dx1[i]);
+    const auto dudy3 = as<S>((Uf(i, j, k) - Uf(i, jm, k)) / dmx2[j]);
+    const auto dudy4 = as<S>((Uf(i, jp, k) - Uf(i, j, k)) / dmx2[jp]);
+    const auto dudz5 = as<S>((Uf(i, j, k) - Uf(i, j, km)) / dmx3[k]);
+    const auto dudz6 = as<S>((Uf(i, j, kp) - Uf(i, j, k)) / dmx3[kp]);
+    const auto dvdx3 = as<S>((Vf(i, j, k) - Vf(im, j, k)) / dmx1[i]);
+    const auto dvdx4 = as<S>((Vf(i, jp, k) - Vf(im, jp, k)) / dmx1[i]);
+    const auto dwdx5 = as<S>((Wf(i, j, k) - Wf(im, j, k)) / dmx1[i]);
+    const auto dwdx6 = as<S>((Wf(i, j, kp) - Wf(im, j, kp)) / dmx1[i]);
 
-    S mua = sc<S>(0.5) * (dx1[im] * MU(jm, k) + dx1[i] * MU(jm, k)) / dmx1[i];
-    S muc = sc<S>(0.5) * (dx1[im] * MU(j, k) + dx1[i] * MU(j, k)) / dmx1[i];
-    S mub = sc<S>(0.5) * (dx1[im] * MU(jp, k) + dx1[i] * MU(jp, k)) / dmx1[i];
-    const S mu3 = sc<S>(0.5) * (dx2[jm] * muc + dx2[j] * mua) / dmx2[j];
-    const S mu4 = sc<S>(0.5) * (dx2[jp] * muc + dx2[j] * mub) / dmx2[jp];
-    mua = sc<S>(0.5) * (dx1[im] * MU(j, km) + dx1[i] * MU(j, km)) / dmx1[i];
-    muc = sc<S>(0.5) * (dx1[im] * MU(j, k) + dx1[i] * MU(j, k)) / dmx1[i];
-    mub = sc<S>(0.5) * (dx1[im] * MU(j, kp) + dx1[i] * MU(j, kp)) / dmx1[i];
-    const S mu5 = sc<S>(0.5) * (dx3[km] * muc + dx3[k] * mua) / dmx3[k];
-    const S mu6 = sc<S>(0.5) * (dx3[kp] * muc + dx3[k] * mub) / dmx3[kp];
+    const auto mua = as<S>(sc<S>(0.5) * (dx1[im] * MU(jm, k) + dx1[i] * MU(jm, k)) / dmx1[i]);
+    const auto muc = as<S>(sc<S>(0.5) * (dx1[im] * MU(j, k) + dx1[i] * MU(j, k)) / dmx1[i]);
+    const auto mub = as<S>(sc<S>(0.5) * (dx1[im] * MU(jp, k) + dx1[i] * MU(jp, k)) / dmx1[i]);
+    const auto mu3 = as<S>(sc<S>(0.5) * (dx2[jm] * muc + dx2[j] * mua) / dmx2[j]);
+    const auto mu4 = as<S>(sc<S>(0.5) * (dx2[jp] * muc + dx2[j] * mub) / dmx2[jp]);
+    const auto mua_2 = as<S>(sc<S>(0.5) * (dx1[im] * MU(j, km) + dx1[i] * MU(j, km)) / dmx1[i]);
+    const auto muc_2 = as<S>(sc<S>(0.5) * (dx1[im] * MU(j, k) + dx1[i] * MU(j, k)) / dmx1[i]);
+    const auto mub_2 = as<S>(sc<S>(0.5) * (dx1[im] * MU(j, kp) + dx1[i] * MU(j, kp)) / dmx1[i]);
+    const auto mu5 = as<S>(sc<S>(0.5) * (dx3[km] * muc_2 + dx3[k] * mua_2) / dmx3[k]);
+    const auto mu6 = as<S>(sc<S>(0.5) * (dx3[kp] * muc_2 + dx3[k] * mub_2) / dmx3[kp]);
 
-    const S invRhoc = sc<S>(0.5) * (dx1[im] * IR(j, k) + dx1[i] * IR(j, k)) / dmx1[i];
-    const S invRhocCmu_half = sc<S>(0.5) * Cmu * invRhoc;
+    const auto invRhoc = as<S>(sc<S>(0.5) * (dx1[im] * IR(j, k) + dx1[i] * IR(j, k)) / dmx1[i]);
+    const auto invRhocCmu_half = as<S>(sc<S>(0.5) * Cmu * invRhoc);
 
-    const S viscous_u1 = sc<S>(1.0) * (MU(j, k) * dudx2 - MU(j, k) * dudx1) / dmx1[i];
-    const S viscous_u2 = sc<S>(1.0) * (mu4 * dudy4 - mu3 * dudy3) / dx2[j];
-    const S viscous_u3 = sc<S>(1.0) * (mu6 * dudz6 - mu5 * dudz5) / dx3[k];
-    const S viscous_u12 = sc<S>(1.0) * (mu4 * dvdx4 - mu3 * dvdx3) / dx2[j];
-    const S viscous_u13 = sc<S>(1.0) * (mu6 * dwdx6 - mu5 * dwdx5) / dx3[k];
+    const auto viscous_u1 = as<S>(sc<S>(1.0) * (MU(j, k) * dudx2 - MU(j, k) * dudx1) / dmx1[i]);
+    const auto viscous_u2 = as<S>(sc<S>(1.0) * (mu4 * dudy4 - mu3 * dudy3) / dx2[j]);
+    const auto viscous_u3 = as<S>(sc<S>(1.0) * (mu6 * dudz6 - mu5 * dudz5) / dx3[k]);
+    const auto viscous_u12 = as<S>(sc<S>(1.0) * (mu4 * dvdx4 - mu3 * dvdx3) / dx2[j]);
+    const auto viscous_u13 = as<S>(sc<S>(1.0) * (mu6 * dwdx6 - mu5 * dwdx5) / dx3[k]);
 
-    S rhs = invRhocCmu_half * (sc<S>(2.0) * viscous_u1 + viscous_u2 + viscous_u3 + viscous_u12 + viscous_u13);
-    rhs = rhs - sc<S>(p.Cmp) * invRhoc * (P[g.ix(i, j, k)] - P[g.ix(im, j, k)]) / dmx1[i];
-    const S Tc = sc<S>(0.5) * (dx1[im] * T[g.ix(i, j, k)] + dx1[i] * T[g.ix(im, j, k)]) / dmx1[i];
-    rhs = rhs + sc<S>(p.Cmt) * (Tc + sc<S>(p.a12pera11) * (Tc * Tc) * sc<S>(p.DeltaT)) * invRhoc;
+    const auto rhs = as<S>(invRhocCmu_half * (sc<S>(2.0) * viscous_u1 + viscous_u2 + viscous_u3 + viscous_u12 + viscous_u13));
+    const auto rhs_2 = as<S>(rhs - sc<S>(p.Cmp) * invRhoc * (P[g.ix(i, j, k)] - P[g.ix(im, j, k)]) / dmx1[i]);
+    const auto Tc = as<S>(sc<S>(0.5) * (dx1[im] * T[g.ix(i, j, k)] + dx1[i] * T[g.ix(im, j, k)]) / dmx1[i]);
+    const auto rhs_3 = as<S>(rhs_2 + sc<S>(p.Cmt) * (Tc + sc<S>(p.a12pera11) * (Tc * Tc) * sc<S>(p.DeltaT)) * invRhoc);
 
     // The wall terms are multiplied by 1 - jum and 1 - jup, zero away from the
     // walls, where rhs + 0 * term = rhs for finite terms.  WM says how a row
@@ -183,42 +183,47 @@ __device__ __forceinline__ void dU_z_row(const Grid &g, const Phys &p, double dt
     // walls (a branch on j, uniform in a wavefront), 2 leaves them out (the
     // caller has checked that j is away from the walls, wall_free); skipped,
     // the loads of the wall arrays are not issued either.
-    if (WM == 0 || (WM == 1 && (jum != 1 || jup != 1))) {
-    S ubc_down = sc<S>(0.25) * v3 / dmx2[j] * UBCbt[g.b2(i, k)]
-                    - sc<S>(0.25) * dudy3 * (dx1[i] * VBCbt[g.b2(im, k)] + dx1[im] * VBCbt[g.b2(i, k)]) / dmx1[i] * sc<S>(0.5);
-    S ubc_up = -sc<S>(0.25) * v4 / dmx2[jp] * UBCup[g.b2(i, k)]
-                  - sc<S>(0.25) * dudy4 * (dx1[i] * VBCup[g.b2(im, k)] + dx1[im] * VBCup[g.b2(i, k)]) / dmx1[i] * sc<S>(0.5);
-    ubc_down = ubc_down + invRhocCmu_half / dx2[j] * mu3 / dmx2[j] * UBCbt[g.b2(i, k)];
-    ubc_down = ubc_down - invRhocCmu_half / dx2[j] * mu3 / dmx1[i] * (VBCbt[g.b2(i, k)] - VBCbt[g.b2(im, k)]);
-    ubc_up = ubc_up + invRhocCmu_half / dx2[j] * mu4 / dmx2[jp] * UBCup[g.b2(i, k)];
-    ubc_up = ubc_up + invRhocCmu_half / dx2[j] * mu4 / dmx1[i] * (VBCup[g.b2(i, k)] - VBCup[g.b2(im, k)]);
-    rhs = rhs + (sc<S>(1.0) - sc<S>(jum)) * ubc_down + (sc<S>(1.0) - sc<S>(jup)) * ubc_up;
-    }
+    const auto wall_terms = [&](const auto &r) {
+        const auto ubc_down = [&] {
+            return sc<S>(0.25) * v3 / dmx2[j] * UBCbt[g.b2(i, k)]
+                 - sc<S>(0.25) * dudy3 * (dx1[i] * VBCbt[g.b2(im, k)] + dx1[im] * VBCbt[g.b2(i, k)]) / dmx1[i] * sc<S>(0.5)
+                 + invRhocCmu_half / dx2[j] * mu3 / dmx2[j] * UBCbt[g.b2(i, k)]
+                 - invRhocCmu_half / dx2[j] * mu3 / dmx1[i] * (VBCbt[g.b2(i, k)] - VBCbt[g.b2(im, k)]);
+        };
+        const auto ubc_up = [&] {
+            return -sc<S>(0.25) * v4 / dmx2[jp] * UBCup[g.b2(i, k)]
+                 - sc<S>(0.25) * dudy4 * (dx1[i] * VBCup[g.b2(im, k)] + dx1[im] * VBCup[g.b2(i, k)]) / dmx1[i] * sc<S>(0.5)
+                 + invRhocCmu_half / dx2[j] * mu4 / dmx2[jp] * UBCup[g.b2(i, k)]
+                 + invRhocCmu_half / dx2[j] * mu4 / dmx1[i] * (VBCup[g.b2(i, k)] - VBCup[g.b2(im, k)]);
+        };
+        return r + (sc<S>(1.0) - sc<S>(jum)) * ubc_down() + (sc<S>(1.0) - sc<S>(jup)) * ubc_up();
+    };
+    const auto rhs_4 = as<S>(with_walls<S, WM>(jum != 1 || jup != 1, rhs_3, wall_terms));
 
-    const S mACI = invRhocCmu_half / dmx1[i] * (MU(j, k) / dx1[i] + MU(j, k) / dx1[im]) * sc<S>(2.0)
-                      + sc<S>(0.25) * (dudx2 * sc<S>(0.5) + dudx1 * sc<S>(0.5) - u2 / dx1[i] + u1 / dx1[im]);
-    const S mAPI = -invRhocCmu_half / dmx1[i] * MU(j, k) / dx1[i] * sc<S>(2.0) + sc<S>(0.25) * (u2 / dx1[i] + dudx2 * sc<S>(0.5));
-    const S mAMI = -invRhocCmu_half / dmx1[i] * MU(j, k) / dx1[im] * sc<S>(2.0) + sc<S>(0.25) * (-u1 / dx1[im] + dudx1 * sc<S>(0.5));
-    const S mACJ = invRhocCmu_half / dx2[j] * (mu4 / dmx2[jp] + mu3 / dmx2[j]) + sc<S>(0.25) * (-v4 / dmx2[jp] + v3 / dmx2[j]);
-    S mAPJ = -invRhocCmu_half / dx2[j] * mu4 / dmx2[jp] + sc<S>(0.25) * (v4 / dmx2[jp]);
-    S mAMJ = -invRhocCmu_half / dx2[j] * mu3 / dmx2[j] + sc<S>(0.25) * (-v3 / dmx2[j]);
-    mAPJ = mAPJ * sc<S>(jup);
-    mAMJ = mAMJ * sc<S>(jum);
-    const S mACK = invRhocCmu_half / dx3[k] * (mu6 / dmx3[kp] + mu5 / dmx3[k]) + sc<S>(0.25) * (-w6 / dmx3[kp] + w5 / dmx3[k]);
-    const S mAPK = -invRhocCmu_half / dx3[k] * mu6 / dmx3[kp] + sc<S>(0.25) * (w6 / dmx3[kp]);
-    const S mAMK = -invRhocCmu_half / dx3[k] * mu5 / dmx3[k] + sc<S>(0.25) * (-w5 / dmx3[k]);
+    const auto mACI = as<S>(invRhocCmu_half / dmx1[i] * (MU(j, k) / dx1[i] + MU(j, k) / dx1[im]) * sc<S>(2.0)
+                      + sc<S>(0.25) * (dudx2 * sc<S>(0.5) + dudx1 * sc<S>(0.5) - u2 / dx1[i] + u1 / dx1[im]));
+    const auto mAPI = as<S>(-invRhocCmu_half / dmx1[i] * MU(j, k) / dx1[i] * sc<S>(2.0) + sc<S>(0.25) * (u2 / dx1[i] + dudx2 * sc<S>(0.5)));
+    const auto mAMI = as<S>(-invRhocCmu_half / dmx1[i] * MU(j, k) / dx1[im] * sc<S>(2.0) + sc<S>(0.25) * (-u1 / dx1[im] + dudx1 * sc<S>(0.5)));
+    const auto mACJ = as<S>(invRhocCmu_half / dx2[j] * (mu4 / dmx2[jp] + mu3 / dmx2[j]) + sc<S>(0.25) * (-v4 / dmx2[jp] + v3 / dmx2[j]));
+    const auto mAPJ = as<S>(-invRhocCmu_half / dx2[j] * mu4 / dmx2[jp] + sc<S>(0.25) * (v4 / dmx2[jp]));
+    const auto mAMJ = as<S>(-invRhocCmu_half / dx2[j] * mu3 / dmx2[j] + sc<S>(0.25) * (-v3 / dmx2[j]));
+    const auto mAPJ_2 = as<S>(mAPJ * sc<S>(jup));
+    const auto mAMJ_2 = as<S>(mAMJ * sc<S>(jum));
+    const auto mACK = as<S>(invRhocCmu_half / dx3[k] * (mu6 / dmx3[kp] + mu5 / dmx3[k]) + sc<S>(0.25) * (-w6 / dmx3[kp] + w5 / dmx3[k]));
+    const auto mAPK = as<S>(-invRhocCmu_half / dx3[k] * mu6 / dmx3[kp] + sc<S>(0.25) * (w6 / dmx3[kp]));
+    const auto mAMK = as<S>(-invRhocCmu_half / dx3[k] * mu5 / dmx3[k] + sc<S>(0.25) * (-w5 / dmx3[k]));
 
-    rhs = rhs - (mAPI * Uf(ip, j, k) + mACI * Uf(i, j, k) + mAMI * Uf(im, j, k)
-                 + mAPJ * Uf(i, jp, k) + mACJ * Uf(i, j, k) + mAMJ * Uf(i, jm, k)
-                 + mAPK * Uf(i, j, kp) + mACK * Uf(i, j, k) + mAMK * Uf(i, j, km));
-    rhs = rhs - (sc<S>(0.25) * (v4 * sc<S>(jup) * dudy4 + v3 * sc<S>(jum) * dudy3)
-                 - invRhocCmu_half / dx2[j] * (mu4 * dvdx4 * sc<S>(jup) - mu3 * dvdx3 * sc<S>(jum)));
-    rhs = rhs - (sc<S>(0.25) * (w6 * dudz6 + w5 * dudz5) - invRhocCmu_half / dx3[k] * (mu6 * dwdx6 - mu5 * dwdx5));
+    const auto rhs_5 = as<S>(rhs_4 - (mAPI * Uf(ip, j, k) + mACI * Uf(i, j, k) + mAMI * Uf(im, j, k)
+                 + mAPJ_2 * Uf(i, jp, k) + mACJ * Uf(i, j, k) + mAMJ_2 * Uf(i, jm, k)
+                 + mAPK * Uf(i, j, kp) + mACK * Uf(i, j, k) + mAMK * Uf(i, j, km)));
+    const auto rhs_6 = as<S>(rhs_5 - (sc<S>(0.25) * (v4 * sc<S>(jup) * dudy4 + v3 * sc<S>(jum) * dudy3)
+                 - invRhocCmu_half / dx2[j] * (mu4 * dvdx4 * sc<S>(jup) - mu3 * dvdx3 * sc<S>(jum))));
+    const auto rhs_7 = as<S>(rhs_6 - (sc<S>(0.25) * (w6 * dudz6 + w5 * dudz5) - invRhocCmu_half / dx3[k] * (mu6 * dwdx6 - mu5 * dwdx5)));
 
     ac = mACK * sc<S>(dt) + sc<S>(1.0);
     ap = mAPK * sc<S>(dt);
     am = mAMK * sc<S>(dt);
-    rhsout = rhs * sc<S>(dt);
+    rhsout = rhs_7 * sc<S>(dt);
 }
 struct DUZ {
     // FP32 lines of the mixed form: the unconditional row loop (2.14 -> 2.03 ms
@@ -230,9 +235,10 @@ struct DUZ {
     double dt;
     const double *U, *V, *W, *P, *T, *Mu, *iR, *UBCup, *UBCbt, *VBCup, *VBCbt;
     static constexpr int NF = 11;  // field inputs, in the order below
+    static constexpr int ND = 7, STALE = -1;  // rev.h
     static constexpr bool FULL = true;  // unconditional row loop in the FP64 z solve
-    template <class S, int WM = -1, class Wr>
-    __device__ __forceinline__ void eval(const Wr &w, int i, int j, int k, S &a, S &b, S &c, S &d) const {
+    template <class S, int WM = -1, class Wr, class I>
+    __device__ __forceinline__ void eval(const Wr &w, I i, I j, I k, S &a, S &b, S &c, S &d) const {
         // WM < 0 (the row's own wall-term mode): terms kept; the FP64 z lines
         // pass 2 or 0 per workgroup (wall_free), the FP32 ones keep them
         dU_z_row<S, (WM >= 0 ? WM : 0)>(g, p, dt, w(0, U), w(1, V), w(2, W), w(3, P), w(4, T), w(5, Mu), w(6, iR), w(7, UBCup), w(8, UBCbt), w(9, VBCup), w(10, VBCbt), i, j, k, a, b, c, d);
@@ -245,22 +251,22 @@ struct DUZ {
     }
 };
 
-template <class S, class FP>
+template <class S, class FP, class I>
 __device__ __forceinline__ void dU_x_row(const Grid &g, const Phys &p, double dt, FP U,
     FP Mu, FP iR,
-    int i, int j, int k, S &am, S &ac, S &ap) {
+    I i, I j, I k, S &am, S &ac, S &ap) {
     ROW_METRICS
-    const int im = i - 1, ip = i + 1;
-    const S u1 = sc<S>(0.5) * (Uf(im, j, k) + Uf(i, j, k));
-    const S u2 = sc<S>(0.5) * (Uf(ip, j, k) + Uf(i, j, k));
-    const S dudx1 = (Uf(i, j, k) - Uf(im, j, k)) / dx1[im];
-    const S dudx2 = (Uf(ip, j, k) - Uf(i, j, k)) / dx1[i];
-    const S invRhoc = sc<S>(0.5) * (dx1[im] * IR(j, k) + dx1[i] * IR(j, k)) / dmx1[i];
-    const S invRhocCmu_half = sc<S>(0.5) * sc<S>(p.Cmu) * invRhoc;
-    const S mACI = invRhocCmu_half / dmx1[i] * (MU(j, k) / dx1[i] + MU(j, k) / dx1[im]) * sc<S>(2.0)
-                      + sc<S>(0.25) * (dudx2 * sc<S>(0.5) + dudx1 * sc<S>(0.5) - u2 / dx1[i] + u1 / dx1[im]);
-    const S mAPI = -invRhocCmu_half / dmx1[i] * MU(j, k) / dx1[i] * sc<S>(2.0) + sc<S>(0.25) * (u2 / dx1[i] + dudx2 * sc<S>(0.5));
-    const S mAMI = -invRhocCmu_half / dmx1[i] * MU(j, k) / dx1[im] * sc<S>(2.0) + sc<S>(0.25) * (-u1 / dx1[im] + dudx1 * sc<S>(0.5));
+    const auto im = i - 1, ip = i + 1;
+    const auto u1 = as<S>(sc<S>(0.5) * (Uf(im, j, k) + Uf(i, j, k)));
+    const auto u2 = as<S>(sc<S>(0.5) * (Uf(ip, j, k) + Uf(i, j, k)));
+    const auto dudx1 = as<S>((Uf(i, j, k) - Uf(im, j, k)) / dx1[im]);
+    const auto dudx2 = as<S>((Uf(ip, j, k) - Uf(i, j, k)) / dx1[i]);
+    const auto invRhoc = as<S>(sc<S>(0.5) * (dx1[im] * IR(j, k) + dx1[i] * IR(j, k)) / dmx1[i]);
+    const auto invRhocCmu_half = as<S>(sc<S>(0.5) * sc<S>(p.Cmu) * invRhoc);
+    const auto mACI = as<S>(invRhocCmu_half / dmx1[i] * (MU(j, k) / dx1[i] + MU(j, k) / dx1[im]) * sc<S>(2.0)
+                      + sc<S>(0.25) * (dudx2 * sc<S>(0.5) + dudx1 * sc<S>(0.5) - u2 / dx1[i] + u1 / dx1[im]));
+    const auto mAPI = as<S>(-invRhocCmu_half / dmx1[i] * MU(j, k) / dx1[i] * sc<S>(2.0) + sc<S>(0.25) * (u2 / dx1[i] + dudx2 * sc<S>(0.5)));
+    const auto mAMI = as<S>(-invRhocCmu_half / dmx1[i] * MU(j, k) / dx1[im] * sc<S>(2.0) + sc<S>(0.25) * (-u1 / dx1[im] + dudx1 * sc<S>(0.5)));
     ac = mACI * sc<S>(dt) + sc<S>(1.0);
     ap = mAPI * sc<S>(dt);
     am = mAMI * sc<S>(dt);
@@ -271,8 +277,9 @@ struct DUX {
     double dt;
     const double *U, *Mu, *iR;
     static constexpr int NF = 3;  // field inputs, in the order below
-    template <class S, class Wr>
-    __device__ __forceinline__ void eval(const Wr &w, int i, int j, int k, S &a, S &b, S &c, S &d) const {
+    static constexpr int ND = 3, STALE = -1;  // rev.h
+    template <class S, class Wr, class I>
+    __device__ __forceinline__ void eval(const Wr &w, I i, I j, I k, S &a, S &b, S &c, S &d) const {
         dU_x_row<S>(g, p, dt, w(0, U), w(1, Mu), w(2, iR), i, j, k, a, b, c);
     }
     __device__ __forceinline__ void operator()(int i, int j, int k, double &a, double &b, double &c,
@@ -281,30 +288,30 @@ struct DUX {
     }
 };
 
-template <class S, class FP>
+template <class S, class FP, class I>
 __device__ __forceinline__ void dU_y_row(const Grid &g, const Phys &p, double dt, FP V,
     FP Mu, FP iR,
-    int i, int j, int k, S &am, S &ac, S &ap) {
+    I i, I j, I k, S &am, S &ac, S &ap) {
     ROW_METRICS
-    const int im = i - 1, jm = j - 1, jp = j + 1;
+    const auto im = i - 1, jm = j - 1, jp = j + 1;
     const int jum = g.jC[jm], jup = g.jC[jp];
-    const S v3 = sc<S>(0.5) * (dx1[im] * Vf(i, j, k) + dx1[i] * Vf(im, j, k)) / dmx1[i];
-    const S v4 = sc<S>(0.5) * (dx1[im] * Vf(i, jp, k) + dx1[i] * Vf(im, jp, k)) / dmx1[i];
-    const S mua = sc<S>(0.5) * (dx1[im] * MU(jm, k) + dx1[i] * MU(jm, k)) / dmx1[i];
-    const S muc = sc<S>(0.5) * (dx1[im] * MU(j, k) + dx1[i] * MU(j, k)) / dmx1[i];
-    const S mub = sc<S>(0.5) * (dx1[im] * MU(jp, k) + dx1[i] * MU(jp, k)) / dmx1[i];
-    const S mu3 = sc<S>(0.5) * (dx2[jm] * muc + dx2[j] * mua) / dmx2[j];
-    const S mu4 = sc<S>(0.5) * (dx2[jp] * muc + dx2[j] * mub) / dmx2[jp];
-    const S invRhoc = sc<S>(0.5) * (dx1[im] * IR(j, k) + dx1[i] * IR(j, k)) / dmx1[i];
-    const S invRhocCmu_half = sc<S>(0.5) * sc<S>(p.Cmu) * invRhoc;
-    const S mACJ = invRhocCmu_half / dx2[j] * (mu4 / dmx2[jp] + mu3 / dmx2[j]) + sc<S>(0.25) * (-v4 / dmx2[jp] + v3 / dmx2[j]);
-    S mAPJ = -invRhocCmu_half / dx2[j] * mu4 / dmx2[jp] + sc<S>(0.25) * (v4 / dmx2[jp]);
-    S mAMJ = -invRhocCmu_half / dx2[j] * mu3 / dmx2[j] + sc<S>(0.25) * (-v3 / dmx2[j]);
-    mAPJ = mAPJ * sc<S>(jup);
-    mAMJ = mAMJ * sc<S>(jum);
+    const auto v3 = as<S>(sc<S>(0.5) * (dx1[im] * Vf(i, j, k) + dx1[i] * Vf(im, j, k)) / dmx1[i]);
+    const auto v4 = as<S>(sc<S>(0.5) * (dx1[im] * Vf(i, jp, k) + dx1[i] * Vf(im, jp, k)) / dmx1[i]);
+    const auto mua = as<S>(sc<S>(0.5) * (dx1[im] * MU(jm, k) + dx1[i] * MU(jm, k)) / dmx1[i]);
+    const auto muc = as<S>(sc<S>(0.5) * (dx1[im] * MU(j, k) + dx1[i] * MU(j, k)) / dmx1[i]);
+    const auto mub = as<S>(sc<S>(0.5) * (dx1[im] * MU(jp, k) + dx1[i] * MU(jp, k)) / dmx1[i]);
+    const auto mu3 = as<S>(sc<S>(0.5) * (dx2[jm] * muc + dx2[j] * mua) / dmx2[j]);
+    const auto mu4 = as<S>(sc<S>(0.5) * (dx2[jp] * muc + dx2[j] * mub) / dmx2[jp]);
+    const auto invRhoc = as<S>(sc<S>(0.5) * (dx1[im] * IR(j, k) + dx1[i] * IR(j, k)) / dmx1[i]);
+    const auto invRhocCmu_half = as<S>(sc<S>(0.5) * sc<S>(p.Cmu) * invRhoc);
+    const auto mACJ = as<S>(invRhocCmu_half / dx2[j] * (mu4 / dmx2[jp] + mu3 / dmx2[j]) + sc<S>(0.25) * (-v4 / dmx2[jp] + v3 / dmx2[j]));
+    const auto mAPJ = as<S>(-invRhocCmu_half / dx2[j] * mu4 / dmx2[jp] + sc<S>(0.25) * (v4 / dmx2[jp]));
+    const auto mAMJ = as<S>(-invRhocCmu_half / dx2[j] * mu3 / dmx2[j] + sc<S>(0.25) * (-v3 / dmx2[j]));
+    const auto mAPJ_2 = as<S>(mAPJ * sc<S>(jup));
+    const auto mAMJ_2 = as<S>(mAMJ * sc<S>(jum));
     ac = mACJ * sc<S>(dt) + sc<S>(1.0);
-    ap = mAPJ * sc<S>(dt);
-    am = mAMJ * sc<S>(dt);
+    ap = mAPJ_2 * sc<S>(dt);
+    am = mAMJ_2 * sc<S>(dt);
 }
 struct DUY {
     // FP32 lines of the mixed form: the unconditional row loop (0.96 -> 0.56 ms
@@ -316,8 +323,9 @@ struct DUY {
     double dt;
     const double *V, *Mu, *iR;
     static constexpr int NF = 3;  // field inputs, in the order below
-    template <class S, class Wr>
-    __device__ __forceinline__ void eval(const Wr &w, int i, int j, int k, S &a, S &b, S &c, S &d) const {
+    static constexpr int ND = 3, STALE = -1;  // rev.h
+    template <class S, class Wr, class I>
+    __device__ __forceinline__ void eval(const Wr &w, I i, I j, I k, S &a, S &b, S &c, S &d) const {
         dU_y_row<S>(g, p, dt, w(0, V), w(1, Mu), w(2, iR), i, j, k, a, b, c);
     }
     __device__ __forceinline__ void operator()(int i, int j, int k, double &a, double &b, double &c,
@@ -339,95 +347,101 @@ __global__ void k_dV_zero_rows(Grid g, E *__restrict__ dV) {
 }
 
 // ---------------------------------------------------------------- dV -------
-template <class S, int WM, class FP>
+template <class S, int WM, class FP, class I>
 __device__ __forceinline__ void dV_z_row(const Grid &g, const Phys &p, double dt, FP U,
     FP V, FP W, FP P,
     FP dU, FP Mu, FP iR,
     FP VBCup, FP VBCbt,
-    int i, int j, int k, S &am, S &ac, S &ap, S &rhsout) {
+    I i, I j, I k, S &am, S &ac, S &ap, S &rhsout) {
     ROW_METRICS_D64
-    const int im = i - 1, ip = i + 1, jm = j - 1, jp = j + 1, km = k - 1, kp = k + 1;
+    const auto im = i - 1, ip = i + 1, jm = j - 1, jp = j + 1, km = k - 1, kp = k + 1;
     const int jvp = g.jS[jm], jvm = g.jS[jp];
-    const S Cmu = sc<S>(p.Cmu);
+    const auto Cmu = as<S>(sc<S>(p.Cmu));
 #define dUf(a, b, c) dU[g.ix(a, b, c)]
-    const S v3 = sc<S>(0.5) * (Vf(i, jm, k) + Vf(i, j, k));
-    const S v4 = sc<S>(0.5) * (Vf(i, j, k) + Vf(i, jp, k));
-    const S u1 = (dx2[jm] * Uf(i, j, k) + dx2[j] * Uf(i, jm, k)) / dmx2[j] * sc<S>(0.5);
-    const S u2 = (dx2[jm] * Uf(ip, j, k) + dx2[j] * Uf(ip, jm, k)) / dmx2[j] * sc<S>(0.5);
-    const S w5 = (dx2[jm] * Wf(i, j, k) + dx2[j] * Wf(i, jm, k)) / dmx2[j] * sc<S>(0.5);
-    const S w6 = (dx2[jm] * Wf(i, j, kp) + dx2[j] * Wf(i, jm, kp)) / dmx2[j] * sc<S>(0.5);
-    const S ddu1 = (dx2[jm] * dUf(i, j, k) + dx2[j] * dUf(i, jm, k)) / dmx2[j] * sc<S>(0.5);
-    const S ddu2 = (dx2[jm] * dUf(ip, j, k) + dx2[j] * dUf(ip, jm, k)) / dmx2[j] * sc<S>(0.5);
+    const auto v3 = as<S>(sc<S>(0.5) * (Vf(i, jm, k) + Vf(i, j, k)));
+    const auto v4 = as<S>(sc<S>(0.5) * (Vf(i, j, k) + Vf(i, jp, k)));
+    const auto u1 = as<S>((dx2[jm] * Uf(i, j, k) + dx2[j] * Uf(i, jm, k)) / dmx2[j] * sc<S>(0.5));
+    const auto u2 = as<S>((dx2[jm] * Uf(ip, j, k) + dx2[j] * Uf(ip, jm, k)) / dmx2[j] * sc<S>(0.5));
+    const auto w5 = as<S>((dx2[jm] * Wf(i, j, k) + dx2[j] * Wf(i, jm, k)) / dmx2[j] * sc<S>(0.5));
+    const auto w6 = as<S>((dx2[jm] * Wf(i, j, kp) + dx2[j] * Wf(i, jm, kp)) / dmx2[j] * sc<S>(0.5));
+    const auto ddu1 = as<S>((dx2[jm] * dUf(i, j, k) + dx2[j] * dUf(i, jm, k)) / dmx2[j] * sc<S>(0.5));
+    const auto ddu2 = as<S>((dx2[jm] * dUf(ip, j, k) + dx2[j] * dUf(ip, jm, k)) / dmx2[j] * sc<S>(0.5));
 
-    const S dvdx1 = (Vf(i, j, k) - Vf(im, j, k)) / dmx1[i];
-    const S dvdx2 = (Vf(ip, j, k) - Vf(i, j, k)) / dmx1[ip];
-    const S dvdy3 = (Vf(i, j, k) - Vf(i, jm, k)) / dx2[jm];
-    const S dvdy4 = (Vf(i, jp, k) - Vf(i, j, k)) / dx2[j];
-    const S dvdz5 = (Vf(i, j, k) - Vf(i, j, km)) / dmx3[k];
-    const S dvdz6 = (Vf(i, j, kp) - Vf(i, j, k)) / dmx3[kp];
-    const S dudy1 = (Uf(i, j, k) - Uf(i, jm, k)) / dmx2[j];
-    const S dudy2 = (Uf(ip, j, k) - Uf(ip, jm, k)) / dmx2[j];
-    const S dwdy5 = (Wf(i, j, k) - Wf(i, jm, k)) / dmx2[j];
-    const S dwdy6 = (Wf(i, j, kp) - Wf(i, jm, kp)) / dmx2[j];
-    const S ddudy1 = (dUf(i, j, k) - dUf(i, jm, k)) / dmx2[j];
-    const S ddudy2 = (dUf(ip, j, k) - dUf(ip, jm, k)) / dmx2[j];
+    const auto dvdx1 = as<S>((Vf(i, j, k) - Vf(im, j, k)) / dmx1[i]);
+    const auto dvdx2 = as<S>((Vf(ip, j, k) - Vf(i, j, k)) / dmx1[ip]);
+    const auto dvdy3 = as<S>((Vf(i, j, k) - Vf(i, jm, k)) / dx2[jm]);
+    const auto dvdy4 = as<S>((Vf(i, jp, k) - Vf(i, j, k)) / dx2[j]);
+    const auto dvdz5 = as<S>((Vf(i, j, k) - Vf(i, j, km)) / dmx3[k]);
+    const auto dvdz6 = as<S>((Vf(i, j, kp) - Vf(i, j, k)) / dmx3[kp]);
+    const auto dudy1 = as<S>((Uf(i, j, k) - Uf(i, jm, k)) / dmx2[j]);
+    const auto dudy2 = as<S>((Uf(ip, j, k) - Uf(ip, jm, k)) / dmx2[j]);
+    const auto dwdy5 = as<S>((Wf(i, j, k) - Wf(i, jm, k)) / dmx2[j]);
+    const auto dwdy6 = as<S>((Wf(i, j, kp) - Wf(i, jm, kp)) / dmx2[j]);
+    const auto ddudy1 = as<S>((dUf(i, j, k) - dUf(i, jm, k)) / dmx2[j]);
+    const auto ddudy2 = as<S>((dUf(ip, j, k) - dUf(ip, jm, k)) / dmx2[j]);
 
-    S mua = sc<S>(0.5) * (dx2[jm] * MU(j, k) + dx2[j] * MU(jm, k)) / dmx2[j];
-    S muc = sc<S>(0.5) * (dx2[jm] * MU(j, k) + dx2[j] * MU(jm, k)) / dmx2[j];
-    S mub = sc<S>(0.5) * (dx2[jm] * MU(j, k) + dx2[j] * MU(jm, k)) / dmx2[j];
-    const S mu1 = sc<S>(0.5) * (dx1[im] * muc + dx1[i] * mua) / dmx1[i];
-    const S mu2 = sc<S>(0.5) * (dx1[ip] * muc + dx1[i] * mub) / dmx1[ip];
-    mua = sc<S>(0.5) * (dx2[jm] * MU(j, km) + dx2[j] * MU(jm, km)) / dmx2[j];
-    muc = sc<S>(0.5) * (dx2[jm] * MU(j, k) + dx2[j] * MU(jm, k)) / dmx2[j];
-    mub = sc<S>(0.5) * (dx2[jm] * MU(j, kp) + dx2[j] * MU(jm, kp)) / dmx2[j];
-    const S mu5 = sc<S>(0.5) * (dx3[km] * muc + dx3[k] * mua) / dmx3[k];
-    const S mu6 = sc<S>(0.5) * (dx3[kp] * muc + dx3[k] * mub) / dmx3[kp];
+    const auto mua = as<S>(sc<S>(0.5) * (dx2[jm] * MU(j, k) + dx2[j] * MU(jm, k)) / dmx2[j]);
+    const auto muc = as<S>(sc<S>(0.5) * (dx2[jm] * MU(j, k) + dx2[j] * MU(jm, k)) / dmx2[j]);
+    const auto mub = as<S>(sc<S>(0.5) * (dx2[jm] * MU(j, k) + dx2[j] * MU(jm, k)) / dmx2[j]);
+    const auto mu1 = as<S>(sc<S>(0.5) * (dx1[im] * muc + dx1[i] * mua) / dmx1[i]);
+    const auto mu2 = as<S>(sc<S>(0.5) * (dx1[ip] * muc + dx1[i] * mub) / dmx1[ip]);
+    const auto mua_2 = as<S>(sc<S>(0.5) * (dx2[jm] * MU(j, km) + dx2[j] * MU(jm, km)) / dmx2[j]);
+    const auto muc_2 = as<S>(sc<S>(0.5) * (dx2[jm] * MU(j, k) + dx2[j] * MU(jm, k)) / dmx2[j]);
+    const auto mub_2 = as<S>(sc<S>(0.5) * (dx2[jm] * MU(j, kp) + dx2[j] * MU(jm, kp)) / dmx2[j]);
+    const auto mu5 = as<S>(sc<S>(0.5) * (dx3[km] * muc_2 + dx3[k] * mua_2) / dmx3[k]);
+    const auto mu6 = as<S>(sc<S>(0.5) * (dx3[kp] * muc_2 + dx3[k] * mub_2) / dmx3[kp]);
 
-    const S invRhoc = sc<S>(0.5) * (dx2[jm] * IR(j, k) + dx2[j] * IR(jm, k)) / dmx2[j];
-    const S invRhocCmu_half = sc<S>(0.5) * Cmu * invRhoc;
+    const auto invRhoc = as<S>(sc<S>(0.5) * (dx2[jm] * IR(j, k) + dx2[j] * IR(jm, k)) / dmx2[j]);
+    const auto invRhocCmu_half = as<S>(sc<S>(0.5) * Cmu * invRhoc);
 
-    const S viscous_v1 = sc<S>(1.0) * (mu2 * dvdx2 - mu1 * dvdx1) / dx1[i];
-    const S viscous_v2 = sc<S>(1.0) * (MU(j, k) * dvdy4 - MU(jm, k) * dvdy3) / dmx2[j];
-    const S viscous_v3 = sc<S>(1.0) * (mu6 * dvdz6 - mu5 * dvdz5) / dx3[k];
-    const S viscous_v21 = sc<S>(1.0) * (mu2 * dudy2 - mu1 * dudy1) / dx1[i];
-    const S viscous_v23 = sc<S>(1.0) * (mu6 * dwdy6 - mu5 * dwdy5) / dx3[k];
+    const auto viscous_v1 = as<S>(sc<S>(1.0) * (mu2 * dvdx2 - mu1 * dvdx1) / dx1[i]);
+    const auto viscous_v2 = as<S>(sc<S>(1.0) * (MU(j, k) * dvdy4 - MU(jm, k) * dvdy3) / dmx2[j]);
+    const auto viscous_v3 = as<S>(sc<S>(1.0) * (mu6 * dvdz6 - mu5 * dvdz5) / dx3[k]);
+    const auto viscous_v21 = as<S>(sc<S>(1.0) * (mu2 * dudy2 - mu1 * dudy1) / dx1[i]);
+    const auto viscous_v23 = as<S>(sc<S>(1.0) * (mu6 * dwdy6 - mu5 * dwdy5) / dx3[k]);
 
-    S rhs = invRhocCmu_half * (viscous_v1 + sc<S>(2.0) * viscous_v2 + viscous_v3 + viscous_v21 + viscous_v23);
-    rhs = rhs - sc<S>(p.Cmp) * invRhoc * (P[g.ix(i, j, k)] - P[g.ix(i, jm, k)]) / dmx2[j];
+    const auto rhs = as<S>(invRhocCmu_half * (viscous_v1 + sc<S>(2.0) * viscous_v2 + viscous_v3 + viscous_v21 + viscous_v23));
+    const auto rhs_2 = as<S>(rhs - sc<S>(p.Cmp) * invRhoc * (P[g.ix(i, j, k)] - P[g.ix(i, jm, k)]) / dmx2[j]);
 
-    if (WM == 0 || (WM == 1 && (jvm != 1 || jvp != 1))) {  // wall terms, as in the dU rows
-    const S vbt = VBCbt[g.b2(i, k)], vup = VBCup[g.b2(i, k)];
-    S vbc_down = (sc<S>(0.25) / dx2[jm] * v3 * vbt - sc<S>(0.25) * sc<S>(0.5) * dvdy3 * vbt);
-    S vbc_up = (-sc<S>(0.25) / dx2[j] * v4 * vup - sc<S>(0.25) * sc<S>(0.5) * dvdy4 * vup);
-    vbc_down = vbc_down + invRhocCmu_half / dmx2[j] * MU(jm, k) / dx2[jm] * vbt * sc<S>(2.0);
-    vbc_up = vbc_up + invRhocCmu_half / dmx2[j] * MU(j, k) / dx2[j] * vup * sc<S>(2.0);
-    rhs = rhs + (sc<S>(1.0) - sc<S>(jvm)) * vbc_down + (sc<S>(1.0) - sc<S>(jvp)) * vbc_up;
-    }
+    const auto wall_terms = [&](const auto &r) {  // as in the dU rows
+        const auto vbt = as<S>(VBCbt[g.b2(i, k)]);
+        const auto vup = as<S>(VBCup[g.b2(i, k)]);
+        const auto vbc_down = [&] {
+            return (sc<S>(0.25) / dx2[jm] * v3 * vbt - sc<S>(0.25) * sc<S>(0.5) * dvdy3 * vbt)
+                 + invRhocCmu_half / dmx2[j] * MU(jm, k) / dx2[jm] * vbt * sc<S>(2.0);
+        };
+        const auto vbc_up = [&] {
+            return (-sc<S>(0.25) / dx2[j] * v4 * vup - sc<S>(0.25) * sc<S>(0.5) * dvdy4 * vup)
+                 + invRhocCmu_half / dmx2[j] * MU(j, k) / dx2[j] * vup * sc<S>(2.0);
+        };
+        return r + (sc<S>(1.0) - sc<S>(jvm)) * vbc_down() + (sc<S>(1.0) - sc<S>(jvp)) * vbc_up();
+    };
+    const auto rhs_3 = as<S>(with_walls<S, WM>(jvm != 1 || jvp != 1, rhs_2, wall_terms));
 
-    const S mACI = invRhocCmu_half / dx1[i] * (mu2 / dmx1[ip] + mu1 / dmx1[i]) + sc<S>(0.25) * (-u2 / dmx1[ip] + u1 / dmx1[i]);
-    const S mAPI = -invRhocCmu_half / dx1[i] * mu2 / dmx1[ip] + sc<S>(0.25) * (u2 / dmx1[ip]);
-    const S mAMI = -invRhocCmu_half / dx1[i] * mu1 / dmx1[i] + sc<S>(0.25) * (-u1 / dmx1[i]);
-    const S mACJ = invRhocCmu_half / dmx2[j] * (MU(j, k) / dx2[j] + MU(jm, k) / dx2[jm]) * sc<S>(2.0)
-                      + sc<S>(0.25) * (dvdy4 * sc<S>(0.5) + dvdy3 * sc<S>(0.5) - v4 / dx2[j] + v3 / dx2[jm]);
-    S mAPJ = -invRhocCmu_half / dmx2[j] * MU(j, k) / dx2[j] * sc<S>(2.0) + sc<S>(0.25) * (v4 / dx2[j] + dvdy4 * sc<S>(0.5));
-    mAPJ = mAPJ * sc<S>(jvp);
-    S mAMJ = -invRhocCmu_half / dmx2[j] * MU(jm, k) / dx2[jm] * sc<S>(2.0) + sc<S>(0.25) * (-v3 / dx2[jm] + dvdy3 * sc<S>(0.5));
-    mAMJ = mAMJ * sc<S>(jvm);
-    const S mACK = invRhocCmu_half / dx3[k] * (mu6 / dmx3[kp] + mu5 / dmx3[k]) + sc<S>(0.25) * (-w6 / dmx3[kp] + w5 / dmx3[k]);
-    const S mAPK = -invRhocCmu_half / dx3[k] * mu6 / dmx3[kp] + sc<S>(0.25) * (w6 / dmx3[kp]);
-    const S mAMK = -invRhocCmu_half / dx3[k] * mu5 / dmx3[k] + sc<S>(0.25) * (-w5 / dmx3[k]);
+    const auto mACI = as<S>(invRhocCmu_half / dx1[i] * (mu2 / dmx1[ip] + mu1 / dmx1[i]) + sc<S>(0.25) * (-u2 / dmx1[ip] + u1 / dmx1[i]));
+    const auto mAPI = as<S>(-invRhocCmu_half / dx1[i] * mu2 / dmx1[ip] + sc<S>(0.25) * (u2 / dmx1[ip]));
+    const auto mAMI = as<S>(-invRhocCmu_half / dx1[i] * mu1 / dmx1[i] + sc<S>(0.25) * (-u1 / dmx1[i]));
+    const auto mACJ = as<S>(invRhocCmu_half / dmx2[j] * (MU(j, k) / dx2[j] + MU(jm, k) / dx2[jm]) * sc<S>(2.0)
+                      + sc<S>(0.25) * (dvdy4 * sc<S>(0.5) + dvdy3 * sc<S>(0.5) - v4 / dx2[j] + v3 / dx2[jm]));
+    const auto mAPJ = as<S>(-invRhocCmu_half / dmx2[j] * MU(j, k) / dx2[j] * sc<S>(2.0) + sc<S>(0.25) * (v4 / dx2[j] + dvdy4 * sc<S>(0.5)));
+    const auto mAPJ_2 = as<S>(mAPJ * sc<S>(jvp));
+    const auto mAMJ = as<S>(-invRhocCmu_half / dmx2[j] * MU(jm, k) / dx2[jm] * sc<S>(2.0) + sc<S>(0.25) * (-v3 / dx2[jm] + dvdy3 * sc<S>(0.5)));
+    const auto mAMJ_2 = as<S>(mAMJ * sc<S>(jvm));
+    const auto mACK = as<S>(invRhocCmu_half / dx3[k] * (mu6 / dmx3[kp] + mu5 / dmx3[k]) + sc<S>(0.25) * (-w6 / dmx3[kp] + w5 / dmx3[k]));
+    const auto mAPK = as<S>(-invRhocCmu_half / dx3[k] * mu6 / dmx3[kp] + sc<S>(0.25) * (w6 / dmx3[kp]));
+    const auto mAMK = as<S>(-invRhocCmu_half / dx3[k] * mu5 / dmx3[k] + sc<S>(0.25) * (-w5 / dmx3[k]));
 
-    rhs = rhs - (mAPI * Vf(ip, j, k) + mACI * Vf(i, j, k) + mAMI * Vf(im, j, k)
-                 + mAPJ * Vf(i, jp, k) + mACJ * Vf(i, j, k) + mAMJ * Vf(i, jm, k)
-                 + mAPK * Vf(i, j, kp) + mACK * Vf(i, j, k) + mAMK * Vf(i, j, km));
-    rhs = rhs - (sc<S>(0.25) * (u2 * dvdx2 + u1 * dvdx1) - invRhocCmu_half / dx1[i] * (mu2 * dudy2 - mu1 * dudy1));
-    rhs = rhs - (sc<S>(0.25) * (w6 * dvdz6 + w5 * dvdz5) - invRhocCmu_half / dx3[k] * (mu6 * dwdy6 - mu5 * dwdy5));
-    rhs = rhs - (sc<S>(0.25) * (ddu2 * dvdx2 + ddu1 * dvdx1) - invRhocCmu_half / dx1[i] * (mu2 * ddudy2 - mu1 * ddudy1));
+    const auto rhs_4 = as<S>(rhs_3 - (mAPI * Vf(ip, j, k) + mACI * Vf(i, j, k) + mAMI * Vf(im, j, k)
+                 + mAPJ_2 * Vf(i, jp, k) + mACJ * Vf(i, j, k) + mAMJ_2 * Vf(i, jm, k)
+                 + mAPK * Vf(i, j, kp) + mACK * Vf(i, j, k) + mAMK * Vf(i, j, km)));
+    const auto rhs_5 = as<S>(rhs_4 - (sc<S>(0.25) * (u2 * dvdx2 + u1 * dvdx1) - invRhocCmu_half / dx1[i] * (mu2 * dudy2 - mu1 * dudy1)));
+    const auto rhs_6 = as<S>(rhs_5 - (sc<S>(0.25) * (w6 * dvdz6 + w5 * dvdz5) - invRhocCmu_half / dx3[k] * (mu6 * dwdy6 - mu5 * dwdy5)));
+    const auto rhs_7 = as<S>(rhs_6 - (sc<S>(0.25) * (ddu2 * dvdx2 + ddu1 * dvdx1) - invRhocCmu_half / dx1[i] * (mu2 * ddudy2 - mu1 * ddudy1)));
 
     ac = mACK * sc<S>(dt) + sc<S>(1.0);
     ap = mAPK * sc<S>(dt);
     am = mAMK * sc<S>(dt);
-    rhsout = rhs * sc<S>(dt);
+    rhsout = rhs_7 * sc<S>(dt);
 }
 struct DVZ {
     // FP32 lines of the mixed form: the unconditional row loop with the
@@ -440,9 +454,10 @@ struct DVZ {
     double dt;
     const double *U, *V, *W, *P, *dU, *Mu, *iR, *VBCup, *VBCbt;
     static constexpr int NF = 9;  // field inputs, in the order below
+    static constexpr int ND = 7, STALE = -1;  // rev.h
     static constexpr bool FULL = true;  // unconditional row loop in the FP64 z solve
-    template <class S, int WM = -1, class Wr>
-    __device__ __forceinline__ void eval(const Wr &w, int i, int j, int k, S &a, S &b, S &c, S &d) const {
+    template <class S, int WM = -1, class Wr, class I>
+    __device__ __forceinline__ void eval(const Wr &w, I i, I j, I k, S &a, S &b, S &c, S &d) const {
         // WM < 0 (the row's own wall-term mode): a branch on j in FP32 rows,
         // terms kept otherwise; the z lines pass 2 or 0 per workgroup
         // (wall_free)
@@ -456,20 +471,21 @@ struct DVZ {
     }
 };
 
-template <class S, class FP>
+template <class S, class FP, class I>
 __device__ __forceinline__ void dV_x_row(const Grid &g, const Phys &p, double dt, FP U,
     FP iR, FP stale,
-    int i, int j, int k, S &am, S &ac, S &ap) {
+    I i, I j, I k, S &am, S &ac, S &ap) {
     ROW_METRICS
-    const int ip = i + 1, jm = j - 1;
-    const S mu1 = stale[0], mu2 = stale[1];
-    const S u1 = (dx2[jm] * Uf(i, j, k) + dx2[j] * Uf(i, jm, k)) / dmx2[j] * sc<S>(0.5);
-    const S u2 = (dx2[jm] * Uf(ip, j, k) + dx2[j] * Uf(ip, jm, k)) / dmx2[j] * sc<S>(0.5);
-    const S invRhoc = sc<S>(0.5) * (dx2[jm] * IR(j, k) + dx2[j] * IR(jm, k)) / dmx2[j];
-    const S invRhocCmu_half = sc<S>(0.5) * sc<S>(p.Cmu) * invRhoc;
-    const S mACI = invRhocCmu_half / dx1[i] * (mu2 / dmx1[ip] + mu1 / dmx1[i]) + sc<S>(0.25) * (-u2 / dmx1[ip] + u1 / dmx1[i]);
-    const S mAPI = -invRhocCmu_half / dx1[i] * mu2 / dmx1[ip] + sc<S>(0.25) * (u2 / dmx1[ip]);
-    const S mAMI = -invRhocCmu_half / dx1[i] * mu1 / dmx1[i] + sc<S>(0.25) * (-u1 / dmx1[i]);
+    const auto ip = i + 1, jm = j - 1;
+    const auto mu1 = as<S>(stale[0]);
+    const auto mu2 = as<S>(stale[1]);
+    const auto u1 = as<S>((dx2[jm] * Uf(i, j, k) + dx2[j] * Uf(i, jm, k)) / dmx2[j] * sc<S>(0.5));
+    const auto u2 = as<S>((dx2[jm] * Uf(ip, j, k) + dx2[j] * Uf(ip, jm, k)) / dmx2[j] * sc<S>(0.5));
+    const auto invRhoc = as<S>(sc<S>(0.5) * (dx2[jm] * IR(j, k) + dx2[j] * IR(jm, k)) / dmx2[j]);
+    const auto invRhocCmu_half = as<S>(sc<S>(0.5) * sc<S>(p.Cmu) * invRhoc);
+    const auto mACI = as<S>(invRhocCmu_half / dx1[i] * (mu2 / dmx1[ip] + mu1 / dmx1[i]) + sc<S>(0.25) * (-u2 / dmx1[ip] + u1 / dmx1[i]));
+    const auto mAPI = as<S>(-invRhocCmu_half / dx1[i] * mu2 / dmx1[ip] + sc<S>(0.25) * (u2 / dmx1[ip]));
+    const auto mAMI = as<S>(-invRhocCmu_half / dx1[i] * mu1 / dmx1[i] + sc<S>(0.25) * (-u1 / dmx1[i]));
     ac = mACI * sc<S>(dt) + sc<S>(1.0);
     ap = mAPI * sc<S>(dt);
     am = mAMI * sc<S>(dt);
@@ -480,8 +496,9 @@ struct DVX {
     double dt;
     const double *U, *iR, *stale;
     static constexpr int NF = 3;  // field inputs, in the order below
-    template <class S, class Wr>
-    __device__ __forceinline__ void eval(const Wr &w, int i, int j, int k, S &a, S &b, S &c, S &d) const {
+    static constexpr int ND = 3, STALE = 2;  // rev.h
+    template <class S, class Wr, class I>
+    __device__ __forceinline__ void eval(const Wr &w, I i, I j, I k, S &a, S &b, S &c, S &d) const {
         dV_x_row<S>(g, p, dt, w(0, U), w(1, iR), w(2, stale), i, j, k, a, b, c);
     }
     __device__ __forceinline__ void operator()(int i, int j, int k, double &a, double &b, double &c,
@@ -490,28 +507,28 @@ struct DVX {
     }
 };
 
-template <class S, class FP>
+template <class S, class FP, class I>
 __device__ __forceinline__ void dV_y_row(const Grid &g, const Phys &p, double dt, FP V,
     FP Mu, FP iR,
-    int i, int j, int k, S &am, S &ac, S &ap) {
+    I i, I j, I k, S &am, S &ac, S &ap) {
     ROW_METRICS
-    const int jm = j - 1, jp = j + 1;
+    const auto jm = j - 1, jp = j + 1;
     const int jvp = g.jS[jm], jvm = g.jS[jp];
-    const S v3 = sc<S>(0.5) * (Vf(i, jm, k) + Vf(i, j, k));
-    const S v4 = sc<S>(0.5) * (Vf(i, j, k) + Vf(i, jp, k));
-    const S dvdy3 = (Vf(i, j, k) - Vf(i, jm, k)) / dx2[jm];
-    const S dvdy4 = (Vf(i, jp, k) - Vf(i, j, k)) / dx2[j];
-    const S invRhoc = sc<S>(0.5) * (dx2[jm] * IR(j, k) + dx2[j] * IR(jm, k)) / dmx2[j];
-    const S invRhocCmu_half = sc<S>(0.5) * sc<S>(p.Cmu) * invRhoc;
-    const S mACJ = invRhocCmu_half / dmx2[j] * (MU(j, k) / dx2[j] + MU(jm, k) / dx2[jm]) * sc<S>(2.0)
-                      + sc<S>(0.25) * (dvdy4 * sc<S>(0.5) + dvdy3 * sc<S>(0.5) - v4 / dx2[j] + v3 / dx2[jm]);
-    S mAPJ = -invRhocCmu_half / dmx2[j] * MU(j, k) / dx2[j] * sc<S>(2.0) + sc<S>(0.25) * (v4 / dx2[j] + dvdy4 * sc<S>(0.5));
-    mAPJ = mAPJ * sc<S>(jvp);
-    S mAMJ = -invRhocCmu_half / dmx2[j] * MU(jm, k) / dx2[jm] * sc<S>(2.0) + sc<S>(0.25) * (-v3 / dx2[jm] + dvdy3 * sc<S>(0.5));
-    mAMJ = mAMJ * sc<S>(jvm);
+    const auto v3 = as<S>(sc<S>(0.5) * (Vf(i, jm, k) + Vf(i, j, k)));
+    const auto v4 = as<S>(sc<S>(0.5) * (Vf(i, j, k) + Vf(i, jp, k)));
+    const auto dvdy3 = as<S>((Vf(i, j, k) - Vf(i, jm, k)) / dx2[jm]);
+    const auto dvdy4 = as<S>((Vf(i, jp, k) - Vf(i, j, k)) / dx2[j]);
+    const auto invRhoc = as<S>(sc<S>(0.5) * (dx2[jm] * IR(j, k) + dx2[j] * IR(jm, k)) / dmx2[j]);
+    const auto invRhocCmu_half = as<S>(sc<S>(0.5) * sc<S>(p.Cmu) * invRhoc);
+    const auto mACJ = as<S>(invRhocCmu_half / dmx2[j] * (MU(j, k) / dx2[j] + MU(jm, k) / dx2[jm]) * sc<S>(2.0)
+                      + sc<S>(0.25) * (dvdy4 * sc<S>(0.5) + dvdy3 * sc<S>(0.5) - v4 / dx2[j] + v3 / dx2[jm]));
+    const auto mAPJ = as<S>(-invRhocCmu_half / dmx2[j] * MU(j, k) / dx2[j] * sc<S>(2.0) + sc<S>(0.25) * (v4 / dx2[j] + dvdy4 * sc<S>(0.5)));
+    const auto mAPJ_2 = as<S>(mAPJ * sc<S>(jvp));
+    const auto mAMJ = as<S>(-invRhocCmu_half / dmx2[j] * MU(jm, k) / dx2[jm] * sc<S>(2.0) + sc<S>(0.25) * (-v3 / dx2[jm] + dvdy3 * sc<S>(0.5)));
+    const auto mAMJ_2 = as<S>(mAMJ * sc<S>(jvm));
     ac = mACJ * sc<S>(dt) + sc<S>(1.0);
-    ap = mAPJ * sc<S>(dt);
-    am = mAMJ * sc<S>(dt);
+    ap = mAPJ_2 * sc<S>(dt);
+    am = mAMJ_2 * sc<S>(dt);
 }
 struct DVY {
     // FP32 lines of the mixed form: the unconditional row loop (0.75 -> 0.53 ms
@@ -523,8 +540,9 @@ struct DVY {
     double dt;
     const double *V, *Mu, *iR;
     static constexpr int NF = 3;  // field inputs, in the order below
-    template <class S, class Wr>
-    __device__ __forceinline__ void eval(const Wr &w, int i, int j, int k, S &a, S &b, S &c, S &d) const {
+    static constexpr int ND = 3, STALE = -1;  // rev.h
+    template <class S, class Wr, class I>
+    __device__ __forceinline__ void eval(const Wr &w, I i, I j, I k, S &a, S &b, S &c, S &d) const {
         dV_y_row<S>(g, p, dt, w(0, V), w(1, Mu), w(2, iR), i, j, k, a, b, c);
     }
     __device__ __forceinline__ void operator()(int i, int j, int k, double &a, double &b, double &c,
@@ -534,111 +552,119 @@ struct DVY {
 };
 
 // ---------------------------------------------------------------- dW -------
-template <class S, int WM, class FP>
+template <class S, int WM, class FP, class I>
 __device__ __forceinline__ void dW_z_row(const Grid &g, const Phys &p, double dt, FP U,
     FP V, FP W, FP P,
     FP dU, FP dV, FP Mu,
     FP iR, FP VBCup, FP VBCbt,
     FP WBCup, FP WBCbt,
-    int i, int j, int k, S &am, S &ac, S &ap, S &rhsout) {
+    I i, I j, I k, S &am, S &ac, S &ap, S &rhsout) {
     ROW_METRICS
-    const int im = i - 1, ip = i + 1, jm = j - 1, jp = j + 1, km = k - 1, kp = k + 1;
+    const auto im = i - 1, ip = i + 1, jm = j - 1, jp = j + 1, km = k - 1, kp = k + 1;
     const int jwp = g.jC[jp], jwm = g.jC[jm];
-    const S Cmu = sc<S>(p.Cmu);
+    const auto Cmu = as<S>(sc<S>(p.Cmu));
 #define dVf(a, b, c) dV[g.ix(a, b, c)]
-    const S w5 = sc<S>(0.5) * (Wf(i, j, k) + Wf(i, j, km));
-    const S w6 = sc<S>(0.5) * (Wf(i, j, k) + Wf(i, j, kp));
-    const S u1 = (dx3[km] * Uf(i, j, k) + dx3[k] * Uf(i, j, km)) / dmx3[k] * sc<S>(0.5);
-    const S u2 = (dx3[km] * Uf(ip, j, k) + dx3[k] * Uf(ip, j, km)) / dmx3[k] * sc<S>(0.5);
-    const S v3 = (dx3[km] * Vf(i, j, k) + dx3[k] * Vf(i, j, km)) / dmx3[k] * sc<S>(0.5);
-    const S v4 = (dx3[km] * Vf(i, jp, k) + dx3[k] * Vf(i, jp, km)) / dmx3[k] * sc<S>(0.5);
+    const auto w5 = as<S>(sc<S>(0.5) * (Wf(i, j, k) + Wf(i, j, km)));
+    const auto w6 = as<S>(sc<S>(0.5) * (Wf(i, j, k) + Wf(i, j, kp)));
+    const auto u1 = as<S>((dx3[km] * Uf(i, j, k) + dx3[k] * Uf(i, j, km)) / dmx3[k] * sc<S>(0.5));
+    const auto u2 = as<S>((dx3[km] * Uf(ip, j, k) + dx3[k] * Uf(ip, j, km)) / dmx3[k] * sc<S>(0.5));
+    const auto v3 = as<S>((dx3[km] * Vf(i, j, k) + dx3[k] * Vf(i, j, km)) / dmx3[k] * sc<S>(0.5));
+    const auto v4 = as<S>((dx3[km] * Vf(i, jp, k) + dx3[k] * Vf(i, jp, km)) / dmx3[k] * sc<S>(0.5));
 
-    const S dwdx1 = (Wf(i, j, k) - Wf(im, j, k)) / dmx1[i];
-    const S dwdx2 = (Wf(ip, j, k) - Wf(i, j, k)) / dmx1[ip];
-    const S dwdy3 = (Wf(i, j, k) - Wf(i, jm, k)) / dmx2[j];
-    const S dwdy4 = (Wf(i, jp, k) - Wf(i, j, k)) / dmx2[jp];
-    const S dwdz5 = (Wf(i, j, k) - Wf(i, j, km)) / dx3[km];
-    const S dwdz6 = (Wf(i, j, kp) - Wf(i, j, k)) / dx3[k];
-    const S dudz1 = (Uf(i, j, k) - Uf(i, j, km)) / dmx3[k];
-    const S dudz2 = (Uf(ip, j, k) - Uf(ip, j, km)) / dmx3[k];
-    const S dvdz3 = (Vf(i, j, k) - Vf(i, j, km)) / dmx3[k];
-    const S dvdz4 = (Vf(i, jp, k) - Vf(i, jp, km)) / dmx3[k];
-    const S ddudz1 = (dUf(i, j, k) - dUf(i, j, km)) / dmx3[k];
-    const S ddudz2 = (dUf(ip, j, k) - dUf(ip, j, km)) / dmx3[k];
-    const S ddvdz3 = (dVf(i, j, k) - dVf(i, j, km)) / dmx3[k];
-    const S ddvdz4 = (dVf(i, jp, k) - dVf(i, jp, km)) / dmx3[k];
-    const S ddu1 = (dx3[km] * dUf(i, j, k) + dx3[k] * dUf(i, j, km)) / dmx3[k] * sc<S>(0.5);
-    const S ddu2 = (dx3[km] * dUf(ip, j, k) + dx3[k] * dUf(ip, j, km)) / dmx3[k] * sc<S>(0.5);
-    const S ddv3 = (dx3[km] * dVf(i, j, k) + dx3[k] * dVf(i, j, km)) / dmx3[k] * sc<S>(0.5) * sc<S>(jwm);
-    const S ddv4 = (dx3[km] * dVf(i, jp, k) + dx3[k] * dVf(i, jp, km)) / dmx3[k] * sc<S>(0.5) * sc<S>(jwp);
+    const auto dwdx1 = as<S>((Wf(i, j, k) - Wf(im, j, k)) / dmx1[i]);
+    const auto dwdx2 = as<S>((Wf(ip, j, k) - Wf(i, j, k)) / dmx1[ip]);
+    const auto dwdy3 = as<S>((Wf(i, j, k) - Wf(i, jm, k)) / dmx2[j]);
+    const auto dwdy4 = as<S>((Wf(i, jp, k) - Wf(i, j, k)) / dmx2[jp]);
+    const auto dwdz5 = as<S>((Wf(i, j, k) - Wf(i, j, km)) / dx3[km]);
+    const auto dwdz6 = as<S>((Wf(i, j, kp) - Wf(i, j, k)) / dx3[k]);
+    const auto dudz1 = as<S>((Uf(i, j, k) - Uf(i, j, km)) / dmx3[k]);
+    const auto dudz2 = as<S>((Uf(ip, j, k) - Uf(ip, j, km)) / dmx3[k]);
+    const auto dvdz3 = as<S>((Vf(i, j, k) - Vf(i, j, km)) / dmx3[k]);
+    const auto dvdz4 = as<S>((Vf(i, jp, k) - Vf(i, jp, km)) / dmx3[k]);
+    const auto ddudz1 = as<S>((dUf(i, j, k) - dUf(i, j, km)) / dmx3[k]);
+    const auto ddudz2 = as<S>((dUf(ip, j, k) - dUf(ip, j, km)) / dmx3[k]);
+    const auto ddvdz3 = as<S>((dVf(i, j, k) - dVf(i, j, km)) / dmx3[k]);
+    const auto ddvdz4 = as<S>((dVf(i, jp, k) - dVf(i, jp, km)) / dmx3[k]);
+    const auto ddu1 = as<S>((dx3[km] * dUf(i, j, k) + dx3[k] * dUf(i, j, km)) / dmx3[k] * sc<S>(0.5));
+    const auto ddu2 = as<S>((dx3[km] * dUf(ip, j, k) + dx3[k] * dUf(ip, j, km)) / dmx3[k] * sc<S>(0.5));
+    const auto ddv3 = as<S>((dx3[km] * dVf(i, j, k) + dx3[k] * dVf(i, j, km)) / dmx3[k] * sc<S>(0.5) * sc<S>(jwm));
+    const auto ddv4 = as<S>((dx3[km] * dVf(i, jp, k) + dx3[k] * dVf(i, jp, km)) / dmx3[k] * sc<S>(0.5) * sc<S>(jwp));
 
-    S mua = sc<S>(0.5) * (dx3[km] * MU(j, k) + dx3[k] * MU(j, km)) / dmx3[k];
-    S muc = sc<S>(0.5) * (dx3[km] * MU(j, k) + dx3[k] * MU(j, km)) / dmx3[k];
-    S mub = sc<S>(0.5) * (dx3[km] * MU(j, k) + dx3[k] * MU(j, km)) / dmx3[k];
-    const S mu1 = sc<S>(0.5) * (dx1[im] * muc + dx1[i] * mua) / dmx1[i];
-    const S mu2 = sc<S>(0.5) * (dx1[ip] * muc + dx1[i] * mub) / dmx1[ip];
-    mua = sc<S>(0.5) * (dx3[km] * MU(jm, k) + dx3[k] * MU(jm, km)) / dmx3[k];
-    muc = sc<S>(0.5) * (dx3[km] * MU(j, k) + dx3[k] * MU(j, km)) / dmx3[k];
-    mub = sc<S>(0.5) * (dx3[km] * MU(jp, k) + dx3[k] * MU(jp, km)) / dmx3[k];
-    const S mu3 = sc<S>(0.5) * (dx2[jm] * muc + dx2[j] * mua) / dmx2[j];
-    const S mu4 = sc<S>(0.5) * (dx2[jp] * muc + dx2[j] * mub) / dmx2[jp];
+    const auto mua = as<S>(sc<S>(0.5) * (dx3[km] * MU(j, k) + dx3[k] * MU(j, km)) / dmx3[k]);
+    const auto muc = as<S>(sc<S>(0.5) * (dx3[km] * MU(j, k) + dx3[k] * MU(j, km)) / dmx3[k]);
+    const auto mub = as<S>(sc<S>(0.5) * (dx3[km] * MU(j, k) + dx3[k] * MU(j, km)) / dmx3[k]);
+    const auto mu1 = as<S>(sc<S>(0.5) * (dx1[im] * muc + dx1[i] * mua) / dmx1[i]);
+    const auto mu2 = as<S>(sc<S>(0.5) * (dx1[ip] * muc + dx1[i] * mub) / dmx1[ip]);
+    const auto mua_2 = as<S>(sc<S>(0.5) * (dx3[km] * MU(jm, k) + dx3[k] * MU(jm, km)) / dmx3[k]);
+    const auto muc_2 = as<S>(sc<S>(0.5) * (dx3[km] * MU(j, k) + dx3[k] * MU(j, km)) / dmx3[k]);
+    const auto mub_2 = as<S>(sc<S>(0.5) * (dx3[km] * MU(jp, k) + dx3[k] * MU(jp, km)) / dmx3[k]);
+    const auto mu3 = as<S>(sc<S>(0.5) * (dx2[jm] * muc_2 + dx2[j] * mua_2) / dmx2[j]);
+    const auto mu4 = as<S>(sc<S>(0.5) * (dx2[jp] * muc_2 + dx2[j] * mub_2) / dmx2[jp]);
 
-    const S invRhoc = sc<S>(0.5) * (dx3[km] * IR(j, k) + dx3[k] * IR(j, km)) / dmx3[k];
-    const S invRhocCmu_half = sc<S>(0.5) * Cmu * invRhoc;
+    const auto invRhoc = as<S>(sc<S>(0.5) * (dx3[km] * IR(j, k) + dx3[k] * IR(j, km)) / dmx3[k]);
+    const auto invRhocCmu_half = as<S>(sc<S>(0.5) * Cmu * invRhoc);
 
-    const S viscous_w1 = sc<S>(1.0) * (mu2 * dwdx2 - mu1 * dwdx1) / dx1[i];
-    const S viscous_w2 = sc<S>(1.0) * (mu4 * dwdy4 - mu3 * dwdy3) / dx2[j];
-    const S viscous_w3 = sc<S>(1.0) * (MU(j, k) * dwdz6 - MU(j, km) * dwdz5) / dmx3[k];
-    const S viscous_w31 = sc<S>(1.0) * (mu2 * dudz2 - mu1 * dudz1) / dx1[i];
-    const S viscous_w32 = sc<S>(1.0) * (mu4 * dvdz4 - mu3 * dvdz3) / dx2[j];
+    const auto viscous_w1 = as<S>(sc<S>(1.0) * (mu2 * dwdx2 - mu1 * dwdx1) / dx1[i]);
+    const auto viscous_w2 = as<S>(sc<S>(1.0) * (mu4 * dwdy4 - mu3 * dwdy3) / dx2[j]);
+    const auto viscous_w3 = as<S>(sc<S>(1.0) * (MU(j, k) * dwdz6 - MU(j, km) * dwdz5) / dmx3[k]);
+    const auto viscous_w31 = as<S>(sc<S>(1.0) * (mu2 * dudz2 - mu1 * dudz1) / dx1[i]);
+    const auto viscous_w32 = as<S>(sc<S>(1.0) * (mu4 * dvdz4 - mu3 * dvdz3) / dx2[j]);
 
-    S rhs = invRhocCmu_half * (viscous_w1 + viscous_w2 + sc<S>(2.0) * viscous_w3 + viscous_w31 + viscous_w32);
-    rhs = rhs - sc<S>(p.Cmp) * invRhoc * (P[g.ix(i, j, k)] - P[g.ix(i, j, km)]) / dmx3[k];
+    const auto rhs = as<S>(invRhocCmu_half * (viscous_w1 + viscous_w2 + sc<S>(2.0) * viscous_w3 + viscous_w31 + viscous_w32));
+    const auto rhs_2 = as<S>(rhs - sc<S>(p.Cmp) * invRhoc * (P[g.ix(i, j, k)] - P[g.ix(i, j, km)]) / dmx3[k]);
 
-    if (WM == 0 || (WM == 1 && (jwm != 1 || jwp != 1))) {  // wall terms, as in the dU rows
-    S zbc_down = sc<S>(0.25) * v3 / dmx2[j] * WBCbt[g.b2(i, k)]
-                    - sc<S>(0.25) * dwdy3 * (dx3[km] * VBCbt[g.b2(i, k)] + dx3[k] * VBCbt[g.b2(i, km)]) / dmx3[k] * sc<S>(0.5);
-    S zbc_up = -sc<S>(0.25) * v4 / dmx2[jp] * WBCup[g.b2(i, k)]
-                  - sc<S>(0.25) * dwdy4 * (dx3[km] * VBCup[g.b2(i, k)] + dx3[k] * VBCup[g.b2(i, km)]) / dmx3[k] * sc<S>(0.5);
-    zbc_down = zbc_down + invRhocCmu_half / dx2[j] * mu3 / dmx2[jp] * WBCbt[g.b2(i, k)];
-    zbc_up = zbc_up + invRhocCmu_half / dx2[j] * mu4 / dmx2[j] * WBCup[g.b2(i, k)];
-    zbc_down = zbc_down - invRhocCmu_half / dx2[j] * mu3 / dmx3[k] * (VBCbt[g.b2(i, k)] - VBCbt[g.b2(i, km)]);
-    zbc_up = zbc_up + invRhocCmu_half / dx2[j] * mu4 / dmx3[k] * (VBCup[g.b2(i, k)] - VBCup[g.b2(i, km)]);
-    rhs = rhs + (sc<S>(1.0) - sc<S>(jwm)) * zbc_down + (sc<S>(1.0) - sc<S>(jwp)) * zbc_up;
-    }
+    const auto wall_terms = [&](const auto &r) {  // as in the dU rows
+        const auto zbc_down = [&] {
+            return sc<S>(0.25) * v3 / dmx2[j] * WBCbt[g.b2(i, k)]
+                 - sc<S>(0.25) * dwdy3 * (dx3[km] * VBCbt[g.b2(i, k)] + dx3[k] * VBCbt[g.b2(i, km)]) / dmx3[k] * sc<S>(0.5)
+                 + invRhocCmu_half / dx2[j] * mu3 / dmx2[jp] * WBCbt[g.b2(i, k)]
+                 - invRhocCmu_half / dx2[j] * mu3 / dmx3[k] * (VBCbt[g.b2(i, k)] - VBCbt[g.b2(i, km)]);
+        };
+        const auto zbc_up = [&] {
+            return -sc<S>(0.25) * v4 / dmx2[jp] * WBCup[g.b2(i, k)]
+                 - sc<S>(0.25) * dwdy4 * (dx3[km] * VBCup[g.b2(i, k)] + dx3[k] * VBCup[g.b2(i, km)]) / dmx3[k] * sc<S>(0.5)
+                 + invRhocCmu_half / dx2[j] * mu4 / dmx2[j] * WBCup[g.b2(i, k)]
+                 + invRhocCmu_half / dx2[j] * mu4 / dmx3[k] * (VBCup[g.b2(i, k)] - VBCup[g.b2(i, km)]);
+        };
+        return r + (sc<S>(1.0) - sc<S>(jwm)) * zbc_down() + (sc<S>(1.0) - sc<S>(jwp)) * zbc_up();
+    };
+    const auto rhs_3 = as<S>(with_walls<S, WM>(jwm != 1 || jwp != 1, rhs_2, wall_terms));
 
-    const S mACI = invRhocCmu_half / dx1[i] * (mu2 / dmx1[ip] + mu1 / dmx1[i]) + sc<S>(0.25) * (-u2 / dmx1[ip] + u1 / dmx1[i]);
-    const S mAPI = -invRhocCmu_half / dx1[i] * mu2 / dmx1[ip] + sc<S>(0.25) * (u2 / dmx1[ip]);
-    const S mAMI = -invRhocCmu_half / dx1[i] * mu1 / dmx1[i] + sc<S>(0.25) * (-u1 / dmx1[i]);
-    const S mACJ = invRhocCmu_half / dx2[j] * (mu4 / dmx2[jp] + mu3 / dmx2[j]) + sc<S>(0.25) * (-v4 / dmx2[jp] + v3 / dmx2[j]);
-    S mAPJ = -invRhocCmu_half / dx2[j] * mu4 / dmx2[jp] + sc<S>(0.25) * (v4 / dmx2[jp]);
-    mAPJ = mAPJ * sc<S>(jwp);
-    S mAMJ = -invRhocCmu_half / dx2[j] * mu3 / dmx2[j] + sc<S>(0.25) * (-v3 / dmx2[j]);
-    mAMJ = mAMJ * sc<S>(jwm);
-    const S mACK = invRhocCmu_half / dmx3[k] * (MU(j, k) / dx3[k] + MU(j, km) / dx3[km]) * sc<S>(2.0)
-                      + sc<S>(0.25) * (-w6 / dx3[k] + w5 / dx3[km] + sc<S>(0.5) * dwdz6 + sc<S>(0.5) * dwdz5);
-    const S mAPK = -invRhocCmu_half / dmx3[k] * MU(j, k) / dx3[k] * sc<S>(2.0) + sc<S>(0.25) * (w6 / dx3[k] + sc<S>(0.5) * dwdz6);
-    const S mAMK = -invRhocCmu_half / dmx3[k] * MU(j, km) / dx3[km] * sc<S>(2.0) + sc<S>(0.25) * (-w5 / dx3[km] + sc<S>(0.5) * dwdz5);
+    const auto mACI = as<S>(invRhocCmu_half / dx1[i] * (mu2 / dmx1[ip] + mu1 / dmx1[i]) + sc<S>(0.25) * (-u2 / dmx1[ip] + u1 / dmx1[i]));
+    const auto mAPI = as<S>(-invRhocCmu_half / dx1[i] * mu2 / dmx1[ip] + sc<S>(0.25) * (u2 / dmx1[ip]));
+    const auto mAMI = as<S>(-invRhocCmu_half / dx1[i] * mu1 / dmx1[i] + sc<S>(0.25) * (-u1 / dmx1[i]));
+    const auto mACJ = as<S>(invRhocCmu_half / dx2[j] * (mu4 / dmx2[jp] + mu3 / dmx2[j]) + sc<S>(0.25) * (-v4 / dmx2[jp] + v3 / dmx2[j]));
+    const auto mAPJ = as<S>(-invRhocCmu_half / dx2[j] * mu4 / dmx2[jp] + sc<S>(0.25) * (v4 / dmx2[jp]));
+    const auto mAPJ_2 = as<S>(mAPJ * sc<S>(jwp));
+    const auto mAMJ = as<S>(-invRhocCmu_half / dx2[j] * mu3 / dmx2[j] + sc<S>(0.25) * (-v3 / dmx2[j]));
+    const auto mAMJ_2 = as<S>(mAMJ * sc<S>(jwm));
+    const auto mACK = as<S>(invRhocCmu_half / dmx3[k] * (MU(j, k) / dx3[k] + MU(j, km) / dx3[km]) * sc<S>(2.0)
+                      + sc<S>(0.25) * (-w6 / dx3[k] + w5 / dx3[km] + sc<S>(0.5) * dwdz6 + sc<S>(0.5) * dwdz5));
+    const auto mAPK = as<S>(-invRhocCmu_half / dmx3[k] * MU(j, k) / dx3[k] * sc<S>(2.0) + sc<S>(0.25) * (w6 / dx3[k] + sc<S>(0.5) * dwdz6));
+    const auto mAMK = as<S>(-invRhocCmu_half / dmx3[k] * MU(j, km) / dx3[km] * sc<S>(2.0) + sc<S>(0.25) * (-w5 / dx3[km] + sc<S>(0.5) * dwdz5));
 
-    rhs = rhs - (mAPI * Wf(ip, j, k) + mACI * Wf(i, j, k) + mAMI * Wf(im, j, k)
-                 + mAPJ * Wf(i, jp, k) + mACJ * Wf(i, j, k) + mAMJ * Wf(i, jm, k)
-                 + mAPK * Wf(i, j, kp) + mACK * Wf(i, j, k) + mAMK * Wf(i, j, km));
-    rhs = rhs - (sc<S>(0.25) * (u2 * dwdx2 + u1 * dwdx1) - invRhocCmu_half / dx1[i] * (mu2 * dudz2 - mu1 * dudz1));
-    rhs = rhs - (sc<S>(0.25) * (v3 * sc<S>(jwm) * dwdy3 + v4 * sc<S>(jwp) * dwdy4)
-                 - invRhocCmu_half / dx2[j] * (mu4 * dvdz4 * sc<S>(jwp) - mu3 * dvdz3 * sc<S>(jwm)));
-    rhs = rhs - (sc<S>(0.25) * (ddu2 * dwdx2 + ddu1 * dwdx1) - invRhocCmu_half / dx1[i] * (mu2 * ddudz2 - mu1 * ddudz1));
-    rhs = rhs - (sc<S>(0.25) * (ddv3 * sc<S>(jwm) * dwdy3 + ddv4 * sc<S>(jwp) * dwdy4)
-                 - invRhocCmu_half / dx2[j] * (mu4 * ddvdz4 * sc<S>(jwp) - mu3 * ddvdz3 * sc<S>(jwm)));
+    const auto rhs_4 = as<S>(rhs_3 - (mAPI * Wf(ip, j, k) + mACI * Wf(i, j, k) + mAMI * Wf(im, j, k)
+                 + mAPJ_2 * Wf(i, jp, k) + mACJ * Wf(i, j, k) + mAMJ_2 * Wf(i, jm, k)
+                 + mAPK * Wf(i, j, kp) + mACK * Wf(i, j, k) + mAMK * Wf(i, j, km)));
+    const auto rhs_5 = as<S>(rhs_4 - (sc<S>(0.25) * (u2 * dwdx2 + u1 * dwdx1) - invRhocCmu_half / dx1[i] * (mu2 * dudz2 - mu1 * dudz1)));
+    const auto rhs_6 = as<S>(rhs_5 - (sc<S>(0.25) * (v3 * sc<S>(jwm) * dwdy3 + v4 * sc<S>(jwp) * dwdy4)
+                 - invRhocCmu_half / dx2[j] * (mu4 * dvdz4 * sc<S>(jwp) - mu3 * dvdz3 * sc<S>(jwm))));
+    const auto rhs_7 = as<S>(rhs_6 - (sc<S>(0.25) * (ddu2 * dwdx2 + ddu1 * dwdx1) - invRhocCmu_half / dx1[i] * (mu2 * ddudz2 - mu1 * ddudz1)));
+    const auto rhs_8 = as<S>(rhs_7 - (sc<S>(0.25) * (ddv3 * sc<S>(jwm) * dwdy3 + ddv4 * sc<S>(jwp) * dwdy4)
+                 - invRhocCmu_half / dx2[j] * (mu4 * ddvdz4 * sc<S>(jwp) - mu3 * ddvdz3 * sc<S>(jwm))));
 
     ac = mACK * sc<S>(dt) + sc<S>(1.0);
     ap = mAPK * sc<S>(dt);
     am = mAMK * sc<S>(dt);
-    rhsout = rhs * sc<S>(dt);
+    rhsout = rhs_8 * sc<S>(dt);
 }
 struct DWZ {
     // FP32 lines of the mixed form: the unconditional row loop with the
     // workgroups split by the wall terms (2.20 -> 1.88 ms at 512^3)
-    static constexpr int W32 = 1;
+    // three waves per SIMD: 168 registers, where the lines are short enough for
+    // several workgroups a CU (without the bound the compiler takes 171:
+    // 0.215 against 0.187 ms at 256^3)
+    static constexpr int W32 = 3;
     static constexpr bool FULL32 = true;
     static constexpr bool WALLS32 = true;
     Grid g;
@@ -646,11 +672,12 @@ struct DWZ {
     double dt;
     const double *U, *V, *W, *P, *dU, *dV, *Mu, *iR, *VBCup, *VBCbt, *WBCup, *WBCbt;
     static constexpr int NF = 12;  // field inputs, in the order below
+    static constexpr int ND = 8, STALE = -1;  // rev.h
     static constexpr bool FULL = true;  // unconditional row loop in the FP64 z solve
-    template <class S, int WM = -1, class Wr>
-    __device__ __forceinline__ void eval(const Wr &w, int i, int j, int k, S &a, S &b, S &c, S &d) const {
+    template <class S, int WM = -1, class Wr, class I>
+    __device__ __forceinline__ void eval(const Wr &w, I i, I j, I k, S &a, S &b, S &c, S &d) const {
         // WM < 0 (the row's own wall-term mode): a branch on j, terms kept in
-        // the adjoint's dual passes; the z lines pass 2 or 0 per workgroup
+        // the adjoint's reverse pass; the z lines pass 2 or 0 per workgroup
         // (wall_free)
         dW_z_row<S, (WM >= 0 ? WM : (is_dual<S>() ? 0 : 1))>(g, p, dt, w(0, U), w(1, V), w(2, W), w(3, P), w(4, dU), w(5, dV), w(6, Mu), w(7, iR), w(8, VBCup), w(9, VBCbt), w(10, WBCup), w(11, WBCbt), i, j, k, a, b, c, d);
     }
@@ -662,20 +689,21 @@ struct DWZ {
     }
 };
 
-template <class S, class FP>
+template <class S, class FP, class I>
 __device__ __forceinline__ void dW_x_row(const Grid &g, const Phys &p, double dt, FP U,
     FP iR, FP stale,
-    int i, int j, int k, S &am, S &ac, S &ap) {
+    I i, I j, I k, S &am, S &ac, S &ap) {
     ROW_METRICS
-    const int ip = i + 1, km = k - 1;
-    const S mu1 = stale[2], mu2 = stale[3];
-    const S u1 = (dx3[km] * Uf(i, j, k) + dx3[k] * Uf(i, j, km)) / dmx3[k] * sc<S>(0.5);
-    const S u2 = (dx3[km] * Uf(ip, j, k) + dx3[k] * Uf(ip, j, km)) / dmx3[k] * sc<S>(0.5);
-    const S invRhoc = sc<S>(0.5) * (dx3[km] * IR(j, k) + dx3[k] * IR(j, km)) / dmx3[k];
-    const S invRhocCmu_half = sc<S>(0.5) * sc<S>(p.Cmu) * invRhoc;
-    const S mACI = invRhocCmu_half / dx1[i] * (mu2 / dmx1[ip] + mu1 / dmx1[i]) + sc<S>(0.25) * (-u2 / dmx1[ip] + u1 / dmx1[i]);
-    const S mAPI = -invRhocCmu_half / dx1[i] * mu2 / dmx1[ip] + sc<S>(0.25) * (u2 / dmx1[ip]);
-    const S mAMI = -invRhocCmu_half / dx1[i] * mu1 / dmx1[i] + sc<S>(0.25) * (-u1 / dmx1[i]);
+    const auto ip = i + 1, km = k - 1;
+    const auto mu1 = as<S>(stale[2]);
+    const auto mu2 = as<S>(stale[3]);
+    const auto u1 = as<S>((dx3[km] * Uf(i, j, k) + dx3[k] * Uf(i, j, km)) / dmx3[k] * sc<S>(0.5));
+    const auto u2 = as<S>((dx3[km] * Uf(ip, j, k) + dx3[k] * Uf(ip, j, km)) / dmx3[k] * sc<S>(0.5));
+    const auto invRhoc = as<S>(sc<S>(0.5) * (dx3[km] * IR(j, k) + dx3[k] * IR(j, km)) / dmx3[k]);
+    const auto invRhocCmu_half = as<S>(sc<S>(0.5) * sc<S>(p.Cmu) * invRhoc);
+    const auto mACI = as<S>(invRhocCmu_half / dx1[i] * (mu2 / dmx1[ip] + mu1 / dmx1[i]) + sc<S>(0.25) * (-u2 / dmx1[ip] + u1 / dmx1[i]));
+    const auto mAPI = as<S>(-invRhocCmu_half / dx1[i] * mu2 / dmx1[ip] + sc<S>(0.25) * (u2 / dmx1[ip]));
+    const auto mAMI = as<S>(-invRhocCmu_half / dx1[i] * mu1 / dmx1[i] + sc<S>(0.25) * (-u1 / dmx1[i]));
     ac = mACI * sc<S>(dt) + sc<S>(1.0);
     ap = mAPI * sc<S>(dt);
     am = mAMI * sc<S>(dt);
@@ -686,8 +714,9 @@ struct DWX {
     double dt;
     const double *U, *iR, *stale;
     static constexpr int NF = 3;  // field inputs, in the order below
-    template <class S, class Wr>
-    __device__ __forceinline__ void eval(const Wr &w, int i, int j, int k, S &a, S &b, S &c, S &d) const {
+    static constexpr int ND = 3, STALE = 2;  // rev.h
+    template <class S, class Wr, class I>
+    __device__ __forceinline__ void eval(const Wr &w, I i, I j, I k, S &a, S &b, S &c, S &d) const {
         dW_x_row<S>(g, p, dt, w(0, U), w(1, iR), w(2, stale), i, j, k, a, b, c);
     }
     __device__ __forceinline__ void operator()(int i, int j, int k, double &a, double &b, double &c,
@@ -696,27 +725,28 @@ struct DWX {
     }
 };
 
-template <class S, class FP>
+template <class S, class FP, class I>
 __device__ __forceinline__ void dW_y_row(const Grid &g, const Phys &p, double dt, FP V,
     FP iR, FP stale,
-    int i, int j, int k, S &am, S &ac, S &ap) {
+    I i, I j, I k, S &am, S &ac, S &ap) {
     ROW_METRICS_D64
-    const int jp = j + 1, jm = j - 1;
-    const int km = g.n3m - 1;  // stale from the x-stage's last k
+    const auto jp = j + 1, jm = j - 1;
+    const auto km = at_plane(k, g.n3m - 1, -1);  // stale from the x-stage's last k
     const int jwp = g.jC[jp], jwm = g.jC[jm];
-    const S mu3 = stale[4], mu4 = stale[5];
-    const S v3 = (dx3[km] * Vf(i, j, k) + dx3[k] * Vf(i, j, km)) / dmx3[k] * sc<S>(0.5);
-    const S v4 = (dx3[km] * Vf(i, jp, k) + dx3[k] * Vf(i, jp, km)) / dmx3[k] * sc<S>(0.5);
-    const S invRhoc = sc<S>(0.5) * (dx3[km] * IR(j, k) + dx3[k] * IR(j, km)) / dmx3[k];
-    const S invRhocCmu_half = sc<S>(0.5) * sc<S>(p.Cmu) * invRhoc;
-    const S mACJ = invRhocCmu_half / dx2[j] * (mu4 / dmx2[jp] + mu3 / dmx2[j]) + sc<S>(0.25) * (-v4 / dmx2[jp] + v3 / dmx2[j]);
-    S mAPJ = -invRhocCmu_half / dx2[j] * mu4 / dmx2[jp] + sc<S>(0.25) * (v4 / dmx2[jp]);
-    mAPJ = mAPJ * sc<S>(jwp);
-    S mAMJ = -invRhocCmu_half / dx2[j] * mu3 / dmx2[j] + sc<S>(0.25) * (-v3 / dmx2[j]);
-    mAMJ = mAMJ * sc<S>(jwm);
+    const auto mu3 = as<S>(stale[4]);
+    const auto mu4 = as<S>(stale[5]);
+    const auto v3 = as<S>((dx3[km] * Vf(i, j, k) + dx3[k] * Vf(i, j, km)) / dmx3[k] * sc<S>(0.5));
+    const auto v4 = as<S>((dx3[km] * Vf(i, jp, k) + dx3[k] * Vf(i, jp, km)) / dmx3[k] * sc<S>(0.5));
+    const auto invRhoc = as<S>(sc<S>(0.5) * (dx3[km] * IR(j, k) + dx3[k] * IR(j, km)) / dmx3[k]);
+    const auto invRhocCmu_half = as<S>(sc<S>(0.5) * sc<S>(p.Cmu) * invRhoc);
+    const auto mACJ = as<S>(invRhocCmu_half / dx2[j] * (mu4 / dmx2[jp] + mu3 / dmx2[j]) + sc<S>(0.25) * (-v4 / dmx2[jp] + v3 / dmx2[j]));
+    const auto mAPJ = as<S>(-invRhocCmu_half / dx2[j] * mu4 / dmx2[jp] + sc<S>(0.25) * (v4 / dmx2[jp]));
+    const auto mAPJ_2 = as<S>(mAPJ * sc<S>(jwp));
+    const auto mAMJ = as<S>(-invRhocCmu_half / dx2[j] * mu3 / dmx2[j] + sc<S>(0.25) * (-v3 / dmx2[j]));
+    const auto mAMJ_2 = as<S>(mAMJ * sc<S>(jwm));
     ac = mACJ * sc<S>(dt) + sc<S>(1.0);
-    ap = mAPJ * sc<S>(dt);
-    am = mAMJ * sc<S>(dt);
+    ap = mAPJ_2 * sc<S>(dt);
+    am = mAMJ_2 * sc<S>(dt);
 }
 struct DWY {
     // FP32 lines of the mixed form: the unconditional row loop (0.74 -> 0.56 ms
@@ -728,8 +758,9 @@ struct DWY {
     double dt;
     const double *V, *iR, *stale;
     static constexpr int NF = 3;  // field inputs, in the order below
-    template <class S, class Wr>
-    __device__ __forceinline__ void eval(const Wr &w, int i, int j, int k, S &a, S &b, S &c, S &d) const {
+    static constexpr int ND = 3, STALE = 2;  // rev.h
+    template <class S, class Wr, class I>
+    __device__ __forceinline__ void eval(const Wr &w, I i, I j, I k, S &a, S &b, S &c, S &d) const {
         dW_y_row<S>(g, p, dt, w(0, V), w(1, iR), w(2, stale), i, j, k, a, b, c);
     }
     __device__ __forceinline__ void operator()(int i, int j, int k, double &a, double &b, double &c,
@@ -740,24 +771,24 @@ struct DWY {
 
 // ------------------------------------------------------- block corrections --
 // mpi_momentum_blockLdV (:1278-1356): the new dV of cell (i,j,k), j >= 2
-template <class S, class FP>
+template <class S, class FP, class I>
 __device__ __forceinline__ void blockLdV_cell(const Grid &g, const Phys &p, double dt, FP V, FP dW, FP Mu,
-                                             FP iR, FP dV, int i, int j, int k, S &out) {
+                                             FP iR, FP dV, I i, I j, I k, S &out) {
     ROW_METRICS
-    const int jm = j - 1, km = k - 1, kp = k + 1;
+    const auto jm = j - 1, km = k - 1, kp = k + 1;
 #define dWf(a, b, c) dW[g.ix(a, b, c)]
-    const S dwm5 = (dx2[jm] * dWf(i, j, k) + dx2[j] * dWf(i, jm, k)) / dmx2[j] * sc<S>(0.5);
-    const S dwm6 = (dx2[jm] * dWf(i, j, kp) + dx2[j] * dWf(i, jm, kp)) / dmx2[j] * sc<S>(0.5);
-    const S ddwdy5 = (dWf(i, j, k) - dWf(i, jm, k)) / dmx2[j];
-    const S ddwdy6 = (dWf(i, j, kp) - dWf(i, jm, kp)) / dmx2[j];
-    const S dvdz5 = (Vf(i, j, k) - Vf(i, j, km)) / dmx3[k];
-    const S dvdz6 = (Vf(i, j, kp) - Vf(i, j, k)) / dmx3[kp];
-    const S invRhoc = sc<S>(0.5) * (dx2[jm] * IR(j, k) + dx2[j] * IR(jm, k)) / dmx2[j];
-    const S mua = sc<S>(0.5) * (dx2[jm] * MU(j, km) + dx2[j] * MU(jm, km)) / dmx2[j];
-    const S muc = sc<S>(0.5) * (dx2[jm] * MU(j, k) + dx2[j] * MU(jm, k)) / dmx2[j];
-    const S mub = sc<S>(0.5) * (dx2[jm] * MU(j, kp) + dx2[j] * MU(jm, kp)) / dmx2[j];
-    const S mu5 = sc<S>(0.5) * (dx3[km] * muc + dx3[k] * mua) / dmx3[k];
-    const S mu6 = sc<S>(0.5) * (dx3[kp] * muc + dx3[k] * mub) / dmx3[kp];
+    const auto dwm5 = as<S>((dx2[jm] * dWf(i, j, k) + dx2[j] * dWf(i, jm, k)) / dmx2[j] * sc<S>(0.5));
+    const auto dwm6 = as<S>((dx2[jm] * dWf(i, j, kp) + dx2[j] * dWf(i, jm, kp)) / dmx2[j] * sc<S>(0.5));
+    const auto ddwdy5 = as<S>((dWf(i, j, k) - dWf(i, jm, k)) / dmx2[j]);
+    const auto ddwdy6 = as<S>((dWf(i, j, kp) - dWf(i, jm, kp)) / dmx2[j]);
+    const auto dvdz5 = as<S>((Vf(i, j, k) - Vf(i, j, km)) / dmx3[k]);
+    const auto dvdz6 = as<S>((Vf(i, j, kp) - Vf(i, j, k)) / dmx3[kp]);
+    const auto invRhoc = as<S>(sc<S>(0.5) * (dx2[jm] * IR(j, k) + dx2[j] * IR(jm, k)) / dmx2[j]);
+    const auto mua = as<S>(sc<S>(0.5) * (dx2[jm] * MU(j, km) + dx2[j] * MU(jm, km)) / dmx2[j]);
+    const auto muc = as<S>(sc<S>(0.5) * (dx2[jm] * MU(j, k) + dx2[j] * MU(jm, k)) / dmx2[j]);
+    const auto mub = as<S>(sc<S>(0.5) * (dx2[jm] * MU(j, kp) + dx2[j] * MU(jm, kp)) / dmx2[j]);
+    const auto mu5 = as<S>(sc<S>(0.5) * (dx3[km] * muc + dx3[k] * mua) / dmx3[k]);
+    const auto mu6 = as<S>(sc<S>(0.5) * (dx3[kp] * muc + dx3[k] * mub) / dmx3[kp]);
     out = dV[g.ix(i, j, k)] - sc<S>(dt) * (sc<S>(0.25) * (dwm5 * dvdz5 + dwm6 * dvdz6)
                           - sc<S>(0.5) * sc<S>(p.Cmu) * invRhoc / dx3[k] * (mu6 * ddwdy6 - mu5 * ddwdy5));
 }
@@ -767,8 +798,9 @@ struct BlockLdV {
     double dt;
     const double *V, *dW, *Mu, *iR, *dV;
     static constexpr int NF = 5;
-    template <class S, class Wr>
-    __device__ __forceinline__ void eval(const Wr &w, int i, int j, int k, S &a, S &b, S &c, S &d) const {
+    static constexpr int ND = 5, STALE = -1;  // rev.h
+    template <class S, class Wr, class I>
+    __device__ __forceinline__ void eval(const Wr &w, I i, I j, I k, S &a, S &b, S &c, S &d) const {
         blockLdV_cell<S>(g, p, dt, w(0, V), w(1, dW), w(2, Mu), w(3, iR), w(4, dV), i, j, k, a);
     }
 };
@@ -788,35 +820,35 @@ __global__ void __launch_bounds__(256) k_blockLdV(BlockLdV cell, Acc acc, E *dV)
 }
 
 // mpi_momentum_blockLdU (:1362-1460): the new dU of cell (i,j,k)
-template <class S, class FP>
+template <class S, class FP, class I>
 __device__ __forceinline__ void blockLdU_cell(const Grid &g, const Phys &p, double dt, FP U, FP dV, FP dW,
-                                             FP Mu, FP iR, FP dU, int i, int j, int k, S &out) {
+                                             FP Mu, FP iR, FP dU, I i, I j, I k, S &out) {
     ROW_METRICS
-    const int im = i - 1, jm = j - 1, jp = j + 1, km = k - 1, kp = k + 1;
+    const auto im = i - 1, jm = j - 1, jp = j + 1, km = k - 1, kp = k + 1;
     const int jum = g.jC[jm], jup = g.jC[jp];
-    const S invRhoc = sc<S>(0.5) * (dx1[im] * IR(j, k) + dx1[i] * IR(j, k)) / dmx1[i];
-    const S dvm3 = (dx1[i] * dVf(im, j, k) + dx1[im] * dVf(i, j, k)) / dmx1[i] * sc<S>(0.5) * sc<S>(jum);
-    const S dvm4 = (dx1[i] * dVf(im, jp, k) + dx1[im] * dVf(i, jp, k)) / dmx1[i] * sc<S>(0.5) * sc<S>(jup);
-    const S dudy3 = (Uf(i, j, k) - Uf(i, jm, k)) / dmx2[j];
-    const S dudy4 = (Uf(i, jp, k) - Uf(i, j, k)) / dmx2[jp];
-    const S dvmdx3 = (dVf(i, j, k) - dVf(im, j, k)) / dmx1[i] * sc<S>(jum);
-    const S dvmdx4 = (dVf(i, jp, k) - dVf(im, jp, k)) / dmx1[i] * sc<S>(jup);
-    S mua = sc<S>(0.5) * (dx1[im] * MU(jm, k) + dx1[i] * MU(jm, k)) / dmx1[i];
-    S muc = sc<S>(0.5) * (dx1[im] * MU(j, k) + dx1[i] * MU(j, k)) / dmx1[i];
-    S mub = sc<S>(0.5) * (dx1[im] * MU(jp, k) + dx1[i] * MU(jp, k)) / dmx1[i];
-    const S mu3 = sc<S>(0.5) * (dx2[jm] * muc + dx2[j] * mua) / dmx2[j];
-    const S mu4 = sc<S>(0.5) * (dx2[jp] * muc + dx2[j] * mub) / dmx2[jp];
-    const S dwm5 = (dx1[i] * dWf(im, j, k) + dx1[im] * dWf(i, j, k)) / dmx1[i] * sc<S>(0.5);
-    const S dwm6 = (dx1[i] * dWf(im, j, kp) + dx1[im] * dWf(i, j, kp)) / dmx1[i] * sc<S>(0.5);
-    const S dudz5 = (Uf(i, j, k) - Uf(i, j, km)) / dmx3[k];
-    const S dudz6 = (Uf(i, j, kp) - Uf(i, j, k)) / dmx3[kp];
-    const S dwmdx5 = (dWf(i, j, k) - dWf(im, j, k)) / dmx1[i];
-    const S dwmdx6 = (dWf(i, j, kp) - dWf(im, j, kp)) / dmx1[i];
-    mua = sc<S>(0.5) * (dx1[im] * MU(j, km) + dx1[i] * MU(j, km)) / dmx1[i];
-    muc = sc<S>(0.5) * (dx1[im] * MU(j, k) + dx1[i] * MU(j, k)) / dmx1[i];
-    mub = sc<S>(0.5) * (dx1[im] * MU(j, kp) + dx1[i] * MU(j, kp)) / dmx1[i];
-    const S mu5 = sc<S>(0.5) * (dx3[km] * muc + dx3[k] * mua) / dmx3[k];
-    const S mu6 = sc<S>(0.5) * (dx3[kp] * muc + dx3[k] * mub) / dmx3[kp];
+    const auto invRhoc = as<S>(sc<S>(0.5) * (dx1[im] * IR(j, k) + dx1[i] * IR(j, k)) / dmx1[i]);
+    const auto dvm3 = as<S>((dx1[i] * dVf(im, j, k) + dx1[im] * dVf(i, j, k)) / dmx1[i] * sc<S>(0.5) * sc<S>(jum));
+    const auto dvm4 = as<S>((dx1[i] * dVf(im, jp, k) + dx1[im] * dVf(i, jp, k)) / dmx1[i] * sc<S>(0.5) * sc<S>(jup));
+    const auto dudy3 = as<S>((Uf(i, j, k) - Uf(i, jm, k)) / dmx2[j]);
+    const auto dudy4 = as<S>((Uf(i, jp, k) - Uf(i, j, k)) / dmx2[jp]);
+    const auto dvmdx3 = as<S>((dVf(i, j, k) - dVf(im, j, k)) / dmx1[i] * sc<S>(jum));
+    const auto dvmdx4 = as<S>((dVf(i, jp, k) - dVf(im, jp, k)) / dmx1[i] * sc<S>(jup));
+    const auto mua = as<S>(sc<S>(0.5) * (dx1[im] * MU(jm, k) + dx1[i] * MU(jm, k)) / dmx1[i]);
+    const auto muc = as<S>(sc<S>(0.5) * (dx1[im] * MU(j, k) + dx1[i] * MU(j, k)) / dmx1[i]);
+    const auto mub = as<S>(sc<S>(0.5) * (dx1[im] * MU(jp, k) + dx1[i] * MU(jp, k)) / dmx1[i]);
+    const auto mu3 = as<S>(sc<S>(0.5) * (dx2[jm] * muc + dx2[j] * mua) / dmx2[j]);
+    const auto mu4 = as<S>(sc<S>(0.5) * (dx2[jp] * muc + dx2[j] * mub) / dmx2[jp]);
+    const auto dwm5 = as<S>((dx1[i] * dWf(im, j, k) + dx1[im] * dWf(i, j, k)) / dmx1[i] * sc<S>(0.5));
+    const auto dwm6 = as<S>((dx1[i] * dWf(im, j, kp) + dx1[im] * dWf(i, j, kp)) / dmx1[i] * sc<S>(0.5));
+    const auto dudz5 = as<S>((Uf(i, j, k) - Uf(i, j, km)) / dmx3[k]);
+    const auto dudz6 = as<S>((Uf(i, j, kp) - Uf(i, j, k)) / dmx3[kp]);
+    const auto dwmdx5 = as<S>((dWf(i, j, k) - dWf(im, j, k)) / dmx1[i]);
+    const auto dwmdx6 = as<S>((dWf(i, j, kp) - dWf(im, j, kp)) / dmx1[i]);
+    const auto mua_2 = as<S>(sc<S>(0.5) * (dx1[im] * MU(j, km) + dx1[i] * MU(j, km)) / dmx1[i]);
+    const auto muc_2 = as<S>(sc<S>(0.5) * (dx1[im] * MU(j, k) + dx1[i] * MU(j, k)) / dmx1[i]);
+    const auto mub_2 = as<S>(sc<S>(0.5) * (dx1[im] * MU(j, kp) + dx1[i] * MU(j, kp)) / dmx1[i]);
+    const auto mu5 = as<S>(sc<S>(0.5) * (dx3[km] * muc_2 + dx3[k] * mua_2) / dmx3[k]);
+    const auto mu6 = as<S>(sc<S>(0.5) * (dx3[kp] * muc_2 + dx3[k] * mub_2) / dmx3[kp]);
     out = dU[g.ix(i, j, k)]
           - sc<S>(dt) * (sc<S>(0.25) * (dvm4 * dudy4 + dvm3 * dudy3) - sc<S>(0.5) * sc<S>(p.Cmu) * invRhoc / dx2[j] * (mu4 * dvmdx4 - mu3 * dvmdx3))
           - sc<S>(dt) * (sc<S>(0.25) * (dwm6 * dudz6 + dwm5 * dudz5) - sc<S>(0.5) * sc<S>(p.Cmu) * invRhoc / dx3[k] * (mu6 * dwmdx6 - mu5 * dwmdx5));
@@ -827,8 +859,9 @@ struct BlockLdU {
     double dt;
     const double *U, *dV, *dW, *Mu, *iR, *dU;
     static constexpr int NF = 6;
-    template <class S, class Wr>
-    __device__ __forceinline__ void eval(const Wr &w, int i, int j, int k, S &a, S &b, S &c, S &d) const {
+    static constexpr int ND = 6, STALE = -1;  // rev.h
+    template <class S, class Wr, class I>
+    __device__ __forceinline__ void eval(const Wr &w, I i, I j, I k, S &a, S &b, S &c, S &d) const {
         blockLdU_cell<S>(g, p, dt, w(0, U), w(1, dV), w(2, dW), w(3, Mu), w(4, iR), w(5, dU), i, j, k, a);
     }
 };

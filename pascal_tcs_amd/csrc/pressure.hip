@@ -139,40 +139,39 @@ __device__ __forceinline__ void lds_fft(double *re, double *im, int n, int nl, c
 // multiplied by 1 - jvm and 1 - jvp, zero away from the walls: with SKIPW
 // the cells there skip it and its two wall-array loads (DivUm - 0 = DivUm;
 // 1.85 -> 1.63 ms for the right-hand side and forward x FFT at 512^3).
-template <class S, bool SKIPW = false, class FP>
+template <class S, bool SKIPW = false, class FP, class I>
 __device__ __forceinline__ void pressure_rhs_cell(const Grid &g, const Phys &p, double dt, FP U, FP V, FP W,
-                                                 FP dPhat, FP iR, FP VBCup, FP VBCbt, int i, int j, int k,
+                                                 FP dPhat, FP iR, FP VBCup, FP VBCbt, I i, I j, I k,
                                                  S &out) {
     const auto dx1 = metric<S, M_DX1>(g), dx2 = metric<S, M_DX2>(g), dx3 = metric<S, M_DX3>(g);
     const auto dmx1 = metric<S, M_DMX1>(g), dmx2 = metric<S, M_DMX2>(g), dmx3 = metric<S, M_DMX3>(g);
-    const int ip = i + 1, im = i - 1, jp = j + 1, jm = j - 1, kp = k + 1, km = k - 1;
+    const auto ip = i + 1, im = i - 1, jp = j + 1, jm = j - 1, kp = k + 1, km = k - 1;
     const int jvm = g.jC[jm], jvp = g.jC[jp];
 #define IRt(jj, kk) iR[g.t2((jj), (kk))]
 #define dPh(a, b, c) dPhat[g.ix(a, b, c)]
-    const S DivUm = (U[g.ix(ip, j, k)] - U[g.ix(i, j, k)]) / dx1[i]
+    const auto DivUm = as<S>((U[g.ix(ip, j, k)] - U[g.ix(i, j, k)]) / dx1[i]
                        + ((double)jvp * V[g.ix(i, jp, k)] - (double)jvm * V[g.ix(i, j, k)]) / dx2[j]
-                       + (W[g.ix(i, j, kp)] - W[g.ix(i, j, k)]) / dx3[k];
-    S div = DivUm;
-    if (!SKIPW || jvm != 1 || jvp != 1) {
-        const S cbc = (1.0 - (double)jvm) * VBCbt[g.b2(i, k)] / dx2[j]
-                         - (1.0 - (double)jvp) * VBCup[g.b2(i, k)] / dx2[j];
-        div = DivUm - cbc;
-    }
-    const S ddpdx1 = (dPh(i, j, k) - dPh(im, j, k)) / dmx1[i];
-    const S ddpdx2 = (dPh(ip, j, k) - dPh(i, j, k)) / dmx1[ip];
-    const S ddpdy3 = (dPh(i, j, k) - dPh(i, jm, k)) / dmx2[j];
-    const S ddpdy4 = (dPh(i, jp, k) - dPh(i, j, k)) / dmx2[jp];
-    const S ddpdz5 = (dPh(i, j, k) - dPh(i, j, km)) / dmx3[k];
-    const S ddpdz6 = (dPh(i, j, kp) - dPh(i, j, k)) / dmx3[kp];
-    const S invRho1 = 0.5 / dmx1[i] * (dx1[im] * IRt(j, k) + dx1[i] * IRt(j, k));
-    const S invRho2 = 0.5 / dmx1[ip] * (dx1[ip] * IRt(j, k) + dx1[i] * IRt(j, k));
-    const S invRho3 = 0.5 / dmx2[j] * (dx2[jm] * IRt(j, k) + dx2[j] * IRt(jm, k));
-    const S invRho4 = 0.5 / dmx2[jp] * (dx2[jp] * IRt(j, k) + dx2[j] * IRt(jp, k));
-    const S invRho5 = 0.5 / dmx3[k] * (dx3[km] * IRt(j, k) + dx3[k] * IRt(j, km));
-    const S invRho6 = 0.5 / dmx3[kp] * (dx3[kp] * IRt(j, k) + dx3[k] * IRt(j, kp));
-    const S ExtraTerm = ((1.0 - invRho2) * ddpdx2 - (1.0 - invRho1) * ddpdx1) / dx1[i]
+                       + (W[g.ix(i, j, kp)] - W[g.ix(i, j, k)]) / dx3[k]);
+    const auto cbc = [&] {
+        return (1.0 - (double)jvm) * VBCbt[g.b2(i, k)] / dx2[j] - (1.0 - (double)jvp) * VBCup[g.b2(i, k)] / dx2[j];
+    };
+    const auto div = with_walls<S, SKIPW ? 1 : 0>(jvm != 1 || jvp != 1, DivUm,
+                                                  [&](const auto &d) { return d - cbc(); });
+    const auto ddpdx1 = as<S>((dPh(i, j, k) - dPh(im, j, k)) / dmx1[i]);
+    const auto ddpdx2 = as<S>((dPh(ip, j, k) - dPh(i, j, k)) / dmx1[ip]);
+    const auto ddpdy3 = as<S>((dPh(i, j, k) - dPh(i, jm, k)) / dmx2[j]);
+    const auto ddpdy4 = as<S>((dPh(i, jp, k) - dPh(i, j, k)) / dmx2[jp]);
+    const auto ddpdz5 = as<S>((dPh(i, j, k) - dPh(i, j, km)) / dmx3[k]);
+    const auto ddpdz6 = as<S>((dPh(i, j, kp) - dPh(i, j, k)) / dmx3[kp]);
+    const auto invRho1 = as<S>(0.5 / dmx1[i] * (dx1[im] * IRt(j, k) + dx1[i] * IRt(j, k)));
+    const auto invRho2 = as<S>(0.5 / dmx1[ip] * (dx1[ip] * IRt(j, k) + dx1[i] * IRt(j, k)));
+    const auto invRho3 = as<S>(0.5 / dmx2[j] * (dx2[jm] * IRt(j, k) + dx2[j] * IRt(jm, k)));
+    const auto invRho4 = as<S>(0.5 / dmx2[jp] * (dx2[jp] * IRt(j, k) + dx2[j] * IRt(jp, k)));
+    const auto invRho5 = as<S>(0.5 / dmx3[k] * (dx3[km] * IRt(j, k) + dx3[k] * IRt(j, km)));
+    const auto invRho6 = as<S>(0.5 / dmx3[kp] * (dx3[kp] * IRt(j, k) + dx3[k] * IRt(j, kp)));
+    const auto ExtraTerm = as<S>(((1.0 - invRho2) * ddpdx2 - (1.0 - invRho1) * ddpdx1) / dx1[i]
                            + ((1.0 - invRho4) * ddpdy4 - (1.0 - invRho3) * ddpdy3) / dx2[j]
-                           + ((1.0 - invRho6) * ddpdz6 - (1.0 - invRho5) * ddpdz5) / dx3[k];
+                           + ((1.0 - invRho6) * ddpdz6 - (1.0 - invRho5) * ddpdz5) / dx3[k]);
     out = div / dt / p.Cmp + ExtraTerm;
 }
 struct PressureRHS {
@@ -181,8 +180,9 @@ struct PressureRHS {
     double dt;
     const double *U, *V, *W, *dPhat, *iR, *VBCup, *VBCbt;
     static constexpr int NF = 7;
-    template <class S, class Wr>
-    __device__ __forceinline__ void eval(const Wr &w, int i, int j, int k, S &a, S &b, S &c, S &d) const {
+    static constexpr int ND = 5, STALE = -1;  // rev.h
+    template <class S, class Wr, class I>
+    __device__ __forceinline__ void eval(const Wr &w, I i, I j, I k, S &a, S &b, S &c, S &d) const {
         pressure_rhs_cell<S, !is_dual<S>()>(g, p, dt, w(0, U), w(1, V), w(2, W), w(3, dPhat), w(4, iR), w(5, VBCup), w(6, VBCbt), i,
                              j, k, a);
     }
@@ -566,35 +566,35 @@ __global__ void k_wall_extrap(Grid g, double *__restrict__ F) {
 // [k>=2] already hold the new value 2 dP - (dPhat + dP0)/2.  This kernel
 // reads only old values and recomputes those neighbours' new values; a
 // second kernel then stores the new dPhat and dP0.
-template <class S>
-__device__ __forceinline__ S dphat_new(S dP, S dPh, S dP0) {
-    const S d0 = (dPh + dP0) / 2.0;
-    return 2.0 * dP - d0;
+template <class A, class B, class C>
+__device__ __forceinline__ auto dphat_new(const A &dP, const B &dPh, const C &dP0) {
+    return 2.0 * dP - (dPh + dP0) / 2.0;
 }
 
-template <class S, class FP>
+template <class S, class FP, class I>
 __device__ __forceinline__ void projection_cell(const Grid &g, const Phys &p, double dt, FP iR, FP dP,
-                                               FP dPhat, FP dP0, FP U, FP V, FP W, FP P, int i, int j, int k,
+                                               FP dPhat, FP dP0, FP U, FP V, FP W, FP P, I i, I j, I k,
                                                S &uo, S &vo, S &wo, S &po) {
     const auto dx1 = metric<S, M_DX1>(g), dx2 = metric<S, M_DX2>(g), dx3 = metric<S, M_DX3>(g);
     const auto dmx1 = metric<S, M_DMX1>(g), dmx2 = metric<S, M_DMX2>(g), dmx3 = metric<S, M_DMX3>(g);
-    const int im = i - 1, jm = j - 1, km = k - 1;
-    const S Cmp = p.Cmp;
-    const size_t q = g.ix(i, j, k);
-    const S dPc = dP[q], dPhc = dPhat[q];
-    const size_t qi = g.ix(im, j, k), qj = g.ix(i, jm, k), qk = g.ix(i, j, km);
-    const S hi = (i >= 2) ? dphat_new(dP[qi], dPhat[qi], dP0[qi]) : dPhat[qi];
-    const S hj = (j >= 3) ? dphat_new(dP[qj], dPhat[qj], dP0[qj]) : dPhat[qj];
-    const S hk = (k >= 2) ? dphat_new(dP[qk], dPhat[qk], dP0[qk]) : dPhat[qk];
-    S invRhoc = 0.5 / dmx1[i] * (dx1[i] * IRt(j, k) + dx1[im] * IRt(j, k));
+    const auto im = i - 1, jm = j - 1, km = k - 1;
+    const auto Cmp = as<S>(p.Cmp);
+    const auto q = g.ix(i, j, k);
+    const auto dPc = as<S>(dP[q]);
+    const auto dPhc = as<S>(dPhat[q]);
+    const auto qi = g.ix(im, j, k), qj = g.ix(i, jm, k), qk = g.ix(i, j, km);
+    const auto before = [&](bool passed, auto o) {
+        return pick<S>(passed, [&] { return dphat_new(dP[o], dPhat[o], dP0[o]); }, [&] { return dPhat[o]; });
+    };
+    const auto hi = as<S>(before(i >= 2, qi));
+    const auto hj = as<S>(before(j >= 3, qj));
+    const auto hk = as<S>(before(k >= 2, qk));
+    const auto invRhoc = as<S>(0.5 / dmx1[i] * (dx1[i] * IRt(j, k) + dx1[im] * IRt(j, k)));
     uo = U[q] - dt * Cmp * ((dPc - dP[qi]) / dmx1[i] + (invRhoc - 1.0) * (dPhc - hi) / dmx1[i]);
-    invRhoc = 0.5 / dmx2[j] * (dx2[j] * IRt(jm, k) + dx2[jm] * IRt(j, k));
-    if (j >= 2)
-        vo = V[q] - dt * Cmp * ((dPc - dP[qj]) / dmx2[j] + (invRhoc - 1.0) * (dPhc - hj) / dmx2[j]);
-    else
-        vo = V[q] - dt * Cmp * ((dPc - dP[qj]) / dmx2[j] + (invRhoc - 1.0) * (dPhc - hj) / dmx2[j]) * 0.0;
-    invRhoc = 0.5 / dmx3[k] * (dx3[k] * IRt(j, km) + dx3[km] * IRt(j, k));
-    wo = W[q] - dt * Cmp * ((dPc - dP[qk]) / dmx3[k] + (invRhoc - 1.0) * (dPhc - hk) / dmx3[k]);
+    const auto invRhoc_2 = as<S>(0.5 / dmx2[j] * (dx2[j] * IRt(jm, k) + dx2[jm] * IRt(j, k)));
+    vo = V[q] - dt * Cmp * ((dPc - dP[qj]) / dmx2[j] + (invRhoc_2 - 1.0) * (dPhc - hj) / dmx2[j]) * (j >= 2 ? 1.0 : 0.0);
+    const auto invRhoc_3 = as<S>(0.5 / dmx3[k] * (dx3[k] * IRt(j, km) + dx3[km] * IRt(j, k)));
+    wo = W[q] - dt * Cmp * ((dPc - dP[qk]) / dmx3[k] + (invRhoc_3 - 1.0) * (dPhc - hk) / dmx3[k]);
     po = P[q] + dPc;
 }
 struct Projection {
@@ -603,8 +603,9 @@ struct Projection {
     double dt;
     const double *iR, *dP, *dPhat, *dP0, *U, *V, *W, *P;
     static constexpr int NF = 8;
-    template <class S, class Wr>
-    __device__ __forceinline__ void eval(const Wr &w, int i, int j, int k, S &a, S &b, S &c, S &d) const {
+    static constexpr int ND = 8, STALE = -1;  // rev.h
+    template <class S, class Wr, class I>
+    __device__ __forceinline__ void eval(const Wr &w, I i, I j, I k, S &a, S &b, S &c, S &d) const {
         projection_cell<S>(g, p, dt, w(0, iR), w(1, dP), w(2, dPhat), w(3, dP0), w(4, U), w(5, V), w(6, W), w(7, P), i,
                            j, k, a, b, c, d);
     }
@@ -626,11 +627,11 @@ __global__ void __launch_bounds__(256) k_projection(Projection cell, double *U, 
 }
 
 // the dPhat and dP0 history after the projection (:846-850)
-template <class S, class FP>
-__device__ __forceinline__ void dphat_cell(const Grid &g, FP dP, FP dPhat, FP dP0, int i, int j, int k, S &hn,
+template <class S, class FP, class I>
+__device__ __forceinline__ void dphat_cell(const Grid &g, FP dP, FP dPhat, FP dP0, I i, I j, I k, S &hn,
                                           S &d0n) {
-    const size_t q = g.ix(i, j, k);
-    const S d0 = (dPhat[q] + dP0[q]) / 2.0;
+    const auto q = g.ix(i, j, k);
+    const auto d0 = as<S>((dPhat[q] + dP0[q]) / 2.0);
     d0n = d0;
     hn = 2.0 * dP[q] - d0;
 }
@@ -638,8 +639,9 @@ struct DPhatUpdate {
     Grid g;
     const double *dP, *dPhat, *dP0;
     static constexpr int NF = 3;
-    template <class S, class Wr>
-    __device__ __forceinline__ void eval(const Wr &w, int i, int j, int k, S &a, S &b, S &c, S &d) const {
+    static constexpr int ND = 3, STALE = -1;  // rev.h
+    template <class S, class Wr, class I>
+    __device__ __forceinline__ void eval(const Wr &w, I i, I j, I k, S &a, S &b, S &c, S &d) const {
         dphat_cell<S>(g, w(0, dP), w(1, dPhat), w(2, dP0), i, j, k, a, b);
     }
 };

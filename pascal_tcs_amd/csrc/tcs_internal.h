@@ -57,6 +57,29 @@ void prof_end(hipStream_t s);
         if (_r != TCS_OK) return _r;                                           \
     } while (0)
 
+// An index of a cell formula in the adjoint's reverse pass: the index v and
+// its constant offset o in {-1, 0, 1} from the cell's own, which names the
+// input on the tape (rev.h).  RelCell: element q of a field, rel from the
+// three offsets; RelRow: element q of a (j, k) table.
+struct Rel {
+    int v, o;
+    __host__ __device__ __forceinline__ operator int() const { return v; }
+};
+__device__ __forceinline__ Rel operator+(Rel a, int d) { return Rel{a.v + d, a.o + d}; }
+__device__ __forceinline__ Rel operator-(Rel a, int d) { return Rel{a.v - d, a.o - d}; }
+struct RelCell {
+    size_t q;
+    int rel;
+};
+struct RelRow {
+    size_t q;
+    int rel;
+};
+// the fixed plane v read by a cell formula in the place of the neighbour at
+// offset o
+__device__ __forceinline__ int at_plane(int, int v, int) { return v; }
+__device__ __forceinline__ Rel at_plane(Rel, int v, int o) { return Rel{v, o}; }
+
 // Grid description passed by value to every stencil kernel.
 // Full fields: (0:n1m+1, 0:n2m+1, 0:n3m+1), i fastest, rows P1 >= N1
 // elements apart (a multiple of 16) and each field allocated FIELD_FRONT
@@ -82,6 +105,13 @@ struct Grid {
     __device__ __forceinline__ size_t t2(int j, int k) const { return (size_t)j + (size_t)N2 * (size_t)k; }
     __device__ __forceinline__ size_t r3(int i, int j, int k) const {
         return (size_t)(i - 1) + (size_t)n1m * ((size_t)(j - 1) + (size_t)n2m * (size_t)(k - 1));
+    }
+    __device__ __forceinline__ RelCell ix(Rel i, Rel j, Rel k) const {
+        return RelCell{ix(i.v, j.v, k.v), (k.o + 1) * 9 + (j.o + 1) * 3 + (i.o + 1)};
+    }
+    __device__ __forceinline__ RelCell b2(Rel i, Rel k) const { return RelCell{b2(i.v, k.v), 13 + i.o}; }
+    __device__ __forceinline__ RelRow t2(Rel j, Rel k) const {
+        return RelRow{t2(j.v, k.v), (k.o + 1) * 3 + (j.o + 1)};
     }
 };
 

@@ -52,20 +52,6 @@ __device__ __forceinline__ void th_kpp(const Phys &p, S T, S &kpp, S &dkpp) {
     dkpp = sc<S>(p.c10) * (sc<S>(p.c11) + sc<S>(2.0) * sc<S>(p.c12) * tmp1 + sc<S>(3.0) * sc<S>(p.c13) * tmp2 + sc<S>(4.0) * sc<S>(p.c14) * tmp3 + sc<S>(5.0) * sc<S>(p.c15) * tmp4) / sc<S>(p.KPP0);
 }
 
-template <class S>
-__device__ __forceinline__ S th_kpp_only(const Phys &p, S T) {
-    S k, dk;
-    th_kpp(p, T, k, dk);
-    return k;
-}
-
-template <class S>
-__device__ __forceinline__ S th_dkpp_only(const Phys &p, S T) {
-    S k, dk;
-    th_kpp(p, T, k, dk);
-    return dk;
-}
-
 // 1/(rho cp) and its derivative term (:116-156); the fast forms take the
 // polynomials in Horner's form, the derivative term's numerator collected
 // by powers of DeltaT*T on the host (Phys::dircN).
@@ -105,6 +91,28 @@ __device__ __forceinline__ void th_rhocp(const Phys &p, S T, S &irc, S &dirc) {
          / (da * da) / (db * db);
 }
 
+// The four property functions of one temperature as values of a cell formula.
+// The reverse pass takes each, a function of T alone, as one operation whose
+// derivative comes from forward-mode numbers.
+#define TH_PROPERTY(name, poly, which)                        \
+    template <class S, class X>                               \
+    __device__ __forceinline__ auto name(const Phys &p, const X &T) { \
+        if constexpr (is_rev<S>()) {                          \
+            Dual a, b;                                        \
+            poly<Dual>(p, Dual(T.v, 1.0), a, b);              \
+            return rev_of(T, which.v, which.d);               \
+        } else {                                              \
+            S a, b;                                           \
+            poly<S>(p, T, a, b);                              \
+            return which;                                     \
+        }                                                     \
+    }
+TH_PROPERTY(th_k, th_kpp, a)
+TH_PROPERTY(th_dk, th_kpp, b)
+TH_PROPERTY(th_irc, th_rhocp, a)
+TH_PROPERTY(th_dirc, th_rhocp, b)
+#undef TH_PROPERTY
+
 // mpi_thermal_coeffi: materialise the four property arrays over the full field
 __global__ void k_thermal_coeffi(Grid g, Phys p, const double *__restrict__ T, double *__restrict__ KPP,
                                  double *__restrict__ dKPP, double *__restrict__ iRC, double *__restrict__ diRC) {
@@ -118,126 +126,142 @@ __global__ void k_thermal_coeffi(Grid g, Phys p, const double *__restrict__ T, d
 }
 
 // stage 1: z (:236-361)
-template <class S, int WM, class FP>
+template <class S, int WM, class FP, class I>
 __device__ __forceinline__ void thermal_z_row(const Grid &g, const Phys &p, double dt,
     FP T, FP U, FP V,
     FP W, FP TBCup, FP TBCbt,
-    int i, int j, int k, S &am, S &ac, S &ap, S &rhsout) {
-    const int im = i - 1, ip = i + 1, jm = j - 1, jp = j + 1, km = k - 1, kp = k + 1;
+    I i, I j, I k, S &am, S &ac, S &ap, S &rhsout) {
+    const auto im = i - 1, ip = i + 1, jm = j - 1, jp = j + 1, km = k - 1, kp = k + 1;
     const int jem = g.jC[jm], jep = g.jC[jp];
     const auto dx1 = metric<S, M_DX1>(g), dx2 = metric<S, M_DX2>(g), dx3 = metric<S, M_DX3>(g);
     const auto dmx1 = metric<S, M_DMX1>(g), dmx2 = metric<S, M_DMX2>(g), dmx3 = metric<S, M_DMX3>(g);
-    const S Ct = sc<S>(p.Ct);
+    const auto Ct = as<S>(sc<S>(p.Ct));
 
-    const S Tc = T[g.ix(i, j, k)];
-    const S Tim = T[g.ix(im, j, k)], Tip = T[g.ix(ip, j, k)];
-    const S Tjm = T[g.ix(i, jm, k)], Tjp = T[g.ix(i, jp, k)];
-    const S Tkm = T[g.ix(i, j, km)], Tkp = T[g.ix(i, j, kp)];
+    const auto Tc = as<S>(T[g.ix(i, j, k)]);
+    const auto Tim = as<S>(T[g.ix(im, j, k)]);
+    const auto Tip = as<S>(T[g.ix(ip, j, k)]);
+    const auto Tjm = as<S>(T[g.ix(i, jm, k)]);
+    const auto Tjp = as<S>(T[g.ix(i, jp, k)]);
+    const auto Tkm = as<S>(T[g.ix(i, j, km)]);
+    const auto Tkp = as<S>(T[g.ix(i, j, kp)]);
 
-    S irc, dirc;
-    th_rhocp(p, Tc, irc, dirc);
-    S Kc, dKc, Kim, dKim, Kip, dKip, Kjm, dKjm, Kjp, dKjp, Kkm, dKkm, Kkp, dKkp;
-    th_kpp(p, Tc, Kc, dKc);
-    th_kpp(p, Tim, Kim, dKim);
-    th_kpp(p, Tip, Kip, dKip);
-    th_kpp(p, Tjm, Kjm, dKjm);
-    th_kpp(p, Tjp, Kjp, dKjp);
-    th_kpp(p, Tkm, Kkm, dKkm);
-    th_kpp(p, Tkp, Kkp, dKkp);
+    const auto irc = th_irc<S>(p, Tc);
+    const auto dirc = th_dirc<S>(p, Tc);
+    const auto Kc = th_k<S>(p, Tc);
+    const auto dKc = th_dk<S>(p, Tc);
+    const auto Kim = th_k<S>(p, Tim);
+    const auto dKim = th_dk<S>(p, Tim);
+    const auto Kip = th_k<S>(p, Tip);
+    const auto dKip = th_dk<S>(p, Tip);
+    const auto Kjm = th_k<S>(p, Tjm);
+    const auto dKjm = th_dk<S>(p, Tjm);
+    const auto Kjp = th_k<S>(p, Tjp);
+    const auto dKjp = th_dk<S>(p, Tjp);
+    const auto Kkm = th_k<S>(p, Tkm);
+    const auto dKkm = th_dk<S>(p, Tkm);
+    const auto Kkp = th_k<S>(p, Tkp);
+    const auto dKkp = th_dk<S>(p, Tkp);
 
-    const S invRhoCpCt_half = sc<S>(0.5) * Ct * irc;
-    const S dinvRhoCpCt_half = sc<S>(0.5) * Ct * dirc;
+    const auto invRhoCpCt_half = as<S>(sc<S>(0.5) * Ct * irc);
+    const auto dinvRhoCpCt_half = as<S>(sc<S>(0.5) * Ct * dirc);
 
-    const S e1 = (dx1[i] * Tim + dx1[im] * Tc) * (sc<S>(0.5) / dmx1[i]);
-    const S e2 = (dx1[ip] * Tc + dx1[i] * Tip) * (sc<S>(0.5) / dmx1[ip]);
-    const S e3 = (dx2[j] * Tjm + dx2[jm] * Tc) * (sc<S>(0.5) / dmx2[j]);
-    const S e4 = (dx2[jp] * Tc + dx2[j] * Tjp) * (sc<S>(0.5) / dmx2[jp]);
-    const S e5 = (dx3[k] * Tkm + dx3[km] * Tc) * (sc<S>(0.5) / dmx3[k]);
-    const S e6 = (dx3[kp] * Tc + dx3[k] * Tkp) * (sc<S>(0.5) / dmx3[kp]);
-    const S dedx1 = (Tc - Tim) / dmx1[i];
-    const S dedx2 = (Tip - Tc) / dmx1[ip];
-    const S dedy3 = (Tc - Tjm) / dmx2[j];
-    const S dedy4 = (Tjp - Tc) / dmx2[jp];
-    const S dedz5 = (Tc - Tkm) / dmx3[k];
-    const S dedz6 = (Tkp - Tc) / dmx3[kp];
+    const auto e1 = as<S>((dx1[i] * Tim + dx1[im] * Tc) * (sc<S>(0.5) / dmx1[i]));
+    const auto e2 = as<S>((dx1[ip] * Tc + dx1[i] * Tip) * (sc<S>(0.5) / dmx1[ip]));
+    const auto e3 = as<S>((dx2[j] * Tjm + dx2[jm] * Tc) * (sc<S>(0.5) / dmx2[j]));
+    const auto e4 = as<S>((dx2[jp] * Tc + dx2[j] * Tjp) * (sc<S>(0.5) / dmx2[jp]));
+    const auto e5 = as<S>((dx3[k] * Tkm + dx3[km] * Tc) * (sc<S>(0.5) / dmx3[k]));
+    const auto e6 = as<S>((dx3[kp] * Tc + dx3[k] * Tkp) * (sc<S>(0.5) / dmx3[kp]));
+    const auto dedx1 = as<S>((Tc - Tim) / dmx1[i]);
+    const auto dedx2 = as<S>((Tip - Tc) / dmx1[ip]);
+    const auto dedy3 = as<S>((Tc - Tjm) / dmx2[j]);
+    const auto dedy4 = as<S>((Tjp - Tc) / dmx2[jp]);
+    const auto dedz5 = as<S>((Tc - Tkm) / dmx3[k]);
+    const auto dedz6 = as<S>((Tkp - Tc) / dmx3[kp]);
 
-    const S Uc = U[g.ix(i, j, k)], Uip = U[g.ix(ip, j, k)];
-    const S Vc = V[g.ix(i, j, k)], Vjp = V[g.ix(i, jp, k)];
-    const S Wc = W[g.ix(i, j, k)], Wkp = W[g.ix(i, j, kp)];
-    const S convect_e1 = (Uc * dedx1 + Uip * dedx2) * sc<S>(0.5);
-    const S convect_e2 = (Vc * dedy3 + Vjp * dedy4) * sc<S>(0.5);
-    const S convect_e3 = (Wc * dedz5 + Wkp * dedz6) * sc<S>(0.5);
-    S rhs = -sc<S>(0.5) * (convect_e1 + convect_e2 + convect_e3);
+    const auto Uc = as<S>(U[g.ix(i, j, k)]);
+    const auto Uip = as<S>(U[g.ix(ip, j, k)]);
+    const auto Vc = as<S>(V[g.ix(i, j, k)]);
+    const auto Vjp = as<S>(V[g.ix(i, jp, k)]);
+    const auto Wc = as<S>(W[g.ix(i, j, k)]);
+    const auto Wkp = as<S>(W[g.ix(i, j, kp)]);
+    const auto convect_e1 = as<S>((Uc * dedx1 + Uip * dedx2) * sc<S>(0.5));
+    const auto convect_e2 = as<S>((Vc * dedy3 + Vjp * dedy4) * sc<S>(0.5));
+    const auto convect_e3 = as<S>((Wc * dedz5 + Wkp * dedz6) * sc<S>(0.5));
+    const auto rhs = as<S>(-sc<S>(0.5) * (convect_e1 + convect_e2 + convect_e3));
 
-    const S kPP1 = sc<S>(0.5) / dmx1[i] * (dx1[i] * Kim + dx1[im] * Kc);
-    const S kPP2 = sc<S>(0.5) / dmx1[ip] * (dx1[ip] * Kc + dx1[i] * Kip);
-    const S kPP3 = sc<S>(0.5) / dmx2[j] * (dx2[j] * Kjm + dx2[jm] * Kc);
-    const S kPP4 = sc<S>(0.5) / dmx2[jp] * (dx2[jp] * Kc + dx2[j] * Kjp);
-    const S kPP5 = sc<S>(0.5) / dmx3[k] * (dx3[k] * Kkm + dx3[km] * Kc);
-    const S kPP6 = sc<S>(0.5) / dmx3[kp] * (dx3[kp] * Kc + dx3[k] * Kkp);
-    const S dkPP1 = sc<S>(0.5) / dmx1[i] * (dx1[i] * dKim + dx1[im] * dKc);
-    const S dkPP2 = sc<S>(0.5) / dmx1[ip] * (dx1[ip] * dKc + dx1[i] * dKip);
-    const S dkPP3 = sc<S>(0.5) / dmx2[j] * (dx2[j] * dKjm + dx2[jm] * dKc);
-    const S dkPP4 = sc<S>(0.5) / dmx2[jp] * (dx2[jp] * dKc + dx2[j] * dKjp);
-    const S dkPP5 = sc<S>(0.5) / dmx3[k] * (dx3[k] * dKkm + dx3[km] * dKc);
-    const S dkPP6 = sc<S>(0.5) / dmx3[kp] * (dx3[kp] * dKc + dx3[k] * dKkp);
+    const auto kPP1 = as<S>(sc<S>(0.5) / dmx1[i] * (dx1[i] * Kim + dx1[im] * Kc));
+    const auto kPP2 = as<S>(sc<S>(0.5) / dmx1[ip] * (dx1[ip] * Kc + dx1[i] * Kip));
+    const auto kPP3 = as<S>(sc<S>(0.5) / dmx2[j] * (dx2[j] * Kjm + dx2[jm] * Kc));
+    const auto kPP4 = as<S>(sc<S>(0.5) / dmx2[jp] * (dx2[jp] * Kc + dx2[j] * Kjp));
+    const auto kPP5 = as<S>(sc<S>(0.5) / dmx3[k] * (dx3[k] * Kkm + dx3[km] * Kc));
+    const auto kPP6 = as<S>(sc<S>(0.5) / dmx3[kp] * (dx3[kp] * Kc + dx3[k] * Kkp));
+    const auto dkPP1 = as<S>(sc<S>(0.5) / dmx1[i] * (dx1[i] * dKim + dx1[im] * dKc));
+    const auto dkPP2 = as<S>(sc<S>(0.5) / dmx1[ip] * (dx1[ip] * dKc + dx1[i] * dKip));
+    const auto dkPP3 = as<S>(sc<S>(0.5) / dmx2[j] * (dx2[j] * dKjm + dx2[jm] * dKc));
+    const auto dkPP4 = as<S>(sc<S>(0.5) / dmx2[jp] * (dx2[jp] * dKc + dx2[j] * dKjp));
+    const auto dkPP5 = as<S>(sc<S>(0.5) / dmx3[k] * (dx3[k] * dKkm + dx3[km] * dKc));
+    const auto dkPP6 = as<S>(sc<S>(0.5) / dmx3[kp] * (dx3[kp] * dKc + dx3[k] * dKkp));
 
-    const S viscous_e1 = (kPP2 * dedx2 - kPP1 * dedx1 - e2 * dkPP2 * dedx2 + e1 * dkPP1 * dedx1) / dx1[i];
-    const S viscous_e2 = (kPP4 * dedy4 - kPP3 * dedy3 - e4 * dkPP4 * dedy4 + e3 * dkPP3 * dedy3) / dx2[j];
-    const S viscous_e3 = (kPP6 * dedz6 - kPP5 * dedz5 - e6 * dkPP6 * dedz6 + e5 * dkPP5 * dedz5) / dx3[k];
+    const auto viscous_e1 = as<S>((kPP2 * dedx2 - kPP1 * dedx1 - e2 * dkPP2 * dedx2 + e1 * dkPP1 * dedx1) / dx1[i]);
+    const auto viscous_e2 = as<S>((kPP4 * dedy4 - kPP3 * dedy3 - e4 * dkPP4 * dedy4 + e3 * dkPP3 * dedy3) / dx2[j]);
+    const auto viscous_e3 = as<S>((kPP6 * dedz6 - kPP5 * dedz5 - e6 * dkPP6 * dedz6 + e5 * dkPP5 * dedz5) / dx3[k]);
 
-    rhs = rhs
+    const auto rhs_2 = as<S>(rhs
         + invRhoCpCt_half * (viscous_e1 + viscous_e2 + viscous_e3)
         - dinvRhoCpCt_half * Tc * ((kPP2 * dedx2 - kPP1 * dedx1) / dx1[i]
                                    + (kPP4 * dedy4 - kPP3 * dedy3) / dx2[j]
-                                   + (kPP6 * dedz6 - kPP5 * dedz5) / dx3[k]);
+                                   + (kPP6 * dedz6 - kPP5 * dedz5) / dx3[k]));
 
     // the wall terms are multiplied by 1 - jem and 1 - jep, zero away from the
     // walls (WM as in the momentum z rows: 0 computes them, 1 skips them
     // there, 2 leaves them out)
-    if (WM == 0 || (WM == 1 && (jem != 1 || jep != 1))) {
-    const S tup = TBCup[g.b2(i, k)], tbt = TBCbt[g.b2(i, k)];
-    S ebc_up = -sc<S>(0.25) * Vjp / dmx2[jp] * tup;
-    S ebc_down = sc<S>(0.25) * Vc / dmx2[j] * tbt;
-    ebc_up = ebc_up
-           + invRhoCpCt_half / dx2[j] * kPP4 / dmx2[jp] * tup
-           + invRhoCpCt_half / dx2[j] * dkPP4 * dedy4 * tup;
-    ebc_down = ebc_down
-             + invRhoCpCt_half / dx2[j] * kPP3 / dmx2[j] * tbt
-             - invRhoCpCt_half / dx2[j] * dkPP3 * dedy3 * tbt;
-    rhs = rhs + sc<S>(1 - jem) * ebc_down + sc<S>(1 - jep) * ebc_up;
-    }
+    const auto wall_terms = [&](const auto &r) {
+        const auto tup = as<S>(TBCup[g.b2(i, k)]);
+        const auto tbt = as<S>(TBCbt[g.b2(i, k)]);
+        const auto ebc_up = [&] {
+            return -sc<S>(0.25) * Vjp / dmx2[jp] * tup
+                 + invRhoCpCt_half / dx2[j] * kPP4 / dmx2[jp] * tup
+                 + invRhoCpCt_half / dx2[j] * dkPP4 * dedy4 * tup;
+        };
+        const auto ebc_down = [&] {
+            return sc<S>(0.25) * Vc / dmx2[j] * tbt
+                 + invRhoCpCt_half / dx2[j] * kPP3 / dmx2[j] * tbt
+                 - invRhoCpCt_half / dx2[j] * dkPP3 * dedy3 * tbt;
+        };
+        return r + sc<S>(1 - jem) * ebc_down() + sc<S>(1 - jep) * ebc_up();
+    };
+    const auto rhs_3 = as<S>(with_walls<S, WM>(jem != 1 || jep != 1, rhs_2, wall_terms));
 
-    const S eACK = invRhoCpCt_half / dx3[k] * (kPP6 / dmx3[kp] + kPP5 / dmx3[k]
+    const auto eACK = as<S>(invRhoCpCt_half / dx3[k] * (kPP6 / dmx3[kp] + kPP5 / dmx3[k]
                                                     - dx3[kp] * (sc<S>(0.5) / dmx3[kp]) * dkPP6 * dedz6
                                                     + dx3[km] * (sc<S>(0.5) / dmx3[k]) * dkPP5 * dedz5)
-                      + (-sc<S>(0.25) * Wkp / dmx3[kp] + sc<S>(0.25) * Wc / dmx3[k]);
-    const S eAPK = -invRhoCpCt_half / dx3[k] * (kPP6 / dmx3[kp] + dx3[k] * (sc<S>(0.5) / dmx3[kp]) * dkPP6 * dedz6) + sc<S>(0.25) * Wkp / dmx3[kp];
-    const S eAMK = -invRhoCpCt_half / dx3[k] * (kPP5 / dmx3[k] - dx3[k] * (sc<S>(0.5) / dmx3[k]) * dkPP5 * dedz5) - sc<S>(0.25) * Wc / dmx3[k];
+                      + (-sc<S>(0.25) * Wkp / dmx3[kp] + sc<S>(0.25) * Wc / dmx3[k]));
+    const auto eAPK = as<S>(-invRhoCpCt_half / dx3[k] * (kPP6 / dmx3[kp] + dx3[k] * (sc<S>(0.5) / dmx3[kp]) * dkPP6 * dedz6) + sc<S>(0.25) * Wkp / dmx3[kp]);
+    const auto eAMK = as<S>(-invRhoCpCt_half / dx3[k] * (kPP5 / dmx3[k] - dx3[k] * (sc<S>(0.5) / dmx3[k]) * dkPP5 * dedz5) - sc<S>(0.25) * Wc / dmx3[k]);
 
-    const S eACI = invRhoCpCt_half / dx1[i] * (kPP2 / dmx1[ip] + kPP1 / dmx1[i]
+    const auto eACI = as<S>(invRhoCpCt_half / dx1[i] * (kPP2 / dmx1[ip] + kPP1 / dmx1[i]
                                                     - dx1[ip] * (sc<S>(0.5) / dmx1[ip]) * dkPP2 * dedx2
                                                     + dx1[im] * (sc<S>(0.5) / dmx1[i]) * dkPP1 * dedx1)
-                      + (sc<S>(0.25) * Uc / dmx1[i] - sc<S>(0.25) * Uip / dmx1[ip]);
-    const S eAPI = -invRhoCpCt_half / dx1[i] * (kPP2 / dmx1[ip] + dx1[i] * (sc<S>(0.5) / dmx1[ip]) * dkPP2 * dedx2) + sc<S>(0.25) * Uip / dmx1[ip];
-    const S eAMI = -invRhoCpCt_half / dx1[i] * (kPP1 / dmx1[i] - dx1[i] * (sc<S>(0.5) / dmx1[i]) * dkPP1 * dedx1) - sc<S>(0.25) * Uc / dmx1[i];
+                      + (sc<S>(0.25) * Uc / dmx1[i] - sc<S>(0.25) * Uip / dmx1[ip]));
+    const auto eAPI = as<S>(-invRhoCpCt_half / dx1[i] * (kPP2 / dmx1[ip] + dx1[i] * (sc<S>(0.5) / dmx1[ip]) * dkPP2 * dedx2) + sc<S>(0.25) * Uip / dmx1[ip]);
+    const auto eAMI = as<S>(-invRhoCpCt_half / dx1[i] * (kPP1 / dmx1[i] - dx1[i] * (sc<S>(0.5) / dmx1[i]) * dkPP1 * dedx1) - sc<S>(0.25) * Uc / dmx1[i]);
 
-    const S eACJ = invRhoCpCt_half / dx2[j] * (kPP4 / dmx2[jp] + kPP3 / dmx2[j]
+    const auto eACJ = as<S>(invRhoCpCt_half / dx2[j] * (kPP4 / dmx2[jp] + kPP3 / dmx2[j]
                                                     - dx2[jp] * (sc<S>(0.5) / dmx2[jp]) * dkPP4 * dedy4 * sc<S>(jep)
                                                     + dx2[jm] * (sc<S>(0.5) / dmx2[j]) * dkPP3 * dedy3 * sc<S>(jem))
-                      + (sc<S>(0.25) * Vc / dmx2[j] - sc<S>(0.25) * Vjp / dmx2[jp]);
-    S eAPJ = -invRhoCpCt_half / dx2[j] * (kPP4 / dmx2[jp] + dx2[j] * (sc<S>(0.5) / dmx2[jp]) * dkPP4 * dedy4) + sc<S>(0.25) * Vjp / dmx2[jp];
-    S eAMJ = -invRhoCpCt_half / dx2[j] * (kPP3 / dmx2[j] - dx2[j] * (sc<S>(0.5) / dmx2[j]) * dkPP3 * dedy3) - sc<S>(0.25) * Vc / dmx2[j];
-    eAPJ = eAPJ * sc<S>(jep);
-    eAMJ = eAMJ * sc<S>(jem);
+                      + (sc<S>(0.25) * Vc / dmx2[j] - sc<S>(0.25) * Vjp / dmx2[jp]));
+    const auto eAPJ = as<S>(-invRhoCpCt_half / dx2[j] * (kPP4 / dmx2[jp] + dx2[j] * (sc<S>(0.5) / dmx2[jp]) * dkPP4 * dedy4) + sc<S>(0.25) * Vjp / dmx2[jp]);
+    const auto eAMJ = as<S>(-invRhoCpCt_half / dx2[j] * (kPP3 / dmx2[j] - dx2[j] * (sc<S>(0.5) / dmx2[j]) * dkPP3 * dedy3) - sc<S>(0.25) * Vc / dmx2[j]);
+    const auto eAPJ_2 = as<S>(eAPJ * sc<S>(jep));
+    const auto eAMJ_2 = as<S>(eAMJ * sc<S>(jem));
 
-    rhs = rhs
+    const auto rhs_4 = as<S>(rhs_3
         - (eAPK * Tkp + eACK * Tc + eAMK * Tkm
-           + eAPJ * Tjp + eACJ * Tc + eAMJ * Tjm
+           + eAPJ_2 * Tjp + eACJ * Tc + eAMJ_2 * Tjm
            + eAPI * Tip + eACI * Tc + eAMI * Tim
            - dinvRhoCpCt_half * Tc * ((kPP2 * dedx2 - kPP1 * dedx1) / dx1[i]
                                       + (kPP4 * dedy4 - kPP3 * dedy3) / dx2[j]
-                                      + (kPP6 * dedz6 - kPP5 * dedz5) / dx3[k]));
+                                      + (kPP6 * dedz6 - kPP5 * dedz5) / dx3[k])));
 
     ac = eACK * sc<S>(dt)
           - sc<S>(0.5) * dinvRhoCpCt_half * ((kPP2 * dedx2 - kPP1 * dedx1) / dx1[i]
@@ -246,7 +270,7 @@ __device__ __forceinline__ void thermal_z_row(const Grid &g, const Phys &p, doub
           + sc<S>(1.0);
     ap = eAPK * sc<S>(dt);
     am = eAMK * sc<S>(dt);
-    rhsout = rhs * sc<S>(dt);
+    rhsout = rhs_4 * sc<S>(dt);
 }
 struct ThermalZ {
     // FP32 lines of the mixed form: 8 lines a workgroup at three waves per
@@ -262,12 +286,13 @@ struct ThermalZ {
     double dt;
     const double *T, *U, *V, *W, *TBCup, *TBCbt;
     static constexpr int NF = 6;  // field inputs, in the order below
+    static constexpr int ND = 6, STALE = -1;  // rev.h
     static constexpr bool FULL = false;  // unconditional row loop in the FP64 z solve
-    template <class S, int WM = -1, class Wr>
-    __device__ __forceinline__ void eval(const Wr &w, int i, int j, int k, S &a, S &b, S &c, S &d) const {
+    template <class S, int WM = -1, class Wr, class I>
+    __device__ __forceinline__ void eval(const Wr &w, I i, I j, I k, S &a, S &b, S &c, S &d) const {
         // WM < 0 (the row's own wall-term mode): a branch on j, skipping the
         // terms away from the walls (FP64 3.44 -> 3.23 ms, FP32 2.33 -> 2.06
-        // ms at 512^3), terms kept in the adjoint's dual passes
+        // ms at 512^3), terms kept in the adjoint's reverse pass
         thermal_z_row<S, (WM >= 0 ? WM : (is_dual<S>() ? 0 : 1))>(g, p, dt, w(0, T), w(1, U), w(2, V), w(3, W), w(4, TBCup), w(5, TBCbt), i, j, k, a, b, c, d);
     }
     // no wall term of row j is weighted (the wall terms' flags are all 1)
@@ -280,55 +305,64 @@ struct ThermalZ {
 
 // stage 2: x (:388-429).  jm,jp,km,kp are the values the reference's loop
 // variables keep after stage 1: n2m-1, n2m+1, n3m-1, n3m+1.
-template <class S, class FP>
+template <class S, class FP, class I>
 __device__ __forceinline__ void thermal_x_row(const Grid &g, const Phys &p, double dt,
     FP T, FP U,
-    int i, int j, int k, S &am, S &ac, S &ap) {
-    const int im = i - 1, ip = i + 1;
-    const int jm = g.n2m - 1, jp = g.n2m + 1, km = g.n3m - 1, kp = g.n3m + 1;
+    I i, I j, I k, S &am, S &ac, S &ap) {
+    const auto im = i - 1, ip = i + 1;
+    const auto jm = at_plane(j, g.n2m - 1, -1), jp = at_plane(j, g.n2m + 1, 1);
+    const auto km = at_plane(k, g.n3m - 1, -1), kp = at_plane(k, g.n3m + 1, 1);
     // the double tables rounded where read (the FP32 rows' faster schedule)
     const auto dx1 = metric<S, M_DX1, true>(g), dx2 = metric<S, M_DX2, true>(g), dx3 = metric<S, M_DX3, true>(g);
     const auto dmx1 = metric<S, M_DMX1, true>(g), dmx2 = metric<S, M_DMX2, true>(g), dmx3 = metric<S, M_DMX3, true>(g);
 
-    const S Tc = T[g.ix(i, j, k)];
-    const S Tim = T[g.ix(im, j, k)], Tip = T[g.ix(ip, j, k)];
-    const S Tjm = T[g.ix(i, jm, k)], Tjp = T[g.ix(i, jp, k)];
-    const S Tkm = T[g.ix(i, j, km)], Tkp = T[g.ix(i, j, kp)];
-    S irc, dirc;
-    th_rhocp(p, Tc, irc, dirc);
-    S Kc, dKc, Kim, dKim, Kip, dKip;
-    th_kpp(p, Tc, Kc, dKc);
-    th_kpp(p, Tim, Kim, dKim);
-    th_kpp(p, Tip, Kip, dKip);
-    const S Kjm = th_kpp_only(p, Tjm), Kjp = th_kpp_only(p, Tjp);
-    const S Kkm = th_kpp_only(p, Tkm), Kkp = th_kpp_only(p, Tkp);
+    const auto Tc = as<S>(T[g.ix(i, j, k)]);
+    const auto Tim = as<S>(T[g.ix(im, j, k)]);
+    const auto Tip = as<S>(T[g.ix(ip, j, k)]);
+    const auto Tjm = as<S>(T[g.ix(i, jm, k)]);
+    const auto Tjp = as<S>(T[g.ix(i, jp, k)]);
+    const auto Tkm = as<S>(T[g.ix(i, j, km)]);
+    const auto Tkp = as<S>(T[g.ix(i, j, kp)]);
+    const auto irc = th_irc<S>(p, Tc);
+    const auto dirc = th_dirc<S>(p, Tc);
+    const auto Kc = th_k<S>(p, Tc);
+    const auto dKc = th_dk<S>(p, Tc);
+    const auto Kim = th_k<S>(p, Tim);
+    const auto dKim = th_dk<S>(p, Tim);
+    const auto Kip = th_k<S>(p, Tip);
+    const auto dKip = th_dk<S>(p, Tip);
+    const auto Kjm = th_k<S>(p, Tjm);
+    const auto Kjp = th_k<S>(p, Tjp);
+    const auto Kkm = th_k<S>(p, Tkm);
+    const auto Kkp = th_k<S>(p, Tkp);
 
-    const S invRhoCpCt_half = sc<S>(0.5) * sc<S>(p.Ct) * irc;
-    const S kPP1 = sc<S>(0.5) / dmx1[i] * (dx1[i] * Kim + dx1[im] * Kc);
-    const S kPP2 = sc<S>(0.5) / dmx1[ip] * (dx1[ip] * Kc + dx1[i] * Kip);
-    const S kPP3 = sc<S>(0.5) / dmx2[j] * (dx2[j] * Kjm + dx2[jm] * Kc);
-    const S kPP4 = sc<S>(0.5) / dmx2[jp] * (dx2[jp] * Kc + dx2[j] * Kjp);
-    const S kPP5 = sc<S>(0.5) / dmx3[k] * (dx3[k] * Kkm + dx3[km] * Kc);
-    const S kPP6 = sc<S>(0.5) / dmx3[kp] * (dx3[kp] * Kc + dx3[k] * Kkp);
-    const S dkPP1 = sc<S>(0.5) / dmx1[i] * (dx1[i] * dKim + dx1[im] * dKc);
-    const S dkPP2 = sc<S>(0.5) / dmx1[ip] * (dx1[ip] * dKc + dx1[i] * dKip);
-    const S dedx1 = (Tc - Tim) / dmx1[i];
-    const S dedx2 = (Tip - Tc) / dmx1[ip];
-    const S dedy3 = (Tc - Tjm) / dmx2[j];
-    const S dedy4 = (Tjp - Tc) / dmx2[jp];
-    const S dedz5 = (Tc - Tkm) / dmx3[k];
-    const S dedz6 = (Tkp - Tc) / dmx3[kp];
-    const S Uc = U[g.ix(i, j, k)], Uip = U[g.ix(ip, j, k)];
+    const auto invRhoCpCt_half = as<S>(sc<S>(0.5) * sc<S>(p.Ct) * irc);
+    const auto kPP1 = as<S>(sc<S>(0.5) / dmx1[i] * (dx1[i] * Kim + dx1[im] * Kc));
+    const auto kPP2 = as<S>(sc<S>(0.5) / dmx1[ip] * (dx1[ip] * Kc + dx1[i] * Kip));
+    const auto kPP3 = as<S>(sc<S>(0.5) / dmx2[j] * (dx2[j] * Kjm + dx2[jm] * Kc));
+    const auto kPP4 = as<S>(sc<S>(0.5) / dmx2[jp] * (dx2[jp] * Kc + dx2[j] * Kjp));
+    const auto kPP5 = as<S>(sc<S>(0.5) / dmx3[k] * (dx3[k] * Kkm + dx3[km] * Kc));
+    const auto kPP6 = as<S>(sc<S>(0.5) / dmx3[kp] * (dx3[kp] * Kc + dx3[k] * Kkp));
+    const auto dkPP1 = as<S>(sc<S>(0.5) / dmx1[i] * (dx1[i] * dKim + dx1[im] * dKc));
+    const auto dkPP2 = as<S>(sc<S>(0.5) / dmx1[ip] * (dx1[ip] * dKc + dx1[i] * dKip));
+    const auto dedx1 = as<S>((Tc - Tim) / dmx1[i]);
+    const auto dedx2 = as<S>((Tip - Tc) / dmx1[ip]);
+    const auto dedy3 = as<S>((Tc - Tjm) / dmx2[j]);
+    const auto dedy4 = as<S>((Tjp - Tc) / dmx2[jp]);
+    const auto dedz5 = as<S>((Tc - Tkm) / dmx3[k]);
+    const auto dedz6 = as<S>((Tkp - Tc) / dmx3[kp]);
+    const auto Uc = as<S>(U[g.ix(i, j, k)]);
+    const auto Uip = as<S>(U[g.ix(ip, j, k)]);
 
-    const S eACI = invRhoCpCt_half / dx1[i] * (kPP2 / dmx1[ip] + kPP1 / dmx1[i]
+    const auto eACI = as<S>(invRhoCpCt_half / dx1[i] * (kPP2 / dmx1[ip] + kPP1 / dmx1[i]
                                                     - dx1[ip] * (sc<S>(0.5) / dmx1[ip]) * dkPP2 * dedx2
                                                     + dx1[im] * (sc<S>(0.5) / dmx1[i]) * dkPP1 * dedx1)
                       + (sc<S>(0.25) * Uc / dmx1[i] - sc<S>(0.25) * Uip / dmx1[ip])
                       - sc<S>(0.5) * invRhoCpCt_half * ((kPP2 * dedx2 - kPP1 * dedx1) / dx1[i]
                                                  + (kPP4 * dedy4 - kPP3 * dedy3) / dx2[j]
-                                                 + (kPP6 * dedz6 - kPP5 * dedz5) / dx3[k]);
-    const S eAPI = -invRhoCpCt_half / dx1[i] * (kPP2 / dmx1[ip] + dx1[i] * (sc<S>(0.5) / dmx1[ip]) * dkPP2 * dedx2) + sc<S>(0.25) * Uip / dmx1[ip];
-    const S eAMI = -invRhoCpCt_half / dx1[i] * (kPP1 / dmx1[i] - dx1[i] * (sc<S>(0.5) / dmx1[i]) * dkPP1 * dedx1) - sc<S>(0.25) * Uc / dmx1[i];
+                                                 + (kPP6 * dedz6 - kPP5 * dedz5) / dx3[k]));
+    const auto eAPI = as<S>(-invRhoCpCt_half / dx1[i] * (kPP2 / dmx1[ip] + dx1[i] * (sc<S>(0.5) / dmx1[ip]) * dkPP2 * dedx2) + sc<S>(0.25) * Uip / dmx1[ip]);
+    const auto eAMI = as<S>(-invRhoCpCt_half / dx1[i] * (kPP1 / dmx1[i] - dx1[i] * (sc<S>(0.5) / dmx1[i]) * dkPP1 * dedx1) - sc<S>(0.25) * Uc / dmx1[i]);
     ac = eACI * sc<S>(dt) + sc<S>(1.0);
     ap = eAPI * sc<S>(dt);
     am = eAMI * sc<S>(dt);
@@ -339,8 +373,9 @@ struct ThermalX {
     double dt;
     const double *T, *U;
     static constexpr int NF = 2;  // field inputs, in the order below
-    template <class S, class Wr>
-    __device__ __forceinline__ void eval(const Wr &w, int i, int j, int k, S &a, S &b, S &c, S &d) const {
+    static constexpr int ND = 2, STALE = -1;  // rev.h
+    template <class S, class Wr, class I>
+    __device__ __forceinline__ void eval(const Wr &w, I i, I j, I k, S &a, S &b, S &c, S &d) const {
         thermal_x_row<S>(g, p, dt, w(0, T), w(1, U), i, j, k, a, b, c);
     }
     __device__ __forceinline__ void operator()(int i, int j, int k, double &a, double &b, double &c,
@@ -350,60 +385,68 @@ struct ThermalX {
 };
 
 // stage 3: y (:456-507); km,kp keep their stage-1 values n3m-1, n3m+1.
-template <class S, class FP>
+template <class S, class FP, class I>
 __device__ __forceinline__ void thermal_y_row(const Grid &g, const Phys &p, double dt,
     FP T, FP V,
-    int i, int j, int k, S &am, S &ac, S &ap) {
-    const int im = i - 1, ip = i + 1, jm = j - 1, jp = j + 1;
-    const int km = g.n3m - 1, kp = g.n3m + 1;
+    I i, I j, I k, S &am, S &ac, S &ap) {
+    const auto im = i - 1, ip = i + 1, jm = j - 1, jp = j + 1;
+    const auto km = at_plane(k, g.n3m - 1, -1), kp = at_plane(k, g.n3m + 1, 1);
     const int jem = g.jC[jm], jep = g.jC[jp];
     const auto dx1 = metric<S, M_DX1>(g), dx2 = metric<S, M_DX2>(g), dx3 = metric<S, M_DX3>(g);
     const auto dmx1 = metric<S, M_DMX1>(g), dmx2 = metric<S, M_DMX2>(g), dmx3 = metric<S, M_DMX3>(g);
 
-    const S Tc = T[g.ix(i, j, k)];
-    const S Tim = T[g.ix(im, j, k)], Tip = T[g.ix(ip, j, k)];
-    const S Tjm = T[g.ix(i, jm, k)], Tjp = T[g.ix(i, jp, k)];
-    const S Tkm = T[g.ix(i, j, km)], Tkp = T[g.ix(i, j, kp)];
-    S irc, dirc;
-    th_rhocp(p, Tc, irc, dirc);
-    S Kc, dKc, Kjm, dKjm, Kjp, dKjp;
-    th_kpp(p, Tc, Kc, dKc);
-    th_kpp(p, Tjm, Kjm, dKjm);
-    th_kpp(p, Tjp, Kjp, dKjp);
-    const S Kim = th_kpp_only(p, Tim), Kip = th_kpp_only(p, Tip);
-    const S Kkm = th_kpp_only(p, Tkm), Kkp = th_kpp_only(p, Tkp);
+    const auto Tc = as<S>(T[g.ix(i, j, k)]);
+    const auto Tim = as<S>(T[g.ix(im, j, k)]);
+    const auto Tip = as<S>(T[g.ix(ip, j, k)]);
+    const auto Tjm = as<S>(T[g.ix(i, jm, k)]);
+    const auto Tjp = as<S>(T[g.ix(i, jp, k)]);
+    const auto Tkm = as<S>(T[g.ix(i, j, km)]);
+    const auto Tkp = as<S>(T[g.ix(i, j, kp)]);
+    const auto irc = th_irc<S>(p, Tc);
+    const auto dirc = th_dirc<S>(p, Tc);
+    const auto Kc = th_k<S>(p, Tc);
+    const auto dKc = th_dk<S>(p, Tc);
+    const auto Kjm = th_k<S>(p, Tjm);
+    const auto dKjm = th_dk<S>(p, Tjm);
+    const auto Kjp = th_k<S>(p, Tjp);
+    const auto dKjp = th_dk<S>(p, Tjp);
+    const auto Kim = th_k<S>(p, Tim);
+    const auto Kip = th_k<S>(p, Tip);
+    const auto Kkm = th_k<S>(p, Tkm);
+    const auto Kkp = th_k<S>(p, Tkp);
 
-    const S invRhoCpCt_half = sc<S>(0.5) * sc<S>(p.Ct) * irc;
-    const S kPP1 = sc<S>(0.5) / dmx1[i] * (dx1[i] * Kim + dx1[im] * Kc);
-    const S kPP2 = sc<S>(0.5) / dmx1[ip] * (dx1[ip] * Kc + dx1[i] * Kip);
-    const S kPP3 = sc<S>(0.5) / dmx2[j] * (dx2[j] * Kjm + dx2[jm] * Kc);
-    const S kPP4 = sc<S>(0.5) / dmx2[jp] * (dx2[jp] * Kc + dx2[j] * Kjp);
-    const S kPP5 = sc<S>(0.5) / dmx3[k] * (dx3[k] * Kkm + dx3[km] * Kc);
-    const S kPP6 = sc<S>(0.5) / dmx3[kp] * (dx3[kp] * Kc + dx3[k] * Kkp);
-    const S dkPP3 = sc<S>(0.5) / dmx2[j] * (dx2[j] * dKjm + dx2[jm] * dKc);
-    const S dkPP4 = sc<S>(0.5) / dmx2[jp] * (dx2[jp] * dKc + dx2[j] * dKjp);
-    const S dedx1 = (Tc - Tim) / dmx1[i];
-    const S dedx2 = (Tip - Tc) / dmx1[ip];
-    const S dedy3 = (Tc - Tjm) / dmx2[j];
-    const S dedy4 = (Tjp - Tc) / dmx2[jp];
-    const S dedz5 = (Tc - Tkm) / dmx3[k];
-    const S dedz6 = (Tkp - Tc) / dmx3[kp];
-    const S Vc = V[g.ix(i, j, k)], Vjp = V[g.ix(i, jp, k)];
+    const auto invRhoCpCt_half = as<S>(sc<S>(0.5) * sc<S>(p.Ct) * irc);
+    const auto kPP1 = as<S>(sc<S>(0.5) / dmx1[i] * (dx1[i] * Kim + dx1[im] * Kc));
+    const auto kPP2 = as<S>(sc<S>(0.5) / dmx1[ip] * (dx1[ip] * Kc + dx1[i] * Kip));
+    const auto kPP3 = as<S>(sc<S>(0.5) / dmx2[j] * (dx2[j] * Kjm + dx2[jm] * Kc));
+    const auto kPP4 = as<S>(sc<S>(0.5) / dmx2[jp] * (dx2[jp] * Kc + dx2[j] * Kjp));
+    const auto kPP5 = as<S>(sc<S>(0.5) / dmx3[k] * (dx3[k] * Kkm + dx3[km] * Kc));
+    const auto kPP6 = as<S>(sc<S>(0.5) / dmx3[kp] * (dx3[kp] * Kc + dx3[k] * Kkp));
+    const auto dkPP3 = as<S>(sc<S>(0.5) / dmx2[j] * (dx2[j] * dKjm + dx2[jm] * dKc));
+    const auto dkPP4 = as<S>(sc<S>(0.5) / dmx2[jp] * (dx2[jp] * dKc + dx2[j] * dKjp));
+    const auto dedx1 = as<S>((Tc - Tim) / dmx1[i]);
+    const auto dedx2 = as<S>((Tip - Tc) / dmx1[ip]);
+    const auto dedy3 = as<S>((Tc - Tjm) / dmx2[j]);
+    const auto dedy4 = as<S>((Tjp - Tc) / dmx2[jp]);
+    const auto dedz5 = as<S>((Tc - Tkm) / dmx3[k]);
+    const auto dedz6 = as<S>((Tkp - Tc) / dmx3[kp]);
+    const auto Vc = as<S>(V[g.ix(i, j, k)]);
+    const auto Vjp = as<S>(V[g.ix(i, jp, k)]);
 
-    const S eACJ = invRhoCpCt_half / dx2[j] * (kPP4 / dmx2[jp] + kPP3 / dmx2[j]
+    const auto eACJ = as<S>(invRhoCpCt_half / dx2[j] * (kPP4 / dmx2[jp] + kPP3 / dmx2[j]
                                                     - dx2[jp] * (sc<S>(0.5) / dmx2[jp]) * dkPP4 * dedy4 * sc<S>(jep)
                                                     + dx2[jm] * (sc<S>(0.5) / dmx2[j]) * dkPP3 * dedy3 * sc<S>(jem))
                       + (sc<S>(0.25) * Vc / dmx2[j] - sc<S>(0.25) * Vjp / dmx2[jp])
                       - sc<S>(0.5) * invRhoCpCt_half * ((kPP2 * dedx2 - kPP1 * dedx1) / dx1[i]
                                                  + (kPP4 * dedy4 - kPP3 * dedy3) / dx2[j]
-                                                 + (kPP6 * dedz6 - kPP5 * dedz5) / dx3[k]);
-    S eAPJ = -invRhoCpCt_half / dx2[j] * (kPP4 / dmx2[jp] + dx2[j] * (sc<S>(0.5) / dmx2[jp]) * dkPP4 * dedy4) + sc<S>(0.25) * Vjp / dmx2[jp];
-    S eAMJ = -invRhoCpCt_half / dx2[j] * (kPP3 / dmx2[j] - dx2[j] * (sc<S>(0.5) / dmx2[j]) * dkPP3 * dedy3) - sc<S>(0.25) * Vc / dmx2[j];
-    eAPJ = eAPJ * sc<S>(jep);
-    eAMJ = eAMJ * sc<S>(jem);
+                                                 + (kPP6 * dedz6 - kPP5 * dedz5) / dx3[k]));
+    const auto eAPJ = as<S>(-invRhoCpCt_half / dx2[j] * (kPP4 / dmx2[jp] + dx2[j] * (sc<S>(0.5) / dmx2[jp]) * dkPP4 * dedy4) + sc<S>(0.25) * Vjp / dmx2[jp]);
+    const auto eAMJ = as<S>(-invRhoCpCt_half / dx2[j] * (kPP3 / dmx2[j] - dx2[j] * (sc<S>(0.5) / dmx2[j]) * dkPP3 * dedy3) - sc<S>(0.25) * Vc / dmx2[j]);
+    const auto eAPJ_2 = as<S>(eAPJ * sc<S>(jep));
+    const auto eAMJ_2 = as<S>(eAMJ * sc<S>(jem));
     ac = eACJ * sc<S>(dt) + sc<S>(1.0);
-    ap = eAPJ * sc<S>(dt);
-    am = eAMJ * sc<S>(dt);
+    ap = eAPJ_2 * sc<S>(dt);
+    am = eAMJ_2 * sc<S>(dt);
 }
 struct ThermalY {
     // FP32 lines of the mixed form at four waves per SIMD (2.54 -> 1.84 ms at
@@ -415,8 +458,9 @@ struct ThermalY {
     double dt;
     const double *T, *V;
     static constexpr int NF = 2;  // field inputs, in the order below
-    template <class S, class Wr>
-    __device__ __forceinline__ void eval(const Wr &w, int i, int j, int k, S &a, S &b, S &c, S &d) const {
+    static constexpr int ND = 2, STALE = -1;  // rev.h
+    template <class S, class Wr, class I>
+    __device__ __forceinline__ void eval(const Wr &w, I i, I j, I k, S &a, S &b, S &c, S &d) const {
         thermal_y_row<S>(g, p, dt, w(0, T), w(1, V), i, j, k, a, b, c);
     }
     __device__ __forceinline__ void operator()(int i, int j, int k, double &a, double &b, double &c,
