@@ -172,7 +172,7 @@ __global__ void k_zero_interior(Grid g, int jlo, double *__restrict__ f) {
 __global__ void k_poisson_tdma_T(int n3m, int h1p, int n2m, int h3p, const double *__restrict__ amj,
                                  const double *__restrict__ apj, const double *__restrict__ acj,
                                  const double *__restrict__ dxk2, const double *__restrict__ dzk,
-                                 double2 *__restrict__ S, double *__restrict__ cw) {
+                                 double2 *S, double *cw) {
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     const int nsys = n3m * h1p;
     if (s >= nsys) return;
@@ -186,27 +186,53 @@ __global__ void k_poisson_tdma_T(int n3m, int h1p, int n2m, int h3p, const doubl
     auto A = [&](int jj) { return (pin && jj == 0) ? 0.0 : amj[jj]; };
     auto B = [&](int jj) { return (pin && jj == 0) ? 1.0 : acj[jj] - shift - zk; };
     auto C = [&](int jj) { return (pin && jj == 0) ? 0.0 : apj[jj]; };
-    // row jj of the transpose: (C(jj-1), B(jj), A(jj+1)); ends dropped (non-cyclic)
+    // row jj of the transpose: (C(jj-1), B(jj), A(jj+1)); ends dropped
+    // (non-cyclic).  The rows come U at a time, the next ones in flight.
+    constexpr int U = 8;
     double cprev = 0.0, dr = 0.0, di = 0.0;
-    for (int jj = 0; jj < n2m; jj++) {
-        const double at = jj > 0 ? C(jj - 1) : 0.0;
-        const double ct = jj < n2m - 1 ? A(jj + 1) : 0.0;
-        const double m = 1.0 / (B(jj) - at * cprev);
-        const double2 v = d[(size_t)jj * rs];
-        const double vi = zim ? 0.0 : v.y;
-        dr = (v.x - at * dr) * m;
-        di = (vi - at * di) * m;
-        cprev = ct * m;
-        cp[(size_t)jj * rs] = cprev;
-        d[(size_t)jj * rs] = make_double2(dr, di);
+    double2 v[U], nv[U];
+#pragma unroll
+    for (int u = 0; u < U; u++)
+        if (u < n2m) v[u] = d[(size_t)u * rs];
+    for (int j0 = 0; j0 < n2m; j0 += U) {
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (j0 + U + u < n2m) nv[u] = d[(size_t)(j0 + U + u) * rs];
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int jj = j0 + u;
+            if (jj >= n2m) break;
+            const double at = jj > 0 ? C(jj - 1) : 0.0;
+            const double ct = jj < n2m - 1 ? A(jj + 1) : 0.0;
+            const double m = 1.0 / (B(jj) - at * cprev);
+            const double vi = zim ? 0.0 : v[u].y;
+            dr = (v[u].x - at * dr) * m;
+            di = (vi - at * di) * m;
+            cprev = ct * m;
+            cp[(size_t)jj * rs] = cprev;
+            d[(size_t)jj * rs] = make_double2(dr, di);
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) v[u] = nv[u];
     }
-    double xr = dr, xi = di;
-    for (int jj = n2m - 2; jj >= 0; jj--) {
-        const double2 v = d[(size_t)jj * rs];
-        const double c_ = cp[(size_t)jj * rs];
-        xr = v.x - c_ * xr;
-        xi = v.y - c_ * xi;
-        d[(size_t)jj * rs] = make_double2(xr, xi);
+    double xr = dr, xi = di, w[U], nw[U];
+#pragma unroll
+    for (int u = 0; u < U; u++)
+        if (n2m - 2 - u >= 0) { v[u] = d[(size_t)(n2m - 2 - u) * rs]; w[u] = cp[(size_t)(n2m - 2 - u) * rs]; }
+    for (int j0 = n2m - 2; j0 >= 0; j0 -= U) {
+#pragma unroll
+        for (int u = 0; u < U; u++)
+            if (j0 - U - u >= 0) { nv[u] = d[(size_t)(j0 - U - u) * rs]; nw[u] = cp[(size_t)(j0 - U - u) * rs]; }
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            const int jj = j0 - u;
+            if (jj < 0) break;
+            xr = v[u].x - w[u] * xr;
+            xi = v[u].y - w[u] * xi;
+            d[(size_t)jj * rs] = make_double2(xr, xi);
+        }
+#pragma unroll
+        for (int u = 0; u < U; u++) { v[u] = nv[u]; w[u] = nw[u]; }
     }
     if (pin) d[0] = make_double2(0.0, d[0].y);
 }
@@ -308,8 +334,8 @@ int stage_adj(tcs_ctx *c, AdjWork *w, const Row &row, int axis, int jlo, bool cy
     TCS_LAUNCH(c->stream, "adj_coef_T", k_coef_T, grd, blk, 0, g, axis, jlo, (int)cyc, am, ap, w->aT, w->cT);
     {
         const LineGeom L = geom(c, axis, jlo);
-        TCS_TRY(ptdma_exact_launch(w->aT + L.off, ac + L.off, w->cT + L.off, w->lam + L.off, L.n0, L.ss0, L.n1, L.ss1,
-                                   L.n_row, L.rs, cyc, c->stream));
+        TCS_TRY(ptdma_exact_launch(w->aT + L.off, ac + L.off, w->cT + L.off, w->lam + L.off, w->lam + L.off, L.n0, L.ss0,
+                                   L.n1, L.ss1, L.n_row, L.rs, cyc, false, c->stream));
     }
     TCS_LAUNCH(c->stream, "adj_row_bars", k_row_bars, grd, blk, 0, g, axis, jlo, (int)cyc, w->lam, X, w->abar, w->bbar,
                w->cbar);
@@ -531,7 +557,7 @@ static int backward(tcs_ctx *c, AdjWork *w, double dt) {
         TCS_TRY(fft_x_fwd_launch(c, "adj_fft_x_fwd", w->rint, spec));
         TCS_TRY(fft_z_launch<-1>(c, "adj_fft_z", spec));
         const int nsys = n3m * h1p;
-        TCS_LAUNCH(c->stream, "adj_poisson_T", k_poisson_tdma_T, dim3((nsys + 255) / 256), dim3(256), 0, n3m, h1p, n2m,
+        TCS_LAUNCH(c->stream, "adj_poisson_T", k_poisson_tdma_T, dim3((nsys + 63) / 64), dim3(64), 0, n3m, h1p, n2m,
                    c->h3p, c->ptab, c->ptab + n2m, c->ptab + 2 * n2m, c->dxk2, c->dzk, spec, c->pC);
         TCS_TRY(fft_z_launch<+1>(c, "adj_fft_z", spec));
         TCS_TRY(fft_x_inv_launch(c, "adj_fft_x_inv", spec, w->tmp[0]));

@@ -19,6 +19,7 @@
 // FFTs are radix-2 Stockham with a host twiddle table, computed in place in
 // LDS with the butterfly outputs staged in registers across barriers.
 #include "ad.h"
+#include "tdma_exact.h"
 #include "tdma_part.h"
 
 #ifndef TCS_FORM
@@ -286,11 +287,17 @@ k_fft_z(int n3m, int h1p, const double2 *__restrict__ tw, double2 *__restrict__ 
 
 // y tridiagonal solves per (kx,kz), PaScaL single-rank order (:599-652).
 // system s = kz + n3m*kx, row j stride n3m*h1p.  amj/apj/acj: 1-D tables.
-__global__ void __launch_bounds__(256)
+// One lane a system, real and imaginary parts as two right-hand sides of
+// one matrix; rows j >= jl of the eliminated form in LDS, the others in pA,
+// pC and the spectrum.
+__global__ void __launch_bounds__(exact_line::EX_W)
 k_poisson_tdma(int n3m, int h1p, int n2m, int h3p, const double *__restrict__ amj, const double *__restrict__ apj,
                const double *__restrict__ acj, const double *__restrict__ dxk2, const double *__restrict__ dzk,
-               double2 *__restrict__ S, double *__restrict__ pA, double *__restrict__ pC) {
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
+               double2 *S, double *pA, double *pC, int jl) {
+    using namespace exact_line;
+    extern __shared__ double lds[];
+    const Kept<2> keep{lds, (int)threadIdx.x};
+    const int s = blockIdx.x * EX_W + threadIdx.x;
     const int nsys = n3m * h1p;
     if (s >= nsys) return;
     const int kx = s / n3m, kz = s - kx * n3m;
@@ -300,79 +307,32 @@ k_poisson_tdma(int n3m, int h1p, int n2m, int h3p, const double *__restrict__ am
     const double shift = dxk2[kx];
     const double zk = dzk[kz];
     const bool pin = (kx == 0 && kz == 0);
-    // row coefficients: A = amj, B = (acj - dxk2) - dzk, C = apj; (1,1,1) pinned
-    auto coef = [&](int jj, double &A, double &B, double &C) {
-        A = amj[jj]; C = apj[jj]; B = acj[jj] - shift - zk;
-        if (pin && jj == 0) { A = 0.0; B = 1.0; C = 0.0; }
-    };
-    double A0, B0, C0, A1, B1, C1;
-    coef(0, A0, B0, C0);
-    coef(1, A1, B1, C1);
-    double2 D0 = d[0], D1 = d[rs];
-    if (pin) D0.x = 0.0;
-    double a0 = A0 / B0;
-    double dr0 = D0.x / B0, di0 = D0.y / B0;
-    double c0 = C0 / B0;
-    const double a1 = A1 / B1;
-    const double dr1 = D1.x / B1, di1 = D1.y / B1;
-    const double c1 = C1 / B1;
-    a[rs] = a1; c[rs] = c1; d[rs] = make_double2(dr1, di1);
-    double ap = a1, cp = c1, drp = dr1, dip = di1;
-    for (int jj = 2; jj < n2m; jj++) {
-        double A, B, C;
-        coef(jj, A, B, C);
-        const double2 Dj = d[(size_t)jj * rs];
-        const double r = 1.0 / (B - A * cp);
-        const double dr = r * (Dj.x - A * drp);
-        const double di = r * (Dj.y - A * dip);
-        const double cn = r * C;
-        const double an = -r * A * ap;
-        a[(size_t)jj * rs] = an; c[(size_t)jj * rs] = cn; d[(size_t)jj * rs] = make_double2(dr, di);
-        ap = an; cp = cn; drp = dr; dip = di;
-    }
-    const double aN = ap, drN = drp, diN = dip;
-    double ax = a1, cx = c1, drx = dr1, dix = di1;
-    if (n2m >= 3) {
-        const size_t o2 = (size_t)(n2m - 2) * rs;
-        ax = a[o2]; cx = c[o2];
-        const double2 v = d[o2];
-        drx = v.x; dix = v.y;
-        for (int jj = n2m - 3; jj >= 1; jj--) {
-            const size_t o = (size_t)jj * rs;
-            const double aj = a[o], cj = c[o];
-            const double2 dj = d[o];
-            const double dr = dj.x - cj * drx;
-            const double di = dj.y - cj * dix;
-            const double an = aj - cj * ax;
-            const double cn = -cj * cx;
-            a[o] = an; c[o] = cn; d[o] = make_double2(dr, di);
-            ax = an; cx = cn; drx = dr; dix = di;
-        }
-    }
-    {
-        const double r = 1.0 / (1.0 - ax * c0);
-        dr0 = r * (dr0 - c0 * drx);
-        di0 = r * (di0 - c0 * dix);
-        a0 = r * a0;
-        c0 = -r * c0 * cx;
-    }
-    const double rr = 1.0 / (1.0 - aN * c0);
-    const double xnr = rr * (drN - aN * dr0);
-    const double xni = rr * (diN - aN * di0);
-    const double x1r = dr0 - c0 * xnr;
-    const double x1i = di0 - c0 * xni;
     // imaginary parts zeroed at kx=0 for kz in {0, h3p-1} (:643-650)
     const bool zim = (kx == 0 && (kz == 0 || kz == h3p - 1));
-    d[0] = make_double2(x1r, zim ? 0.0 : x1i);
-    d[(size_t)(n2m - 1) * rs] = make_double2(xnr, zim ? 0.0 : xni);
-    for (int jj = 1; jj < n2m - 1; jj++) {
-        const size_t o = (size_t)jj * rs;
-        const double aj = a[o], cj = c[o];
-        const double2 dj = d[o];
-        const double vr = dj.x - aj * x1r - cj * xnr;
-        const double vi = dj.y - aj * x1i - cj * xni;
-        d[o] = make_double2(vr, zim ? 0.0 : vi);
-    }
+    solve<false, 2>(
+        n2m,
+        [&](int j) {
+            // A = amj, B = (acj - dxk2) - dzk, C = apj; (1,1,1) pinned
+            const double2 v = d[(size_t)j * rs];
+            Row<2> w{amj[j], acj[j] - shift - zk, apj[j], {v.x, v.y}};
+            if (pin && j == 0) { w.a = 0.0; w.b = 1.0; w.c = 0.0; w.d[0] = 0.0; }
+            return w;
+        },
+        [&](int j, const Elim<2> &e) {
+            if (j >= jl) {
+                keep.put(j - jl, e);
+            } else {
+                const size_t o = (size_t)j * rs;
+                a[o] = e.a; c[o] = e.c; d[o] = make_double2(e.d[0], e.d[1]);
+            }
+        },
+        [&](int j) {
+            if (j >= jl) return keep.get(j - jl);
+            const size_t o = (size_t)j * rs;
+            const double2 v = d[o];
+            return Elim<2>{a[o], c[o], {v.x, v.y}};
+        },
+        [&](int j, const Elim<2> &, const double (&x)[2]) { d[(size_t)j * rs] = make_double2(x[0], zim ? 0.0 : x[1]); });
 }
 
 // The same y solves with split lines (tdma_split): PaScaL_TDMA's multi-rank
@@ -788,8 +748,16 @@ static int poisson_after_x(tcs_ctx *c) {
         TCS_LAUNCH(c->stream, "poisson_part", k_poisson_part, dim3((nsys + PT_SX - 1) / PT_SX), dim3(PT_SX * P), 0,
                    n3m, h1p, c->h3p, c->ptab, c->ptab + n2m, c->ptab + 2 * n2m, c->dxk2, c->dzk, spec, P, w1, w2);
     } else {
-        TCS_LAUNCH(c->stream, "poisson_tdma", k_poisson_tdma, dim3((nsys + 255) / 256), dim3(256), 0, n3m, h1p, n2m,
-                   c->h3p, c->ptab, c->ptab + n2m, c->ptab + 2 * n2m, c->dxk2, c->dzk, spec, c->pA, c->pC);
+        const int kept = exact_line::kept_rows<2>(nsys, n2m), lds = kept * exact_line::Kept<2>::ROW_BYTES;
+        static bool lds_raised = false;  // more than 64 KiB of dynamic LDS (gfx950: 160 KiB per CU)
+        if (!lds_raised) {
+            TCS_HIP(hipFuncSetAttribute((const void *)k_poisson_tdma, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                        exact_line::KEPT_LDS));
+            lds_raised = true;
+        }
+        TCS_LAUNCH(c->stream, "poisson_tdma", k_poisson_tdma, dim3((nsys + exact_line::EX_W - 1) / exact_line::EX_W),
+                   dim3(exact_line::EX_W), lds, n3m, h1p, n2m, c->h3p, c->ptab, c->ptab + n2m, c->ptab + 2 * n2m,
+                   c->dxk2, c->dzk, spec, c->pA, c->pC, n2m - kept);
     }
     TCS_TRY(fft_z_launch<+1>(c, "fft_z<+1>", spec));
     if (SPECTRAL_MEAN)

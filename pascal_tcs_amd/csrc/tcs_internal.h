@@ -234,9 +234,10 @@ inline dim3 cell_grid(int nx, int ny, int nz, int kb, dim3 blk = interior_block(
 
 // TDMA launcher (exact PaScaL order) on strided systems:
 //   system (s0, s1) starts at base + s0*ss0 + s1*ss1, rows step rs.
-int ptdma_exact_launch(double *A, const double *B, double *C, double *D,
-                       int n0, long ss0, int n1, long ss1, int n_row, long rs,
-                       bool cyclic, hipStream_t st);
+// Right-hand sides from Din, solutions to Dout (which may be Din); A and C
+// are overwritten, with keep by the reference's modified coefficients.
+int ptdma_exact_launch(double *A, const double *B, double *C, const double *Din, double *Dout, int n0, long ss0,
+                       int n1, long ss1, int n_row, long rs, bool cyclic, bool keep, hipStream_t st);
 // Where a split solve puts its solution: back into D (mode 0), or into an
 // FP64 field F at F[base + s0*ss0 + s1*ss1 + row*rs], stored (mode 1),
 // added to what F holds (mode 2), or added to what Fin holds at the same
@@ -266,7 +267,7 @@ inline int ptdma_sweep(const tcs_ctx *c, double *A, const double *B, double *C, 
     int P, w1, w2;
     if (c->tdma_split && ptdma_part_plan(n_row, P, w1, w2) && (rs == 1 || ss0 == 1))
         return ptdma_part_launch(A, B, C, D, n0, ss0, n1, ss1, n_row, rs, cyclic, c->stream);
-    return ptdma_exact_launch(A, B, C, D, n0, ss0, n1, ss1, n_row, rs, cyclic, c->stream);
+    return ptdma_exact_launch(A, B, C, D, D, n0, ss0, n1, ss1, n_row, rs, cyclic, false, c->stream);
 }
 // FP32 sweep of the mixed form: always the split solve (lines <= 512 rows).
 inline int ptdma_sweep(const tcs_ctx *c, float *A, const float *B, float *C, float *D, int n0, long ss0, int n1,

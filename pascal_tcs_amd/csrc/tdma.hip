@@ -2,293 +2,220 @@
 // operation order (PaScaL_TDMA/src/pascal_tdma.f90:487-578 and :715-806,
 // reduced 2-row solves of PaScaL_TDMA/src/tdmas.f90:113-212).
 //
-// One thread owns one system and walks its rows; consecutive threads own
-// systems that are adjacent in memory wherever the caller's layout allows
-// (the z and y sweeps of a field), so every row step is one coalesced
-// 512-byte wavefront access per array.  The three passes of the modified
-// Thomas algorithm (forward elimination with A fill-in, backward elimination
-// with C fill-in, update from the reduced solution) keep their operands in
-// place, exactly as the reference does with its A, C, D arrays.
-#include "tcs_internal.h"
+// The kernels here move rows between memory and the one-lane lines of
+// tdma_exact.h.
+#include "tdma_exact.h"
 
 #include <mutex>
 
 namespace tcs {
 
-template <bool CYC>
-__global__ void __launch_bounds__(256)
-k_ptdma_exact(double *__restrict__ A, const double *__restrict__ B, double *__restrict__ C,
-              double *__restrict__ D, int n0, long ss0, long ss1, int n_row, long rs) {
-    const int s0 = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s0 >= n0) return;
-    const long base = (long)s0 * ss0 + (long)blockIdx.y * ss1;
-    double *a = A + base;
-    const double *b = B + base;
-    double *c = C + base;
-    double *d = D + base;
+namespace {
 
-    // rows 1 and 2 normalised by their own diagonal (:503-511)
-    const double b0 = b[0], b1 = b[rs];
-    double a0 = a[0] / b0;
-    double d0 = d[0] / b0;
-    double c0 = c[0] / b0;
-    const double a1 = a[rs] / b1;
-    const double d1 = d[rs] / b1;
-    const double c1 = c[rs] / b1;
-    a[rs] = a1; d[rs] = d1; c[rs] = c1;
+using namespace exact_line;
 
-    // forward elimination j = 3..n_row (:513-520)
-    double ap = a1, cp = c1, dp = d1;
-    for (int j = 2; j < n_row; j++) {
-        const long o = (long)j * rs;
-        const double aj = a[o], bj = b[o], cj = c[o], dj = d[o];
-        const double r = 1.0 / (bj - aj * cp);
-        const double dn = r * (dj - aj * dp);
-        const double cn = r * cj;
-        const double an = -r * aj * ap;
-        a[o] = an; c[o] = cn; d[o] = dn;
-        ap = an; cp = cn; dp = dn;
-    }
-    const double aN = ap, cN = cp, dN = dp;  // last row (forward values)
-
-    // backward elimination j = n_row-2..2 (:523-529)
-    double ax = a1, cx = c1, dx = d1;  // row 2 after the backward sweep
-    if (n_row >= 3) {
-        const long o2 = (long)(n_row - 2) * rs;
-        ax = a[o2]; cx = c[o2]; dx = d[o2];
-        for (int j = n_row - 3; j >= 1; j--) {
+// Lines strided in memory: line l = s0 + n0*s1 starts at s0*ss0 + s1*ss1,
+// rows rs apart.  A, C and Dout also hold the eliminated rows j < jl (the
+// rows j >= jl are kept in LDS); KEEP: A and C come back as the reference
+// leaves them.
+template <bool CYC, bool KEEP>
+__global__ void __launch_bounds__(EX_W)
+k_ptdma_exact(double *A, const double *B, double *C, const double *Din, double *Dout, int n0, long ss0, long ss1,
+              long lines, int n_row, long rs, int jl) {
+    extern __shared__ double lds[];
+    const Kept<1> keep{lds, (int)threadIdx.x};
+    const long line = (long)blockIdx.x * EX_W + threadIdx.x;
+    if (line >= lines) return;  // no barrier below: a lane reads only what it wrote
+    const long s1 = line / n0, base = (line - s1 * n0) * ss0 + s1 * ss1;
+    double *a = A + base, *c = C + base, *d = Dout + base;
+    const double *b = B + base, *din = Din + base;
+    solve<CYC, 1>(
+        n_row,
+        [&](int j) {
             const long o = (long)j * rs;
-            const double aj = a[o], cj = c[o], dj = d[o];
-            const double dn = dj - cj * dx;
-            const double an = aj - cj * ax;
-            const double cn = -cj * cx;
-            a[o] = an; c[o] = cn; d[o] = dn;
-            ax = an; cx = cn; dx = dn;
-        }
-    }
-
-    // row 1 and the reduced 2-row system (:531-542)
-    {
-        const double r = 1.0 / (1.0 - ax * c0);
-        d0 = r * (d0 - c0 * dx);
-        a0 = r * a0;
-        c0 = -r * c0 * cx;
-    }
-    a[0] = a0; c[0] = c0;
-
-    double x1, xn;
-    if (!CYC) {
-        // tdma_many with n2=2, b=1 (tdmas.f90:113-146); x/1.0 is exact
-        const double r = 1.0 / (1.0 - aN * c0);
-        xn = r * (dN - aN * d0);
-        x1 = d0 - c0 * xn;
-    } else {
-        // tdma_cycl_many with n2=2 (tdmas.f90:159-212): e(2) is set to -a(2)
-        // and then overwritten by e(n2) = -c(n2)
-        const double e2 = -cN;
-        x1 = (d0 - a0 * dN - c0 * dN) / (1.0 + a0 * e2 + c0 * e2);
-        xn = dN + x1 * e2;
-    }
-    d[0] = x1;
-    d[(long)(n_row - 1) * rs] = xn;
-
-    // update of the inner rows (:572-576)
-    for (int j = 1; j < n_row - 1; j++) {
-        const long o = (long)j * rs;
-        d[o] = d[o] - a[o] * x1 - c[o] * xn;
-    }
+            return Row<1>{a[o], b[o], c[o], {din[o]}};
+        },
+        [&](int j, const Elim<1> &e) {
+            if (j >= jl) {
+                keep.put(j - jl, e);
+            } else {
+                const long o = (long)j * rs;
+                a[o] = e.a; c[o] = e.c; d[o] = e.d[0];
+            }
+        },
+        [&](int j) {
+            if (j >= jl) return keep.get(j - jl);
+            const long o = (long)j * rs;
+            return Elim<1>{a[o], c[o], {d[o]}};
+        },
+        [&](int j, const Elim<1> &e, const double (&x)[1]) {
+            const long o = (long)j * rs;
+            d[o] = x[0];
+            if constexpr (KEEP) { a[o] = e.a; c[o] = e.c; }
+        });
 }
 
 // Systems whose rows are contiguous in memory (the x sweep of an (i,j,k)
-// array): one wavefront owns 64 systems and streams their rows through LDS
-// in chunks of ROWS_R, so every global access is a coalesced run of
-// ROWS_R doubles per line while each lane still walks its own system row by
-// row in the reference's order.  LDS rows are padded to ROWS_R+1 doubles.
-constexpr int ROWS_R = 16;
-constexpr int ROWS_P = ROWS_R + 1;
-
-// tile slot a holds array a of {A, B, C, D}; MASK selects the arrays moved
-template <int MASK>
-__device__ __forceinline__ void rows_load(double (*tile)[64 * ROWS_P], double *A, double *B, double *C, double *D,
-                                          long lbase0, long ss0, int nlines, int r0, int nr) {
-    const int t = threadIdx.x;
-    double *const src[4] = {A, B, C, D};
-    for (int q = 0; q < ROWS_R; q++) {
-        const int idx = q * 64 + t;
-        const int l = idx / ROWS_R, rr = idx - l * ROWS_R;
-        if (l < nlines && rr < nr) {
-            const long g = lbase0 + (long)l * ss0 + r0 + rr;
+// array): line (s0, s1) starts at s0*ss0 + s1*ss1.  The rows come in chunks
+// of EX_R of the workgroup's 64 lines, loaded along the lines (128-byte
+// segments) one chunk ahead and turned through LDS, so each lane still walks
+// its own line.  The eliminated rows of a chunk go back to the chunk's own
+// memory in the order of the lanes (lane l of row r is value r*64 + l of the
+// chunk), where the backward passes read them without turning; only the
+// solution (and with KEEP a and c) is turned back.
+template <bool CYC, bool KEEP>
+__global__ void __launch_bounds__(EX_W)
+k_ptdma_exact_rows(double *A, const double *B, double *C, const double *Din, double *Dout, int n0, long ss0,
+                   long ss1, int n_row) {
+    constexpr int P = EX_R + 1;  // padded row of the tile
+    __shared__ double tile[4][EX_W * P];
+    const int lane = threadIdx.x;
+    const int s0a = blockIdx.x * EX_W;
+    const int nl = min(EX_W, n0 - s0a);  // lines here
+    const long lb = (long)s0a * ss0 + (long)blockIdx.y * ss1;
+    const bool act = lane < nl;
+    const int nch = (n_row + EX_R - 1) / EX_R;
+    double *TA = tile[0] + lane * P, *TB = tile[1] + lane * P, *TC = tile[2] + lane * P, *TD = tile[3] + lane * P;
+    const int ql = lane / EX_R, qr = lane % EX_R;  // along the lines: line 4q + ql, row qr of the chunk
+    // value (r, lane) of the chunk at row r0 with nr rows
+    auto spot = [&](int r0, int nr, int r) {
+        if (nl == EX_W && nr == EX_R) return lb + (long)(r * 4 + ql) * ss0 + r0 + qr;
+        const int v = r * nl + lane;
+        return lb + (long)(v / nr) * ss0 + r0 + v % nr;
+    };
+    double va[EX_R], vb[EX_R], vc[EX_R], vd[EX_R];
+    auto fetch = [&](int ch) {  // a chunk's rows into registers, along the lines
+        const int r0 = ch * EX_R;
 #pragma unroll
-            for (int a = 0; a < 4; a++)
-                if (MASK & (1 << a)) tile[a][l * ROWS_P + rr] = src[a][g];
+        for (int q = 0; q < EX_R; q++) {
+            const int l = q * 4 + ql;
+            if (l < nl && r0 + qr < n_row) {
+                const long o = lb + (long)l * ss0 + r0 + qr;
+                va[q] = A[o]; vb[q] = B[o]; vc[q] = C[o]; vd[q] = Din[o];
+            }
         }
-    }
-}
-
-// stores tile rows [lo, hi) of the chunk starting at global row r0
-template <int MASK>
-__device__ __forceinline__ void rows_store(double (*tile)[64 * ROWS_P], double *A, double *B, double *C, double *D,
-                                           long lbase0, long ss0, int nlines, int r0, int lo, int hi) {
-    const int t = threadIdx.x;
-    double *const dst[4] = {A, B, C, D};
-    for (int q = 0; q < ROWS_R; q++) {
-        const int idx = q * 64 + t;
-        const int l = idx / ROWS_R, rr = idx - l * ROWS_R;
-        if (l < nlines && rr >= lo && rr < hi) {
-            const long g = lbase0 + (long)l * ss0 + r0 + rr;
-#pragma unroll
-            for (int a = 0; a < 4; a++)
-                if (MASK & (1 << a)) dst[a][g] = tile[a][l * ROWS_P + rr];
-        }
-    }
-}
-
-constexpr int M_ABCD = 15, M_ACD = 13, M_D = 8;
-
-template <bool CYC>
-__global__ void __launch_bounds__(64)
-k_ptdma_rows(double *__restrict__ A, double *__restrict__ B, double *__restrict__ C, double *__restrict__ D,
-             int n0, long ss0, long ss1, int n_row) {
-    __shared__ double tile[4][64 * ROWS_P];
-    const int t = threadIdx.x;
-    const int s0a = blockIdx.x * 64;
-    const int nlines = min(64, n0 - s0a);
-    const long lbase0 = (long)s0a * ss0 + (long)blockIdx.y * ss1;
-    const bool active = t < nlines;
-    double *TA = tile[0] + t * ROWS_P;
-    double *TB = tile[1] + t * ROWS_P;
-    double *TC = tile[2] + t * ROWS_P;
-    double *TD = tile[3] + t * ROWS_P;
-    const int nch = (n_row + ROWS_R - 1) / ROWS_R;
-
-    // forward elimination (rows 1,2 normalised; j = 3..n_row)
-    double a0 = 0, c0 = 0, d0 = 0, a1 = 0, c1 = 0, d1 = 0;
-    double ap = 0, cp = 0, dp = 0;
+    };
+    Elim<1> e0{}, e1{}, p{}, pp{};
+    fetch(0);
     for (int ch = 0; ch < nch; ch++) {
-        const int r0 = ch * ROWS_R, nr = min(ROWS_R, n_row - r0);
-        rows_load<M_ABCD>(tile, A, B, C, D, lbase0, ss0, nlines, r0, nr);
+        const int r0 = ch * EX_R, nr = min(EX_R, n_row - r0);
+#pragma unroll
+        for (int q = 0; q < EX_R; q++) {
+            const int o = (q * 4 + ql) * P + qr;
+            tile[0][o] = va[q]; tile[1][o] = vb[q]; tile[2][o] = vc[q]; tile[3][o] = vd[q];
+        }
         __syncthreads();
-        if (active) {
-            for (int rr = 0; rr < nr; rr++) {
-                const int j = r0 + rr;
-                const double aj = TA[rr], bj = TB[rr], cj = TC[rr], dj = TD[rr];
-                if (j == 0) {
-                    a0 = aj / bj; d0 = dj / bj; c0 = cj / bj;
-                } else if (j == 1) {
-                    a1 = aj / bj; d1 = dj / bj; c1 = cj / bj;
-                    TA[rr] = a1; TC[rr] = c1; TD[rr] = d1;
-                    ap = a1; cp = c1; dp = d1;
+        if (ch + 1 < nch) fetch(ch + 1);
+        if (act) {
+            auto row = [&](int r) {
+                const int j = r0 + r;
+                const Row<1> w{TA[r], TB[r], TC[r], {TD[r]}};
+                pp = p;
+                if (j >= 2) {
+                    p = fwd_row<1>(w, p);
                 } else {
-                    const double r = 1.0 / (bj - aj * cp);
-                    const double dn = r * (dj - aj * dp);
-                    const double cn = r * cj;
-                    const double an = -r * aj * ap;
-                    TA[rr] = an; TC[rr] = cn; TD[rr] = dn;
-                    ap = an; cp = cn; dp = dn;
+                    p = first_row<1>(w);
+                    if (j == 0) e0 = p;
+                    else e1 = p;
                 }
+                const long o = spot(r0, nr, r);
+                A[o] = p.a; C[o] = p.c; Dout[o] = p.d[0];
+            };
+            if (nr == EX_R) {
+#pragma unroll
+                for (int r = 0; r < EX_R; r++) row(r);
+            } else {
+                for (int r = 0; r < nr; r++) row(r);
             }
         }
         __syncthreads();
-        // row 0 is written back after the row-1 fix-up; keep its input bits here
-        rows_store<M_ACD>(tile, A, B, C, D, lbase0, ss0, nlines, r0, ch == 0 ? 1 : 0, nr);
-        __syncthreads();
     }
-    (void)a0;
-    const double aN = ap, cN = cp, dN = dp;
+    const Elim<1> eN = p, eT = n_row >= 3 ? pp : e1;
 
-    // backward elimination j = n_row-2..2 (1-based)
-    double ax = a1, cx = c1, dx = d1;
-    if (n_row >= 3) {
-        const int jtop = n_row - 2;  // 0-based row whose forward values seed the sweep
-        for (int ch = jtop / ROWS_R; ch >= 0; ch--) {
-            const int r0 = ch * ROWS_R, nr = min(ROWS_R, n_row - r0);
-            rows_load<M_ACD>(tile, A, B, C, D, lbase0, ss0, nlines, r0, nr);
-            __syncthreads();
-            if (active) {
-                const int hi = min(r0 + nr - 1, jtop);
-                for (int j = hi; j >= max(r0, 1); j--) {
-                    const int rr = j - r0;
-                    if (j == jtop) {
-                        ax = TA[rr]; cx = TC[rr]; dx = TD[rr];
-                        continue;
+    double x1[1] = {0.0}, xn[1] = {0.0};
+    auto backward = [&](auto out) {
+        constexpr bool OUT = decltype(out)::value;
+        Elim<1> x = eT, q[EX_R];
+        auto get = [&](int ch) {
+            const int r0 = ch * EX_R, nr = min(EX_R, n_row - r0);
+#pragma unroll
+            for (int r = 0; r < EX_R; r++)
+                if (act && r < nr) {
+                    const long o = spot(r0, nr, r);
+                    q[r].a = A[o]; q[r].c = C[o]; q[r].d[0] = Dout[o];
+                }
+        };
+        get(nch - 1);
+        for (int ch = nch - 1; ch >= 0; ch--) {
+            const int r0 = ch * EX_R, nr = min(EX_R, n_row - r0);
+            Elim<1> w[EX_R];
+#pragma unroll
+            for (int r = 0; r < EX_R; r++) w[r] = q[r];
+            if (ch > 0) get(ch - 1);
+#pragma unroll
+            for (int r = EX_R - 1; r >= 0; r--) {
+                const int j = r0 + r;
+                if (r >= nr) continue;
+                if (j >= 1 && j <= n_row - 3) x = back_row<1>(w[r], x);
+                if constexpr (OUT) {
+                    double v = x.d[0] - x.a * x1[0] - x.c * xn[0], ka = x.a, kc = x.c;
+                    if (j == n_row - 1) { v = xn[0]; ka = eN.a; kc = eN.c; }
+                    if (j == 0) { v = x1[0]; ka = e0.a; kc = e0.c; }
+                    TD[r] = v;
+                    if constexpr (KEEP) { TA[r] = ka; TC[r] = kc; }
+                }
+            }
+            if constexpr (OUT) {
+                // every lane has its own rows of this chunk in registers before
+                // the solution takes their place in memory
+                __syncthreads();
+#pragma unroll
+                for (int u = 0; u < EX_R; u++) {
+                    const int l = u * 4 + ql, o = l * P + qr;
+                    if (l < nl && qr < nr) {
+                        const long t = lb + (long)l * ss0 + r0 + qr;
+                        Dout[t] = tile[3][o];
+                        if constexpr (KEEP) { A[t] = tile[0][o]; C[t] = tile[2][o]; }
                     }
-                    const double aj = TA[rr], cj = TC[rr], dj = TD[rr];
-                    const double dn = dj - cj * dx;
-                    const double an = aj - cj * ax;
-                    const double cn = -cj * cx;
-                    TA[rr] = an; TC[rr] = cn; TD[rr] = dn;
-                    ax = an; cx = cn; dx = dn;
                 }
-            }
-            __syncthreads();
-            rows_store<M_ACD>(tile, A, B, C, D, lbase0, ss0, nlines, r0, ch == 0 ? 1 : 0, nr);
-            __syncthreads();
-        }
-    }
-
-    // row 1 fix-up and the reduced 2-row system
-    double x1 = 0, xn = 0;
-    {
-        const double r = 1.0 / (1.0 - ax * c0);
-        d0 = r * (d0 - c0 * dx);
-        a0 = r * a0;
-        c0 = -r * c0 * cx;
-    }
-    if (!CYC) {
-        const double r = 1.0 / (1.0 - aN * c0);
-        xn = r * (dN - aN * d0);
-        x1 = d0 - c0 * xn;
-    } else {
-        const double e2 = -cN;
-        x1 = (d0 - a0 * dN - c0 * dN) / (1.0 + a0 * e2 + c0 * e2);
-        xn = dN + x1 * e2;
-    }
-
-    // update pass: rows 2..n_row-1 (1-based), rows 1 and n_row from the reduced solve
-    for (int ch = 0; ch < nch; ch++) {
-        const int r0 = ch * ROWS_R, nr = min(ROWS_R, n_row - r0);
-        rows_load<M_ACD>(tile, A, B, C, D, lbase0, ss0, nlines, r0, nr);
-        __syncthreads();
-        if (active) {
-            for (int rr = 0; rr < nr; rr++) {
-                const int j = r0 + rr;
-                if (j == 0) {
-                    TA[rr] = a0; TC[rr] = c0; TD[rr] = x1;
-                } else if (j == n_row - 1) {
-                    TD[rr] = xn;
-                } else {
-                    TD[rr] = TD[rr] - TA[rr] * x1 - TC[rr] * xn;
-                }
+                __syncthreads();
             }
         }
-        __syncthreads();
-        if (ch == 0) rows_store<M_ACD>(tile, A, B, C, D, lbase0, ss0, nlines, r0, 0, 1);  // row 1: A, C, D
-        rows_store<M_D>(tile, A, B, C, D, lbase0, ss0, nlines, r0, ch == 0 ? 1 : 0, nr);
-        __syncthreads();
-    }
+        return x;
+    };
+    const Elim<1> x2 = backward(std::integral_constant<bool, false>());
+    line_ends<CYC, 1>(e0, x2, eN, x1, xn);
+    backward(std::integral_constant<bool, true>());
 }
 
-int ptdma_exact_launch(double *A, const double *B, double *C, double *D,
-                       int n0, long ss0, int n1, long ss1, int n_row, long rs,
-                       bool cyclic, hipStream_t st) {
+}  // namespace
+
+int ptdma_exact_launch(double *A, const double *B, double *C, const double *Din, double *Dout, int n0, long ss0,
+                       int n1, long ss1, int n_row, long rs, bool cyclic, bool keep, hipStream_t st) {
     if (n0 <= 0 || n1 <= 0) return TCS_OK;
     if (n_row < 2 || n1 > 65535) {
         set_error("ptdma: n_row must be >= 2 and the outer system count <= 65535");
         return TCS_E_ARG;
     }
-    if (rs == 1 && n_row >= 2) {
-        dim3 rblk(64), rgrd((unsigned)((n0 + 63) / 64), (unsigned)n1);
-        if (cyclic)
-            TCS_LAUNCH(st, "ptdma_rows_cyclic", k_ptdma_rows<true>, rgrd, rblk, 0, A, (double *)B, C, D, n0, ss0, ss1, n_row);
-        else
-            TCS_LAUNCH(st, "ptdma_rows", k_ptdma_rows<false>, rgrd, rblk, 0, A, (double *)B, C, D, n0, ss0, ss1, n_row);
+#define EXACT_PICK(kern) \
+    (cyclic ? (keep ? kern<true, true> : kern<true, false>) : (keep ? kern<false, true> : kern<false, false>))
+    if (rs == 1) {
+        const dim3 grd((unsigned)((n0 + EX_W - 1) / EX_W), (unsigned)n1);
+        TCS_LAUNCH(st, cyclic ? "ptdma_rows_cyclic" : "ptdma_rows", EXACT_PICK(k_ptdma_exact_rows), grd, dim3(EX_W),
+                   0, A, B, C, Din, Dout, n0, ss0, ss1, n_row);
         return TCS_OK;
     }
-    dim3 blk(256), grd((unsigned)((n0 + 255) / 256), (unsigned)n1);
-    if (cyclic)
-        TCS_LAUNCH(st, "ptdma_cyclic", k_ptdma_exact<true>, grd, blk, 0, A, B, C, D, n0, ss0, ss1, n_row, rs);
-    else
-        TCS_LAUNCH(st, "ptdma", k_ptdma_exact<false>, grd, blk, 0, A, B, C, D, n0, ss0, ss1, n_row, rs);
+    const long lines = (long)n0 * n1;
+    const int kept = kept_rows<1>(lines, n_row), lds = kept * Kept<1>::ROW_BYTES;
+    const auto kern = EXACT_PICK(k_ptdma_exact);
+    static bool raised[4];  // more than 64 KiB of dynamic LDS (gfx950: 160 KiB per CU)
+    if (!raised[2 * cyclic + keep]) {
+        TCS_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, KEPT_LDS));
+        raised[2 * cyclic + keep] = true;
+    }
+    TCS_LAUNCH(st, cyclic ? "ptdma_cyclic" : "ptdma", kern, dim3((unsigned)((lines + EX_W - 1) / EX_W)), dim3(EX_W),
+               lds, A, B, C, Din, Dout, n0, ss0, ss1, lines, n_row, rs, n_row - kept);
+#undef EXACT_PICK
     return TCS_OK;
 }
 
@@ -302,20 +229,10 @@ static int many_solve(double *A, const double *B, double *C, double *D, int32_t 
         set_error("ptdma_many_solve: null pointer or n_row < 2");
         return TCS_E_ARG;
     }
-    // (n_sys, n_row): systems contiguous; split n_sys into (n0 = chunk) x n1
-    // so the outer count stays within the grid's y limit.
-    const int chunk = 65536;
-    int n0 = n_sys < chunk ? n_sys : chunk;
-    int n1 = (n_sys + chunk - 1) / chunk;
-    if (n_sys % n0 != 0) {
-        // ragged tail: two launches
-        int full = n_sys / n0;
-        TCS_TRY(ptdma_exact_launch(A, B, C, D, n0, 1, full, n0, n_row, n_sys, cyc, (hipStream_t)stream));
-        long off = (long)full * n0;
-        return ptdma_exact_launch(A + off, B + off, C + off, D + off, n_sys - (int)off, 1, 1, 0, n_row,
-                                  n_sys, cyc, (hipStream_t)stream);
-    }
-    return ptdma_exact_launch(A, B, C, D, n0, 1, n1, n0, n_row, n_sys, cyc, (hipStream_t)stream);
+    // (n_sys, n_row): the systems adjacent, their rows n_sys apart
+    if (n_sys == 1)  // one system: its rows are contiguous
+        return ptdma_exact_launch(A, B, C, D, D, 1, 1, 1, 0, n_row, 1, cyc, true, (hipStream_t)stream);
+    return ptdma_exact_launch(A, B, C, D, D, n_sys, 1, 1, 0, n_row, n_sys, cyc, true, (hipStream_t)stream);
 }
 
 extern "C" int ptdma_many_solve_dev(double *A, const double *B, double *C, double *D, int32_t n_sys,
@@ -446,10 +363,10 @@ extern "C" int ptdma_axis_solve_dev(double *A, const double *B, double *C, doubl
     long s1 = n1, s2 = (long)n1 * n2;
     switch (axis) {
     case 0:  // rows along i: systems (j,k)
-        return ptdma_exact_launch(A, B, C, D, n2, s1, n3, s2, n1, 1, cyclic != 0, st);
+        return ptdma_exact_launch(A, B, C, D, D, n2, s1, n3, s2, n1, 1, cyclic != 0, true, st);
     case 1:  // rows along j: systems (i,k)
-        return ptdma_exact_launch(A, B, C, D, n1, 1, n3, s2, n2, s1, cyclic != 0, st);
+        return ptdma_exact_launch(A, B, C, D, D, n1, 1, n3, s2, n2, s1, cyclic != 0, true, st);
     default:  // rows along k: systems (i,j)
-        return ptdma_exact_launch(A, B, C, D, n1, 1, n2, s1, n3, s2, cyclic != 0, st);
+        return ptdma_exact_launch(A, B, C, D, D, n1, 1, n2, s1, n3, s2, cyclic != 0, true, st);
     }
 }
