@@ -227,7 +227,7 @@ struct RhsCell {
 
 // x r2c: TX k-lines (k0..k0+TX-1) of row j per workgroup.
 // spec[(k + n3m*(kx + h1p*(j-1)))] complex, k 0-based.
-template <int NT, class Src>
+template <int NT, int MB, class Src>
 __global__ void __launch_bounds__(NT)
 k_fft_x_fwd(Grid g, int h1p, int TX, Src src, const double2 *__restrict__ tw, double2 *__restrict__ spec) {
     extern __shared__ double lds[];
@@ -260,7 +260,7 @@ k_fft_x_fwd(Grid g, int h1p, int TX, Src src, const double2 *__restrict__ tw, do
         }
     }
     __syncthreads();
-    lds_fft<-1, NT, FFT_MAXB_FWD>(re, im, n, TX, tw);
+    lds_fft<-1, NT, MB>(re, im, n, TX, tw);
     const size_t rowbase = (size_t)g.n3m * h1p * (j - 1);
     for (int e = tid; e < TX * h1p; e += NT) {
         const int kx = e / TX, l = e - kx * TX;
@@ -678,8 +678,13 @@ template <class Src>
 static int fft_x_fwd_src_launch(tcs_ctx *c, const char *label, const Src &src, double2 *spec) {
     const int TX = fft_tile(c->n1m, c->n3m, FFT_MAXB_FWD);
     const size_t lds = (size_t)fft_lds_len(TX * c->n1m) * 2 * sizeof(double);
-    TCS_LAUNCH(c->stream, label, (k_fft_x_fwd<FFT_X_THREADS, Src>), dim3(c->n3m / TX, c->n2m), dim3(FFT_X_THREADS),
-               lds, c->grid(), c->h1p, TX, src, (const double2 *)c->tw1, spec);
+    const dim3 grd(c->n3m / TX, c->n2m), blk(FFT_X_THREADS);
+    if (c->n1m > 2 * FFT_MAXB_FWD * FFT_X_THREADS)  // 4096 points: twice the butterflies a thread
+        TCS_LAUNCH(c->stream, label, (k_fft_x_fwd<FFT_X_THREADS, FFT_MAXB, Src>), grd, blk, lds, c->grid(), c->h1p, TX,
+                   src, (const double2 *)c->tw1, spec);
+    else
+        TCS_LAUNCH(c->stream, label, (k_fft_x_fwd<FFT_X_THREADS, FFT_MAXB_FWD, Src>), grd, blk, lds, c->grid(), c->h1p,
+                   TX, src, (const double2 *)c->tw1, spec);
     return TCS_OK;
 }
 static int fft_x_fwd_launch(tcs_ctx *c, const char *label, const double *in, double2 *spec) {
