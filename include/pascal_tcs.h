@@ -47,9 +47,12 @@ typedef struct tcs_params {
                                      2: mixed, FP32 stage rows, line solves and
                                         increments, FP64 state and pressure */
     int32_t tdma_split;           /* 0: every ADI line solved as on one rank;
-                                     1: lines of up to 512 rows split into
+                                     1: lines of up to 512 rows (precision 1:
+                                     ADI lines of up to 2048) split into
                                      parts as PaScaL_TDMA splits them over
-                                     ranks (see ptdma_many_solve_part_dev) */
+                                     ranks (see ptdma_many_solve_part_dev;
+                                     precision 1 and 2 choose the parts by
+                                     the number of lines) */
     double Ct, Cmu, Cmt, Cmp;     /* :139-141 */
     double DeltaT;                /* namelist sim_parameter */
     double a10, a11, a12, a13, a14, a15;  /* density polynomial   :117 */

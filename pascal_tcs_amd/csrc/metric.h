@@ -9,6 +9,14 @@
 #include <type_traits>
 
 //
+// Whether the form's split lines may be split in any way (part_plan_any); the
+// exact form's splits are the oracle's.
+#ifdef TCS_RECIP
+constexpr bool ANY_SPLIT = true;
+#else
+constexpr bool ANY_SPLIT = false;
+#endif
+//
 // sc<S>(x): a constant of the formulas (a literal, a physical constant, dt,
 // a mask) in the arithmetic of S: float for S = float, else the double
 // itself (also in the reverse pass).

@@ -971,13 +971,14 @@ static int launch_stale(tcs_ctx *c) {
 // when all n2m rows fit a split line (dV y at 512^3: 1.56 -> 1.0 ms, whole
 // 16-row parts and the unconditional row loop); dV's wall row is zero
 // either way.
-template <int SX, class Row>
+template <int SX, bool LEAD = false, class Row>
 static int y_stage(tcs_ctx *c, const char *label_rows, const char *label_solve, const Row &row, int jlo, double *F) {
     scr_t *am = SCR(c->am), *ac = SCR(c->ac), *ap = SCR(c->ap), *rhs = SCR(c->rhs);
     const int nrows = c->n2m - jlo + 1;
-    if (jlo == 2 && rows_in_solve<scr_t>(c, c->n2m))
-        return y_stage_in_solve<SX>(c, label_solve, row, 1, c->n2m, rhs, F, 1, jlo);
-    if (rows_in_solve<scr_t>(c, nrows)) return y_stage_in_solve<SX>(c, label_solve, row, jlo, nrows, rhs, F, 1);
+    if constexpr (LEAD)
+        if (rows_in_solve<scr_t, ANY_SPLIT>(c, c->n2m))
+            return y_stage_in_solve<ANY_SPLIT, SX, true>(c, label_solve, row, 1, c->n2m, rhs, F, 1, jlo);
+    if (rows_in_solve<scr_t, ANY_SPLIT>(c, nrows)) return y_stage_in_solve<ANY_SPLIT, SX>(c, label_solve, row, jlo, nrows, rhs, F, 1);
     TCS_TRY(rows3d_launch<false>(c, label_rows, row, jlo, am, ac, ap, rhs));
     return sweep_y_field(c, jlo, nrows, F, 1);
 }
@@ -989,8 +990,8 @@ int momentum_solvedU(tcs_ctx *c, double dt) {
     scr_t *am = SCR(c->am), *ac = SCR(c->ac), *ap = SCR(c->ap), *rhs = SCR(c->rhs);
     const DUZ z{g, c->phys, dt, f[TCS_U], f[TCS_V], f[TCS_W], f[TCS_P], f[TCS_T], f[TCS_MU], f[TCS_INVRHO],
                 c->wall[TCS_UBCUP], c->wall[TCS_UBCBT], c->wall[TCS_VBCUP], c->wall[TCS_VBCBT]};
-    TCS_TRY(z_stage(c, "dU_z", "dU_z_solve", z, 1, am, ac, ap, rhs));
-    TCS_TRY(x_stage(c, "dU_x", "dU_x_solve", DUX{g, c->phys, dt, f[TCS_U], f[TCS_MU], f[TCS_INVRHO]}, 1, am, ac, ap,
+    TCS_TRY(z_stage<ANY_SPLIT>(c, "dU_z", "dU_z_solve", z, 1, am, ac, ap, rhs));
+    TCS_TRY(x_stage<ANY_SPLIT>(c, "dU_x", "dU_x_solve", DUX{g, c->phys, dt, f[TCS_U], f[TCS_MU], f[TCS_INVRHO]}, 1, am, ac, ap,
                     rhs));
     return y_stage<sizeof(scr_t) == 8 ? 8 : 16>(c, "dU_y", "dU_y_solve", DUY{g, c->phys, dt, f[TCS_V], f[TCS_MU], f[TCS_INVRHO]}, 1, f[TCS_DU]);
 }
@@ -1004,12 +1005,12 @@ int momentum_solvedV(tcs_ctx *c, double dt) {
     // rows j = 1 are not part of the dV systems: every stage covers j = 2..n2m
     const DVZ z{g, c->phys, dt, f[TCS_U], f[TCS_V], f[TCS_W], f[TCS_P], f[TCS_DU], f[TCS_MU], f[TCS_INVRHO],
                 c->wall[TCS_VBCUP], c->wall[TCS_VBCBT]};
-    TCS_TRY(z_stage(c, "dV_z", "dV_z_solve", z, 2, am, ac, ap, rhs));
-    TCS_TRY(x_stage(c, "dV_x", "dV_x_solve", DVX{g, c->phys, dt, f[TCS_U], f[TCS_INVRHO], c->stale}, 2, am, ac, ap,
+    TCS_TRY(z_stage<ANY_SPLIT>(c, "dV_z", "dV_z_solve", z, 2, am, ac, ap, rhs));
+    TCS_TRY(x_stage<ANY_SPLIT>(c, "dV_x", "dV_x_solve", DVX{g, c->phys, dt, f[TCS_U], f[TCS_INVRHO], c->stale}, 2, am, ac, ap,
                     rhs));
     TCS_LAUNCH(c->stream, "dV_zero_rows", k_dV_zero_rows<inc_t>, dim3((c->N1 + 63) / 64, c->N3), dim3(64), 0, g,
                inc(c, TCS_DV));
-    return y_stage<sizeof(scr_t) == 8 ? 8 : 16>(c, "dV_y", "dV_y_solve", DVY{g, c->phys, dt, f[TCS_V], f[TCS_MU], f[TCS_INVRHO]}, 2, f[TCS_DV]);
+    return y_stage<sizeof(scr_t) == 8 ? 8 : 16, true>(c, "dV_y", "dV_y_solve", DVY{g, c->phys, dt, f[TCS_V], f[TCS_MU], f[TCS_INVRHO]}, 2, f[TCS_DV]);
 }
 
 int momentum_solvedW(tcs_ctx *c, double dt) {
@@ -1020,8 +1021,8 @@ int momentum_solvedW(tcs_ctx *c, double dt) {
     TCS_TRY(ensure_twins(c, MOMENTUM_TWINS | TWIN_STALE));
     const DWZ z{g, c->phys, dt, f[TCS_U], f[TCS_V], f[TCS_W], f[TCS_P], f[TCS_DU], f[TCS_DV], f[TCS_MU],
                 f[TCS_INVRHO], c->wall[TCS_VBCUP], c->wall[TCS_VBCBT], c->wall[TCS_WBCUP], c->wall[TCS_WBCBT]};
-    TCS_TRY(z_stage(c, "dW_z", "dW_z_solve", z, 1, am, ac, ap, rhs));
-    TCS_TRY(x_stage(c, "dW_x", "dW_x_solve", DWX{g, c->phys, dt, f[TCS_U], f[TCS_INVRHO], c->stale}, 1, am, ac, ap,
+    TCS_TRY(z_stage<ANY_SPLIT>(c, "dW_z", "dW_z_solve", z, 1, am, ac, ap, rhs));
+    TCS_TRY(x_stage<ANY_SPLIT>(c, "dW_x", "dW_x_solve", DWX{g, c->phys, dt, f[TCS_U], f[TCS_INVRHO], c->stale}, 1, am, ac, ap,
                     rhs));
     return y_stage<16>(c, "dW_y", "dW_y_solve", DWY{g, c->phys, dt, f[TCS_V], f[TCS_INVRHO], c->stale}, 1, f[TCS_DW]);
 }

@@ -346,7 +346,7 @@ __global__ void __launch_bounds__(PT_SX * PT_PMAX)
 k_poisson_part(int n3m, int h1p, int h3p, const double *__restrict__ amj, const double *__restrict__ apj,
                const double *__restrict__ acj, const double *__restrict__ dxk2, const double *__restrict__ dzk,
                double2 *__restrict__ S, int P, int w1, int w2) {
-    __shared__ part::RedLDS<double, PT_SX, 2> red;
+    __shared__ part::RedLDS<double, PT_SX, 2, PT_PMAX> red;
     const int t = threadIdx.x;
     const int line = t % PT_SX, p = t / PT_SX;
     const int nsys = n3m * h1p;
@@ -375,17 +375,17 @@ k_poisson_part(int n3m, int h1p, int h3p, const double *__restrict__ amj, const 
                 }
             }
         }
-        part::reduce<double, 2>(a, b, c, d, m);
+        part::reduce<double, 2, PT_MMAX>(a, b, c, d, m);
     }
     double xf[2], xl[2];
-    part::exchange<double, false, PT_SX, 2>(red, line, p, P, a, c, d, m, xf, xl);
+    part::exchange<double, false, PT_SX, 2, PT_MMAX, PT_PMAX>(red, line, p, P, a, c, d, m, xf, xl);
     if (!act) return;
     const bool zim = (kx == 0 && (kz == 0 || kz == h3p - 1));
 #pragma unroll
     for (int r = 0; r < PT_MMAX; r++) {
         if (r < m) {
-            const double vr = part::x_of<double, 2>(a, c, d, 0, r, m, xf[0], xl[0]);
-            const double vi = part::x_of<double, 2>(a, c, d, 1, r, m, xf[1], xl[1]);
+            const double vr = part::x_of<double, 2, PT_MMAX>(a, c, d, 0, r, m, xf[0], xl[0]);
+            const double vi = part::x_of<double, 2, PT_MMAX>(a, c, d, 1, r, m, xf[1], xl[1]);
             S[s + (size_t)(j0 + r) * rs] = make_double2(vr, zim ? 0.0 : vi);
         }
     }
@@ -748,6 +748,10 @@ static int poisson_after_x(tcs_ctx *c) {
     double2 *spec = (double2 *)c->spec_x;
     TCS_TRY(fft_z_launch<-1>(c, "fft_z<-1>", spec));
     const int nsys = n3m * h1p;
+    // (parts of 16 rows and at most 32 of them in every form: the nearly
+    // singular systems of the small wavenumbers lose digits with more parts,
+    // the error of V against 64 bits 6e-13 -> 6e-12 at 32x600x32, of P 5e-14 ->
+    // 1.6e-13 with 4-row parts at 64^3)
     int P, w1, w2;
     if (c->tdma_split && ptdma_part_plan(n2m, P, w1, w2)) {
         TCS_LAUNCH(c->stream, "poisson_part", k_poisson_part, dim3((nsys + PT_SX - 1) / PT_SX), dim3(PT_SX * P), 0,

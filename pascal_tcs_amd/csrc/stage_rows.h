@@ -228,23 +228,24 @@ struct XLineRows {
 
 // Whether a stage's lines of n_row rows are solved with their rows computed
 // in the solve: split solves are asked for (the mixed form always splits)
-// and the lines are short enough to split.
-template <typename S>
+// and the lines are short enough to split (ANY: the form takes
+// part_plan_any's splits).
+template <typename S, bool ANY>
 inline bool rows_in_solve(const tcs_ctx *c, int n_row) {
-    int P, w1, w2;
-    return (c->tdma_split || sizeof(S) == sizeof(float)) && ptdma_part_plan(n_row, P, w1, w2);
+    PartPlan q;
+    return (c->tdma_split || sizeof(S) == sizeof(float)) && part_plan_for<ANY>(n_row, 1, q);
 }
 
 // z stage over the z lines of rows j >= jlo, solution into the scratch rhs:
 // rows computed in the split solve (label_solve), or written by k_rows3d
 // (label_rows) and swept.
-template <class Row, typename S>
+template <bool ANY, class Row, typename S>
 int z_stage(tcs_ctx *c, const char *label_rows, const char *label_solve, const Row &row, int jlo, S *am, S *ac,
             S *ap, S *rhs) {
     const long n1 = c->n1m, n12 = (long)c->n1m * c->n2m, off = (long)(jlo - 1) * n1;
     constexpr int SX = std::is_same<S, float>::value ? RowSX32<Row>::value : RowSX64<Row>::value;
-    if (rows_in_solve<S>(c, c->n3m))
-        return ptdma_part_src_launch<true, SX>(c->stream, label_solve, ZLineRows<Row, S>{row, twin_w(c), jlo},
+    if (rows_in_solve<S, ANY>(c, c->n3m))
+        return ptdma_part_src_launch<true, SX, ANY>(c->stream, label_solve, ZLineRows<Row, S>{row, twin_w(c), jlo},
                                                rhs + off, c->n1m, c->n2m - jlo + 1, n1, c->n3m, n12);
     TCS_TRY(rows3d_launch<true>(c, label_rows, row, jlo, am, ac, ap, rhs));
     return ptdma_sweep(c, am + off, ac + off, ap + off, rhs + off, c->n1m, 1, c->n2m - jlo + 1, n1, c->n3m, n12,
@@ -253,13 +254,13 @@ int z_stage(tcs_ctx *c, const char *label_rows, const char *label_solve, const R
 
 // x stage over the x lines of rows j >= jlo (right-hand side and solution in
 // the scratch rhs), in either of the two ways.
-template <class Row, typename S>
+template <bool ANY, class Row, typename S>
 int x_stage(tcs_ctx *c, const char *label_rows, const char *label_solve, const Row &row, int jlo, S *am, S *ac,
             S *ap, S *rhs) {
     const long n1 = c->n1m, n12 = (long)c->n1m * c->n2m, off = (long)(jlo - 1) * n1;
     const int nl = c->n2m - jlo + 1;
-    if (rows_in_solve<S>(c, c->n1m))
-        return ptdma_part_rows_src_launch<true>(c->stream, label_solve, XLineRows<Row, S>{row, twin_w(c), rhs, jlo},
+    if (rows_in_solve<S, ANY>(c, c->n1m))
+        return ptdma_part_rows_src_launch<true, ANY>(c->stream, label_solve, XLineRows<Row, S>{row, twin_w(c), rhs, jlo},
                                                 rhs + off, nl, n1, c->n3m, n12, c->n1m);
     TCS_TRY(rows3d_launch<false>(c, label_rows, row, jlo, am, ac, ap, rhs));
     return ptdma_sweep(c, am + off, ac + off, ap + off, rhs + off, nl, n1, c->n3m, n12, c->n1m, 1, true);
@@ -269,8 +270,8 @@ int x_stage(tcs_ctx *c, const char *label_rows, const char *label_solve, const R
 // the y lines of rows j = jlo..jlo+nrows-1, right-hand side from the scratch
 // rhs.  The solution is stored into (mode 1) or added to (mode 2) the
 // interior of the field F, or, with F null, written back into rhs.  Rows
-// j < jrow are identity rows (YLineRowsLead) when jrow > jlo.
-template <int SX = PT_SX, class Row, typename S>
+// j < jrow are identity rows (YLineRowsLead) with LEAD.
+template <bool ANY, int SX = PT_SX, bool LEAD = false, class Row, typename S>
 int y_stage_in_solve(tcs_ctx *c, const char *label, const Row &row, int jlo, int nrows, S *rhs, double *F,
                      int mode, int jrow = 0) {
     const long n1 = c->n1m, n12 = (long)c->n1m * c->n2m, off = (long)(jlo - 1) * n1;
@@ -293,10 +294,10 @@ int y_stage_in_solve(tcs_ctx *c, const char *label, const Row &row, int jlo, int
             out.mode = 4;
         }
     }
-    if (jrow > jlo)
-        return ptdma_part_src_launch<false, SX>(c->stream, label, YLineRowsLead<Row, S>{row, twin_w(c), rhs, jlo, jrow},
+    if constexpr (LEAD)
+        return ptdma_part_src_launch<false, SX, ANY>(c->stream, label, YLineRowsLead<Row, S>{row, twin_w(c), rhs, jlo, jrow},
                                                 rhs + off, c->n1m, c->n3m, n12, nrows, n1, out);
-    return ptdma_part_src_launch<false, SX>(c->stream, label, YLineRows<Row, S>{row, twin_w(c), rhs, jlo}, rhs + off,
+    return ptdma_part_src_launch<false, SX, ANY>(c->stream, label, YLineRows<Row, S>{row, twin_w(c), rhs, jlo}, rhs + off,
                                             c->n1m, c->n3m, n12, nrows, n1, out);
 }
 

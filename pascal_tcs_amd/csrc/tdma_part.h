@@ -18,8 +18,47 @@ namespace tcs {
 
 constexpr int PT_MMAX = 16;               // rows per part
 constexpr int PT_PMAX = 32;               // parts per line (n_row <= 512)
-constexpr int PT_RS = 2 * PT_PMAX + 1;    // reduced-row stride in LDS (odd: no bank conflicts)
 constexpr int PT_SX = 16;                 // lines per workgroup
+
+// How a line of n_row rows is split: P parts (a power of two) of w1 or w1 + 1
+// rows, at most mm, P <= pm.
+struct PartPlan {
+    int P, w1, w2, mm, pm;
+};
+inline PartPlan part_plan(int n_row, int mm, int pm) {
+    PartPlan q{1, 0, 0, mm, pm};
+    while (q.P * mm < n_row) q.P <<= 1;
+    q.w1 = n_row / q.P;
+    q.w2 = n_row % q.P;
+    return q;
+}
+// The plan of the forms that are bound to no particular split (the fast
+// forms; the exact form keeps ptdma_part_plan's, which the oracle restates):
+//   * lines of 513..2048 rows: 64 or 128 parts of 16 rows, fewer lines a
+//     workgroup (momentum x lines of 1024 rows at 1024x128x256: 845 us as
+//     single-rank lines after 200 us for their rows, 271-295 us split);
+//   * few lines: parts of 8 or 4 rows while 16-row parts leave the chip short
+//     of wavefronts (PART_FILL threads are 8 wavefronts a CU): a thread
+//     makes its part's rows one after the other, which is what a small grid
+//     waits for (64^3: dW z 42 -> 13 us, dU z 24 -> 13, dW x 25 -> 12).  No
+//     part gets fewer than three rows.
+// The lines' errors against 64 bits stay where they were (16x40x32 to
+// 2048x40x16 and 16x1100x16).
+constexpr long PART_FILL = 8L * 64 * 256;
+inline bool part_plan_any(int n_row, long lines, PartPlan &q) {
+    if (n_row < 2 || n_row > 4 * PT_MMAX * PT_PMAX) return false;
+    if (n_row > PT_MMAX * PT_PMAX) {
+        q = part_plan(n_row, PT_MMAX, n_row > 2 * PT_MMAX * PT_PMAX ? 4 * PT_PMAX : 2 * PT_PMAX);
+        return true;
+    }
+    q = part_plan(n_row, PT_MMAX, PT_PMAX);
+    while (q.mm > 4 && lines * q.P < PART_FILL && n_row <= q.mm / 2 * PT_PMAX) {
+        const PartPlan h = part_plan(n_row, q.mm / 2, PT_PMAX);
+        if (h.P > 1 && h.w1 < 3) break;  // a part of two rows couples past its neighbour (row 1's fix-up)
+        q = h;
+    }
+    return true;
+}
 
 namespace part {
 
@@ -32,9 +71,9 @@ __device__ __forceinline__ void range(int p, int w1, int w2, int &j0, int &m) {
 // pascal_tdma.f90:501-536 on a part held in registers: row r (coefficients
 // ar, br, cr, dr) enters the forward elimination, rows < r already hold
 // their eliminated form.  Rows 0 and 1 are only normalised.
-template <typename T, int NR>
-__device__ __forceinline__ void reduce_row(int r, T ar, T br, T cr, const T (&dr)[NR], T (&a)[PT_MMAX],
-                                           T (&c)[PT_MMAX], T (&d)[NR][PT_MMAX]) {
+template <typename T, int NR, int MM>
+__device__ __forceinline__ void reduce_row(int r, T ar, T br, T cr, const T (&dr)[NR], T (&a)[MM],
+                                           T (&c)[MM], T (&d)[NR][MM]) {
     if (r < 2) {
         a[r] = ar / br;
 #pragma unroll
@@ -52,10 +91,10 @@ __device__ __forceinline__ void reduce_row(int r, T ar, T br, T cr, const T (&dr
 // The rest of the per-rank algorithm once rows 0..m-1 have been through
 // reduce_row: backward elimination and the fix-up of row 0.  a, c, d come
 // back as the reduced-form coefficients.
-template <typename T, int NR>
-__device__ __forceinline__ void reduce_back(T (&a)[PT_MMAX], T (&c)[PT_MMAX], T (&d)[NR][PT_MMAX], int m) {
+template <typename T, int NR, int MM>
+__device__ __forceinline__ void reduce_back(T (&a)[MM], T (&c)[MM], T (&d)[NR][MM], int m) {
 #pragma unroll
-    for (int r = PT_MMAX - 3; r >= 1; r--) {
+    for (int r = MM - 3; r >= 1; r--) {
         if (r <= m - 3) {
 #pragma unroll
             for (int k = 0; k < NR; k++) d[k][r] = d[k][r] - c[r] * d[k][r + 1];
@@ -72,33 +111,33 @@ __device__ __forceinline__ void reduce_back(T (&a)[PT_MMAX], T (&c)[PT_MMAX], T 
 
 // One part (rows 0..m-1, m >= 2) in registers, all rows loaded: b is
 // consumed; a, c, d come back as the reduced-form coefficients.
-template <typename T, int NR>
-__device__ __forceinline__ void reduce(T (&a)[PT_MMAX], T (&b)[PT_MMAX], T (&c)[PT_MMAX],
-                                       T (&d)[NR][PT_MMAX], int m) {
+template <typename T, int NR, int MM>
+__device__ __forceinline__ void reduce(T (&a)[MM], T (&b)[MM], T (&c)[MM],
+                                       T (&d)[NR][MM], int m) {
 #pragma unroll
-    for (int r = 0; r < PT_MMAX; r++) {
+    for (int r = 0; r < MM; r++) {
         if (r < m) {
             T dr[NR];
 #pragma unroll
             for (int k = 0; k < NR; k++) dr[k] = d[k][r];
-            reduce_row<T, NR>(r, a[r], b[r], c[r], dr, a, c, d);
+            reduce_row<T, NR, MM>(r, a[r], b[r], c[r], dr, a, c, d);
         }
     }
-    reduce_back<T, NR>(a, c, d, m);
+    reduce_back<T, NR, MM>(a, c, d, m);
 }
 
 // a, c, d at row m-1 (a runtime index) in one unrolled pass: selecting all
 // of them together keeps the arrays in registers (a separate select per
 // array lets the compiler turn it into a dynamically indexed private array)
-template <typename T, int NR>
-__device__ __forceinline__ void lasts(const T (&a)[PT_MMAX], const T (&c)[PT_MMAX], const T (&d)[NR][PT_MMAX],
+template <typename T, int NR, int MM>
+__device__ __forceinline__ void lasts(const T (&a)[MM], const T (&c)[MM], const T (&d)[NR][MM],
                                       int m, T &la, T &lc, T (&ld)[NR]) {
     la = a[0];
     lc = c[0];
 #pragma unroll
     for (int k = 0; k < NR; k++) ld[k] = d[k][0];
 #pragma unroll
-    for (int r = 1; r < PT_MMAX; r++) {
+    for (int r = 1; r < MM; r++) {
         if (r == m - 1) {
             la = a[r];
             lc = c[r];
@@ -110,8 +149,8 @@ __device__ __forceinline__ void lasts(const T (&a)[PT_MMAX], const T (&c)[PT_MMA
 
 // x(r) of right-hand side k from the part's reduced solution xf (row 0)
 // and xl (row m-1): pascal_tdma.f90:567-576
-template <typename T, int NR>
-__device__ __forceinline__ T x_of(const T (&a)[PT_MMAX], const T (&c)[PT_MMAX], const T (&d)[NR][PT_MMAX],
+template <typename T, int NR, int MM>
+__device__ __forceinline__ T x_of(const T (&a)[MM], const T (&c)[MM], const T (&d)[NR][MM],
                                   int k, int r, int m, T xf, T xl) {
     if (r == 0) return xf;
     if (r == m - 1) return xl;
@@ -120,10 +159,11 @@ __device__ __forceinline__ T x_of(const T (&a)[PT_MMAX], const T (&c)[PT_MMAX], 
 
 // Reduced arrays of a workgroup, [array][line][row]: a, c, b (or the e
 // scratch of the serial cyclic solve), then the NR right-hand sides.
-template <typename T, int SX, int NR>
+template <typename T, int SX, int NR, int PM>
 struct RedLDS {
-    T v[(3 + NR) * SX * PT_RS];
-    __device__ T *q(int which, int line) { return v + ((size_t)which * SX + line) * PT_RS; }
+    static constexpr int RS = 2 * PM + 1;  // odd: no bank conflicts
+    T v[(3 + NR) * SX * RS];
+    __device__ T *q(int which, int line) { return v + ((size_t)which * SX + line) * RS; }
 };
 
 // The 2-row reduced system of a single part, serially: tdma_many
@@ -182,16 +222,16 @@ __device__ void reduced_serial(T *ra, T *rc, T *re, T *const (&rd)[NR], int n2) 
 // row i couples only to j = i + N/2 and the pair is solved directly,
 // x_i = (d_i b_j - e_i d_j)/(b_i b_j - e_i e_j), e = a + c.
 // Every thread of the workgroup must call this (it synchronises).
-template <typename T, bool CYC, int SX, int NR>
-__device__ __forceinline__ void exchange(RedLDS<T, SX, NR> &red, int line, int p, int P, const T (&a)[PT_MMAX],
-                                         const T (&c)[PT_MMAX], const T (&d)[NR][PT_MMAX], int m, T (&xf)[NR],
+template <typename T, bool CYC, int SX, int NR, int MM, int PM>
+__device__ __forceinline__ void exchange(RedLDS<T, SX, NR, PM> &red, int line, int p, int P, const T (&a)[MM],
+                                         const T (&c)[MM], const T (&d)[NR][MM], int m, T (&xf)[NR],
                                          T (&xl)[NR]) {
     T *ra = red.q(0, line), *rc = red.q(1, line), *rb = red.q(2, line);
     T *rd[NR];
 #pragma unroll
     for (int k = 0; k < NR; k++) rd[k] = red.q(3 + k, line);
     T la, lc, ld[NR];
-    lasts<T, NR>(a, c, d, m, la, lc, ld);
+    lasts<T, NR, MM>(a, c, d, m, la, lc, ld);
     ra[2 * p] = a[0]; rc[2 * p] = c[0];
     ra[2 * p + 1] = la; rc[2 * p + 1] = lc;
 #pragma unroll
@@ -266,29 +306,29 @@ __device__ __forceinline__ void exchange(RedLDS<T, SX, NR> &red, int line, int p
 
 // The solution of a part of line (s0, s1): into D at dbase + row*rs
 // (out.mode 0), or into the field of out (modes 1, 2, 3).
-template <typename T>
-__device__ __forceinline__ void store(const T (&a)[PT_MMAX], const T (&c)[PT_MMAX], const T (&d)[1][PT_MMAX],
+template <typename T, int MM>
+__device__ __forceinline__ void store(const T (&a)[MM], const T (&c)[MM], const T (&d)[1][MM],
                                       int j0, int m, T xf, T xl, T *D, long dbase, long rs, const LineOut &out,
                                       int s0, int s1) {
     if constexpr (sizeof(T) == sizeof(float)) {
         if (out.mode == 4) {  // FP32 lines only: the mixed form's increments
             const long fb = out.base + (long)s0 * out.ss0 + (long)s1 * out.ss1;
 #pragma unroll
-            for (int r = 0; r < PT_MMAX; r++)
-                if (r < m) out.G[fb + (long)(j0 + r) * out.rs] = x_of<T, 1>(a, c, d, 0, r, m, xf, xl);
+            for (int r = 0; r < MM; r++)
+                if (r < m) out.G[fb + (long)(j0 + r) * out.rs] = x_of<T, 1, MM>(a, c, d, 0, r, m, xf, xl);
             return;
         }
     }
     if (out.mode == 0) {
 #pragma unroll
-        for (int r = 0; r < PT_MMAX; r++)
-            if (r < m) D[dbase + (long)(j0 + r) * rs] = x_of<T, 1>(a, c, d, 0, r, m, xf, xl);
+        for (int r = 0; r < MM; r++)
+            if (r < m) D[dbase + (long)(j0 + r) * rs] = x_of<T, 1, MM>(a, c, d, 0, r, m, xf, xl);
     } else {
         const long fb = out.base + (long)s0 * out.ss0 + (long)s1 * out.ss1;
 #pragma unroll
-        for (int r = 0; r < PT_MMAX; r++) {
+        for (int r = 0; r < MM; r++) {
             if (r < m) {
-                const double x = (double)x_of<T, 1>(a, c, d, 0, r, m, xf, xl);
+                const double x = (double)x_of<T, 1, MM>(a, c, d, 0, r, m, xf, xl);
                 const long o = fb + (long)(j0 + r) * out.rs;
                 const double v = out.mode == 1 ? x : (out.mode == 2 ? out.F[o] : out.Fin[o]) + x;
                 out.F[o] = v;
@@ -301,6 +341,14 @@ __device__ __forceinline__ void store(const T (&a)[PT_MMAX], const T (&c)[PT_MMA
 }
 
 }  // namespace part
+
+// the plan of a stage's lines: part_plan_any's (ANY) or ptdma_part_plan's
+template <bool ANY>
+inline bool part_plan_for(int n_row, long lines, PartPlan &q) {
+    if constexpr (ANY) return part_plan_any(n_row, lines, q);
+    q = PartPlan{0, 0, 0, PT_MMAX, PT_PMAX};
+    return ptdma_part_plan(n_row, q.P, q.w1, q.w2);
+}
 
 // Workgroup order for the solves that compute their rows.  Workgroups go
 // to the 8 XCDs round-robin in dispatch order, and the rows of a line group
@@ -346,45 +394,45 @@ __device__ __forceinline__ void src_row(const Src &src, int s0, int s1, int row,
 // they share once; otherwise guarded by r < m.  (The row loop in a function
 // of its own, taking the part arrays by reference, put them in scratch
 // memory.)
-template <int WM, typename T, bool CYC, class Src, int SX, bool FULL>
-__device__ __forceinline__ void part_src_lines(const Src &src, part::RedLDS<T, SX, 1> &red, T *D, int n0, long ss1, long rs,
+template <int WM, typename T, bool CYC, class Src, int SX, bool FULL, int MM, int PM>
+__device__ __forceinline__ void part_src_lines(const Src &src, part::RedLDS<T, SX, 1, PM> &red, T *D, int n0, long ss1, long rs,
                                                int P, int w1, int w2, const LineOut &out, int line, int p, int s0,
                                                int s1) {
     using namespace part;
     const bool act = s0 < n0;
     int j0, m;
     range(p, w1, w2, j0, m);
-    T a[PT_MMAX], c[PT_MMAX], d[1][PT_MMAX];
+    T a[MM], c[MM], d[1][MM];
     if (FULL && act) {
 #pragma unroll
-        for (int r = 0; r < PT_MMAX; r++) {
+        for (int r = 0; r < MM; r++) {
             T ar, br, cr, dr[1];
             src_row<WM>(src, s0, s1, j0 + r, ar, br, cr, dr[0]);
-            reduce_row<T, 1>(r, ar, br, cr, dr, a, c, d);
+            reduce_row<T, 1, MM>(r, ar, br, cr, dr, a, c, d);
         }
     } else if (FULL && sizeof(T) == sizeof(float)) {
         // padding lines of FP32 solves: zero rows (the guarded loop below
         // puts the FP32 arrays on the stack in this instantiation; the FP64
         // ones keep it, dU y 1.02 against 1.14 ms with the zero rows)
 #pragma unroll
-        for (int r = 0; r < PT_MMAX; r++) { a[r] = T(0); c[r] = T(0); d[0][r] = T(0); }
+        for (int r = 0; r < MM; r++) { a[r] = T(0); c[r] = T(0); d[0][r] = T(0); }
     } else {
 #pragma unroll
-        for (int r = 0; r < PT_MMAX; r++) {
+        for (int r = 0; r < MM; r++) {
             if (r < m) {
                 T ar = T(0), br = T(1), cr = T(0), dr[1] = {T(0)};
                 if (act) src_row<WM>(src, s0, s1, j0 + r, ar, br, cr, dr[0]);
-                reduce_row<T, 1>(r, ar, br, cr, dr, a, c, d);
+                reduce_row<T, 1, MM>(r, ar, br, cr, dr, a, c, d);
             } else {
                 a[r] = T(0); c[r] = T(0); d[0][r] = T(0);
             }
         }
     }
-    reduce_back<T, 1>(a, c, d, m);
+    reduce_back<T, 1, MM>(a, c, d, m);
     T xf[1], xl[1];
-    exchange<T, CYC, SX, 1>(red, line, p, P, a, c, d, m, xf, xl);
+    exchange<T, CYC, SX, 1, MM, PM>(red, line, p, P, a, c, d, m, xf, xl);
     if (!act) return;
-    store<T>(a, c, d, j0, m, xf[0], xl[0], D, (long)s0 + (long)s1 * ss1, rs, out, s0, s1);
+    store<T, MM>(a, c, d, j0, m, xf[0], xl[0], D, (long)s0 + (long)s1 * ss1, rs, out, s0, s1);
 }
 
 // Lines strided in memory whose rows are computed, not read: src(s0, s1,
@@ -396,10 +444,10 @@ __device__ __forceinline__ void part_src_lines(const Src &src, part::RedLDS<T, S
 // those of the split solve of stored lines.  Sources with wall terms
 // (SrcWalls) make the rows of a workgroup whose j is away from the walls
 // without them.
-template <typename T, bool CYC, class Src, int SX, bool FULL>
-__global__ void __launch_bounds__(SX * PT_PMAX) __attribute__((amdgpu_waves_per_eu(Src::waves)))
+template <typename T, bool CYC, class Src, int SX, bool FULL, int MM, int PM>
+__global__ void __launch_bounds__(SX * PM) __attribute__((amdgpu_waves_per_eu(Src::waves)))
 k_ptdma_part_src(Src src, T *D, int n0, int n1, long ss1, long rs, int P, int w1, int w2, LineOut out) {
-    __shared__ part::RedLDS<T, SX, 1> red;
+    __shared__ part::RedLDS<T, SX, 1, PM> red;
     const int t = threadIdx.x;
     const int line = t % SX, p = t / SX;
     int bx, by;
@@ -409,11 +457,11 @@ k_ptdma_part_src(Src src, T *D, int n0, int n1, long ss1, long rs, int P, int w1
     if constexpr (SrcWalls<Src>::value) {
         // s1 is the workgroup's: one branch for the whole workgroup
         if (src.wall_free(s1))
-            part_src_lines<2, T, CYC, Src, SX, FULL>(src, red, D, n0, ss1, rs, P, w1, w2, out, line, p, s0, s1);
+            part_src_lines<2, T, CYC, Src, SX, FULL, MM, PM>(src, red, D, n0, ss1, rs, P, w1, w2, out, line, p, s0, s1);
         else
-            part_src_lines<0, T, CYC, Src, SX, FULL>(src, red, D, n0, ss1, rs, P, w1, w2, out, line, p, s0, s1);
+            part_src_lines<0, T, CYC, Src, SX, FULL, MM, PM>(src, red, D, n0, ss1, rs, P, w1, w2, out, line, p, s0, s1);
     } else {
-        part_src_lines<-1, T, CYC, Src, SX, FULL>(src, red, D, n0, ss1, rs, P, w1, w2, out, line, p, s0, s1);
+        part_src_lines<-1, T, CYC, Src, SX, FULL, MM, PM>(src, red, D, n0, ss1, rs, P, w1, w2, out, line, p, s0, s1);
     }
 }
 
@@ -426,7 +474,8 @@ inline int stage_len(int rows) { return rows - 1 + ((rows - 1) >> 4) + 1; }
 // parts [g*P/nb, (g+1)*P/nb) and so rows [row0(g), row0(g+1)).
 constexpr int PT_RBLK = 4;
 constexpr int PT_EU = 2;    // rows a thread makes at once
-constexpr int PT_XRUN = 4;  // consecutive rows a thread makes when a block divides evenly
+// consecutive rows a thread makes when a block divides evenly (parts of mm rows)
+constexpr int xrun(int mm) { return mm / PT_RBLK; }
 __host__ __device__ inline int rblocks(int P) { return P < PT_RBLK ? P : PT_RBLK; }
 __host__ __device__ inline int rblock_row0(int g, int P, int w1, int w2) {
     const int p = g * (P / rblocks(P));
@@ -437,7 +486,9 @@ __host__ __device__ inline int rblock_row0(int g, int P, int w1, int w2) {
 // rows are made along the lines, so fewer lines cost no coalescing, and the
 // small workgroups (PT_XSX * P threads, one wavefront for 512 rows) with
 // their small stages share a CU, one's memory waits covered by the others'
-// work (at 512^3: 2 lines 12-30% faster than 16).
+// work (at 512^3: 2 lines 12-30% faster than 16).  Shorter lines take as many
+// as fill a wavefront (16 four-part lines of 64 rows: 8 threads a workgroup
+// with two, 23 us at 64^3).
 constexpr int PT_XSX = 2;
 
 // Contiguous lines (rows 1 apart, x sweeps) whose rows are computed:
@@ -448,52 +499,53 @@ constexpr int PT_XSX = 2;
 // four arrays of the block together; the threads whose parts lie in the
 // block take their rows from there.  Then the solve of k_ptdma_part_rows,
 // whose LDS stage also takes the solution out.
-template <typename T, bool CYC, class Src>
-__global__ void __launch_bounds__(PT_XSX * PT_PMAX)
+template <typename T, bool CYC, class Src, int XSX, int MM, int PM>
+__global__ void __launch_bounds__(XSX * PM)
 k_ptdma_part_rows_src(Src src, T *D, int n0, long ss0, long ss1, int n_row, int ls, int lsb, int P, int w1,
                       int w2) {
     using namespace part;
+    constexpr int XRUN = xrun(MM);
     extern __shared__ __align__(16) unsigned char stage_raw[];
     T *stage = reinterpret_cast<T *>(stage_raw);
-    __shared__ RedLDS<T, PT_XSX, 1> red;
+    __shared__ RedLDS<T, XSX, 1, PM> red;
     const int t = threadIdx.x, nt = blockDim.x;
-    const int line = t % PT_XSX, p = t / PT_XSX;
+    const int line = t % XSX, p = t / XSX;
     int bx, s1;
     xcd_tiles(bx, s1);
-    const int s0 = bx * PT_XSX + line;
+    const int s0 = bx * XSX + line;
     const bool act = s0 < n0;
-    const int nl = min(PT_XSX, n0 - bx * PT_XSX);  // lines present in this workgroup
+    const int nl = min(XSX, n0 - bx * XSX);  // lines present in this workgroup
     int j0, m;
     range(p, w1, w2, j0, m);
     const int nb = rblocks(P), mygrp = p / (P / nb);
 
-    T a[PT_MMAX], b[PT_MMAX], c[PT_MMAX], d[1][PT_MMAX];
+    T a[MM], b[MM], c[MM], d[1][MM];
     for (int g = 0; g < nb; g++) {
         const int r0 = rblock_row0(g, P, w1, w2), nr = rblock_row0(g + 1, P, w1, w2) - r0;
         if (g > 0) __syncthreads();  // the previous block has been read
-        // stage[(q*PT_XSX + l)*lsb + stage_pos(r - r0)], q = a, b, c, d
-        if (sizeof(T) == 8 && nr * PT_XSX == PT_XRUN * nt && nl == PT_XSX) {
-            // a whole block, PT_XRUN consecutive rows of one line per thread,
+        // stage[(q*XSX + l)*lsb + stage_pos(r - r0)], q = a, b, c, d
+        if (sizeof(T) == 8 && nr * XSX == XRUN * nt && nl == XSX) {
+            // a whole block, XRUN consecutive rows of one line per thread,
             // made unconditionally: consecutive rows share their loads and
             // terms (FP64 dU/dV/dW x solves 1.58-1.72 -> 1.08-1.11 ms at
             // 512^3)
-            const int per = nt / PT_XSX;  // threads per line
-            const int l = t / per, rb = (t - l * per) * PT_XRUN;
-            T ar[PT_XRUN], br[PT_XRUN], cr[PT_XRUN], dr[PT_XRUN];
+            const int per = nt / XSX;  // threads per line
+            const int l = t / per, rb = (t - l * per) * XRUN;
+            T ar[XRUN], br[XRUN], cr[XRUN], dr[XRUN];
 #pragma unroll
-            for (int u = 0; u < PT_XRUN; u++) src(bx * PT_XSX + l, s1, r0 + rb + u, ar[u], br[u], cr[u], dr[u]);
+            for (int u = 0; u < XRUN; u++) src(bx * XSX + l, s1, r0 + rb + u, ar[u], br[u], cr[u], dr[u]);
 #pragma unroll
-            for (int u = 0; u < PT_XRUN; u++) {
+            for (int u = 0; u < XRUN; u++) {
                 const int o = l * lsb + stage_pos(rb + u);
                 stage[o] = ar[u];
-                stage[o + PT_XSX * lsb] = br[u];
-                stage[o + 2 * PT_XSX * lsb] = cr[u];
-                stage[o + 3 * PT_XSX * lsb] = dr[u];
+                stage[o + XSX * lsb] = br[u];
+                stage[o + 2 * XSX * lsb] = cr[u];
+                stage[o + 3 * XSX * lsb] = dr[u];
             }
         } else {
         // otherwise a thread makes PT_EU rows (nt apart) before it stores any,
         // so their reads overlap
-        for (int e0 = t; e0 < nr * PT_XSX; e0 += PT_EU * nt) {
+        for (int e0 = t; e0 < nr * XSX; e0 += PT_EU * nt) {
             T ar[PT_EU], br[PT_EU], cr[PT_EU], dr[PT_EU];
             int o[PT_EU];
 #pragma unroll
@@ -501,9 +553,9 @@ k_ptdma_part_rows_src(Src src, T *D, int n0, long ss0, long ss1, int n_row, int 
                 const int e = e0 + u * nt;
                 ar[u] = T(0); br[u] = T(1); cr[u] = T(0); dr[u] = T(0);
                 o[u] = -1;
-                if (e < nr * PT_XSX) {
+                if (e < nr * XSX) {
                     const int l = e / nr, r = e - l * nr;
-                    if (l < nl) src(bx * PT_XSX + l, s1, r0 + r, ar[u], br[u], cr[u], dr[u]);
+                    if (l < nl) src(bx * XSX + l, s1, r0 + r, ar[u], br[u], cr[u], dr[u]);
                     o[u] = l * lsb + stage_pos(r);
                 }
             }
@@ -511,9 +563,9 @@ k_ptdma_part_rows_src(Src src, T *D, int n0, long ss0, long ss1, int n_row, int 
             for (int u = 0; u < PT_EU; u++) {
                 if (o[u] >= 0) {
                     stage[o[u]] = ar[u];
-                    stage[o[u] + PT_XSX * lsb] = br[u];
-                    stage[o[u] + 2 * PT_XSX * lsb] = cr[u];
-                    stage[o[u] + 3 * PT_XSX * lsb] = dr[u];
+                    stage[o[u] + XSX * lsb] = br[u];
+                    stage[o[u] + 2 * XSX * lsb] = cr[u];
+                    stage[o[u] + 3 * XSX * lsb] = dr[u];
                 }
             }
         }
@@ -521,47 +573,42 @@ k_ptdma_part_rows_src(Src src, T *D, int n0, long ss0, long ss1, int n_row, int 
         __syncthreads();
         if (mygrp == g) {
 #pragma unroll
-            for (int r = 0; r < PT_MMAX; r++) {
+            for (int r = 0; r < MM; r++) {
                 const bool in = r < m;
                 const T *q = stage + line * lsb + stage_pos(j0 - r0 + r);
                 a[r] = in ? q[0] : T(0);
-                b[r] = in ? q[PT_XSX * lsb] : T(1);
-                c[r] = in ? q[2 * PT_XSX * lsb] : T(0);
-                d[0][r] = in ? q[3 * PT_XSX * lsb] : T(0);
+                b[r] = in ? q[XSX * lsb] : T(1);
+                c[r] = in ? q[2 * XSX * lsb] : T(0);
+                d[0][r] = in ? q[3 * XSX * lsb] : T(0);
             }
         }
     }
-    reduce<T, 1>(a, b, c, d, m);
+    reduce<T, 1, MM>(a, b, c, d, m);
     T xf[1], xl[1];
-    exchange<T, CYC, PT_XSX, 1>(red, line, p, P, a, c, d, m, xf, xl);
+    exchange<T, CYC, XSX, 1, MM, PM>(red, line, p, P, a, c, d, m, xf, xl);
     // every thread has read the stage before exchange's first barrier
     if (act) {
 #pragma unroll
-        for (int r = 0; r < PT_MMAX; r++)
-            if (r < m) stage[line * ls + stage_pos(j0 + r)] = x_of<T, 1>(a, c, d, 0, r, m, xf[0], xl[0]);
+        for (int r = 0; r < MM; r++)
+            if (r < m) stage[line * ls + stage_pos(j0 + r)] = x_of<T, 1, MM>(a, c, d, 0, r, m, xf[0], xl[0]);
     }
     __syncthreads();
-    const long gbase = (long)bx * PT_XSX * ss0 + (long)s1 * ss1;
+    const long gbase = (long)bx * XSX * ss0 + (long)s1 * ss1;
     for (int r = t; r < n_row; r += nt) {
 #pragma unroll
-        for (int l = 0; l < PT_XSX; l++)
+        for (int l = 0; l < XSX; l++)
             if (l < nl) D[gbase + l * ss0 + r] = stage[l * ls + stage_pos(r)];
     }
 }
 
-// Launch of k_ptdma_part_src over n0 x n1 lines of n_row rows (n_row in
-// [2, 512]), SX lines per workgroup (16: four 128-byte row segments per
-// wavefront load; 8: 64-byte segments, but two workgroups per CU); returns
-// TCS_E_ARG outside the split range.
-template <bool CYC, int SX = PT_SX, typename T, class Src>
-int ptdma_part_src_launch(hipStream_t st, const char *label, const Src &src, T *D, int n0, int n1, long ss1,
-                          int n_row, long rs, const LineOut &out = LineOut()) {
-    int P, w1, w2;
-    if (n0 <= 0 || n1 <= 0) return TCS_OK;
-    if (!ptdma_part_plan(n_row, P, w1, w2) || n1 > 65535) {
-        set_error("ptdma_part: n_row must be in [2, 512] and the outer line count <= 65535");
-        return TCS_E_ARG;
-    }
+// Launch of k_ptdma_part_src over n0 x n1 lines of n_row rows, SX lines per
+// workgroup (16: four 128-byte row segments per wavefront load; 8: 64-byte
+// segments, but two workgroups per CU; fewer where a line has more than
+// PT_PMAX parts); ANY: the plan is part_plan_any's, else ptdma_part_plan's.
+// Returns TCS_E_ARG outside the split range.
+template <bool CYC, int SX, int MM, int PM, typename T, class Src>
+int part_src_launch(hipStream_t st, const char *label, const Src &src, const PartPlan &q, T *D, int n0, int n1,
+                    long ss1, long rs, const LineOut &out) {
     // the outer line count padded to whole XCD tiles (the padding
     // workgroups return at once): a dV stage's 511 lines then take the tiled
     // order too
@@ -569,48 +616,84 @@ int ptdma_part_src_launch(hipStream_t st, const char *label, const Src &src, T *
     unsigned gy = (unsigned)n1;
     const unsigned gyp = (gy + XT_Y - 1) / XT_Y * XT_Y;
     if (gx % XT_X == 0 && (gx * gyp) % (8 * XT_X * XT_Y) == 0 && gyp <= 65535) gy = gyp;
-    const dim3 blk(SX * P), grd(gx, gy);
-    // FP64 lines whose parts all hold PT_MMAX rows take the unconditional
+    const dim3 blk(SX * q.P), grd(gx, gy);
+    // FP64 lines whose parts all hold MM rows take the unconditional
     // row loop where the source asks for it (Src::full_rows: every y stage,
     // thermal y 2.63 -> 2.00 ms, dU y 1.52 -> 1.02 ms, dW y 1.43 -> 1.29 ms
     // at 512^3; the dU z stage, 4.14 -> 3.14 ms); FP32 lines (the mixed
     // form) where the row asks for it as well (Src::full_rows32)
-    if (Src::full_rows && (sizeof(T) == 8 || Src::full_rows32) && w1 == PT_MMAX && w2 == 0)
-        TCS_LAUNCH(st, label, (k_ptdma_part_src<T, CYC, Src, SX, true>), grd, blk, 0, src, D, n0, n1, ss1, rs, P, w1, w2,
-                   out);
-    else
-        TCS_LAUNCH(st, label, (k_ptdma_part_src<T, CYC, Src, SX, false>), grd, blk, 0, src, D, n0, n1, ss1, rs, P, w1, w2,
-                   out);
+    if constexpr (Src::full_rows && (sizeof(T) == 8 || Src::full_rows32))
+        if (q.w1 == MM && q.w2 == 0) {
+            TCS_LAUNCH(st, label, (k_ptdma_part_src<T, CYC, Src, SX, true, MM, PM>), grd, blk, 0, src, D, n0, n1, ss1,
+                       rs, q.P, q.w1, q.w2, out);
+            return TCS_OK;
+        }
+    TCS_LAUNCH(st, label, (k_ptdma_part_src<T, CYC, Src, SX, false, MM, PM>), grd, blk, 0, src, D, n0, n1, ss1, rs,
+               q.P, q.w1, q.w2, out);
     return TCS_OK;
 }
-
-// Launch of k_ptdma_part_rows_src over n0 x n1 contiguous lines of n_row
-// rows (n_row in [2, 512]).
-template <bool CYC, typename T, class Src>
-int ptdma_part_rows_src_launch(hipStream_t st, const char *label, const Src &src, T *D, int n0, long ss0, int n1,
-                               long ss1, int n_row) {
-    int P, w1, w2;
+template <bool CYC, int SX, bool ANY, typename T, class Src>
+int ptdma_part_src_launch(hipStream_t st, const char *label, const Src &src, T *D, int n0, int n1, long ss1,
+                          int n_row, long rs, const LineOut &out = LineOut()) {
+    PartPlan q;
     if (n0 <= 0 || n1 <= 0) return TCS_OK;
-    if (!ptdma_part_plan(n_row, P, w1, w2) || n1 > 65535) {
-        set_error("ptdma_part: n_row must be in [2, 512] and the outer line count <= 65535");
+    if (!part_plan_for<ANY>(n_row, (long)n0 * n1, q) || n1 > 65535) {
+        set_error("ptdma_part: line length outside the split range or outer line count > 65535");
         return TCS_E_ARG;
     }
+    if constexpr (ANY) {
+        constexpr int M = PT_MMAX, PP = PT_PMAX;
+        if constexpr (sizeof(T) == 8)
+            if (q.pm == 2 * PP) return part_src_launch<CYC, 8, M, 2 * PP>(st, label, src, q, D, n0, n1, ss1, rs, out);
+        if constexpr (sizeof(T) == 8)
+            if (q.pm == 4 * PP) return part_src_launch<CYC, 4, M, 4 * PP>(st, label, src, q, D, n0, n1, ss1, rs, out);
+        if (q.mm == 8) return part_src_launch<CYC, 16, 8, PP>(st, label, src, q, D, n0, n1, ss1, rs, out);
+        if (q.mm == 4) return part_src_launch<CYC, 16, 4, PP>(st, label, src, q, D, n0, n1, ss1, rs, out);
+    }
+    return part_src_launch<CYC, SX, PT_MMAX, PT_PMAX>(st, label, src, q, D, n0, n1, ss1, rs, out);
+}
+
+// Launch of k_ptdma_part_rows_src over n0 x n1 contiguous lines of n_row rows.
+template <bool CYC, int XSX, int MM, int PM, typename T, class Src>
+int part_rows_src_launch(hipStream_t st, const char *label, const Src &src, const PartPlan &q, T *D, int n0, long ss0,
+                         int n1, long ss1, int n_row) {
     int lsb = 0;
-    for (int g = 0; g < rblocks(P); g++)
-        lsb = std::max(lsb, stage_len(rblock_row0(g + 1, P, w1, w2) - rblock_row0(g, P, w1, w2)));
+    for (int g = 0; g < rblocks(q.P); g++)
+        lsb = std::max(lsb, stage_len(rblock_row0(g + 1, q.P, q.w1, q.w2) - rblock_row0(g, q.P, q.w1, q.w2)));
     const int ls = stage_len(n_row);
-    const int lds = (int)sizeof(T) * std::max(PT_XSX * ls, 4 * PT_XSX * lsb);
+    const int lds = (int)sizeof(T) * std::max(XSX * ls, 4 * XSX * lsb);
     static bool lds_raised = false;  // more than 64 KiB of dynamic LDS (gfx950: 160 KiB per CU)
     if (!lds_raised) {
-        const int most = std::max(PT_XSX * stage_len(PT_MMAX * PT_PMAX), 4 * PT_XSX * stage_len(PT_MMAX * PT_PMAX / PT_RBLK));
-        TCS_HIP(hipFuncSetAttribute((const void *)k_ptdma_part_rows_src<T, CYC, Src>,
+        const int most = std::max(XSX * stage_len(MM * PM), 4 * XSX * stage_len(MM * PM / PT_RBLK));
+        TCS_HIP(hipFuncSetAttribute((const void *)k_ptdma_part_rows_src<T, CYC, Src, XSX, MM, PM>,
                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(T) * most));
         lds_raised = true;
     }
-    const dim3 blk(PT_XSX * P), grd((unsigned)((n0 + PT_XSX - 1) / PT_XSX), (unsigned)n1);
-    TCS_LAUNCH(st, label, (k_ptdma_part_rows_src<T, CYC, Src>), grd, blk, lds, src, D, n0, ss0, ss1, n_row, ls, lsb,
-               P, w1, w2);
+    const dim3 blk(XSX * q.P), grd((unsigned)((n0 + XSX - 1) / XSX), (unsigned)n1);
+    TCS_LAUNCH(st, label, (k_ptdma_part_rows_src<T, CYC, Src, XSX, MM, PM>), grd, blk, lds, src, D, n0, ss0, ss1, n_row,
+               ls, lsb, q.P, q.w1, q.w2);
     return TCS_OK;
+}
+template <bool CYC, bool ANY, typename T, class Src>
+int ptdma_part_rows_src_launch(hipStream_t st, const char *label, const Src &src, T *D, int n0, long ss0, int n1,
+                               long ss1, int n_row) {
+    PartPlan q;
+    if (n0 <= 0 || n1 <= 0) return TCS_OK;
+    if (!part_plan_for<ANY>(n_row, (long)n0 * n1, q) || n1 > 65535) {
+        set_error("ptdma_part: line length outside the split range or outer line count > 65535");
+        return TCS_E_ARG;
+    }
+    constexpr int M = PT_MMAX, PP = PT_PMAX, X = PT_XSX;
+    if constexpr (ANY) {
+        if constexpr (sizeof(T) == 8)
+            if (q.pm == 2 * PP) return part_rows_src_launch<CYC, X, M, 2 * PP>(st, label, src, q, D, n0, ss0, n1, ss1, n_row);
+        if constexpr (sizeof(T) == 8)
+            if (q.pm == 4 * PP) return part_rows_src_launch<CYC, X, M, 4 * PP>(st, label, src, q, D, n0, ss0, n1, ss1, n_row);
+        if (q.mm == 8) return part_rows_src_launch<CYC, 8, 8, PP>(st, label, src, q, D, n0, ss0, n1, ss1, n_row);
+        if (q.mm == 4) return part_rows_src_launch<CYC, 8, 4, PP>(st, label, src, q, D, n0, ss0, n1, ss1, n_row);
+    }
+    if (q.P < PP / 2) return part_rows_src_launch<CYC, 8, M, PP>(st, label, src, q, D, n0, ss0, n1, ss1, n_row);
+    return part_rows_src_launch<CYC, X, M, PP>(st, label, src, q, D, n0, ss0, n1, ss1, n_row);
 }
 
 }  // namespace tcs

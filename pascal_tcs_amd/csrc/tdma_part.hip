@@ -36,10 +36,8 @@ namespace tcs {
 
 bool ptdma_part_plan(int n_row, int &P, int &w1, int &w2) {
     if (n_row < 2 || n_row > PT_MMAX * PT_PMAX) return false;
-    P = 1;
-    while (P * PT_MMAX < n_row) P <<= 1;  // power of two: the cyclic reduction pairs rows i, i + P
-    w1 = n_row / P;
-    w2 = n_row % P;
+    const PartPlan q = part_plan(n_row, PT_MMAX, PT_PMAX);
+    P = q.P; w1 = q.w1; w2 = q.w2;
     return true;
 }
 
@@ -64,7 +62,7 @@ template <typename T, bool CYC, int SX>
 __global__ void __launch_bounds__(SX * PT_PMAX)
 k_ptdma_part(const T *__restrict__ A, const T *__restrict__ B, const T *__restrict__ C,
              T *__restrict__ D, int n0, long ss1, long rs, int P, int w1, int w2, LineOut out) {
-    __shared__ RedLDS<T, SX, 1> red;
+    __shared__ RedLDS<T, SX, 1, PT_PMAX> red;
     const int t = threadIdx.x;
     const int line = t % SX, p = t / SX;
     const int s0 = line_group<SX>(blockIdx.x, gridDim.x) * SX + line;
@@ -85,12 +83,12 @@ k_ptdma_part(const T *__restrict__ A, const T *__restrict__ B, const T *__restri
                 a[r] = T(0); b[r] = T(1); c[r] = T(0); d[0][r] = T(0);
             }
         }
-        reduce<T, 1>(a, b, c, d, m);
+        reduce<T, 1, PT_MMAX>(a, b, c, d, m);
     }
     T xf[1], xl[1];
-    exchange<T, CYC, SX, 1>(red, line, p, P, a, c, d, m, xf, xl);
+    exchange<T, CYC, SX, 1, PT_MMAX, PT_PMAX>(red, line, p, P, a, c, d, m, xf, xl);
     if (!act) return;
-    store<T>(a, c, d, j0, m, xf[0], xl[0], D, base, rs, out, s0, blockIdx.y);
+    store<T, PT_MMAX>(a, c, d, j0, m, xf[0], xl[0], D, base, rs, out, s0, blockIdx.y);
 }
 
 // Contiguous lines (rows 1 apart): line (s0, s1) starts at s0*ss0 + s1*ss1.
@@ -107,7 +105,7 @@ k_ptdma_part_rows(const T *__restrict__ A, const T *__restrict__ B, const T *__r
                   int n0, long ss0, long ss1, int n_row, int ls, int P, int w1, int w2) {
     extern __shared__ __align__(16) unsigned char stage_raw[];
     T *stage = reinterpret_cast<T *>(stage_raw);
-    __shared__ RedLDS<T, PT_SX, 1> red;
+    __shared__ RedLDS<T, PT_SX, 1, PT_PMAX> red;
     const int t = threadIdx.x;
     const int line = t % PT_SX, p = t / PT_SX;
     const int s0 = blockIdx.x * PT_SX + line;
@@ -140,14 +138,14 @@ k_ptdma_part_rows(const T *__restrict__ A, const T *__restrict__ B, const T *__r
 #pragma unroll
         for (int r = 0; r < PT_MMAX; r++) dst[r] = (act && r < m) ? stage[line * ls + stage_pos(j0 + r)] : pad;
     }
-    reduce<T, 1>(a, b, c, d, m);
+    reduce<T, 1, PT_MMAX>(a, b, c, d, m);
     T xf[1], xl[1];
-    exchange<T, CYC, PT_SX, 1>(red, line, p, P, a, c, d, m, xf, xl);
+    exchange<T, CYC, PT_SX, 1, PT_MMAX, PT_PMAX>(red, line, p, P, a, c, d, m, xf, xl);
     // every thread has read the stage before exchange's first barrier
     if (act) {
 #pragma unroll
         for (int r = 0; r < PT_MMAX; r++)
-            if (r < m) stage[line * ls + stage_pos(j0 + r)] = x_of<T, 1>(a, c, d, 0, r, m, xf[0], xl[0]);
+            if (r < m) stage[line * ls + stage_pos(j0 + r)] = x_of<T, 1, PT_MMAX>(a, c, d, 0, r, m, xf[0], xl[0]);
     }
     __syncthreads();
     if (row_ok) {

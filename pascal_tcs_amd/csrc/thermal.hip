@@ -517,6 +517,20 @@ int thermal_coeffi(tcs_ctx *c) {
     return TCS_OK;
 }
 
+// The x rows evaluate seven property polynomials each: made by the workgroup
+// inside the contiguous-line solve they leave it waiting on them, so they go
+// through the scratch as a kernel of their own (2.59 against 2.74 ms at
+// 512^3) -- except for lines too long for the stored-line split, which
+// otherwise would be solved as single-rank lines.
+static int thermal_x_stage(tcs_ctx *c, const ThermalX &row) {
+    scr_t *am = SCR(c->am), *ac = SCR(c->ac), *ap = SCR(c->ap), *rhs = SCR(c->rhs);
+    if constexpr (ANY_SPLIT && sizeof(scr_t) == 8)
+        if (c->n1m > PT_MMAX * PT_PMAX && rows_in_solve<scr_t, ANY_SPLIT>(c, c->n1m))
+            return x_stage<ANY_SPLIT>(c, "thermal_x", "thermal_x_solve", row, 1, am, ac, ap, rhs);
+    TCS_TRY(rows3d_launch<false>(c, "thermal_x", row, 1, am, ac, ap, rhs));
+    return ptdma_sweep(c, am, ac, ap, rhs, c->n2m, c->n1m, c->n3m, (long)c->n1m * c->n2m, c->n1m, 1, true);
+}
+
 int thermal_solver(tcs_ctx *c, double dt) {
     TCS_TRY(ensure_twins(c, TWIN_T | TWIN_U | TWIN_V | TWIN_W | TWIN_WALL));  // the mixed form's FP32 rows
     c->twin_ok &= ~(unsigned)TWIN_T;
@@ -524,17 +538,13 @@ int thermal_solver(tcs_ctx *c, double dt) {
     double *T = c->f[TCS_T];
     scr_t *am = SCR(c->am), *ac = SCR(c->ac), *ap = SCR(c->ap), *rhs = SCR(c->rhs);
     const ThermalZ z{g, c->phys, dt, T, c->f[TCS_U], c->f[TCS_V], c->f[TCS_W], c->wall[TCS_TBCUP], c->wall[TCS_TBCBT]};
-    TCS_TRY(z_stage(c, "thermal_z", "thermal_z_solve", z, 1, am, ac, ap, rhs));
-    // The x rows evaluate seven property polynomials each: made by the
-    // workgroup inside the contiguous-line solve they leave it waiting on
-    // them, so here they go through the scratch as a kernel of their own.
-    TCS_TRY(rows3d_launch<false>(c, "thermal_x", ThermalX{g, c->phys, dt, T, c->f[TCS_U]}, 1, am, ac, ap, rhs));
-    TCS_TRY(ptdma_sweep(c, am, ac, ap, rhs, c->n2m, c->n1m, c->n3m, (long)c->n1m * c->n2m, c->n1m, 1, true));
+    TCS_TRY(z_stage<ANY_SPLIT>(c, "thermal_z", "thermal_z_solve", z, 1, am, ac, ap, rhs));
+    TCS_TRY(thermal_x_stage(c, ThermalX{g, c->phys, dt, T, c->f[TCS_U]}));
     const ThermalY y{g, c->phys, dt, T, c->f[TCS_V]};
-    if (rows_in_solve<scr_t>(c, c->n2m)) {
+    if (rows_in_solve<scr_t, ANY_SPLIT>(c, c->n2m)) {
         // the y rows read T around every cell, so the increment goes through
         // the scratch and is added once every line is solved
-        TCS_TRY(y_stage_in_solve(c, "thermal_y_solve", y, 1, c->n2m, rhs, nullptr, 0));
+        TCS_TRY(y_stage_in_solve<ANY_SPLIT>(c, "thermal_y_solve", y, 1, c->n2m, rhs, nullptr, 0));
         TCS_LAUNCH(c->stream, "add_interior", k_interior_out<2>, interior_grid(c->n1m, c->n2m, c->n3m),
                    interior_block(), 0, g, 1, T, rhs);
         return TCS_OK;
@@ -548,16 +558,15 @@ int thermal_solver(tcs_ctx *c, double dt) {
 // otherwise the plain routine (*written = false, T updated in place).
 int thermal_solver_into(tcs_ctx *c, double dt, double *Tn, bool *written) {
     *written = false;
-    if (!rows_in_solve<scr_t>(c, c->n2m)) return thermal_solver(c, dt);
+    if (!rows_in_solve<scr_t, ANY_SPLIT>(c, c->n2m)) return thermal_solver(c, dt);
     TCS_TRY(ensure_twins(c, TWIN_T | TWIN_U | TWIN_V | TWIN_W | TWIN_WALL));  // the mixed form's FP32 rows
     c->twin_ok &= ~(unsigned)TWIN_T;
     const Grid g = c->grid();
     double *T = c->f[TCS_T];
     scr_t *am = SCR(c->am), *ac = SCR(c->ac), *ap = SCR(c->ap), *rhs = SCR(c->rhs);
     const ThermalZ z{g, c->phys, dt, T, c->f[TCS_U], c->f[TCS_V], c->f[TCS_W], c->wall[TCS_TBCUP], c->wall[TCS_TBCBT]};
-    TCS_TRY(z_stage(c, "thermal_z", "thermal_z_solve", z, 1, am, ac, ap, rhs));
-    TCS_TRY(rows3d_launch<false>(c, "thermal_x", ThermalX{g, c->phys, dt, T, c->f[TCS_U]}, 1, am, ac, ap, rhs));
-    TCS_TRY(ptdma_sweep(c, am, ac, ap, rhs, c->n2m, c->n1m, c->n3m, (long)c->n1m * c->n2m, c->n1m, 1, true));
+    TCS_TRY(z_stage<ANY_SPLIT>(c, "thermal_z", "thermal_z_solve", z, 1, am, ac, ap, rhs));
+    TCS_TRY(thermal_x_stage(c, ThermalX{g, c->phys, dt, T, c->f[TCS_U]}));
     TCS_TRY(copy_shell(c, T, Tn));
     const long n1 = c->n1m, n12 = (long)c->n1m * c->n2m;
     LineOut out;
@@ -572,7 +581,7 @@ int thermal_solver_into(tcs_ctx *c, double dt, double *Tn, bool *written) {
     // FP64 lines 8 a workgroup (1.96 -> 1.91 ms at 512^3), FP32 lines 16
     // (8: 1.52 -> 1.96 ms)
     constexpr int SX = sizeof(scr_t) == 8 ? 8 : PT_SX;
-    const int rc = ptdma_part_src_launch<false, SX>(c->stream, "thermal_y_solve",
+    const int rc = ptdma_part_src_launch<false, SX, ANY_SPLIT>(c->stream, "thermal_y_solve",
                                                     YLineRows<ThermalY, scr_t>{ThermalY{g, c->phys, dt, T, c->f[TCS_V]},
                                                                                twin_w(c), rhs, 1},
                                                     rhs, c->n1m, c->n3m, n12, c->n2m, n1, out);
