@@ -46,18 +46,6 @@ __device__ __forceinline__ void mu_ir_of_T(const Phys &p, S T, S &mu, S &ir) {
     ir = sc<S>(p.Rho0) / (sc<S>(p.a10) + sc<S>(p.a10) * (sc<S>(p.a11) * tmp1 + sc<S>(p.a12) * tmp2 + sc<S>(p.a13) * tmp3 + sc<S>(p.a14) * tmp4 + sc<S>(p.a15) * tmp5));
 }
 
-// on the (j,k) table from T(n1sub,j,k)
-__global__ void k_momentum_coeffi(Grid g, Phys p, const double *__restrict__ T, double *__restrict__ Mu,
-                                  double *__restrict__ iR) {
-    const int j = blockIdx.x * blockDim.x + threadIdx.x;
-    const int k = blockIdx.y;
-    if (j >= g.N2) return;
-    double mu, ir;
-    mu_ir_of_T(p, T[g.ix(g.n1m + 1, j, k)], mu, ir);
-    Mu[g.t2(j, k)] = mu;
-    iR[g.t2(j, k)] = ir;
-}
-
 // the stage-1 last-point viscosities that later stages reuse
 template <class S, class FP>
 __device__ __forceinline__ void stale_values(const Grid &g, FP Mu, S (&out)[6]) {
@@ -87,10 +75,60 @@ __device__ __forceinline__ void stale_values(const Grid &g, FP Mu, S (&out)[6]) 
     }
 }
 
-__global__ void k_momentum_stale(Grid g, const double *__restrict__ Mu, double *__restrict__ out) {
+// The Mu table for the stale scalars, read (T null) or as its entries are
+// made: the same scalars to the last bit either way, so neither the value nor
+// its uses may be merged with what is around them where the arithmetic is
+// contracted.
+struct MuTable {
+    const Grid &g;
+    const Phys &p;
+    const double *T, *Mu;
+    __device__ __forceinline__ double operator[](size_t q) const {
+        double mu, ir;
+        if (T) {
+            double t = T[g.ix(g.n1m + 1, (int)(q % g.N2), (int)(q / g.N2))];
+            asm volatile("" : "+v"(t));
+            mu_ir_of_T(p, t, mu, ir);
+        } else {
+            mu = Mu[q];
+        }
+        asm volatile("" : "+v"(mu));
+        return mu;
+    }
+};
+
+// on the (j,k) table from T(n1sub,j,k); the workgroups past the last k make
+// the stale scalars from the same temperatures
+__global__ void k_momentum_coeffi(Grid g, Phys p, const double *__restrict__ T, double *__restrict__ Mu,
+                                  double *__restrict__ iR, double *__restrict__ stale, float *Mu32, float *iR32,
+                                  float *stale32) {
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    const int k = blockIdx.y;
+    if (k == g.N3) {
+        if (j != 0) return;
+        double v[6];
+        stale_values<double>(g, MuTable{g, p, T, nullptr}, v);
+        for (int q = 0; q < 6; q++) {
+            stale[q] = v[q];
+            if (stale32) stale32[q] = (float)v[q];
+        }
+        return;
+    }
+    if (j >= g.N2) return;
+    double mu, ir;
+    mu_ir_of_T(p, T[g.ix(g.n1m + 1, j, k)], mu, ir);
+    Mu[g.t2(j, k)] = mu;
+    iR[g.t2(j, k)] = ir;
+    if (Mu32) {  // the mixed form: the FP32 copies as well
+        Mu32[g.t2(j, k)] = (float)mu;
+        iR32[g.t2(j, k)] = (float)ir;
+    }
+}
+
+__global__ void k_momentum_stale(Grid g, Phys p, const double *__restrict__ Mu, double *__restrict__ out) {
     if (threadIdx.x != 0 || blockIdx.x != 0) return;
     double v[6];
-    stale_values<double>(g, Mu, v);
+    stale_values<double>(g, MuTable{g, p, nullptr, Mu}, v);
     for (int q = 0; q < 6; q++) out[q] = v[q];
 }
 
@@ -903,6 +941,16 @@ __global__ void __launch_bounds__(256) k_blockLdV_pseudo(BlockLdV cell, Acc acc,
         if (j >= 2) dV[q] = o[c];
         Vn[q] = vn[c];
     }
+    if (g.edge(i0, LDV_IB, j, blockIdx.z * LDV_KB + 1, LDV_KB)) {
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+            const int i = i0 + c % LDV_IB, k = blockIdx.z * LDV_KB + c / LDV_IB + 1;
+            const size_t q = g.ix(i, j, k);
+            if (j >= 2) g.images(dV, i, k, q, o[c]);
+            g.images(Vn, i, k, q, vn[c]);
+            g.wall(Vn, cell.V, i, j, k);
+        }
+    }
 }
 
 template <typename E, class Acc>
@@ -951,15 +999,17 @@ static inline auto cell_access(const tcs_ctx *c) {
 constexpr unsigned MOMENTUM_TWINS = TWIN_U | TWIN_V | TWIN_W | TWIN_P | TWIN_T | TWIN_TAB | TWIN_WALL;
 
 int momentum_coeffi(tcs_ctx *c) {
-    c->twin_ok &= ~(unsigned)TWIN_TAB;
-    TCS_LAUNCH(c->stream, "momentum_coeffi", k_momentum_coeffi, dim3((c->N2 + 63) / 64, c->N3), dim3(64), 0, c->grid(),
-                       c->phys, c->f[TCS_T], c->f[TCS_MU], c->f[TCS_INVRHO]);
+    TCS_LAUNCH(c->stream, "momentum_coeffi", k_momentum_coeffi, dim3((c->N2 + 63) / 64, c->N3 + 1), dim3(64), 0,
+               c->grid(), c->phys, c->f[TCS_T], c->f[TCS_MU], c->f[TCS_INVRHO], c->stale, twin(c, c->f[TCS_MU]),
+               twin(c, c->f[TCS_INVRHO]), twin(c, c->stale));
+    if (c->a32) c->twin_ok |= TWIN_TAB | TWIN_STALE;
     return TCS_OK;
 }
 
 static int launch_stale(tcs_ctx *c) {
+    if (c->wrap) return TCS_OK;  // a step: made with the table
     c->twin_ok &= ~(unsigned)TWIN_STALE;
-    TCS_LAUNCH(c->stream, "momentum_stale", k_momentum_stale, dim3(1), dim3(64), 0, c->grid(), c->f[TCS_MU], c->stale);
+    TCS_LAUNCH(c->stream, "momentum_stale", k_momentum_stale, dim3(1), dim3(64), 0, c->grid(), c->phys, c->f[TCS_MU], c->stale);
     return TCS_OK;
 }
 
@@ -1008,8 +1058,10 @@ int momentum_solvedV(tcs_ctx *c, double dt) {
     TCS_TRY(z_stage<ANY_SPLIT>(c, "dV_z", "dV_z_solve", z, 2, am, ac, ap, rhs));
     TCS_TRY(x_stage<ANY_SPLIT>(c, "dV_x", "dV_x_solve", DVX{g, c->phys, dt, f[TCS_U], f[TCS_INVRHO], c->stale}, 2, am, ac, ap,
                     rhs));
-    TCS_LAUNCH(c->stream, "dV_zero_rows", k_dV_zero_rows<inc_t>, dim3((c->N1 + 63) / 64, c->N3), dim3(64), 0, g,
-               inc(c, TCS_DV));
+    if (!(c->kept >> TCS_DV & 1))
+        TCS_LAUNCH(c->stream, "dV_zero_rows", k_dV_zero_rows<inc_t>, dim3((c->N1 + 63) / 64, c->N3), dim3(64), 0, g,
+                   inc(c, TCS_DV));
+    if (c->wrap) c->kept |= 1u << TCS_DV;
     return y_stage<sizeof(scr_t) == 8 ? 8 : 16, true>(c, "dV_y", "dV_y_solve", DVY{g, c->phys, dt, f[TCS_V], f[TCS_MU], f[TCS_INVRHO]}, 2, f[TCS_DV]);
 }
 
@@ -1077,6 +1129,17 @@ __global__ void __launch_bounds__(256) k_blockLdU_pseudo(BlockLdU cell, Acc acc,
         Un[q] = un[c];
         Wn[q] = wn[c];
     }
+    if (g.edge(i0, LDU_IB, j, blockIdx.z * LDU_KB + 1, LDU_KB)) {
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+            const int i = i0 + c % LDU_IB, k = blockIdx.z * LDU_KB + c / LDU_IB + 1;
+            const size_t q = g.ix(i, j, k);
+            g.images(Un, i, k, q, un[c]);
+            g.images(Wn, i, k, q, wn[c]);
+            g.wall(Un, cell.U, i, j, k);
+            g.wall(Wn, W, i, j, k);
+        }
+    }
 }
 
 int momentum_blockLdV_pseudo(tcs_ctx *c, double dt, double *Vn) {
@@ -1084,7 +1147,7 @@ int momentum_blockLdV_pseudo(tcs_ctx *c, double dt, double *Vn) {
     const BlockLdV cell{c->grid(), c->phys, dt, c->f[TCS_V], c->f[TCS_DW], c->f[TCS_MU], c->f[TCS_INVRHO], c->f[TCS_DV]};
     TCS_TRY(ensure_twins(c, TWIN_V | TWIN_TAB));
     c->twin_ok &= ~(unsigned)TWIN_V;  // Vn becomes V
-    TCS_TRY(copy_shell(c, c->f[TCS_V], Vn));
+    if (!c->wrap) TCS_TRY(copy_shell(c, {TCS_V}));
     auto acc = cell_access(c);
     TCS_LAUNCH(c->stream, "blockLdV", (k_blockLdV_pseudo<inc_t, decltype(acc)>), grd, blk, 0, cell, acc,
                inc(c, TCS_DV), Vn);
@@ -1097,7 +1160,7 @@ int momentum_blockLdU_pseudo(tcs_ctx *c, double dt, double *Un, double *Wn) {
                         c->f[TCS_MU], c->f[TCS_INVRHO], c->f[TCS_DU]};
     TCS_TRY(ensure_twins(c, TWIN_U | TWIN_TAB));
     c->twin_ok &= ~(unsigned)(TWIN_U | TWIN_W);  // Un, Wn become U, W
-    TCS_TRY(copy_shell(c, {{c->f[TCS_U], Un}, {c->f[TCS_W], Wn}}));
+    if (!c->wrap) TCS_TRY(copy_shell(c, {TCS_U, TCS_W}));
     auto acc = cell_access(c);
     TCS_LAUNCH(c->stream, "blockLdU", (k_blockLdU_pseudo<inc_t, decltype(acc)>), grd, blk, 0, cell, acc,
                c->f[TCS_W], inc(c, TCS_DW), inc(c, TCS_DU), Un, Wn);

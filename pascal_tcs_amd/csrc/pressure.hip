@@ -438,6 +438,21 @@ k_fft_x_inv(Grid g, int h1p, int TX, const double2 *__restrict__ spec, const dou
             const int l = e / n, t = e - l * n;
             dP[g.ix(t + 1, j, k0 + l + 1)] = re[fpad(e)] / fn1 / fn3 - mean;
         }
+        if (!g.wrap) return;
+        // the periodic ghosts: the rows' two ends, then whole ghost rows
+        for (int e = tid; e < 2 * TX; e += NT) {
+            const int l = e / 2, t = e % 2 ? 0 : n - 1, k = k0 + l + 1;
+            const double v = re[fpad(l * n + t)] / fn1 / fn3 - mean;
+            const long q = (long)g.ix(t ? 0 : n + 1, j, k);
+            dP[q] = v;
+            if (k == 1 || k == g.n3m) dP[q + (k == 1 ? (long)g.n3m : -(long)g.n3m) * g.P1 * g.N2] = v;
+        }
+        for (int l = 0; l < TX; l++) {
+            const int k = k0 + l + 1;
+            if (k != 1 && k != g.n3m) continue;
+            const int kg = k == 1 ? g.n3m + 1 : 0;
+            for (int t = tid; t < n; t += NT) dP[g.ix(t + 1, j, kg)] = re[fpad(l * n + t)] / fn1 / fn3 - mean;
+        }
         return;
     }
     for (int e = tid; e < TX * n; e += NT) {
@@ -457,54 +472,79 @@ k_fft_x_inv(Grid g, int h1p, int TX, const double2 *__restrict__ spec, const dou
     for (int l = tid; l < TX; l += NT) linesum[(size_t)(j - 1) + (size_t)g.n2m * (k0 + l)] = im[l * n];
 }
 
+// pairwise sum of the P values in buf (P a power of two); every thread gets it
+__device__ double block_tree_fold(double *buf, int P) {
+    for (int h = P / 2; h >= 1; h >>= 1) {
+        for (int t = threadIdx.x; t < h; t += blockDim.x) buf[t] = buf[t] + buf[t + h];
+        __syncthreads();
+    }
+    const double s = buf[0];
+    __syncthreads();  // buf may be filled again
+    return s;
+}
+
 // pairwise sum of `cnt` values at src + q*stride, zero padded to a power of two
 __device__ double block_tree_sum(const double *__restrict__ src, int cnt, size_t stride, double *buf) {
     int P = 1;
     while (P < cnt) P <<= 1;
     for (int t = threadIdx.x; t < P; t += blockDim.x) buf[t] = (t < cnt) ? src[(size_t)t * stride] : 0.0;
     __syncthreads();
-    for (int h = P / 2; h >= 1; h >>= 1) {
-        for (int t = threadIdx.x; t < h; t += blockDim.x) buf[t] = buf[t] + buf[t + h];
-        __syncthreads();
-    }
-    return buf[0];
+    return block_tree_fold(buf, P);
 }
 
-// The fast forms' line sums from the spectrum after the z c2c: line (j, k)
-// sums to the kx = 0 coefficient over n3m (see SPECTRAL_MEAN).
-__global__ void k_spec_linesum(int n2m, int n3m, int h1p, const double2 *__restrict__ spec,
-                               double *__restrict__ linesum) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = blockIdx.y;  // 0-based
-    if (k >= n3m) return;
-    linesum[(size_t)j + (size_t)n2m * k] = spec[(size_t)n3m * h1p * j + k].x / (double)n3m;
-}
-
-__global__ void k_plane_sum(int n2m, const double *__restrict__ linesum, double *__restrict__ planesum) {
-    extern __shared__ double buf[];
+// Line sums -> plane sums -> the mean, in one launch: workgroup k sums plane
+// k (its lines in pairs, as the reference's sums are taken here), and the
+// last workgroup to finish sums the planes.  SPEC
+// (the fast forms): line (j, k) sums to the kx = 0 coefficient over n3m (see
+// SPECTRAL_MEAN), read from the spectrum; otherwise linesum holds the lines.
+template <bool SPEC>
+__global__ void __launch_bounds__(256)
+k_mean(int n1m, int n2m, int n3m, int h1p, const double2 *__restrict__ spec, const double *__restrict__ linesum,
+       double *planesum, double *scal, unsigned *count) {
+    extern __shared__ double buf[];  // a power of two >= n2m and >= n3m
     const int k = blockIdx.x;
-    const double s = block_tree_sum(linesum + (size_t)n2m * k, n2m, 1, buf);
-    if (threadIdx.x == 0) planesum[k] = s;
-}
-
-__global__ void k_total_mean(int n1m, int n2m, int n3m, const double *__restrict__ planesum,
-                             double *__restrict__ scal) {
-    extern __shared__ double buf[];
-    const double s = block_tree_sum(planesum, n3m, 1, buf);
+    double s;
+    if (SPEC) {
+        int P = 1;
+        while (P < n2m) P <<= 1;
+        for (int t = threadIdx.x; t < P; t += blockDim.x)
+            buf[t] = t < n2m ? spec[(size_t)n3m * h1p * t + k].x / (double)n3m : 0.0;
+        __syncthreads();
+        s = block_tree_fold(buf, P);
+    } else {
+        s = block_tree_sum(linesum + (size_t)n2m * k, n2m, 1, buf);
+    }
+    if (threadIdx.x == 0) {
+        last_put(planesum + k, s);
+        buf[0] = last_arrive(count, gridDim.x);
+    }
+    __syncthreads();
+    const bool last = buf[0] != 0.0;
+    __syncthreads();
+    if (!last) return;
+    int P = 1;
+    while (P < n3m) P <<= 1;
+    for (int t = threadIdx.x; t < P; t += blockDim.x)
+        buf[t] = t < n3m ? last_get(planesum + t) : 0.0;
+    __syncthreads();
+    s = block_tree_fold(buf, P);
     if (threadIdx.x == 0) scal[0] = s / (double)n1m / (double)n2m / (double)n3m;
 }
 
-__global__ void k_dp_subtract(Grid g, const double *__restrict__ scal, double *__restrict__ dP) {
+__global__ void k_dp_subtract(Grid g, const double *__restrict__ scal, double *dP) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
     const int j = blockIdx.y * blockDim.y + threadIdx.y + 1;
     const int k = blockIdx.z + 1;
     if (i > g.n1m || j > g.n2m) return;
     const size_t q = g.ix(i, j, k);
-    dP[q] = dP[q] - scal[0];
+    const double v = dP[q] - scal[0];
+    dP[q] = v;
+    if (g.edge(i, 1, j, k, 1)) g.images(dP, i, k, q, v);
 }
 
-// quadratic wall extrapolation (:719-736) of dP (mode 0) or P (mode 1)
-__global__ void k_wall_extrap(Grid g, double *__restrict__ F) {
+// quadratic wall extrapolation (:719-736) of dP or P, with the wall rows'
+// periodic ghosts; F32 (the mixed form, not null): the FP32 copy as well
+__global__ void k_wall_extrap(Grid g, double *F, float *F32) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
     const int k = blockIdx.y + 1;
     if (i > g.n1m) return;
@@ -513,11 +553,22 @@ __global__ void k_wall_extrap(Grid g, double *__restrict__ F) {
     const double s = dmx2[1] + dmx2[2];
     const double a0 = (s * s) / ((s * s) - (dmx2[1] * dmx2[1]));
     const double b0 = (dmx2[1] * dmx2[1]) / ((s * s) - (dmx2[1] * dmx2[1]));
-    F[g.ix(i, 0, k)] = a0 * F[g.ix(i, 1, k)] - b0 * F[g.ix(i, 2, k)];
+    const double lo = a0 * F[g.ix(i, 1, k)] - b0 * F[g.ix(i, 2, k)];
+    const size_t q0 = g.ix(i, 0, k), q1 = g.ix(i, n2sub, k);
+    F[q0] = lo;
     const double t = dmx2[n2sub] + dmx2[n2msub];
     const double a1 = (t * t) / ((t * t) - (dmx2[n2sub] * dmx2[n2sub]));
     const double b1 = (dmx2[n2sub] * dmx2[n2sub]) / ((t * t) - (dmx2[n2sub] * dmx2[n2sub]));
-    F[g.ix(i, n2sub, k)] = a1 * F[g.ix(i, n2msub, k)] - b1 * F[g.ix(i, n2sub - 2, k)];
+    const double hi = a1 * F[g.ix(i, n2msub, k)] - b1 * F[g.ix(i, n2sub - 2, k)];
+    F[q1] = hi;
+    if (F32) F32[q0] = (float)lo, F32[q1] = (float)hi;
+    if (!g.wrap) return;
+    g.images(F, i, k, q0, lo);
+    g.images(F, i, k, q1, hi);
+    if (F32) {
+        g.images(F32, i, k, q0, (float)lo);
+        g.images(F32, i, k, q1, (float)hi);
+    }
 }
 
 // projection (:793-851).  The reference overwrites dPhat(i,j,k) inside the
@@ -645,6 +696,28 @@ __global__ void __launch_bounds__(256) k_projection_into(Projection cell, DPhatU
             tw.f[3][o] = (float)q[c];
         }
     }
+    if (g.edge(i0, PROJ_IB, j, blockIdx.z * PROJ_KB + 1, PROJ_KB)) {
+#pragma unroll
+        for (int c = 0; c < NC; c++) {
+            const int i = i0 + c % PROJ_IB, k = blockIdx.z * PROJ_KB + c / PROJ_IB + 1;
+            const size_t o = g.ix(i, j, k);
+            g.images(U, i, k, o, u[c]);
+            g.images(V, i, k, o, v[c]);
+            g.images(W, i, k, o, w[c]);
+            g.images(P, i, k, o, q[c]);
+            g.images(dPhatn, i, k, o, h[c]);
+            g.wall(dPhatn, cell.dPhat, i, j, k);
+            if (TW) {
+                g.images(tw.f[0], i, k, o, (float)u[c]);
+                g.images(tw.f[1], i, k, o, (float)v[c]);
+                g.images(tw.f[2], i, k, o, (float)w[c]);
+                g.images(tw.f[3], i, k, o, (float)q[c]);
+                g.wall(tw.f[0], U, i, j, k);
+                g.wall(tw.f[1], V, i, j, k);
+                g.wall(tw.f[2], W, i, j, k);
+            }
+        }
+    }
 }
 
 __global__ void __launch_bounds__(256) k_dphat_update(DPhatUpdate cell, double *dPhat, double *dP0) {
@@ -769,26 +842,19 @@ static int poisson_after_x(tcs_ctx *c) {
                    c->dxk2, c->dzk, spec, c->pA, c->pC, n2m - kept);
     }
     TCS_TRY(fft_z_launch<+1>(c, "fft_z<+1>", spec));
-    if (SPECTRAL_MEAN)
-        TCS_LAUNCH(c->stream, "spec_linesum", k_spec_linesum, dim3((n3m + 255) / 256, n2m), dim3(256), 0, n2m, n3m,
-                   h1p, spec, c->linesum);
-    else
-        TCS_TRY(fft_x_inv_launch(c, "fft_x_inv", spec, c->f[TCS_DP]));
-    int P2 = 1;
-    while (P2 < n2m) P2 <<= 1;
-    TCS_LAUNCH(c->stream, "plane_sum", k_plane_sum, dim3(n3m), dim3(256), P2 * sizeof(double), n2m, c->linesum,
-                       c->planesum);
-    int P3 = 1;
-    while (P3 < n3m) P3 <<= 1;
-    TCS_LAUNCH(c->stream, "total_mean", k_total_mean, dim3(1), dim3(256), P3 * sizeof(double), n1m, n2m, n3m,
-                       c->planesum, c->scal);
+    if (!SPECTRAL_MEAN) TCS_TRY(fft_x_inv_launch(c, "fft_x_inv", spec, c->f[TCS_DP]));
+    int PM = 1;
+    while (PM < std::max(n2m, n3m)) PM <<= 1;
+    TCS_LAUNCH(c->stream, "mean", k_mean<SPECTRAL_MEAN>, dim3(n3m), dim3(256), PM * sizeof(double), n1m, n2m, n3m, h1p,
+               spec, c->linesum, c->planesum, c->scal, (unsigned *)(c->scal + 1));
     if (SPECTRAL_MEAN) {
         TCS_TRY(fft_x_inv_launch(c, "fft_x_inv", spec, c->f[TCS_DP], true));
     } else {
         const dim3 blk = interior_block(), grd = interior_grid(n1m, n2m, n3m);
         TCS_LAUNCH(c->stream, "dp_subtract", k_dp_subtract, grd, blk, 0, g, c->scal, c->f[TCS_DP]);
     }
-    TCS_LAUNCH(c->stream, "wall_extrap", k_wall_extrap, dim3((n1m + 63) / 64, n3m), dim3(64), 0, g, c->f[TCS_DP]);
+    TCS_LAUNCH(c->stream, "wall_extrap", k_wall_extrap, dim3((n1m + 63) / 64, n3m), dim3(64), 0, g, c->f[TCS_DP],
+               (float *)nullptr);
     return TCS_OK;
 }
 
@@ -814,7 +880,8 @@ int pressure_projection(tcs_ctx *c, double dt) {
                c->f[TCS_P]);
     TCS_LAUNCH(c->stream, "dphat_update", k_dphat_update, grd, blk, 0, DPhatUpdate{g, c->f[TCS_DP], c->f[TCS_DPHAT],
                c->f[TCS_DP0]}, c->f[TCS_DPHAT], c->f[TCS_DP0]);
-    TCS_LAUNCH(c->stream, "wall_extrap", k_wall_extrap, dim3((c->n1m + 63) / 64, c->n3m), dim3(64), 0, g, c->f[TCS_P]);
+    TCS_LAUNCH(c->stream, "wall_extrap", k_wall_extrap, dim3((c->n1m + 63) / 64, c->n3m), dim3(64), 0, g, c->f[TCS_P],
+               twin(c, c->f[TCS_P]));
     return TCS_OK;
 }
 
@@ -824,7 +891,9 @@ int pressure_projection_into(tcs_ctx *c, double dt, double *dPhatn, double *dP0n
     const dim3 blk = interior_block(), grd = cell_grid(c->n1m, c->n2m, c->n3m, PROJ_KB, interior_block(), PROJ_IB);
     const Projection cell{g, c->phys, dt, c->f[TCS_INVRHO], c->f[TCS_DP], c->f[TCS_DPHAT], c->f[TCS_DP0],
                           c->f[TCS_U], c->f[TCS_V], c->f[TCS_W], c->f[TCS_P]};
-    TCS_TRY(copy_shell(c, {{c->f[TCS_DPHAT], dPhatn}, {c->f[TCS_DP0], dP0n}}));
+    if (!c->wrap) TCS_TRY(copy_shell(c, {TCS_DPHAT, TCS_DP0}));
+    else if (!(c->kept >> TCS_DP0 & 1)) TCS_TRY(copy_shell(c, {TCS_DP0}));
+    if (c->wrap) c->kept |= 1u << TCS_DP0;
     const DPhatUpdate hist{g, c->f[TCS_DP], c->f[TCS_DPHAT], c->f[TCS_DP0]};
     if (c->a32) {
         const FieldSet32 tw{{twin(c, c->f[TCS_U]), twin(c, c->f[TCS_V]), twin(c, c->f[TCS_W]), twin(c, c->f[TCS_P])}};
@@ -834,7 +903,8 @@ int pressure_projection_into(tcs_ctx *c, double dt, double *dPhatn, double *dP0n
         TCS_LAUNCH(c->stream, "projection", k_projection_into<false>, grd, blk, 0, cell, hist, c->f[TCS_U], c->f[TCS_V],
                    c->f[TCS_W], c->f[TCS_P], dPhatn, dP0n, FieldSet32{});
     }
-    TCS_LAUNCH(c->stream, "wall_extrap", k_wall_extrap, dim3((c->n1m + 63) / 64, c->n3m), dim3(64), 0, g, c->f[TCS_P]);
+    TCS_LAUNCH(c->stream, "wall_extrap", k_wall_extrap, dim3((c->n1m + 63) / 64, c->n3m), dim3(64), 0, g, c->f[TCS_P],
+               twin(c, c->f[TCS_P]));
     return TCS_OK;
 }
 

@@ -138,10 +138,9 @@ __global__ void k_halo(Grid g, Set fs) {
 // the cells of a full field outside the interior: the faces i in {0, n1m+1}
 // (all j, k), then j in {0, n2m+1} (interior i, all k), then k in {0, n3m+1}
 // (interior i and j)
-template <typename E, class DstSet>
-__global__ void k_copy_shell(Grid g, FieldSet src_set, DstSet dst_set) {
+__global__ void k_copy_shell(Grid g, FieldSet src_set, FieldSet dst_set) {
     const double *__restrict__ src = src_set.f[blockIdx.y];  // one pair per grid row
-    E *__restrict__ dst = dst_set.f[blockIdx.y];
+    double *__restrict__ dst = dst_set.f[blockIdx.y];
     const int N1 = g.N1, N2 = g.N2, N3 = g.N3, n1m = g.n1m, n2m = g.n2m;
     const size_t fi = (size_t)2 * N2 * N3, fj = (size_t)2 * n1m * N3, fk = (size_t)2 * n1m * n2m;
     size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -161,24 +160,22 @@ __global__ void k_copy_shell(Grid g, FieldSet src_set, DstSet dst_set) {
     } else {
         return;
     }
-    dst[o] = (E)src[o];
+    dst[o] = src[o];
 }
 
-int copy_shell(tcs_ctx *c, std::initializer_list<std::pair<const double *, double *>> pairs) {
+int copy_shell(tcs_ctx *c, std::initializer_list<int> ids) {
     FieldSet src{}, dst{};
     int nf = 0;
-    for (const auto &pr : pairs) {
+    for (int id : ids) {
         if (nf == FieldSet::MAX) return TCS_E_ARG;
-        src.f[nf] = const_cast<double *>(pr.first);
-        dst.f[nf++] = pr.second;
+        src.f[nf] = c->f[id];
+        dst.f[nf++] = c->spare[id];
     }
     const size_t n = (size_t)2 * c->N2 * c->N3 + (size_t)2 * c->n1m * c->N3 + (size_t)2 * c->n1m * c->n2m;
-    TCS_LAUNCH(c->stream, "copy_shell", (k_copy_shell<double, FieldSet>), dim3((unsigned)((n + 255) / 256), (unsigned)nf),
-               dim3(256), 0, c->grid(), src, dst);
+    TCS_LAUNCH(c->stream, "copy_shell", k_copy_shell, dim3((unsigned)((n + 255) / 256), (unsigned)nf), dim3(256), 0,
+               c->grid(), src, dst);
     return TCS_OK;
 }
-int copy_shell(tcs_ctx *c, const double *src, double *dst) { return copy_shell(c, {{src, dst}}); }
-
 
 int halo(tcs_ctx *c, std::initializer_list<double *> fields) {
     FieldSet fs{};
@@ -219,26 +216,6 @@ static unsigned twin_bit(int id) {
     case TCS_MU: case TCS_INVRHO: return TWIN_TAB;
     default: return 0;
     }
-}
-
-// The cells outside the interior of fields into their FP32 twins (the
-// interior's twins written by the kernel that updated it): the twins of
-// those fields are current afterwards.
-static int shell_to_twins(tcs_ctx *c, std::initializer_list<int> ids) {
-    FieldSet src{};
-    FieldSet32 dst{};
-    int nf = 0;
-    unsigned bits = 0;
-    for (int id : ids) {
-        if (nf == FieldSet::MAX || !(dst.f[nf] = twin(c, c->f[id]))) return TCS_E_ARG;
-        src.f[nf++] = c->f[id];
-        bits |= twin_bit(id);
-    }
-    const size_t n = (size_t)2 * c->N2 * c->N3 + (size_t)2 * c->n1m * c->N3 + (size_t)2 * c->n1m * c->n2m;
-    TCS_LAUNCH(c->stream, "twin_shell", (k_copy_shell<float, FieldSet32>), dim3((unsigned)((n + 255) / 256), (unsigned)nf),
-               dim3(256), 0, c->grid(), src, dst);
-    c->twin_ok |= bits;
-    return TCS_OK;
 }
 
 __global__ void k_to_f32(const double *__restrict__ src, float *__restrict__ dst, size_t n) {
@@ -336,10 +313,13 @@ k_post_max(Grid g, const double *__restrict__ U, const double *__restrict__ V, c
 }
 
 // both maxima in one pass over U, V, W: partial[b] (divergence) and
-// partial[RED_BLOCKS + b] (sum |u|/dx)
+// partial[RED_BLOCKS + b] (sum |u|/dx); the last workgroup to finish takes
+// the maxima of those into out (pinned host memory).  Rows shorter than a
+// workgroup go several at a time.
+template <bool SHORT>
 __global__ void __launch_bounds__(256)
 k_post_both(Grid g, const double *__restrict__ U, const double *__restrict__ V, const double *__restrict__ W,
-            double *__restrict__ partial) {
+            double *partial, double *out, unsigned *count) {
     __shared__ double s0[256], s1[256];
     // Workgroups go to the 8 XCDs round-robin.  When n2m divides by 8, XCD x
     // serves the rows j of band x (n2m/8 of them) at every k, so the V(j+1)
@@ -350,10 +330,13 @@ k_post_both(Grid g, const double *__restrict__ U, const double *__restrict__ V, 
     const int band = banded ? g.n2m / 8 : g.n2m, x = banded ? (int)blockIdx.x % 8 : 0;
     const int q = banded ? (int)blockIdx.x / 8 : (int)blockIdx.x, nq = banded ? (int)gridDim.x / 8 : (int)gridDim.x;
     const int nrows = band * g.n3m;
+    // threads along a row, rows at a time
+    const int nt = SHORT ? g.n1m : (int)blockDim.x, rt = SHORT ? (int)blockDim.x / nt : 1;
+    const int t0 = SHORT ? (int)threadIdx.x % nt : (int)threadIdx.x, r0 = SHORT ? (int)threadIdx.x / nt : 0;
     double m0 = -INFINITY, m1 = -INFINITY;
-    for (int r = q; r < nrows; r += nq) {
+    for (int r = q * rt + r0; r < nrows; r += nq * rt) {
         const int j = x * band + r % band + 1, k = r / band + 1;
-        for (int i = threadIdx.x + 1; i <= g.n1m; i += blockDim.x) {
+        for (int i = t0 + 1; i <= g.n1m; i += nt) {
             const double u0 = U[g.ix(i, j, k)], u1 = U[g.ix(i + 1, j, k)];
             const double v0 = V[g.ix(i, j, k)], v1 = V[g.ix(i, j + 1, k)];
             const double w0 = W[g.ix(i, j, k)], w1 = W[g.ix(i, j, k + 1)];
@@ -365,16 +348,35 @@ k_post_both(Grid g, const double *__restrict__ U, const double *__restrict__ V, 
     s0[threadIdx.x] = m0;
     s1[threadIdx.x] = m1;
     __syncthreads();
-    for (int h = 128; h >= 1; h >>= 1) {
-        if ((int)threadIdx.x < h) {
-            s0[threadIdx.x] = fmax(s0[threadIdx.x], s0[threadIdx.x + h]);
-            s1[threadIdx.x] = fmax(s1[threadIdx.x], s1[threadIdx.x + h]);
+    auto fold = [&] {
+        for (int h = 128; h >= 1; h >>= 1) {
+            if ((int)threadIdx.x < h) {
+                s0[threadIdx.x] = fmax(s0[threadIdx.x], s0[threadIdx.x + h]);
+                s1[threadIdx.x] = fmax(s1[threadIdx.x], s1[threadIdx.x + h]);
+            }
+            __syncthreads();
         }
-        __syncthreads();
-    }
+    };
+    fold();
+    __shared__ bool last;
     if (threadIdx.x == 0) {
-        partial[blockIdx.x] = s0[0];
-        partial[RED_BLOCKS + blockIdx.x] = s1[0];
+        last_put(partial + blockIdx.x, s0[0], partial + RED_BLOCKS + blockIdx.x, s1[0]);
+        last = last_arrive(count, gridDim.x);
+    }
+    __syncthreads();
+    if (!last) return;
+    m0 = m1 = -INFINITY;
+    for (int b = threadIdx.x; b < (int)gridDim.x; b += blockDim.x) {
+        m0 = fmax(m0, last_get(partial + b));
+        m1 = fmax(m1, last_get(partial + RED_BLOCKS + b));
+    }
+    s0[threadIdx.x] = m0;
+    s1[threadIdx.x] = m1;
+    __syncthreads();
+    fold();
+    if (threadIdx.x == 0) {
+        out[0] = s0[0];
+        out[1] = s1[0];
     }
 }
 
@@ -405,14 +407,12 @@ static int post_max(tcs_ctx *c, double *out) {
 // mpi_Post_Div's pass also gives mpi_Post_CFL's maximum (the same U, V, W
 // reads), kept until an entry that may change the fields runs
 int post_div(tcs_ctx *c, double *out) {
-    TCS_LAUNCH(c->stream, "post_div_cfl", k_post_both, dim3(RED_BLOCKS), dim3(256), 0, c->grid(), c->f[TCS_U],
-               c->f[TCS_V], c->f[TCS_W], c->red);
-    TCS_LAUNCH(c->stream, "final_max", k_final_max, dim3(1), dim3(256), 0, RED_BLOCKS, c->red,
-               c->red + 2 * RED_BLOCKS);
-    TCS_LAUNCH(c->stream, "final_max", k_final_max, dim3(1), dim3(256), 0, RED_BLOCKS, c->red + RED_BLOCKS,
-               c->red + 2 * RED_BLOCKS + 1);
-    TCS_HIP(hipMemcpyAsync(c->h_pinned, c->red + 2 * RED_BLOCKS, 2 * sizeof(double), hipMemcpyDeviceToHost,
-                           c->stream));
+    // at least 8 cells a thread: the values of more workgroups take longer to
+    // gather than they save (64^3: 128 workgroups)
+    const size_t nb = (c->nint + 2047) / 2048;
+    TCS_LAUNCH(c->stream, "post_div_cfl", (c->n1m < 256 ? k_post_both<true> : k_post_both<false>),
+               dim3((unsigned)std::min<size_t>(RED_BLOCKS, (nb + 7) / 8 * 8)), dim3(256), 0, c->grid(), c->f[TCS_U], c->f[TCS_V],
+               c->f[TCS_W], c->red, c->h_pinned, (unsigned *)(c->scal + 2));
     TCS_HIP(hipStreamSynchronize(c->stream));
     *out = c->h_pinned[0];
     c->cfl_max = c->h_pinned[1];
@@ -867,6 +867,7 @@ static int check_field(tcs_ctx *c, int id) {
         return TCS_E_ARG;
     }
     TCS_TRY(flush_pending(c));
+    c->kept &= ~(1u << id);
     c->cfl_valid = 0;  // the field may change (upload, halo, a handed-out pointer)
     c->twin_ok &= ~twin_bit(id);  // and with it the mixed form's FP32 copy
     return TCS_OK;
@@ -941,6 +942,7 @@ extern "C" int tcs_field_copy_device(tcs_ctx *c, int32_t id, int32_t to_field, d
 extern "C" int tcs_fields_touched(tcs_ctx *c) {
     if (!c) return TCS_E_ARG;
     TCS_TRY(flush_pending(c));
+    c->kept = 0;
     c->cfl_valid = 0;
     c->twin_ok = 0;
     for (int q : {TCS_DU, TCS_DV, TCS_DW}) TCS_TRY(increment_from_fp64(c, q));
@@ -1015,9 +1017,11 @@ extern "C" int tcs_momentum_boundary(tcs_ctx *c, double Uup, double Ubt, double 
 #define CTX_CHECK(c) \
     if (!(c)) { set_error("null context"); return TCS_E_ARG; } \
     TCS_TRY(flush_pending(c));
-// entries that may change fields drop the kept CFL maximum
+// entries that may change fields drop the kept CFL maximum and what a step
+// keeps for the next
 #define CTX_GUARD(c) \
     CTX_CHECK(c) \
+    (c)->kept = 0; \
     (c)->cfl_valid = 0;
 
 #define STAGE(label) ProfStage _stage(c, label)
@@ -1196,39 +1200,41 @@ extern "C" int tcs_nusselt(tcs_ctx *c, double Tup, double Tbt, double *nb, doubl
         TCS_TRY(expr);                \
     } while (0)
 
+namespace {
+struct Wrap {  // tcs_ctx::wrap for a scope
+    tcs_ctx *c;
+    explicit Wrap(tcs_ctx *c) : c(c) { c->wrap = 1; }
+    ~Wrap() { c->wrap = 0; }
+};
+}  // namespace
+
+// Every ghost-cell update of main's order is made by the kernel that writes
+// the field (tcs_ctx::wrap).
 extern "C" int tcs_step(tcs_ctx *c, double dt) {
-    CTX_GUARD(c);
+    CTX_CHECK(c);
+    c->cfl_valid = 0;
     STAGE("step");
-    const char *H = "update ghostcell";
+    const Wrap wrap(c);
     bool swap_T = false;
     RUN("thermal solve", FORM(c, thermal_solver_into, dt, c->spare[TCS_T], &swap_T));
     if (swap_T) std::swap(c->f[TCS_T], c->spare[TCS_T]);
-    RUN(H, halo(c, c->f[TCS_T]));
-    // the mixed form: the last thermal sweep wrote T's FP32 copy inside; now its shell
-    if (c->a32 && swap_T) RUN(H, shell_to_twins(c, {TCS_T}));
+    if (c->a32 && swap_T) c->twin_ok |= TWIN_T;  // the mixed form: written by the last thermal sweep
     RUN("momentum coeff", FORM(c, momentum_coeffi));
     RUN("momentum solvedU", FORM(c, momentum_solvedU, dt));
-    RUN(H, halo_field(c, TCS_DU));
     RUN("momentum solvedV", FORM(c, momentum_solvedV, dt));
-    RUN(H, halo_field(c, TCS_DV));
     RUN("momentum solvedW", FORM(c, momentum_solvedW, dt));
-    RUN(H, halo_field(c, TCS_DW));
     // block corrections with the pseudo-update (U + dU, V + dV, W + dW into
     // the second buffers; the corrections read the old U, V)
     RUN("momentum blockLdV", FORM(c, momentum_blockLdV_pseudo, dt, c->spare[TCS_V]));
-    RUN(H, halo_field(c, TCS_DV));
     RUN("momentum blockLdU", FORM(c, momentum_blockLdU_pseudo, dt, c->spare[TCS_U], c->spare[TCS_W]));
     for (int q : {TCS_U, TCS_V, TCS_W}) std::swap(c->f[q], c->spare[q]);
-    RUN(H, halo(c, {c->f[TCS_U], c->f[TCS_V], c->f[TCS_W]}));
     // the right-hand side is made inside the solve's x transform
     RUN("pressure PoissonSolve", FORM(c, pressure_poisson_rhs, dt));
-    RUN(H, halo(c, c->f[TCS_DP]));
     RUN("pressure projection", FORM(c, pressure_projection_into, dt, c->spare[TCS_DPHAT], c->spare[TCS_DP0]));
     std::swap(c->f[TCS_DPHAT], c->spare[TCS_DPHAT]);
     std::swap(c->f[TCS_DP0], c->spare[TCS_DP0]);
-    RUN(H, halo(c, {c->f[TCS_U], c->f[TCS_V], c->f[TCS_W], c->f[TCS_P], c->f[TCS_DPHAT]}));
-    // the mixed form: the projection wrote the FP32 copies of U, V, W, P inside
-    if (c->a32) RUN(H, shell_to_twins(c, {TCS_U, TCS_V, TCS_W, TCS_P}));
+    // the mixed form: the projection wrote the FP32 copies of U, V, W, P
+    if (c->a32) c->twin_ok |= TWIN_U | TWIN_V | TWIN_W | TWIN_P;
     return TCS_OK;
 }
 

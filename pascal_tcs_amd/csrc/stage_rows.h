@@ -283,6 +283,7 @@ int y_stage_in_solve(tcs_ctx *c, const char *label, const Row &row, int jlo, int
         out.ss0 = 1;
         out.ss1 = (long)c->P1 * c->N2;
         out.rs = c->P1;
+        out.wrap_to(c, nrows);
         if constexpr (sizeof(S) == sizeof(float)) {
             // the mixed form stores its increments into their FP32 twins
             out.G = twin(c, F);

@@ -92,6 +92,7 @@ struct Grid {
     int n1m, n2m, n3m;
     int N1, N2, N3;  // full extents n?m+2
     int P1;          // row pitch of the full fields
+    int wrap;        // kernels write the periodic ghosts (tcs_ctx::wrap)
     const double *dx1, *dx2, *dx3, *dmx1, *dmx2, *dmx3;
     const double *rdx1, *rdx2, *rdx3, *rdmx1, *rdmx2, *rdmx3;  // their reciprocals
     // the six tables (dx1, dmx1, dx2, dmx2, dx3, dmx3) back to back rounded to
@@ -105,6 +106,39 @@ struct Grid {
     __device__ __forceinline__ size_t t2(int j, int k) const { return (size_t)j + (size_t)N2 * (size_t)k; }
     __device__ __forceinline__ size_t r3(int i, int j, int k) const {
         return (size_t)(i - 1) + (size_t)n1m * ((size_t)(j - 1) + (size_t)n2m * (size_t)(k - 1));
+    }
+    // The periodic images in x and z of F(i, j, k) = v (element q): a kernel
+    // that makes a whole field leaves its rows as the ghost-cell update would.
+    // Called in a branch of the few wavefronts for which edge() holds, after
+    // the stores of the cells themselves: tested cell by cell at each store,
+    // the images cost blockLdU 0.5 of 1.8 ms at 512^3.
+    template <class E>
+    __device__ __forceinline__ void images(E *F, int i, int k, size_t q, E v) const {
+        const long di = i == 1 ? n1m : i == n1m ? -n1m : 0;
+        if (di) F[(long)q + di] = v;
+        if (k == 1 || k == n3m) {
+            const long dk = (k == 1 ? (long)n3m : -(long)n3m) * P1 * N2;
+            F[(long)q + dk] = v;
+            if (di) F[(long)q + dk + di] = v;
+        }
+    }
+    // (wrap) whether cells i0..i0+ib-1, j, k0..k0+kb-1 touch the edge of the
+    // interior; ib and kb divide n1m and n3m
+    __device__ __forceinline__ bool edge(int i0, int ib, int j, int k0, int kb) const {
+        return wrap && (i0 == 1 || i0 + ib > n1m || j == 1 || j == n2m || k0 == 1 || k0 + kb > n3m);
+    }
+    // F's wall row next to row j, if there is one, from src's, with its
+    // images: the thread of an edge row brings over the wall row of a second
+    // buffer, or with src = F renews a wall row's ghosts
+    template <class E, class E0>
+    __device__ __forceinline__ void wall(E *F, const E0 *src, int i, int j, int k) const {
+        for (int s = 0; s < 2; s++) {
+            if (s ? j != n2m : j != 1) continue;
+            const size_t q = ix(i, s ? j + 1 : 0, k);
+            const E v = (E)src[q];
+            F[q] = v;
+            images(F, i, k, q, v);
+        }
     }
     __device__ __forceinline__ RelCell ix(Rel i, Rel j, Rel k) const {
         return RelCell{ix(i.v, j.v, k.v), (k.o + 1) * 9 + (j.o + 1) * 3 + (i.o + 1)};
@@ -191,6 +225,19 @@ struct tcs_ctx {
     // (the FP64 arrays are filled from them on download); the others are
     // FP32 copies of the FP64 arrays, current while their TWIN_* bit is set
     // in twin_ok.  Null / 0 in the FP64 forms.
+    // Set within tcs_step, which knows that every field a kernel writes whole
+    // is followed by its ghost-cell update: the kernels write the periodic
+    // ghosts and the wall rows themselves (Grid::edge, images, wall; LineOut::gx)
+    // instead of 13 launches that cost 5 us each on a small grid (a step at
+    // 64^3 294 -> 264 us with the reductions' single launches; 256x193x128
+    // 2.07 -> 2.03 ms; 512^3 32.8 -> 32.4 ms).  The routines
+    // called one by one leave the ghosts to tcs_ghostcell_update, as a caller
+    // may look at them in between.
+    int wrap;
+    // For steps in a row, cleared by every other entry that may write the
+    // field or hands out its address, bits 1 << id: dP0's second buffer holds
+    // the same shell as dP0; dV's rows 0, 1 and n2m+1 are zero.
+    unsigned kept;
     double *a64;
     float *a32;
     size_t an, aused;
@@ -201,6 +248,7 @@ struct tcs_ctx {
         g.n1m = n1m; g.n2m = n2m; g.n3m = n3m;
         g.N1 = N1; g.N2 = N2; g.N3 = N3;
         g.P1 = P1;
+        g.wrap = wrap;
         g.dx1 = dx1; g.dx2 = dx2; g.dx3 = dx3;
         g.rdx1 = rmet; g.rdmx1 = rmet + N1; g.rdx2 = rmet + 2 * N1; g.rdmx2 = g.rdx2 + N2;
         g.rdx3 = g.rdx2 + 2 * N2; g.rdmx3 = g.rdx3 + N3;
@@ -212,6 +260,34 @@ struct tcs_ctx {
 };
 
 namespace tcs {
+
+// Reductions that end in the same launch: thread 0 of each workgroup leaves
+// its value(s) with last_put and then asks last_arrive, true in the workgroup
+// that arrives last, whose threads read every value with last_get.  A
+// put's exchange has been performed where all XCDs see it when its old value
+// is back, and last_arrive's add is issued after that, so no fence is needed:
+// a release per workgroup writes back and an acquire drops the whole of its
+// XCD's L2 (1024 workgroups of a reduction over 64^3 cells: 31 us).
+__device__ __forceinline__ unsigned long long last_swap(double *p, double v) {
+    return __hip_atomic_exchange(reinterpret_cast<unsigned long long *>(p), (unsigned long long)__double_as_longlong(v),
+                                 __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void last_put(double *p, double v) {
+    const unsigned long long old = last_swap(p, v);
+    asm volatile("" ::"v"(old) : "memory");  // wait for it
+}
+__device__ __forceinline__ void last_put(double *p, double v, double *p1, double v1) {
+    const unsigned long long old = last_swap(p, v), old1 = last_swap(p1, v1);
+    asm volatile("" ::"v"(old), "v"(old1) : "memory");
+}
+__device__ __forceinline__ bool last_arrive(unsigned *count, unsigned n) {
+    const bool last = __hip_atomic_fetch_add(count, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == n - 1;
+    if (last) __hip_atomic_store(count, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    return last;
+}
+__device__ __forceinline__ double last_get(const double *p) {
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 
 // launch helpers -------------------------------------------------------------
 inline dim3 interior_block() { return dim3(64, 4, 1); }
@@ -251,6 +327,12 @@ struct LineOut {
                          // lines: G (when set) also receives the FP32 copy of the FP64 value
     long base = 0, ss0 = 0, ss1 = 0, rs = 0;
     int mode = 0;
+    // > 0: gx x gz lines of n_row rows, written with their periodic ghosts in
+    // s0 and s1 and with the wall rows before and after them (mode 3: Fin's)
+    int gx = 0, gz = 0, n_row = 0;
+    void wrap_to(const tcs_ctx *c, int nr) {
+        if (c->wrap) { gx = c->n1m; gz = c->n3m; n_row = nr; }
+    }
 };
 // The same systems split into parts (PaScaL_TDMA's multi-rank algorithm,
 // one thread per rank); n_row in [2, 512]; strided lines need ss0 = 1.
@@ -334,9 +416,9 @@ int ensure_twins(tcs_ctx *c, unsigned bits);
 // form) and back (uploads)
 int increment_to_fp64(tcs_ctx *c, int id);
 int increment_from_fp64(tcs_ctx *c, int id);
-// copy the cells outside the interior (x/z ghosts, wall rows) of a full field
-int copy_shell(tcs_ctx *c, const double *src, double *dst);
-int copy_shell(tcs_ctx *c, std::initializer_list<std::pair<const double *, double *>> pairs);
+// copy the cells outside the interior (x/z ghosts, wall rows) of fields into
+// the second buffers that are to become them
+int copy_shell(tcs_ctx *c, std::initializer_list<int> ids);
 // Routine entries that hold their launches back: tcs_momentum_blockLdV, the
 // ghost-cell update of dV after it and tcs_momentum_blockLdU wait for
 // tcs_momentum_pseudoupdateUVW (which then runs the block corrections with

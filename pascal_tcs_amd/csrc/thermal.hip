@@ -472,14 +472,19 @@ struct ThermalY {
 // T(i,j,k) += RHSJ (:518-524)
 // F(i,j,k) = inc (MODE 1) or F(i,j,k) += inc (MODE 2) over interior rows j >= j0
 template <int MODE>
-__global__ void k_interior_out(Grid g, int j0, double *__restrict__ F, const scr_t *__restrict__ inc) {
+__global__ void k_interior_out(Grid g, int j0, double *F, const scr_t *__restrict__ inc) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
     const int j = blockIdx.y * blockDim.y + threadIdx.y + 1;
     const int k = blockIdx.z + 1;
     if (i > g.n1m || j > g.n2m || j < j0) return;
     const size_t q = g.ix(i, j, k);
-    if (MODE == 1) F[q] = inc[g.r3(i, j, k)];
-    else F[q] = F[q] + inc[g.r3(i, j, k)];
+    const double v = inc[g.r3(i, j, k)];
+    const double f = MODE == 1 ? v : F[q] + v;
+    F[q] = f;
+    if (g.edge(i, 1, j, k, 1)) {
+        g.images(F, i, k, q, f);
+        g.wall(F, F, i, j, k);
+    }
 }
 
 // y sweep of rows j = j0..j0+nrows-1 (1-based) whose solution ends the
@@ -498,6 +503,7 @@ int sweep_y_field(tcs_ctx *c, int j0, int nrows, double *F, int mode) {
         out.ss0 = 1;
         out.ss1 = (long)c->P1 * c->N2;
         out.rs = c->P1;
+        out.wrap_to(c, nrows);
         return ptdma_part_launch(SCR(c->am) + off, SCR(c->ac) + off, SCR(c->ap) + off, SCR(c->rhs) + off, c->n1m, 1,
                                  c->n3m, n12, nrows, n1, false, c->stream, out);
     }
@@ -567,7 +573,7 @@ int thermal_solver_into(tcs_ctx *c, double dt, double *Tn, bool *written) {
     const ThermalZ z{g, c->phys, dt, T, c->f[TCS_U], c->f[TCS_V], c->f[TCS_W], c->wall[TCS_TBCUP], c->wall[TCS_TBCBT]};
     TCS_TRY(z_stage<ANY_SPLIT>(c, "thermal_z", "thermal_z_solve", z, 1, am, ac, ap, rhs));
     TCS_TRY(thermal_x_stage(c, ThermalX{g, c->phys, dt, T, c->f[TCS_U]}));
-    TCS_TRY(copy_shell(c, T, Tn));
+    if (!c->wrap) TCS_TRY(copy_shell(c, {TCS_T}));
     const long n1 = c->n1m, n12 = (long)c->n1m * c->n2m;
     LineOut out;
     out.F = Tn;
@@ -578,6 +584,7 @@ int thermal_solver_into(tcs_ctx *c, double dt, double *Tn, bool *written) {
     out.ss0 = 1;
     out.ss1 = (long)c->P1 * c->N2;
     out.rs = c->P1;
+    out.wrap_to(c, c->n2m);
     // FP64 lines 8 a workgroup (1.96 -> 1.91 ms at 512^3), FP32 lines 16
     // (8: 1.52 -> 1.96 ms)
     constexpr int SX = sizeof(scr_t) == 8 ? 8 : PT_SX;
