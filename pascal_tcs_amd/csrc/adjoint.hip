@@ -49,10 +49,12 @@ struct AdjWork {
     double *bwall[TCS_NWALL];       // of the wall arrays
     double *tmp[4];                 // full-size work
     double *s0[adj::NSTATE];        // state at the start of the step
-    double *sT1, *sdU1, *sdV1, *sdW1, *sdV2, *sdU2, *sU1, *sV1, *sW1, *sdP, *sMu, *siR, *sstale;
+    // and within it, of what a later stage overwrites: dU and dV as solved,
+    // U, V, W before the projection
+    double *sdU1, *sdV1, *sU1, *sV1, *sW1;
     double *X[4][3];                // ADI stage solutions (interior layout)
-    double *lam, *abar, *bbar, *cbar, *aT, *cT, *rint;  // interior layout
-    double *scal;
+    double *lam, *rint;             // interior layout
+    double *psum;                   // partial sums of the dP mean, then the mean; a counter
     std::vector<void *> all;
 };
 
@@ -62,7 +64,8 @@ namespace adj {
 
 // k_halo transposed: every ghost's adjoint goes to its periodic source (the
 // same enumeration as k_halo; sources are never x or z ghosts)
-__global__ void k_halo_adj(Grid g, double *__restrict__ b) {
+__global__ void k_halo_adj(Grid g, FieldSet fs) {
+    double *__restrict__ b = fs.f[blockIdx.y];  // one field per grid row
     const int N1 = g.N1, N2 = g.N2, N3 = g.N3;
     const int n1m = g.n1m, n3m = g.n3m;
     const size_t nx = (size_t)2 * N2 * N3, nz = (size_t)2 * N1 * N2;
@@ -91,9 +94,16 @@ __global__ void k_halo_adj(Grid g, double *__restrict__ b) {
     if (v != 0.0) unsafeAtomicAdd(b + src, v);  // the L2's FP64 atomic (not a compare-and-swap loop)
 }
 
-int halo_adj(tcs_ctx *c, double *b) {
+int halo_adj(tcs_ctx *c, std::initializer_list<double *> fields) {
+    FieldSet fs{};
+    int nf = 0;
+    for (double *b : fields) {
+        if (nf == FieldSet::MAX) return TCS_E_ARG;
+        fs.f[nf++] = b;
+    }
     const size_t n = (size_t)2 * c->N2 * c->N3 + (size_t)2 * c->N1 * c->N2;
-    TCS_LAUNCH(c->stream, "adj_halo", k_halo_adj, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, c->grid(), b);
+    TCS_LAUNCH(c->stream, "adj_halo", k_halo_adj, dim3((unsigned)((n + 255) / 256), (unsigned)nf), dim3(256), 0,
+               c->grid(), fs);
     return TCS_OK;
 }
 
@@ -125,45 +135,120 @@ int wall_extrap_adj(tcs_ctx *c, double *b) {
     return TCS_OK;
 }
 
-// interior sum (one atomic per workgroup) and the mean projection
-__global__ void k_interior_sum(Grid g, const double *__restrict__ b, double *__restrict__ sum) {
-    __shared__ double s[256];
-    const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    const int j = blockIdx.y * blockDim.y + threadIdx.y + 1;
-    const int k = blockIdx.z + 1;
-    const int t = threadIdx.x + blockDim.x * threadIdx.y;
-    s[t] = (i <= g.n1m && j <= g.n2m) ? b[g.ix(i, j, k)] : 0.0;
+// The interior's mean into out[SUM_BLOCKS] (out: partial sums, the mean, a
+// counter): the last workgroup adds the partial sums in their order.
+constexpr int SUM_BLOCKS = 512;
+__device__ __forceinline__ double block_sum(double v, double *s) {
+    s[threadIdx.x] = v;
     __syncthreads();
     for (int h = 128; h >= 1; h >>= 1) {
-        if (t < h) s[t] += s[t + h];
+        if ((int)threadIdx.x < h) s[threadIdx.x] += s[threadIdx.x + h];
         __syncthreads();
     }
-    if (t == 0) unsafeAtomicAdd(sum, s[0]);
+    v = s[0];
+    __syncthreads();
+    return v;
 }
-__global__ void k_interior_sub(Grid g, const double *__restrict__ sum, double *__restrict__ b) {
+__global__ void __launch_bounds__(256) k_interior_mean(Grid g, const double *__restrict__ b, double *out) {
+    __shared__ double s[256];
+    __shared__ bool last;
+    const size_t n = (size_t)g.n1m * g.n2m * g.n3m;
+    double v = 0.0;
+    for (size_t q = (size_t)blockIdx.x * 256 + threadIdx.x; q < n; q += (size_t)gridDim.x * 256) {
+        const size_t r = q / g.n1m;
+        v += b[g.ix((int)(q - r * g.n1m) + 1, (int)(r % g.n2m) + 1, (int)(r / g.n2m) + 1)];
+    }
+    v = block_sum(v, s);
+    if (threadIdx.x == 0) {
+        last_put(out + blockIdx.x, v);
+        last = last_arrive(reinterpret_cast<unsigned *>(out + SUM_BLOCKS + 1), gridDim.x);
+    }
+    __syncthreads();
+    if (!last) return;
+    v = 0.0;
+    for (unsigned q = threadIdx.x; q < gridDim.x; q += 256) v += last_get(out + q);
+    v = block_sum(v, s);
+    if (threadIdx.x == 0) out[SUM_BLOCKS] = v / ((double)g.n1m * (double)g.n2m * (double)g.n3m);
+}
+
+// r (interior layout) = the interior of b minus the mean, and b's interior 0
+__global__ void k_take_mean(Grid g, const double *__restrict__ mean, double *__restrict__ b, double *__restrict__ r) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
     const int j = blockIdx.y * blockDim.y + threadIdx.y + 1;
     const int k = blockIdx.z + 1;
     if (i > g.n1m || j > g.n2m) return;
-    b[g.ix(i, j, k)] -= sum[0] / ((double)g.n1m * (double)g.n2m * (double)g.n3m);
+    const size_t q = g.ix(i, j, k);
+    r[g.r3(i, j, k)] = b[q] - mean[0];
+    b[q] = 0.0;
 }
 
-// full-field layout <-> interior layout
-__global__ void k_full_to_int(Grid g, int jlo, const double *__restrict__ f, double *__restrict__ r) {
+// b at (i, j, k), element q, plus what its periodic images hold, which are
+// set to zero: k_halo_adj's fold for the one cell that has those images
+__device__ __forceinline__ double fold_images(const Grid &g, double *b, int i, int k, size_t q) {
+    double v = b[q];
+    auto take = [&](long d) {
+        v += b[(long)q + d];
+        b[(long)q + d] = 0.0;
+    };
+    const long di = i == 1 ? g.n1m : i == g.n1m ? -g.n1m : 0;
+    if (di) take(di);
+    if (k == 1 || k == g.n3m) {
+        const long dk = (k == 1 ? (long)g.n3m : -(long)g.n3m) * g.P1 * g.N2;
+        take(dk);
+        if (di) take(dk + di);
+    }
+    return v;
+}
+// The ghost-cell update of b transposed, then r (interior layout) = its
+// interior (0 for rows j < jlo).  ZERO: b (ghosts and wall rows too) ends
+// as zero, the stage having replaced the field; otherwise b stays.
+template <bool ZERO>
+__global__ void k_take(Grid g, int jlo, double *b, double *__restrict__ r) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
     const int j = blockIdx.y * blockDim.y + threadIdx.y + 1;
     const int k = blockIdx.z + 1;
     if (i > g.n1m || j > g.n2m) return;
-    r[g.r3(i, j, k)] = j >= jlo ? f[g.ix(i, j, k)] : 0.0;
+    const size_t q = g.ix(i, j, k);
+    const double v = fold_images(g, b, i, k, q);
+    b[q] = ZERO ? 0.0 : v;
+    r[g.r3(i, j, k)] = j >= jlo ? v : 0.0;
+    for (int s = 0; s < 2; s++) {
+        if (s ? j != g.n2m : j != 1) continue;
+        const size_t o = g.ix(i, s ? j + 1 : 0, k);
+        const double w = fold_images(g, b, i, k, o);
+        b[o] = ZERO ? 0.0 : w;
+    }
 }
 
-// zero the interior cells j >= jlo of a full field
-__global__ void k_zero_interior(Grid g, int jlo, double *__restrict__ f) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    const int j = blockIdx.y * blockDim.y + threadIdx.y + 1;
-    const int k = blockIdx.z + 1;
-    if (i > g.n1m || j > g.n2m || j < jlo) return;
-    f[g.ix(i, j, k)] = 0.0;
+// Work on several arrays in one launch, an array a grid row
+struct Arrays {
+    static constexpr int MAX = 20;
+    double *dst[MAX];
+    const double *src[MAX];
+    size_t n[MAX];
+    int count = 0;
+    void add(double *d, const double *s, size_t len) {
+        dst[count] = d;
+        src[count] = s;
+        n[count++] = len;
+    }
+};
+// dst = src, or 0 where src is null
+__global__ void __launch_bounds__(256) k_copy_arrays(Arrays a) {
+    double *__restrict__ dst = a.dst[blockIdx.y];
+    const double *__restrict__ src = a.src[blockIdx.y];
+    const size_t n = a.n[blockIdx.y], st = (size_t)gridDim.x * 256;
+    if (src)
+        for (size_t q = (size_t)blockIdx.x * 256 + threadIdx.x; q < n; q += st) dst[q] = src[q];
+    else
+        for (size_t q = (size_t)blockIdx.x * 256 + threadIdx.x; q < n; q += st) dst[q] = 0.0;
+}
+static int copy_arrays(tcs_ctx *c, const Arrays &a) {
+    size_t most = 1;
+    for (int q = 0; q < a.count; q++) most = std::max(most, a.n[q]);
+    TCS_LAUNCH(c->stream, "adj_copy", k_copy_arrays, dim3((unsigned)std::min<size_t>((most + 1023) / 1024, 1024), a.count),
+               dim3(256), 0, a);
+    return TCS_OK;
 }
 
 // transposed Poisson y-systems, one (kx, kz) system per thread (the rows of
@@ -239,52 +324,29 @@ __global__ void k_poisson_tdma_T(int n3m, int h1p, int n2m, int h3p, const doubl
 
 // ---- ADI stage transposes ------------------------------------------------------
 
-// the line through interior cell q along `axis` (0 x, 1 y, 2 z), rows j >= jlo:
-// position, length and stride of the line
-struct LinePos {
-    int pos, n;
-    long stride;
-};
-__device__ __forceinline__ LinePos line_pos(const Grid &g, int axis, int jlo, int i, int j, int k) {
-    const long n1 = g.n1m, n12 = (long)g.n1m * g.n2m;
-    if (axis == 0) return {i - 1, g.n1m, 1};
-    if (axis == 1) return {j - jlo, g.n2m - jlo + 1, n1};
-    return {k - 1, g.n3m, n12};
-}
-
-// transposed rows in place of the stage's rows: aT_i = c_{i-1}, cT_i = a_{i+1}
-__global__ void k_coef_T(Grid g, int axis, int jlo, int cyc, const double *__restrict__ am, const double *__restrict__ ap,
-                         double *__restrict__ aT, double *__restrict__ cT) {
+// A stage's rows (rows3d's) with the transposed systems' coefficients: aT_i =
+// c_{i-1} and cT_i = a_{i+1}, each coefficient stored where the transposed
+// row has it
+template <class Row>
+__global__ void __launch_bounds__(256) k_rows3d_T(Row row, int axis, int jlo, int cyc, double *__restrict__ aT,
+                                                  double *__restrict__ b, double *__restrict__ cT) {
+    const Grid &g = row.g;
     const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    const int j = blockIdx.y * blockDim.y + threadIdx.y + 1;
-    const int k = blockIdx.z + 1;
+    const int j = wave_row_j();
     if (i > g.n1m || j > g.n2m || j < jlo) return;
-    const size_t q = g.r3(i, j, k);
-    const LinePos L = line_pos(g, axis, jlo, i, j, k);
-    const bool hp = L.pos > 0 || cyc, hn = L.pos < L.n - 1 || cyc;
-    const long qp = L.pos > 0 ? (long)q - L.stride : (long)q + (long)(L.n - 1) * L.stride;
-    const long qn = L.pos < L.n - 1 ? (long)q + L.stride : (long)q - (long)(L.n - 1) * L.stride;
-    aT[q] = hp ? ap[qp] : 0.0;
-    cT[q] = hn ? am[qn] : 0.0;
-}
-
-// row adjoints of a solved stage from lambda = A^-T xbar and the solution x
-__global__ void k_row_bars(Grid g, int axis, int jlo, int cyc, const double *__restrict__ lam,
-                           const double *__restrict__ x, double *__restrict__ ab, double *__restrict__ bb,
-                           double *__restrict__ cb) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
-    const int j = blockIdx.y * blockDim.y + threadIdx.y + 1;
-    const int k = blockIdx.z + 1;
-    if (i > g.n1m || j > g.n2m || j < jlo) return;
-    const size_t q = g.r3(i, j, k);
-    const LinePos L = line_pos(g, axis, jlo, i, j, k);
-    const bool hp = L.pos > 0 || cyc, hn = L.pos < L.n - 1 || cyc;
-    const long qp = L.pos > 0 ? (long)q - L.stride : (long)q + (long)(L.n - 1) * L.stride;
-    const long qn = L.pos < L.n - 1 ? (long)q + L.stride : (long)q - (long)(L.n - 1) * L.stride;
-    const double l = lam[q];
-    ab[q] = hp ? -l * x[qp] : 0.0;
-    bb[q] = -l * x[q];
-    cb[q] = hn ? -l * x[qn] : 0.0;
+#pragma unroll
+    for (int q = 0; q < ROWS3D_KB; q++) {
+        const int k = blockIdx.z * ROWS3D_KB + q + 1;
+        double am, ac, ap, d;
+        row(i, j, k, am, ac, ap, d);
+        const LinePos L = line_pos(g, axis, jlo, cyc, i, j, k);
+        const size_t o = g.r3(i, j, k);
+        b[o] = ac;
+        if (L.hp) cT[L.prev] = am;
+        else aT[o] = 0.0;
+        if (L.hn) aT[L.next] = ap;
+        else cT[o] = 0.0;
+    }
 }
 
 template <class Cell>
@@ -315,9 +377,10 @@ static LineGeom geom(const tcs_ctx *c, int axis, int jlo) {
     return {off, c->n1m, 1, c->n3m, n12, nl, n1};
 }
 
-static int sweep(tcs_ctx *c, double *A, const double *B, double *C, double *D, int axis, int jlo, bool cyc) {
+static int sweep(tcs_ctx *c, double *A, const double *B, double *C, const double *Din, double *Dout, int axis,
+                 int jlo, bool cyc) {
     const LineGeom L = geom(c, axis, jlo);
-    return ptdma_sweep(c, A + L.off, B + L.off, C + L.off, D + L.off, L.n0, L.ss0, L.n1, L.ss1, L.n_row, L.rs, cyc);
+    return ptdma_sweep(c, A + L.off, B + L.off, C + L.off, Din + L.off, Dout + L.off, L.n0, L.ss0, L.n1, L.ss1, L.n_row, L.rs, cyc);
 }
 
 // One stage backwards.  On entry w->lam holds xbar (interior layout, rows
@@ -327,19 +390,11 @@ static int sweep(tcs_ctx *c, double *A, const double *B, double *C, double *D, i
 template <bool HAS_D, class Row>
 int stage_adj(tcs_ctx *c, AdjWork *w, const Row &row, int axis, int jlo, bool cyc, const double *X,
               InBars<Row::NF> ib) {
-    const Grid g = c->grid();
-    const dim3 blk = interior_block(), grd = interior_grid(c->n1m, c->n2m, c->n3m);
-    double *am = c->am, *ac = c->ac, *ap = c->ap;
-    TCS_TRY(rows3d_launch<HAS_D>(c, "adj_rows", row, jlo, am, ac, ap, w->rint));
-    TCS_LAUNCH(c->stream, "adj_coef_T", k_coef_T, grd, blk, 0, g, axis, jlo, (int)cyc, am, ap, w->aT, w->cT);
-    {
-        const LineGeom L = geom(c, axis, jlo);
-        TCS_TRY(ptdma_exact_launch(w->aT + L.off, ac + L.off, w->cT + L.off, w->lam + L.off, w->lam + L.off, L.n0, L.ss0,
-                                   L.n1, L.ss1, L.n_row, L.rs, cyc, false, c->stream));
-    }
-    TCS_LAUNCH(c->stream, "adj_row_bars", k_row_bars, grd, blk, 0, g, axis, jlo, (int)cyc, w->lam, X, w->abar, w->bbar,
-               w->cbar);
-    OutBars ob{{w->abar, w->bbar, w->cbar, HAS_D ? w->lam : nullptr}, 0};
+    TCS_LAUNCH(c->stream, "adj_rows", k_rows3d_T<Row>,
+               cell_grid(c->n1m, c->n2m, c->n3m, ROWS3D_KB, interior_block(), 1), interior_block(), 0, row, axis, jlo,
+               (int)cyc, c->am, c->ac, c->ap);
+    TCS_TRY(sweep(c, c->am, c->ac, c->ap, w->lam, w->lam, axis, jlo, cyc));
+    const OutBars ob{{}, 0, w->lam, X, axis, jlo, (int)cyc, (int)HAS_D};
     return cell_vjp(c, w, row, jlo, ob, ib);
 }
 
@@ -407,109 +462,158 @@ __global__ void k_nusselt_adj(Grid g, double wgt, double *__restrict__ bT, doubl
 
 // ---- the step forward, keeping what the adjoint needs ----------------------------
 
-static int copy(tcs_ctx *c, double *dst, const double *src, size_t n) {
-    TCS_HIP(hipMemcpyAsync(dst, src, n * sizeof(double), hipMemcpyDeviceToDevice, c->stream));
+// A stage's increment (interior layout) into its field: stored (MODE 1, 0 in
+// rows j < j0 and, with j0 > 1, in the wall rows) or added (MODE 2), with the
+// field's ghost-cell update; S (not null) keeps a copy of the whole field.
+template <int MODE>
+__global__ void k_store_keep(Grid g, int j0, const double *__restrict__ inc, double *F, double *S) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
+    const int j = blockIdx.y * blockDim.y + threadIdx.y + 1;
+    const int k = blockIdx.z + 1;
+    if (i > g.n1m || j > g.n2m) return;
+    auto put = [&](size_t q, double v) {
+        F[q] = v;
+        g.images(F, i, k, q, v);
+        if (!S) return;
+        S[q] = v;
+        g.images(S, i, k, q, v);
+    };
+    const size_t q = g.ix(i, j, k);
+    const double v = j >= j0 ? inc[g.r3(i, j, k)] : 0.0;
+    put(q, MODE == 1 ? v : F[q] + v);
+    for (int s = 0; s < 2; s++) {
+        if (s ? j != g.n2m : j != 1) continue;
+        const size_t o = g.ix(i, s ? j + 1 : 0, k);
+        put(o, j0 > 1 ? 0.0 : F[o]);
+    }
+}
+template <int MODE>
+static int store_keep(tcs_ctx *c, int j0, const double *inc, double *F, double *S) {
+    TCS_LAUNCH(c->stream, "adj_fwd_store", k_store_keep<MODE>, interior_grid(c->n1m, c->n2m, c->n3m),
+               interior_block(), 0, c->grid(), j0, inc, F, S);
     return TCS_OK;
 }
 
-// ADI of one increment (or of T), forward: the three solutions into X[0..2]
+// the fields' ghost-cell updates, and copies of the whole fields
+__global__ void k_halo_keep(Grid g, Arrays a) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
+    const int j = blockIdx.y * blockDim.y + threadIdx.y + 1;
+    const int k = blockIdx.z % g.n3m + 1, f = blockIdx.z / g.n3m;
+    if (i > g.n1m || j > g.n2m) return;
+    double *S = a.dst[f], *F = const_cast<double *>(a.src[f]);
+    const int w0 = j == 1 ? 0 : j, w1 = j == g.n2m ? j + 1 : j;
+    for (int jj = w0; jj <= w1; jj++) {
+        const size_t q = g.ix(i, jj, k);
+        const double v = F[q];
+        S[q] = v;
+        g.images(F, i, k, q, v);
+        g.images(S, i, k, q, v);
+    }
+}
+
+// ADI of one increment (or of T), forward: the three solutions into X[0..2],
+// each solve from the one before it
 template <class RZ, class RX, class RY>
 static int adi_forward(tcs_ctx *c, const RZ &rz, const RX &rx, const RY &ry, int jlo, double *const (&X)[3]) {
-    double *am = c->am, *ac = c->ac, *ap = c->ap, *rhs = c->rhs;
-    TCS_TRY(rows3d_launch<true>(c, "adj_fwd_rows", rz, jlo, am, ac, ap, rhs));
-    TCS_TRY(sweep(c, am, ac, ap, rhs, 2, jlo, true));
-    TCS_TRY(copy(c, X[0], rhs, c->nint));
-    TCS_TRY(rows3d_launch<false>(c, "adj_fwd_rows", rx, jlo, am, ac, ap, rhs));
-    TCS_TRY(sweep(c, am, ac, ap, rhs, 0, jlo, true));
-    TCS_TRY(copy(c, X[1], rhs, c->nint));
-    TCS_TRY(rows3d_launch<false>(c, "adj_fwd_rows", ry, jlo, am, ac, ap, rhs));
-    TCS_TRY(sweep(c, am, ac, ap, rhs, 1, jlo, false));
-    TCS_TRY(copy(c, X[2], rhs, c->nint));
+    double *am = c->am, *ac = c->ac, *ap = c->ap;
+    TCS_TRY(rows3d_launch<true>(c, "adj_fwd_rows", rz, jlo, am, ac, ap, X[0]));
+    TCS_TRY(sweep(c, am, ac, ap, X[0], X[0], 2, jlo, true));
+    TCS_TRY(rows3d_launch<false>(c, "adj_fwd_rows", rx, jlo, am, ac, ap, X[1]));
+    TCS_TRY(sweep(c, am, ac, ap, X[0], X[1], 0, jlo, true));
+    TCS_TRY(rows3d_launch<false>(c, "adj_fwd_rows", ry, jlo, am, ac, ap, X[2]));
+    TCS_TRY(sweep(c, am, ac, ap, X[1], X[2], 1, jlo, false));
     return TCS_OK;
 }
 
+// T, dW, the tables, the stale scalars and dP keep the values that the
+// backward pass needs until the step's end; what is overwritten is copied.
+// (A copy and a solve's right-hand side or increment moved by launches of
+// their own, and the adjoints' folds, packs and clears likewise: 286 kernels
+// and copies a step, 139 now; a backward step at 32x45x64 0.91 -> 0.52 ms, at
+// 128^3 4.84 -> 3.76 ms, the transposed systems split as the forward ones are.)
 static int forward_keep(tcs_ctx *c, AdjWork *w, double dt) {
     const Grid g = c->grid();
     double **f = c->f;
-    const dim3 blk = interior_block(), grd = interior_grid(c->n1m, c->n2m, c->n3m);
-    for (int s = 0; s < NSTATE; s++) TCS_TRY(copy(c, w->s0[s], f[STATE_IDS[s]], c->nfull));
+    {
+        Arrays a;
+        for (int s = 0; s < NSTATE; s++) a.add(w->s0[s], f[STATE_IDS[s]], c->nfull);
+        TCS_TRY(copy_arrays(c, a));
+    }
     // thermal
     TCS_TRY(adi_forward(c, ThermalZ{g, c->phys, dt, f[TCS_T], f[TCS_U], f[TCS_V], f[TCS_W], c->wall[TCS_TBCUP],
                                     c->wall[TCS_TBCBT]},
                         ThermalX{g, c->phys, dt, f[TCS_T], f[TCS_U]}, ThermalY{g, c->phys, dt, f[TCS_T], f[TCS_V]}, 1,
                         w->X[STG_T]));
-    TCS_LAUNCH(c->stream, "adj_fwd_add", k_interior_out<2>, grd, blk, 0, g, 1, f[TCS_T], w->X[STG_T][2]);
-    TCS_TRY(halo(c, f[TCS_T]));
-    TCS_TRY(copy(c, w->sT1, f[TCS_T], c->nfull));
+    TCS_TRY(store_keep<2>(c, 1, w->X[STG_T][2], f[TCS_T], nullptr));
     TCS_TRY(momentum_coeffi(c));
-    TCS_TRY(copy(c, w->sMu, f[TCS_MU], c->ntab));
-    TCS_TRY(copy(c, w->siR, f[TCS_INVRHO], c->ntab));
     // solvedU
     TCS_TRY(adi_forward(c, DUZ{g, c->phys, dt, f[TCS_U], f[TCS_V], f[TCS_W], f[TCS_P], f[TCS_T], f[TCS_MU],
                                f[TCS_INVRHO], c->wall[TCS_UBCUP], c->wall[TCS_UBCBT], c->wall[TCS_VBCUP],
                                c->wall[TCS_VBCBT]},
                         DUX{g, c->phys, dt, f[TCS_U], f[TCS_MU], f[TCS_INVRHO]},
                         DUY{g, c->phys, dt, f[TCS_V], f[TCS_MU], f[TCS_INVRHO]}, 1, w->X[STG_U]));
-    TCS_LAUNCH(c->stream, "adj_fwd_store", k_interior_out<1>, grd, blk, 0, g, 1, f[TCS_DU], w->X[STG_U][2]);
-    TCS_TRY(halo(c, f[TCS_DU]));
-    TCS_TRY(copy(c, w->sdU1, f[TCS_DU], c->nfull));
+    TCS_TRY(store_keep<1>(c, 1, w->X[STG_U][2], f[TCS_DU], w->sdU1));
     // solvedV (rows j >= 2)
-    TCS_TRY(launch_stale(c));
-    TCS_TRY(copy(c, w->sstale, c->stale, 6));
     TCS_TRY(adi_forward(c, DVZ{g, c->phys, dt, f[TCS_U], f[TCS_V], f[TCS_W], f[TCS_P], f[TCS_DU], f[TCS_MU],
                                f[TCS_INVRHO], c->wall[TCS_VBCUP], c->wall[TCS_VBCBT]},
                         DVX{g, c->phys, dt, f[TCS_U], f[TCS_INVRHO], c->stale},
                         DVY{g, c->phys, dt, f[TCS_V], f[TCS_MU], f[TCS_INVRHO]}, 2, w->X[STG_V]));
-    TCS_LAUNCH(c->stream, "adj_fwd_zero", k_dV_zero_rows, dim3((c->N1 + 63) / 64, c->N3), dim3(64), 0, g, f[TCS_DV]);
-    TCS_LAUNCH(c->stream, "adj_fwd_store", k_interior_out<1>, grd, blk, 0, g, 2, f[TCS_DV], w->X[STG_V][2]);
-    TCS_TRY(halo(c, f[TCS_DV]));
-    TCS_TRY(copy(c, w->sdV1, f[TCS_DV], c->nfull));
+    TCS_TRY(store_keep<1>(c, 2, w->X[STG_V][2], f[TCS_DV], w->sdV1));
     // solvedW
-    TCS_TRY(launch_stale(c));
     TCS_TRY(adi_forward(c, DWZ{g, c->phys, dt, f[TCS_U], f[TCS_V], f[TCS_W], f[TCS_P], f[TCS_DU], f[TCS_DV],
                                f[TCS_MU], f[TCS_INVRHO], c->wall[TCS_VBCUP], c->wall[TCS_VBCBT],
                                c->wall[TCS_WBCUP], c->wall[TCS_WBCBT]},
                         DWX{g, c->phys, dt, f[TCS_U], f[TCS_INVRHO], c->stale},
                         DWY{g, c->phys, dt, f[TCS_V], f[TCS_INVRHO], c->stale}, 1, w->X[STG_W]));
-    TCS_LAUNCH(c->stream, "adj_fwd_store", k_interior_out<1>, grd, blk, 0, g, 1, f[TCS_DW], w->X[STG_W][2]);
-    TCS_TRY(halo(c, f[TCS_DW]));
-    TCS_TRY(copy(c, w->sdW1, f[TCS_DW], c->nfull));
+    TCS_TRY(store_keep<1>(c, 1, w->X[STG_W][2], f[TCS_DW], nullptr));
     // block corrections, pseudo-update
     TCS_TRY(momentum_blockLdV(c, dt));
     TCS_TRY(halo(c, f[TCS_DV]));
-    TCS_TRY(copy(c, w->sdV2, f[TCS_DV], c->nfull));
     TCS_TRY(momentum_blockLdU(c, dt));
-    TCS_TRY(copy(c, w->sdU2, f[TCS_DU], c->nfull));
     TCS_TRY(momentum_pseudoupdate(c));
-    TCS_TRY(halo(c, f[TCS_U]));
-    TCS_TRY(halo(c, f[TCS_V]));
-    TCS_TRY(halo(c, f[TCS_W]));
-    TCS_TRY(copy(c, w->sU1, f[TCS_U], c->nfull));
-    TCS_TRY(copy(c, w->sV1, f[TCS_V], c->nfull));
-    TCS_TRY(copy(c, w->sW1, f[TCS_W], c->nfull));
+    {
+        Arrays a;
+        a.add(w->sU1, f[TCS_U], c->nfull);
+        a.add(w->sV1, f[TCS_V], c->nfull);
+        a.add(w->sW1, f[TCS_W], c->nfull);
+        TCS_LAUNCH(c->stream, "adj_fwd_keep", k_halo_keep, interior_grid(c->n1m, c->n2m, c->n3m * a.count),
+                   interior_block(), 0, g, a);
+    }
     // pressure
     TCS_TRY(pressure_rhs(c, dt));
     TCS_TRY(pressure_poisson(c));
     TCS_TRY(halo(c, f[TCS_DP]));
-    TCS_TRY(copy(c, w->sdP, f[TCS_DP], c->nfull));
     TCS_TRY(pressure_projection(c, dt));
-    TCS_TRY(halo(c, f[TCS_U]));
-    TCS_TRY(halo(c, f[TCS_V]));
-    TCS_TRY(halo(c, f[TCS_W]));
-    TCS_TRY(halo(c, f[TCS_P]));
-    TCS_TRY(halo(c, f[TCS_DPHAT]));
-    return TCS_OK;
+    return halo(c, {f[TCS_U], f[TCS_V], f[TCS_W], f[TCS_P], f[TCS_DPHAT]});
 }
 
 // ---- the step backwards ----------------------------------------------------------
 
-// Before a cell update that overwrites field F's interior rows j >= jlo: its
-// new adjoint starts as the old one outside those cells (untouched values
-// pass through) and zero inside (filled by the update's product).
-static int overwrite_begin(tcs_ctx *c, double *tmp, const double *bar, int jlo) {
-    TCS_TRY(copy(c, tmp, bar, c->nfull));
-    TCS_LAUNCH(c->stream, "adj_zero", k_zero_interior, interior_grid(c->n1m, c->n2m, c->n3m), interior_block(), 0,
-               c->grid(), jlo, tmp);
+// Before a cell update that overwrites fields' interior rows j >= jlo: their
+// new adjoints (dst) start as the old ones (src) outside those cells
+// (untouched values pass through) and zero inside (filled by the update's
+// product).
+__global__ void k_overwrite_begin(Grid g, int jlo, Arrays a) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    const int j = blockIdx.y * blockDim.y + threadIdx.y;
+    const int k = blockIdx.z % g.N3, f = blockIdx.z / g.N3;
+    if (i >= g.N1 || j >= g.N2) return;
+    const bool in = i >= 1 && i <= g.n1m && j >= jlo && j <= g.n2m && k >= 1 && k <= g.n3m;
+    const size_t q = g.ix(i, j, k);
+    a.dst[f][q] = in ? 0.0 : a.src[f][q];
+}
+static int overwrite_begin(tcs_ctx *c, int jlo, std::initializer_list<std::pair<double *, const double *>> fields) {
+    Arrays a;
+    for (const auto &f : fields) a.add(f.first, f.second, c->nfull);
+    TCS_LAUNCH(c->stream, "adj_begin", k_overwrite_begin, interior_grid(c->N1, c->N2, c->N3 * a.count),
+               interior_block(), 0, c->grid(), jlo, a);
+    return TCS_OK;
+}
+
+template <bool ZERO>
+static int take(tcs_ctx *c, int jlo, double *b, double *r) {
+    TCS_LAUNCH(c->stream, "adj_take", k_take<ZERO>, interior_grid(c->n1m, c->n2m, c->n3m), interior_block(), 0,
+               c->grid(), jlo, b, r);
     return TCS_OK;
 }
 
@@ -517,43 +621,39 @@ static int backward(tcs_ctx *c, AdjWork *w, double dt) {
     const Grid g = c->grid();
     const dim3 blk = interior_block(), grd = interior_grid(c->n1m, c->n2m, c->n3m);
     double **b = w->b;
+    const double *Mu = c->f[TCS_MU], *iR = c->f[TCS_INVRHO];
     const double *TBCup = c->wall[TCS_TBCUP], *TBCbt = c->wall[TCS_TBCBT];
     // halos after the projection
-    TCS_TRY(halo_adj(c, b[ST_DPHAT]));
-    TCS_TRY(halo_adj(c, b[ST_P]));
-    TCS_TRY(halo_adj(c, b[ST_W]));
-    TCS_TRY(halo_adj(c, b[ST_V]));
-    TCS_TRY(halo_adj(c, b[ST_U]));
+    TCS_TRY(halo_adj(c, {b[ST_DPHAT], b[ST_P], b[ST_W], b[ST_V], b[ST_U]}));
     // P wall extrapolation; dPhat / dP0 history; projection
     TCS_TRY(wall_extrap_adj(c, b[ST_P]));
     {
-        const DPhatUpdate cell{g, w->sdP, w->s0[ST_DPHAT], w->s0[ST_DP0]};
-        TCS_TRY(overwrite_begin(c, w->tmp[0], b[ST_DPHAT], 1));
-        TCS_TRY(overwrite_begin(c, w->tmp[1], b[ST_DP0], 1));
+        const DPhatUpdate cell{g, c->f[TCS_DP], w->s0[ST_DPHAT], w->s0[ST_DP0]};
+        TCS_TRY(overwrite_begin(c, 1, {{w->tmp[0], b[ST_DPHAT]}, {w->tmp[1], b[ST_DP0]}}));
         TCS_TRY(cell_vjp(c, w, cell, 1, OutBars{{b[ST_DPHAT], b[ST_DP0], nullptr, nullptr}, 1},
                          InBars<3>{{w->bdP, w->tmp[0], w->tmp[1]}}));
         std::swap(b[ST_DPHAT], w->tmp[0]);
         std::swap(b[ST_DP0], w->tmp[1]);
     }
     {
-        const Projection cell{g, c->phys, dt, w->siR, w->sdP, w->s0[ST_DPHAT], w->s0[ST_DP0],
+        const Projection cell{g, c->phys, dt, iR, c->f[TCS_DP], w->s0[ST_DPHAT], w->s0[ST_DP0],
                               w->sU1, w->sV1, w->sW1, w->s0[ST_P]};
-        for (int q = 0; q < 4; q++) TCS_TRY(overwrite_begin(c, w->tmp[q], b[ST_U + q], 1));
+        TCS_TRY(overwrite_begin(c, 1, {{w->tmp[0], b[ST_U]}, {w->tmp[1], b[ST_V]}, {w->tmp[2], b[ST_W]},
+                                       {w->tmp[3], b[ST_P]}}));
         TCS_TRY(cell_vjp(c, w, cell, 1, OutBars{{b[ST_U], b[ST_V], b[ST_W], b[ST_P]}, 1},
                          InBars<8>{{w->biR, w->bdP, b[ST_DPHAT], b[ST_DP0], w->tmp[0], w->tmp[1], w->tmp[2],
                                     w->tmp[3]}}));
         for (int q = 0; q < 4; q++) std::swap(b[ST_U + q], w->tmp[q]);
     }
     // Poisson: halo(dP), wall extrapolation, mean, then the transposed solve
-    TCS_TRY(halo_adj(c, w->bdP));
+    TCS_TRY(halo_adj(c, {w->bdP}));
     TCS_TRY(wall_extrap_adj(c, w->bdP));
-    TCS_HIP(hipMemsetAsync(w->scal, 0, sizeof(double), c->stream));
-    TCS_LAUNCH(c->stream, "adj_sum", k_interior_sum, grd, blk, 0, g, w->bdP, w->scal);
-    TCS_LAUNCH(c->stream, "adj_sub", k_interior_sub, grd, blk, 0, g, w->scal, w->bdP);
+    TCS_LAUNCH(c->stream, "adj_mean", k_interior_mean, dim3((unsigned)std::min<size_t>(SUM_BLOCKS, (c->nint + 2047) / 2048)),
+               dim3(256), 0, g, w->bdP, w->psum);
+    TCS_LAUNCH(c->stream, "adj_take_mean", k_take_mean, grd, blk, 0, g, w->psum + SUM_BLOCKS, w->bdP, w->rint);
     {
         const int n2m = c->n2m, n3m = c->n3m, h1p = c->h1p;
         double2 *spec = (double2 *)c->spec_x;
-        TCS_LAUNCH(c->stream, "adj_pack", k_full_to_int, grd, blk, 0, g, 1, w->bdP, w->rint);
         TCS_TRY(fft_x_fwd_launch(c, "adj_fft_x_fwd", w->rint, spec));
         TCS_TRY(fft_z_launch<-1>(c, "adj_fft_z", spec));
         const int nsys = n3m * h1p;
@@ -561,47 +661,41 @@ static int backward(tcs_ctx *c, AdjWork *w, double dt) {
                    c->h3p, c->ptab, c->ptab + n2m, c->ptab + 2 * n2m, c->dxk2, c->dzk, spec, c->pC);
         TCS_TRY(fft_z_launch<+1>(c, "adj_fft_z", spec));
         TCS_TRY(fft_x_inv_launch(c, "adj_fft_x_inv", spec, w->tmp[0]));
-        TCS_LAUNCH(c->stream, "adj_pack", k_full_to_int, grd, blk, 0, g, 1, w->tmp[0], w->rint);
-        TCS_HIP(hipMemsetAsync(w->bdP, 0, c->nfull * sizeof(double), c->stream));
     }
     // pressure right-hand side
     {
-        const PressureRHS cell{g, c->phys, dt, w->sU1, w->sV1, w->sW1, w->s0[ST_DPHAT], w->siR,
+        const PressureRHS cell{g, c->phys, dt, w->sU1, w->sV1, w->sW1, w->s0[ST_DPHAT], iR,
                                c->wall[TCS_VBCUP], c->wall[TCS_VBCBT]};
-        TCS_TRY(cell_vjp(c, w, cell, 1, OutBars{{w->rint, nullptr, nullptr, nullptr}, 0},
+        TCS_TRY(cell_vjp(c, w, cell, 1, OutBars{{w->tmp[0], nullptr, nullptr, nullptr}, 1},
                          InBars<7>{{b[ST_U], b[ST_V], b[ST_W], b[ST_DPHAT], w->biR, nullptr, nullptr}}));
     }
     // halos of U, V, W; pseudo-update
-    TCS_TRY(halo_adj(c, b[ST_W]));
-    TCS_TRY(halo_adj(c, b[ST_V]));
-    TCS_TRY(halo_adj(c, b[ST_U]));
+    TCS_TRY(halo_adj(c, {b[ST_W], b[ST_V], b[ST_U]}));
     TCS_LAUNCH(c->stream, "adj_pseudo", k_pseudo_adj, grd, blk, 0, g, b[ST_U], b[ST_V], b[ST_W], w->bdU, w->bdV,
                w->bdW);
     // blockLdU, halo(dV), blockLdV, halo(dW)
     {
-        const BlockLdU cell{g, c->phys, dt, w->s0[ST_U], w->sdV2, w->sdW1, w->sMu, w->siR, w->sdU1};
-        TCS_TRY(overwrite_begin(c, w->tmp[0], w->bdU, 1));
+        const BlockLdU cell{g, c->phys, dt, w->s0[ST_U], c->f[TCS_DV], c->f[TCS_DW], Mu, iR, w->sdU1};
+        TCS_TRY(overwrite_begin(c, 1, {{w->tmp[0], w->bdU}}));
         TCS_TRY(cell_vjp(c, w, cell, 1, OutBars{{w->bdU, nullptr, nullptr, nullptr}, 1},
                          InBars<6>{{b[ST_U], w->bdV, w->bdW, w->bMu, w->biR, w->tmp[0]}}));
         std::swap(w->bdU, w->tmp[0]);
     }
-    TCS_TRY(halo_adj(c, w->bdV));
+    TCS_TRY(halo_adj(c, {w->bdV}));
     {
-        const BlockLdV cell{g, c->phys, dt, w->s0[ST_V], w->sdW1, w->sMu, w->siR, w->sdV1};
-        TCS_TRY(overwrite_begin(c, w->tmp[0], w->bdV, 2));
+        const BlockLdV cell{g, c->phys, dt, w->s0[ST_V], c->f[TCS_DW], Mu, iR, w->sdV1};
+        TCS_TRY(overwrite_begin(c, 2, {{w->tmp[0], w->bdV}}));
         TCS_TRY(cell_vjp(c, w, cell, 2, OutBars{{w->bdV, nullptr, nullptr, nullptr}, 1},
                          InBars<5>{{b[ST_V], w->bdW, w->bMu, w->biR, w->tmp[0]}}));
         std::swap(w->bdV, w->tmp[0]);
     }
-    TCS_TRY(halo_adj(c, w->bdW));
     // solvedW: dW's interior is the y stage's solution
-    TCS_LAUNCH(c->stream, "adj_pack", k_full_to_int, grd, blk, 0, g, 1, w->bdW, w->lam);
-    TCS_HIP(hipMemsetAsync(w->bdW, 0, c->nfull * sizeof(double), c->stream));
+    TCS_TRY(take<true>(c, 1, w->bdW, w->lam));
     {
-        const DWZ rz{g, c->phys, dt, w->s0[ST_U], w->s0[ST_V], w->s0[ST_W], w->s0[ST_P], w->sdU1, w->sdV1, w->sMu,
-                     w->siR, c->wall[TCS_VBCUP], c->wall[TCS_VBCBT], c->wall[TCS_WBCUP], c->wall[TCS_WBCBT]};
-        const DWX rx{g, c->phys, dt, w->s0[ST_U], w->siR, w->sstale};
-        const DWY ry{g, c->phys, dt, w->s0[ST_V], w->siR, w->sstale};
+        const DWZ rz{g, c->phys, dt, w->s0[ST_U], w->s0[ST_V], w->s0[ST_W], w->s0[ST_P], w->sdU1, w->sdV1, Mu,
+                     iR, c->wall[TCS_VBCUP], c->wall[TCS_VBCBT], c->wall[TCS_WBCUP], c->wall[TCS_WBCBT]};
+        const DWX rx{g, c->phys, dt, w->s0[ST_U], iR, c->stale};
+        const DWY ry{g, c->phys, dt, w->s0[ST_V], iR, c->stale};
         TCS_TRY(stage_adj<false>(c, w, ry, 1, 1, false, w->X[STG_W][2], InBars<3>{{b[ST_V], w->biR, w->bstale}}));
         TCS_TRY(stage_adj<false>(c, w, rx, 0, 1, true, w->X[STG_W][1], InBars<3>{{b[ST_U], w->biR, w->bstale}}));
         TCS_TRY(stage_adj<true>(c, w, rz, 2, 1, true, w->X[STG_W][0],
@@ -609,14 +703,12 @@ static int backward(tcs_ctx *c, AdjWork *w, double dt) {
                                             nullptr, nullptr, nullptr, nullptr}}));
     }
     // solvedV: rows j >= 2; dV's other rows are zeroed in the forward step
-    TCS_TRY(halo_adj(c, w->bdV));
-    TCS_LAUNCH(c->stream, "adj_pack", k_full_to_int, grd, blk, 0, g, 2, w->bdV, w->lam);
-    TCS_HIP(hipMemsetAsync(w->bdV, 0, c->nfull * sizeof(double), c->stream));
+    TCS_TRY(take<true>(c, 2, w->bdV, w->lam));
     {
-        const DVZ rz{g, c->phys, dt, w->s0[ST_U], w->s0[ST_V], w->s0[ST_W], w->s0[ST_P], w->sdU1, w->sMu, w->siR,
+        const DVZ rz{g, c->phys, dt, w->s0[ST_U], w->s0[ST_V], w->s0[ST_W], w->s0[ST_P], w->sdU1, Mu, iR,
                      c->wall[TCS_VBCUP], c->wall[TCS_VBCBT]};
-        const DVX rx{g, c->phys, dt, w->s0[ST_U], w->siR, w->sstale};
-        const DVY ry{g, c->phys, dt, w->s0[ST_V], w->sMu, w->siR};
+        const DVX rx{g, c->phys, dt, w->s0[ST_U], iR, c->stale};
+        const DVY ry{g, c->phys, dt, w->s0[ST_V], Mu, iR};
         TCS_TRY(stage_adj<false>(c, w, ry, 1, 2, false, w->X[STG_V][2], InBars<3>{{b[ST_V], w->bMu, w->biR}}));
         TCS_TRY(stage_adj<false>(c, w, rx, 0, 2, true, w->X[STG_V][1], InBars<3>{{b[ST_U], w->biR, w->bstale}}));
         TCS_TRY(stage_adj<true>(c, w, rz, 2, 2, true, w->X[STG_V][0],
@@ -624,14 +716,12 @@ static int backward(tcs_ctx *c, AdjWork *w, double dt) {
                                            nullptr}}));
     }
     // solvedU
-    TCS_TRY(halo_adj(c, w->bdU));
-    TCS_LAUNCH(c->stream, "adj_pack", k_full_to_int, grd, blk, 0, g, 1, w->bdU, w->lam);
-    TCS_HIP(hipMemsetAsync(w->bdU, 0, c->nfull * sizeof(double), c->stream));
+    TCS_TRY(take<true>(c, 1, w->bdU, w->lam));
     {
-        const DUZ rz{g, c->phys, dt, w->s0[ST_U], w->s0[ST_V], w->s0[ST_W], w->s0[ST_P], w->sT1, w->sMu, w->siR,
+        const DUZ rz{g, c->phys, dt, w->s0[ST_U], w->s0[ST_V], w->s0[ST_W], w->s0[ST_P], c->f[TCS_T], Mu, iR,
                      c->wall[TCS_UBCUP], c->wall[TCS_UBCBT], c->wall[TCS_VBCUP], c->wall[TCS_VBCBT]};
-        const DUX rx{g, c->phys, dt, w->s0[ST_U], w->sMu, w->siR};
-        const DUY ry{g, c->phys, dt, w->s0[ST_V], w->sMu, w->siR};
+        const DUX rx{g, c->phys, dt, w->s0[ST_U], Mu, iR};
+        const DUY ry{g, c->phys, dt, w->s0[ST_V], Mu, iR};
         TCS_TRY(stage_adj<false>(c, w, ry, 1, 1, false, w->X[STG_U][2], InBars<3>{{b[ST_V], w->bMu, w->biR}}));
         TCS_TRY(stage_adj<false>(c, w, rx, 0, 1, true, w->X[STG_U][1], InBars<3>{{b[ST_U], w->bMu, w->biR}}));
         TCS_TRY(stage_adj<true>(c, w, rz, 2, 1, true, w->X[STG_U][0],
@@ -639,12 +729,11 @@ static int backward(tcs_ctx *c, AdjWork *w, double dt) {
                                             nullptr, nullptr, nullptr}}));
     }
     // stale viscosities and the Mu / invRho tables (from T after the thermal stage)
-    TCS_LAUNCH(c->stream, "adj_stale", k_stale_adj, dim3(1), dim3(64), 0, g, w->sMu, w->bstale, w->bMu);
-    TCS_LAUNCH(c->stream, "adj_coeffi", k_coeffi_adj, dim3((c->N2 + 63) / 64, c->N3), dim3(64), 0, g, c->phys, w->sT1,
+    TCS_LAUNCH(c->stream, "adj_stale", k_stale_adj, dim3(1), dim3(64), 0, g, Mu, w->bstale, w->bMu);
+    TCS_LAUNCH(c->stream, "adj_coeffi", k_coeffi_adj, dim3((c->N2 + 63) / 64, c->N3), dim3(64), 0, g, c->phys, c->f[TCS_T],
                w->bMu, w->biR, b[ST_T]);
-    TCS_TRY(halo_adj(c, b[ST_T]));
     // thermal: T1 = T0 + x3 on the interior
-    TCS_LAUNCH(c->stream, "adj_pack", k_full_to_int, grd, blk, 0, g, 1, b[ST_T], w->lam);
+    TCS_TRY(take<false>(c, 1, b[ST_T], w->lam));
     {
         const ThermalZ rz{g, c->phys, dt, w->s0[ST_T], w->s0[ST_U], w->s0[ST_V], w->s0[ST_W], TBCup, TBCbt};
         const ThermalX rx{g, c->phys, dt, w->s0[ST_T], w->s0[ST_U]};
@@ -656,10 +745,11 @@ static int backward(tcs_ctx *c, AdjWork *w, double dt) {
                                            w->bwall[TCS_TBCBT]}}));
     }
     // the step's own tables and scalars start from zero next time
-    TCS_HIP(hipMemsetAsync(w->bMu, 0, c->ntab * sizeof(double), c->stream));
-    TCS_HIP(hipMemsetAsync(w->biR, 0, c->ntab * sizeof(double), c->stream));
-    TCS_HIP(hipMemsetAsync(w->bstale, 0, REV_STALE * REV_STALE_STRIDE * sizeof(double), c->stream));
-    return TCS_OK;
+    Arrays z;
+    z.add(w->bMu, nullptr, c->ntab);
+    z.add(w->biR, nullptr, c->ntab);
+    z.add(w->bstale, nullptr, REV_STALE * REV_STALE_STRIDE);
+    return copy_arrays(c, z);
 }
 
 }  // namespace adj
@@ -687,15 +777,15 @@ static int adjoint_alloc(tcs_ctx *c) {
     };
     int rc = TCS_OK;
     for (int s = 0; s < adj::NSTATE && rc == TCS_OK; s++) rc |= get(&w->b[s], c->nfull) | get(&w->s0[s], c->nfull);
-    for (double **p : {&w->bdU, &w->bdV, &w->bdW, &w->bdP, &w->sT1, &w->sdU1, &w->sdV1, &w->sdW1, &w->sdV2, &w->sdU2,
-                       &w->sU1, &w->sV1, &w->sW1, &w->sdP, &w->tmp[0], &w->tmp[1], &w->tmp[2], &w->tmp[3]})
+    for (double **p : {&w->bdU, &w->bdV, &w->bdW, &w->bdP, &w->sdU1, &w->sdV1, &w->sU1, &w->sV1, &w->sW1, &w->tmp[0],
+                        &w->tmp[1], &w->tmp[2], &w->tmp[3]})
         rc |= get(p, c->nfull);
-    for (double **p : {&w->bMu, &w->biR, &w->sMu, &w->siR}) rc |= get(p, c->ntab);
-    rc |= get(&w->bstale, (size_t)REV_STALE * REV_STALE_STRIDE) | get(&w->sstale, 6) | get(&w->scal, 1);
+    for (double **p : {&w->bMu, &w->biR}) rc |= get(p, c->ntab);
+    rc |= get(&w->bstale, (size_t)REV_STALE * REV_STALE_STRIDE) | get(&w->psum, adj::SUM_BLOCKS + 2);
     for (int q = 0; q < TCS_NWALL; q++) rc |= get(&w->bwall[q], c->nwall);
     for (int s = 0; s < 4; s++)
         for (int q = 0; q < 3; q++) rc |= get(&w->X[s][q], c->nint);
-    for (double **p : {&w->lam, &w->abar, &w->bbar, &w->cbar, &w->aT, &w->cT, &w->rint}) rc |= get(p, c->nint);
+    for (double **p : {&w->lam, &w->rint}) rc |= get(p, c->nint);
     if (rc != TCS_OK) {
         adjoint_free(c);
         set_error("tcs_adjoint: device allocation failed");
@@ -714,12 +804,12 @@ extern "C" int tcs_adjoint_zero(tcs_ctx *c) {
     c->kept = 0;
     TCS_TRY(adjoint_alloc(c));
     AdjWork *w = c->adj;
-    for (int s = 0; s < adj::NSTATE; s++) TCS_HIP(hipMemsetAsync(w->b[s], 0, c->nfull * sizeof(double), c->stream));
-    for (int q = 0; q < TCS_NWALL; q++)
-        TCS_HIP(hipMemsetAsync(w->bwall[q], 0, c->nwall * sizeof(double), c->stream));
-    for (double *p : {w->bdU, w->bdV, w->bdW, w->bdP})
-        TCS_HIP(hipMemsetAsync(p, 0, c->nfull * sizeof(double), c->stream));
-    return TCS_OK;
+    adj::Arrays z;
+    static_assert(adj::NSTATE + TCS_NWALL + 4 <= adj::Arrays::MAX, "one launch");
+    for (int s = 0; s < adj::NSTATE; s++) z.add(w->b[s], nullptr, c->nfull);
+    for (int q = 0; q < TCS_NWALL; q++) z.add(w->bwall[q], nullptr, c->nwall);
+    for (double *p : {w->bdU, w->bdV, w->bdW, w->bdP}) z.add(p, nullptr, c->nfull);
+    return adj::copy_arrays(c, z);
 }
 
 static double *adjoint_array(tcs_ctx *c, int32_t kind, int32_t id, size_t &n) {

@@ -195,9 +195,32 @@ struct RevW {
 };
 
 struct OutBars {
-    const double *p[4];  // output adjoints (null: no such output)
-    int full;            // 1: full-field layout, 0: interior layout
+    const double *p[4];
+    int full;  // p in the fields' layout (1) or the interior layout (0)
+    // rows of a solved stage instead (lam not null): their adjoints from
+    // lambda = A^-T xbar and the solution x, -lambda x' with x' the solution
+    // at the row before, at the row and after it on the stage's line, and
+    // lambda for the right-hand side (has_d)
+    const double *lam, *x;
+    int axis, jlo, cyc, has_d;
 };
+// the line through interior cell q along `axis` (0 x, 1 y, 2 z), rows j >= jlo:
+// position, length and stride of the line, and the cells before and after q
+// on it (cyclically), with hp, hn whether the line has them
+struct LinePos {
+    int pos, n;
+    long prev, next;
+    bool hp, hn;
+};
+__device__ __forceinline__ LinePos line_pos(const Grid &g, int axis, int jlo, int cyc, int i, int j, int k) {
+    const long n1 = g.n1m, q = (long)g.r3(i, j, k);
+    const long stride = axis == 0 ? 1 : axis == 1 ? n1 : n1 * g.n2m;
+    const int n = axis == 0 ? g.n1m : axis == 1 ? g.n2m - jlo + 1 : g.n3m;
+    const int pos = axis == 0 ? i - 1 : axis == 1 ? j - jlo : k - 1;
+    const long wrap = (long)(n - 1) * stride;
+    return {pos, n, pos > 0 ? q - stride : q + wrap, pos < n - 1 ? q + stride : q - wrap, pos > 0 || cyc,
+            pos < n - 1 || cyc};
+}
 template <int NF>
 struct InBars {
     double *p[NF];  // adjoints of the input fields (the first Cell::ND are used)
@@ -324,12 +347,18 @@ k_cell_vjp(Cell cell, int jlo, int jhi, int lw, OutBars ob, InBars<Cell::NF> ib)
         const int k = blockIdx.z * VJP_KB + kk + 1;
         const size_t q = ob.full ? g.ix(i, j, k) : g.r3(i, j, k);
         double w[4];
-        bool any = false;
+        if (ob.lam) {
+            const LinePos L = line_pos(g, ob.axis, ob.jlo, ob.cyc, i, j, k);
+            const double l = act ? ob.lam[q] : 0.0;
+            w[0] = L.hp ? -l * ob.x[L.prev] : 0.0;
+            w[1] = -l * ob.x[q];
+            w[2] = L.hn ? -l * ob.x[L.next] : 0.0;
+            w[3] = ob.has_d ? l : 0.0;
+        } else {
 #pragma unroll
-        for (int o = 0; o < 4; o++) {
-            w[o] = (act && ob.p[o]) ? ob.p[o][q] : 0.0;
-            any = any || w[o] != 0.0;
+            for (int o = 0; o < 4; o++) w[o] = (act && ob.p[o]) ? ob.p[o][q] : 0.0;
         }
+        const bool any = w[0] != 0.0 || w[1] != 0.0 || w[2] != 0.0 || w[3] != 0.0;
         if (__ballot(any) == 0) continue;
         if constexpr (HasWalls<Cell>::value) {
             if (__ballot(!cell.wall_free(j)) == 0) cell_reverse<2>(cell, i, j, k, w, ib, lw, lane, act, all);

@@ -339,17 +339,24 @@ struct LineOut {
 bool ptdma_part_plan(int n_row, int &P, int &w1, int &w2);
 int ptdma_part_launch(double *A, const double *B, double *C, double *D, int n0, long ss0, int n1, long ss1,
                       int n_row, long rs, bool cyclic, hipStream_t st, const LineOut &out = LineOut());
+// right-hand sides from Din, solutions to Dout (which may be Din)
+int ptdma_part_launch(const double *A, const double *B, const double *C, const double *Din, double *Dout, int n0,
+                      long ss0, int n1, long ss1, int n_row, long rs, bool cyclic, hipStream_t st);
 // FP32 lines (the mixed form's ADI solves), same algorithm and layouts.
 int ptdma_part_launch(float *A, const float *B, float *C, float *D, int n0, long ss0, int n1, long ss1,
                       int n_row, long rs, bool cyclic, hipStream_t st, const LineOut &out = LineOut());
 // ADI sweep of a context: split solve when the context asks for it and the
 // line length allows, else the single-rank order.
-inline int ptdma_sweep(const tcs_ctx *c, double *A, const double *B, double *C, double *D, int n0, long ss0,
-                       int n1, long ss1, int n_row, long rs, bool cyclic) {
+inline int ptdma_sweep(const tcs_ctx *c, double *A, const double *B, double *C, const double *Din, double *Dout,
+                       int n0, long ss0, int n1, long ss1, int n_row, long rs, bool cyclic) {
     int P, w1, w2;
     if (c->tdma_split && ptdma_part_plan(n_row, P, w1, w2) && (rs == 1 || ss0 == 1))
-        return ptdma_part_launch(A, B, C, D, n0, ss0, n1, ss1, n_row, rs, cyclic, c->stream);
-    return ptdma_exact_launch(A, B, C, D, D, n0, ss0, n1, ss1, n_row, rs, cyclic, false, c->stream);
+        return ptdma_part_launch(A, B, C, Din, Dout, n0, ss0, n1, ss1, n_row, rs, cyclic, c->stream);
+    return ptdma_exact_launch(A, B, C, Din, Dout, n0, ss0, n1, ss1, n_row, rs, cyclic, false, c->stream);
+}
+inline int ptdma_sweep(const tcs_ctx *c, double *A, const double *B, double *C, double *D, int n0, long ss0,
+                       int n1, long ss1, int n_row, long rs, bool cyclic) {
+    return ptdma_sweep(c, A, B, C, D, D, n0, ss0, n1, ss1, n_row, rs, cyclic);
 }
 // FP32 sweep of the mixed form: always the split solve (lines <= 512 rows).
 inline int ptdma_sweep(const tcs_ctx *c, float *A, const float *B, float *C, float *D, int n0, long ss0, int n1,

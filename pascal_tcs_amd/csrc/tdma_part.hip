@@ -61,7 +61,7 @@ __device__ __forceinline__ int line_group(int bx, int nbx) {
 template <typename T, bool CYC, int SX>
 __global__ void __launch_bounds__(SX * PT_PMAX)
 k_ptdma_part(const T *__restrict__ A, const T *__restrict__ B, const T *__restrict__ C,
-             T *__restrict__ D, int n0, long ss1, long rs, int P, int w1, int w2, LineOut out) {
+             const T *Din, T *D, int n0, long ss1, long rs, int P, int w1, int w2, LineOut out) {
     __shared__ RedLDS<T, SX, 1, PT_PMAX> red;
     const int t = threadIdx.x;
     const int line = t % SX, p = t / SX;
@@ -78,7 +78,7 @@ k_ptdma_part(const T *__restrict__ A, const T *__restrict__ B, const T *__restri
         for (int r = 0; r < PT_MMAX; r++) {
             if (act && r < m) {
                 const long o = base + (long)(j0 + r) * rs;
-                a[r] = A[o]; b[r] = B[o]; c[r] = C[o]; d[0][r] = D[o];
+                a[r] = A[o]; b[r] = B[o]; c[r] = C[o]; d[0][r] = Din[o];
             } else {
                 a[r] = T(0); b[r] = T(1); c[r] = T(0); d[0][r] = T(0);
             }
@@ -101,7 +101,7 @@ k_ptdma_part(const T *__restrict__ A, const T *__restrict__ B, const T *__restri
 // through the stage the same way.
 template <typename T, bool CYC>
 __global__ void __launch_bounds__(PT_SX * PT_PMAX)
-k_ptdma_part_rows(const T *__restrict__ A, const T *__restrict__ B, const T *__restrict__ C, T *__restrict__ D,
+k_ptdma_part_rows(const T *__restrict__ A, const T *__restrict__ B, const T *__restrict__ C, const T *Din, T *D,
                   int n0, long ss0, long ss1, int n_row, int ls, int P, int w1, int w2) {
     extern __shared__ __align__(16) unsigned char stage_raw[];
     T *stage = reinterpret_cast<T *>(stage_raw);
@@ -128,7 +128,7 @@ k_ptdma_part_rows(const T *__restrict__ A, const T *__restrict__ B, const T *__r
             for (int l = 0; l < PT_SX; l++) stage[l * ls + stage_pos(t)] = v[l];
         }
         if (q < 3) {
-            const T *g = q == 0 ? B : (q == 1 ? C : D);
+            const T *g = q == 0 ? B : (q == 1 ? C : Din);
 #pragma unroll
             for (int l = 0; l < PT_SX; l++) v[l] = (l < nl && row_ok) ? g[gbase + l * ss0 + t] : T(0);
         }
@@ -175,7 +175,7 @@ template <> struct PartLabels<float> {
 // Partitioned solve of n0 x n1 lines (see the kernels for the layouts).
 // Returns TCS_E_ARG when the line length is outside the partitioned range.
 template <typename T>
-static int part_launch(T *A, const T *B, T *C, T *D, int n0, long ss0, int n1, long ss1, int n_row, long rs,
+static int part_launch(const T *A, const T *B, const T *C, const T *Din, T *D, int n0, long ss0, int n1, long ss1, int n_row, long rs,
                        bool cyclic, hipStream_t st, const LineOut &out) {
     int P, w1, w2;
     if (n0 <= 0 || n1 <= 0) return TCS_OK;
@@ -202,10 +202,10 @@ static int part_launch(T *A, const T *B, T *C, T *D, int n0, long ss0, int n1, l
         }
         dim3 blk(PT_SX * P), grd((unsigned)((n0 + PT_SX - 1) / PT_SX), (unsigned)n1);
         if (cyclic)
-            TCS_LAUNCH(st, L::rows_cyc, (k_ptdma_part_rows<T, true>), grd, blk, lds, A, B, C, D, n0, ss0, ss1, n_row,
+            TCS_LAUNCH(st, L::rows_cyc, (k_ptdma_part_rows<T, true>), grd, blk, lds, A, B, C, Din, D, n0, ss0, ss1, n_row,
                        ls, P, w1, w2);
         else
-            TCS_LAUNCH(st, L::rows, (k_ptdma_part_rows<T, false>), grd, blk, lds, A, B, C, D, n0, ss0, ss1, n_row, ls,
+            TCS_LAUNCH(st, L::rows, (k_ptdma_part_rows<T, false>), grd, blk, lds, A, B, C, Din, D, n0, ss0, ss1, n_row, ls,
                        P, w1, w2);
         return TCS_OK;
     }
@@ -215,22 +215,27 @@ static int part_launch(T *A, const T *B, T *C, T *D, int n0, long ss0, int n1, l
     }
     dim3 blk(PT_SX * P), grd((unsigned)((n0 + PT_SX - 1) / PT_SX), (unsigned)n1);
     if (cyclic)
-        TCS_LAUNCH(st, L::cyc, (k_ptdma_part<T, true, PT_SX>), grd, blk, 0, A, B, C, D, n0, ss1, rs, P, w1, w2,
+        TCS_LAUNCH(st, L::cyc, (k_ptdma_part<T, true, PT_SX>), grd, blk, 0, A, B, C, Din, D, n0, ss1, rs, P, w1, w2,
                    out);
     else
-        TCS_LAUNCH(st, L::plain, (k_ptdma_part<T, false, PT_SX>), grd, blk, 0, A, B, C, D, n0, ss1, rs, P, w1, w2,
+        TCS_LAUNCH(st, L::plain, (k_ptdma_part<T, false, PT_SX>), grd, blk, 0, A, B, C, Din, D, n0, ss1, rs, P, w1, w2,
                    out);
     return TCS_OK;
 }
 
 int ptdma_part_launch(double *A, const double *B, double *C, double *D, int n0, long ss0, int n1, long ss1,
                       int n_row, long rs, bool cyclic, hipStream_t st, const LineOut &out) {
-    return part_launch<double>(A, B, C, D, n0, ss0, n1, ss1, n_row, rs, cyclic, st, out);
+    return part_launch<double>(A, B, C, D, D, n0, ss0, n1, ss1, n_row, rs, cyclic, st, out);
+}
+
+int ptdma_part_launch(const double *A, const double *B, const double *C, const double *Din, double *Dout, int n0,
+                      long ss0, int n1, long ss1, int n_row, long rs, bool cyclic, hipStream_t st) {
+    return part_launch<double>(A, B, C, Din, Dout, n0, ss0, n1, ss1, n_row, rs, cyclic, st, LineOut());
 }
 
 int ptdma_part_launch(float *A, const float *B, float *C, float *D, int n0, long ss0, int n1, long ss1,
                       int n_row, long rs, bool cyclic, hipStream_t st, const LineOut &out) {
-    return part_launch<float>(A, B, C, D, n0, ss0, n1, ss1, n_row, rs, cyclic, st, out);
+    return part_launch<float>(A, B, C, D, D, n0, ss0, n1, ss1, n_row, rs, cyclic, st, out);
 }
 
 }  // namespace tcs
