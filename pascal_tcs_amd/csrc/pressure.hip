@@ -225,28 +225,43 @@ struct RhsCell {
     }
 };
 
+// The shape of the x transforms of N points: TX k-lines a workgroup (at most
+// 4: more leave too few workgroups per CU) and as many threads as the radix-8
+// groups of a pass.  With the length a constant
+// the passes' positions and twiddle steps are too, and all threads have work:
+// 256 threads over a runtime length took 21 ps a cell forward (right-hand side
+// included) at 256 and 1024 points and 12 at the 512 they fit, now 13.9, 12.7
+// and 11.6; backward 8 and 6, now 6 to 7.  N = 0: the
+// other lengths (4 to 32 points, 4096), read from the grid.
+template <int N>
+struct XFft {
+    static constexpr int TX = N <= 1024 ? 4 : 2;
+    static constexpr int NT = N == 0 || N == 512 ? 256 : N > 512 ? 512 : N == 256 ? 128 : 64;
+    static int tile(int n1m) { return N ? TX : n1m > 1024 ? 1 : 4; }
+};
+
 // x r2c: TX k-lines (k0..k0+TX-1) of row j per workgroup.
 // spec[(k + n3m*(kx + h1p*(j-1)))] complex, k 0-based.
-template <int NT, int MB, class Src>
-__global__ void __launch_bounds__(NT)
-k_fft_x_fwd(Grid g, int h1p, int TX, Src src, const double2 *__restrict__ tw, double2 *__restrict__ spec) {
+template <int N, class Src>
+__global__ void __launch_bounds__(XFft<N>::NT)
+k_fft_x_fwd(Grid g, int h1p, int tx, Src src, const double2 *__restrict__ tw, double2 *__restrict__ spec) {
     extern __shared__ double lds[];
-    const int n = g.n1m;
+    constexpr int NT = XFft<N>::NT, MB = N ? FFT_MAXB_FWD : FFT_MAXB;
+    const int n = N ? N : g.n1m, TX = N ? XFft<N>::TX : tx;
     double *re = lds, *im = lds + fft_lds_len(TX * n);
     int kb, jb;
     xcd_tiles(kb, jb);  // neighbouring rows j on one XCD: the right-hand side's stencil
     const int j = jb + 1;
     const int k0 = kb * TX;  // 0-based
     const int tid = threadIdx.x;
-    if (TX == 4 && n == 2 * NT) {
-        // the 512-point shape: a thread's two x positions one after the
-        // other, each over the four k-lines, so the k-lines share their
-        // loads (both positions at once hold more registers: 145 against
-        // 121, 2.42 against 1.85 ms with the transform's 4 butterflies)
+    // a thread's x positions one after the other, each over all the k-lines,
+    // so the k-lines share their loads and terms (two positions at once at 512
+    // points hold more registers: 145 against 121, 2.42 against 1.85 ms)
+    if constexpr (N >= 128) {
 #pragma unroll 1
-        for (int h = 0; h < 2; h++) {
+        for (int h = 0; h < N / NT; h++) {
 #pragma unroll
-            for (int l = 0; l < 4; l++) {
+            for (int l = 0; l < XFft<N>::TX; l++) {
                 const int t = tid + h * NT;
                 re[fpad(l * n + t)] = src(t + 1, j, k0 + l + 1);
                 im[fpad(l * n + t)] = 0.0;
@@ -268,21 +283,32 @@ k_fft_x_fwd(Grid g, int h1p, int TX, Src src, const double2 *__restrict__ tw, do
     }
 }
 
-// z c2c in place along the contiguous axis: one (kx, j) line per workgroup
-template <int SIGN, int NT>
+// z c2c in place along the contiguous axis: NL (kx, j) lines per workgroup.
+// One wavefront where a pass has no more radix-8 groups than 64: then 512 / N
+// lines of N points, so that every lane has a group (one line of 128 points
+// left three quarters idle: 36 -> 24 us at 256x193x128).  N = 0: the other lengths, one line of
+// length n3m.
+template <int N>
+struct ZFft {
+    static constexpr int NL = N == 0 || N >= 512 ? 1 : 512 / N;
+};
+template <int SIGN, int NT, int N>
 __global__ void __launch_bounds__(NT)
 k_fft_z(int n3m, int h1p, const double2 *__restrict__ tw, double2 *__restrict__ spec) {
     extern __shared__ double lds[];
-    double *re = lds, *im = lds + fft_lds_len(n3m);
-    const size_t base = (size_t)n3m * ((size_t)blockIdx.x + (size_t)h1p * blockIdx.y);
+    constexpr int NL = ZFft<N>::NL;
+    const int n = N ? N : n3m;
+    double *re = lds, *im = lds + fft_lds_len(NL * n);
+    const size_t base = (size_t)n * ((size_t)blockIdx.x * NL + (size_t)h1p * blockIdx.y);
+    const int count = min(NL, h1p - (int)blockIdx.x * NL) * n;  // values present
     const int tid = threadIdx.x;
-    for (int t = tid; t < n3m; t += NT) {
-        const double2 v = spec[base + t];
+    for (int t = tid; t < NL * n; t += NT) {
+        const double2 v = t < count ? spec[base + t] : make_double2(0.0, 0.0);
         re[fpad(t)] = v.x; im[fpad(t)] = v.y;
     }
     __syncthreads();
-    lds_fft<SIGN, NT>(re, im, n3m, 1, tw);
-    for (int t = tid; t < n3m; t += NT) spec[base + t] = make_double2(re[fpad(t)], im[fpad(t)]);
+    lds_fft<SIGN, NT>(re, im, n, NL, tw);
+    for (int t = tid; t < count; t += NT) spec[base + t] = make_double2(re[fpad(t)], im[fpad(t)]);
 }
 
 // y tridiagonal solves per (kx,kz), PaScaL single-rank order (:599-652).
@@ -407,12 +433,13 @@ constexpr bool SPECTRAL_MEAN = false;
 // x c2r of TX k-lines of row j, scaling by 1/n1m/n3m into dP's interior,
 // and the per-line pairwise sums for the mean (SUB: the mean scal[0] is
 // known and subtracted instead).
-template <int NT, bool SUB>
-__global__ void __launch_bounds__(NT)
-k_fft_x_inv(Grid g, int h1p, int TX, const double2 *__restrict__ spec, const double2 *__restrict__ tw,
+template <int N, bool SUB>
+__global__ void __launch_bounds__(XFft<N>::NT)
+k_fft_x_inv(Grid g, int h1p, int tx, const double2 *__restrict__ spec, const double2 *__restrict__ tw,
             double *__restrict__ dP, double *__restrict__ linesum, const double *__restrict__ scal) {
     extern __shared__ double lds[];
-    const int n = g.n1m;
+    constexpr int NT = XFft<N>::NT;
+    const int n = N ? N : g.n1m, TX = N ? XFft<N>::TX : tx;
     double *re = lds, *im = lds + fft_lds_len(TX * n);
     const int j = blockIdx.y + 1;
     const int k0 = blockIdx.x * TX;
@@ -734,31 +761,41 @@ __global__ void __launch_bounds__(256) k_dphat_update(DPhatUpdate cell, double *
 }
 
 // ---------------------------------------------------------------- host -----
-// x FFTs: 256 threads (the strided gather of the k-lines wants them all)
-// over TX k-lines of n1m points per workgroup, at most 4 (more leaves too
-// few workgroups per CU), within one pass's butterflies and 64 KiB of LDS
-constexpr int FFT_X_THREADS = 256;
-static int fft_tile(int n1m, int n3m, int mb) {
-    int tx = 1;
-    while (tx < 4 && tx * 2 <= n3m && (tx * 2) * (n1m / 2) <= mb * FFT_X_THREADS &&
-           (size_t)fft_lds_len(tx * 2 * n1m) * 16 <= 65536)
-        tx *= 2;
-    return tx;
+// An x transform's workgroups may need more than 64 KiB of LDS (1024 and 2048
+// points; gfx950: 160 KiB per CU): the kernel's limit raised
+template <class K>
+static int lds_limit(K kernel, size_t bytes) {
+    if (bytes > 65536)
+        TCS_HIP(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+    return TCS_OK;
+}
+
+// f(length): the length as a constant where the transforms have it
+template <class F>
+static int with_length(int n, F f) {
+    switch (n) {
+    case 64: return f(std::integral_constant<int, 64>());
+    case 128: return f(std::integral_constant<int, 128>());
+    case 256: return f(std::integral_constant<int, 256>());
+    case 512: return f(std::integral_constant<int, 512>());
+    case 1024: return f(std::integral_constant<int, 1024>());
+    case 2048: return f(std::integral_constant<int, 2048>());
+    default: return f(std::integral_constant<int, 0>());
+    }
 }
 
 // r2c along x of the interior-layout values src(i, j, k) into the spectrum
 template <class Src>
 static int fft_x_fwd_src_launch(tcs_ctx *c, const char *label, const Src &src, double2 *spec) {
-    const int TX = fft_tile(c->n1m, c->n3m, FFT_MAXB_FWD);
-    const size_t lds = (size_t)fft_lds_len(TX * c->n1m) * 2 * sizeof(double);
-    const dim3 grd(c->n3m / TX, c->n2m), blk(FFT_X_THREADS);
-    if (c->n1m > 2 * FFT_MAXB_FWD * FFT_X_THREADS)  // 4096 points: twice the butterflies a thread
-        TCS_LAUNCH(c->stream, label, (k_fft_x_fwd<FFT_X_THREADS, FFT_MAXB, Src>), grd, blk, lds, c->grid(), c->h1p, TX,
-                   src, (const double2 *)c->tw1, spec);
-    else
-        TCS_LAUNCH(c->stream, label, (k_fft_x_fwd<FFT_X_THREADS, FFT_MAXB_FWD, Src>), grd, blk, lds, c->grid(), c->h1p,
-                   TX, src, (const double2 *)c->tw1, spec);
-    return TCS_OK;
+    return with_length(c->n1m, [&](auto len) {
+        constexpr int N = decltype(len)::value;
+        const int TX = XFft<N>::tile(c->n1m);
+        const size_t lds = (size_t)fft_lds_len(TX * c->n1m) * 2 * sizeof(double);
+        TCS_TRY(lds_limit(k_fft_x_fwd<N, Src>, lds));
+        TCS_LAUNCH(c->stream, label, (k_fft_x_fwd<N, Src>), dim3(c->n3m / TX, c->n2m), dim3(XFft<N>::NT), lds, c->grid(),
+                   c->h1p, TX, src, (const double2 *)c->tw1, spec);
+        return TCS_OK;
+    });
 }
 static int fft_x_fwd_launch(tcs_ctx *c, const char *label, const double *in, double2 *spec) {
     return fft_x_fwd_src_launch(c, label, RhsArray{c->grid(), in}, spec);
@@ -767,39 +804,31 @@ static int fft_x_fwd_launch(tcs_ctx *c, const char *label, const double *in, dou
 // c2r along x into the full-layout field `out`, with the per-line sums
 // (sub: subtracting the mean c->scal[0] instead)
 static int fft_x_inv_launch(tcs_ctx *c, const char *label, const double2 *spec, double *out, bool sub = false) {
-    const int TX = fft_tile(c->n1m, c->n3m, FFT_MAXB);
-    const size_t lds = (size_t)fft_lds_len(TX * c->n1m) * 2 * sizeof(double);
-    if (sub)
-        TCS_LAUNCH(c->stream, label, (k_fft_x_inv<FFT_X_THREADS, true>), dim3(c->n3m / TX, c->n2m),
-                   dim3(FFT_X_THREADS), lds, c->grid(), c->h1p, TX, spec, (const double2 *)c->tw1, out, c->linesum,
+    return with_length(c->n1m, [&](auto len) {
+        constexpr int N = decltype(len)::value;
+        const int TX = XFft<N>::tile(c->n1m);
+        const size_t lds = (size_t)fft_lds_len(TX * c->n1m) * 2 * sizeof(double);
+        const auto kernel = sub ? k_fft_x_inv<N, true> : k_fft_x_inv<N, false>;
+        TCS_TRY(lds_limit(kernel, lds));
+        TCS_LAUNCH(c->stream, label, kernel, dim3(c->n3m / TX, c->n2m),
+                   dim3(XFft<N>::NT), lds, c->grid(), c->h1p, TX, spec, (const double2 *)c->tw1, out, c->linesum,
                    c->scal);
-    else
-        TCS_LAUNCH(c->stream, label, (k_fft_x_inv<FFT_X_THREADS, false>), dim3(c->n3m / TX, c->n2m),
-                   dim3(FFT_X_THREADS), lds, c->grid(), c->h1p, TX, spec, (const double2 *)c->tw1, out, c->linesum,
-                   c->scal);
-    return TCS_OK;
+        return TCS_OK;
+    });
 }
 
-// z FFTs: the fewest threads (64, 128 or 256) that hold a pass's
-// butterflies at FFT_MAXB per thread (one wave for 512 points: small
-// workgroups, more of them per CU)
-static int fft_threads(int butterflies) {
-    int nt = 64;
-    while (nt < 256 && FFT_MAXB * nt < butterflies) nt <<= 1;
-    return nt;
-}
-
-// c2c along z in place, one (kx, j) line per workgroup
+// c2c along z in place
 template <int SIGN>
 static int fft_z_launch(tcs_ctx *c, const char *label, double2 *spec) {
-    const int NT = fft_threads(c->n3m / 2);
-    const size_t lds = (size_t)fft_lds_len(c->n3m) * 2 * sizeof(double);
-    const dim3 grd(c->h1p, c->n2m);
-    const double2 *tw = (const double2 *)c->tw3;
-    if (NT == 64) TCS_LAUNCH(c->stream, label, (k_fft_z<SIGN, 64>), grd, dim3(64), lds, c->n3m, c->h1p, tw, spec);
-    else if (NT == 128) TCS_LAUNCH(c->stream, label, (k_fft_z<SIGN, 128>), grd, dim3(128), lds, c->n3m, c->h1p, tw, spec);
-    else TCS_LAUNCH(c->stream, label, (k_fft_z<SIGN, 256>), grd, dim3(256), lds, c->n3m, c->h1p, tw, spec);
-    return TCS_OK;
+    return with_length(c->n3m, [&](auto len) {
+        constexpr int N = decltype(len)::value, NL = ZFft<N>::NL;
+        // the fewest threads that hold a pass's butterflies at FFT_MAXB each
+        constexpr int NT = N == 0 ? 256 : N <= 1024 ? 64 : 128;
+        const size_t lds = (size_t)fft_lds_len(NL * c->n3m) * 2 * sizeof(double);
+        TCS_LAUNCH(c->stream, label, (k_fft_z<SIGN, NT, N>), dim3((c->h1p + NL - 1) / NL, c->n2m), dim3(NT), lds,
+                   c->n3m, c->h1p, (const double2 *)c->tw3, spec);
+        return TCS_OK;
+    });
 }
 
 static PressureRHS rhs_cell(tcs_ctx *c, double dt) {

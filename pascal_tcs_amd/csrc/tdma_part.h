@@ -521,8 +521,9 @@ __host__ __device__ inline int rblock_row0(int g, int P, int w1, int w2) {
 // small workgroups (PT_XSX * P threads, one wavefront for 512 rows) with
 // their small stages share a CU, one's memory waits covered by the others'
 // work (at 512^3: 2 lines 12-30% faster than 16).  Shorter lines take as many
-// as fill a wavefront (16 four-part lines of 64 rows: 8 threads a workgroup
-// with two, 23 us at 64^3).
+// as fill a wavefront: four of 16 parts (two left half of it idle, the three
+// momentum x solves at 256x193x128 280 -> 170 us), eight of fewer (four-part
+// lines of 64 rows two at a time: 8 threads a workgroup, 23 us at 64^3).
 constexpr int PT_XSX = 2;
 
 // Contiguous lines (rows 1 apart, x sweeps) whose rows are computed:
@@ -726,6 +727,7 @@ int ptdma_part_rows_src_launch(hipStream_t st, const char *label, const Src &src
         if (q.mm == 8) return part_rows_src_launch<CYC, 8, 8, PP>(st, label, src, q, D, n0, ss0, n1, ss1, n_row);
         if (q.mm == 4) return part_rows_src_launch<CYC, 8, 4, PP>(st, label, src, q, D, n0, ss0, n1, ss1, n_row);
     }
+    if (q.P == PP / 2) return part_rows_src_launch<CYC, 2 * X, M, PP>(st, label, src, q, D, n0, ss0, n1, ss1, n_row);
     if (q.P < PP / 2) return part_rows_src_launch<CYC, 8, M, PP>(st, label, src, q, D, n0, ss0, n1, ss1, n_row);
     return part_rows_src_launch<CYC, X, M, PP>(st, label, src, q, D, n0, ss0, n1, ss1, n_row);
 }
