@@ -423,12 +423,14 @@ __device__ __forceinline__ void src_row(const Src &src, int s0, int s1, int row,
 
 // One workgroup's lines: rows in wall-term mode WM, each entering the
 // forward elimination as it is made, then the reduced system and the
-// solution.  FULL (every part holds PT_MMAX rows): one unconditional run of
+// solution.  ROWS_FULL (every part holds MM rows): one unconditional run of
 // rows for the active lines, so consecutive rows make the loads and terms
-// they share once; otherwise guarded by r < m.  (The row loop in a function
+// they share once; ROWS_MOST (MM - 1 rows or MM): the same with the last row
+// guarded; ROWS_GUARD: every row guarded by r < m.  (The row loop in a function
 // of its own, taking the part arrays by reference, put them in scratch
 // memory.)
-template <int WM, typename T, bool CYC, class Src, int SX, bool FULL, int MM, int PM>
+enum { ROWS_GUARD, ROWS_FULL, ROWS_MOST };
+template <int WM, typename T, bool CYC, class Src, int SX, int ROWS, int MM, int PM>
 __device__ __forceinline__ void part_src_lines(const Src &src, part::RedLDS<T, SX, 1, PM> &red, T *D, int n0, long ss1, long rs,
                                                int P, int w1, int w2, const LineOut &out, int line, int p, int s0,
                                                int s1) {
@@ -437,14 +439,23 @@ __device__ __forceinline__ void part_src_lines(const Src &src, part::RedLDS<T, S
     int j0, m;
     range(p, w1, w2, j0, m);
     T a[MM], c[MM], d[1][MM];
-    if (FULL && act) {
+    if (ROWS != ROWS_GUARD && act) {
+        constexpr int MU = ROWS == ROWS_FULL ? MM : MM - 1;  // unconditional rows
 #pragma unroll
-        for (int r = 0; r < MM; r++) {
+        for (int r = 0; r < MU; r++) {
             T ar, br, cr, dr[1];
             src_row<WM>(src, s0, s1, j0 + r, ar, br, cr, dr[0]);
             reduce_row<T, 1, MM>(r, ar, br, cr, dr, a, c, d);
         }
-    } else if (FULL && sizeof(T) == sizeof(float)) {
+        if (MU < MM) {
+            a[MM - 1] = T(0); c[MM - 1] = T(0); d[0][MM - 1] = T(0);
+            if (m == MM) {
+                T ar, br, cr, dr[1];
+                src_row<WM>(src, s0, s1, j0 + MM - 1, ar, br, cr, dr[0]);
+                reduce_row<T, 1, MM>(MM - 1, ar, br, cr, dr, a, c, d);
+            }
+        }
+    } else if (ROWS == ROWS_MOST || (ROWS == ROWS_FULL && sizeof(T) == sizeof(float))) {
         // padding lines of FP32 solves: zero rows (the guarded loop below
         // puts the FP32 arrays on the stack in this instantiation; the FP64
         // ones keep it, dU y 1.02 against 1.14 ms with the zero rows)
@@ -478,7 +489,7 @@ __device__ __forceinline__ void part_src_lines(const Src &src, part::RedLDS<T, S
 // those of the split solve of stored lines.  Sources with wall terms
 // (SrcWalls) make the rows of a workgroup whose j is away from the walls
 // without them.
-template <typename T, bool CYC, class Src, int SX, bool FULL, int MM, int PM>
+template <typename T, bool CYC, class Src, int SX, int ROWS, int MM, int PM>
 __global__ void __launch_bounds__(SX * PM) __attribute__((amdgpu_waves_per_eu(Src::waves)))
 k_ptdma_part_src(Src src, T *D, int n0, int n1, long ss1, long rs, int P, int w1, int w2, LineOut out) {
     __shared__ part::RedLDS<T, SX, 1, PM> red;
@@ -491,11 +502,11 @@ k_ptdma_part_src(Src src, T *D, int n0, int n1, long ss1, long rs, int P, int w1
     if constexpr (SrcWalls<Src>::value) {
         // s1 is the workgroup's: one branch for the whole workgroup
         if (src.wall_free(s1))
-            part_src_lines<2, T, CYC, Src, SX, FULL, MM, PM>(src, red, D, n0, ss1, rs, P, w1, w2, out, line, p, s0, s1);
+            part_src_lines<2, T, CYC, Src, SX, ROWS, MM, PM>(src, red, D, n0, ss1, rs, P, w1, w2, out, line, p, s0, s1);
         else
-            part_src_lines<0, T, CYC, Src, SX, FULL, MM, PM>(src, red, D, n0, ss1, rs, P, w1, w2, out, line, p, s0, s1);
+            part_src_lines<0, T, CYC, Src, SX, ROWS, MM, PM>(src, red, D, n0, ss1, rs, P, w1, w2, out, line, p, s0, s1);
     } else {
-        part_src_lines<-1, T, CYC, Src, SX, FULL, MM, PM>(src, red, D, n0, ss1, rs, P, w1, w2, out, line, p, s0, s1);
+        part_src_lines<-1, T, CYC, Src, SX, ROWS, MM, PM>(src, red, D, n0, ss1, rs, P, w1, w2, out, line, p, s0, s1);
     }
 }
 
@@ -641,7 +652,7 @@ k_ptdma_part_rows_src(Src src, T *D, int n0, long ss0, long ss1, int n_row, int 
 // segments, but two workgroups per CU; fewer where a line has more than
 // PT_PMAX parts); ANY: the plan is part_plan_any's, else ptdma_part_plan's.
 // Returns TCS_E_ARG outside the split range.
-template <bool CYC, int SX, int MM, int PM, typename T, class Src>
+template <bool CYC, int SX, bool MOST, int MM, int PM, typename T, class Src>
 int part_src_launch(hipStream_t st, const char *label, const Src &src, const PartPlan &q, T *D, int n0, int n1,
                     long ss1, long rs, const LineOut &out) {
     // the outer line count padded to whole XCD tiles (the padding
@@ -657,15 +668,30 @@ int part_src_launch(hipStream_t st, const char *label, const Src &src, const Par
     // thermal y 2.63 -> 2.00 ms, dU y 1.52 -> 1.02 ms, dW y 1.43 -> 1.29 ms
     // at 512^3; the dU z stage, 4.14 -> 3.14 ms); FP32 lines (the mixed
     // form) where the row asks for it as well (Src::full_rows32)
-    if constexpr (Src::full_rows && (sizeof(T) == 8 || Src::full_rows32))
-        if (q.w1 == MM && q.w2 == 0) {
-            TCS_LAUNCH(st, label, (k_ptdma_part_src<T, CYC, Src, SX, true, MM, PM>), grd, blk, 0, src, D, n0, n1, ss1,
-                       rs, q.P, q.w1, q.w2, out);
-            return TCS_OK;
+    auto launch = [&](auto kernel) {
+        TCS_LAUNCH(st, label, kernel, grd, blk, 0, src, D, n0, n1, ss1, rs, q.P, q.w1, q.w2, out);
+        return TCS_OK;
+    };
+    if constexpr (Src::full_rows && (sizeof(T) == 8 || Src::full_rows32)) {
+        if (q.w1 == MM && q.w2 == 0) return launch(k_ptdma_part_src<T, CYC, Src, SX, ROWS_FULL, MM, PM>);
+        // Lines of any length along y: a kernel for each part size from 8
+        // rows (two parts or more hold 8 to 16), the same rows in the same
+        // order (at 256x193x128: T 147 -> 114 us, dU 89 -> 67, dV 74 -> 57; the
+        // rows guarded one by one share no loads or terms)
+        if constexpr (MOST && MM == PT_MMAX) {
+            switch (q.w1) {
+            case 8: return launch(k_ptdma_part_src<T, CYC, Src, SX, ROWS_MOST, 9, PM>);
+            case 9: return launch(k_ptdma_part_src<T, CYC, Src, SX, ROWS_MOST, 10, PM>);
+            case 10: return launch(k_ptdma_part_src<T, CYC, Src, SX, ROWS_MOST, 11, PM>);
+            case 11: return launch(k_ptdma_part_src<T, CYC, Src, SX, ROWS_MOST, 12, PM>);
+            case 12: return launch(k_ptdma_part_src<T, CYC, Src, SX, ROWS_MOST, 13, PM>);
+            case 13: return launch(k_ptdma_part_src<T, CYC, Src, SX, ROWS_MOST, 14, PM>);
+            case 14: return launch(k_ptdma_part_src<T, CYC, Src, SX, ROWS_MOST, 15, PM>);
+            case 15: return launch(k_ptdma_part_src<T, CYC, Src, SX, ROWS_MOST, 16, PM>);
+            }
         }
-    TCS_LAUNCH(st, label, (k_ptdma_part_src<T, CYC, Src, SX, false, MM, PM>), grd, blk, 0, src, D, n0, n1, ss1, rs,
-               q.P, q.w1, q.w2, out);
-    return TCS_OK;
+    }
+    return launch(k_ptdma_part_src<T, CYC, Src, SX, ROWS_GUARD, MM, PM>);
 }
 template <bool CYC, int SX, bool ANY, typename T, class Src>
 int ptdma_part_src_launch(hipStream_t st, const char *label, const Src &src, T *D, int n0, int n1, long ss1,
@@ -679,13 +705,13 @@ int ptdma_part_src_launch(hipStream_t st, const char *label, const Src &src, T *
     if constexpr (ANY) {
         constexpr int M = PT_MMAX, PP = PT_PMAX;
         if constexpr (sizeof(T) == 8)
-            if (q.pm == 2 * PP) return part_src_launch<CYC, 8, M, 2 * PP>(st, label, src, q, D, n0, n1, ss1, rs, out);
+            if (q.pm == 2 * PP) return part_src_launch<CYC, 8, false, M, 2 * PP>(st, label, src, q, D, n0, n1, ss1, rs, out);
         if constexpr (sizeof(T) == 8)
-            if (q.pm == 4 * PP) return part_src_launch<CYC, 4, M, 4 * PP>(st, label, src, q, D, n0, n1, ss1, rs, out);
-        if (q.mm == 8) return part_src_launch<CYC, 16, 8, PP>(st, label, src, q, D, n0, n1, ss1, rs, out);
-        if (q.mm == 4) return part_src_launch<CYC, 16, 4, PP>(st, label, src, q, D, n0, n1, ss1, rs, out);
+            if (q.pm == 4 * PP) return part_src_launch<CYC, 4, false, M, 4 * PP>(st, label, src, q, D, n0, n1, ss1, rs, out);
+        if (q.mm == 8) return part_src_launch<CYC, 16, false, 8, PP>(st, label, src, q, D, n0, n1, ss1, rs, out);
+        if (q.mm == 4) return part_src_launch<CYC, 16, false, 4, PP>(st, label, src, q, D, n0, n1, ss1, rs, out);
     }
-    return part_src_launch<CYC, SX, PT_MMAX, PT_PMAX>(st, label, src, q, D, n0, n1, ss1, rs, out);
+    return part_src_launch<CYC, SX, ANY && !CYC, PT_MMAX, PT_PMAX>(st, label, src, q, D, n0, n1, ss1, rs, out);
 }
 
 // Launch of k_ptdma_part_rows_src over n0 x n1 contiguous lines of n_row rows.
