@@ -308,13 +308,7 @@ inline dim3 cell_grid(int nx, int ny, int nz, int kb, dim3 blk = interior_block(
     return dim3((unsigned)((nx / ib + blk.x - 1) / blk.x), (unsigned)((ny + blk.y - 1) / blk.y), (unsigned)(nz / kb));
 }
 
-// TDMA launcher (exact PaScaL order) on strided systems:
-//   system (s0, s1) starts at base + s0*ss0 + s1*ss1, rows step rs.
-// Right-hand sides from Din, solutions to Dout (which may be Din); A and C
-// are overwritten, with keep by the reference's modified coefficients.
-int ptdma_exact_launch(double *A, const double *B, double *C, const double *Din, double *Dout, int n0, long ss0,
-                       int n1, long ss1, int n_row, long rs, bool cyclic, bool keep, hipStream_t st);
-// Where a split solve puts its solution: back into D (mode 0), or into an
+// Where a solve puts its solution: back into D (mode 0), or into an
 // FP64 field F at F[base + s0*ss0 + s1*ss1 + row*rs], stored (mode 1),
 // added to what F holds (mode 2), or added to what Fin holds at the same
 // place (mode 3: F a second buffer of the field), or stored into the FP32
@@ -334,6 +328,31 @@ struct LineOut {
         if (c->wrap) { gx = c->n1m; gz = c->n3m; n_row = nr; }
     }
 };
+namespace part {
+// F[o] = v and its images on the periodic ghost lines di in s0 and dk in s1
+// away (0: none), stored with the value still in registers: read back from the
+// line's own stores afterwards, the images took 50 us of a 110 us solve at
+// 256^3, in the few workgroups that have them.
+template <typename E>
+__device__ __forceinline__ void put_line(E *F, long o, E v, long di, long dk) {
+    F[o] = v;
+    if (di) F[o + di] = v;
+    if (dk) {
+        F[o + dk] = v;
+        if (di) F[o + dk + di] = v;
+    }
+}
+}  // namespace part
+
+// TDMA launcher (exact PaScaL order) on strided systems:
+//   system (s0, s1) starts at base + s0*ss0 + s1*ss1, rows step rs.
+// Right-hand sides from Din, solutions to Dout (which may be Din); A and C
+// are overwritten, with keep by the reference's modified coefficients.  out
+// (mode 1, non-cyclic strided systems): the solutions into a field instead,
+// Dout overwritten.
+int ptdma_exact_launch(double *A, const double *B, double *C, const double *Din, double *Dout, int n0, long ss0,
+                       int n1, long ss1, int n_row, long rs, bool cyclic, bool keep, hipStream_t st,
+                       const LineOut &out = LineOut());
 // The same systems split into parts (PaScaL_TDMA's multi-rank algorithm,
 // one thread per rank); n_row in [2, 512]; strided lines need ss0 = 1.
 bool ptdma_part_plan(int n_row, int &P, int &w1, int &w2);

@@ -17,11 +17,14 @@ using namespace exact_line;
 // Lines strided in memory: line l = s0 + n0*s1 starts at s0*ss0 + s1*ss1,
 // rows rs apart.  A, C and Dout also hold the eliminated rows j < jl (the
 // rows j >= jl are kept in LDS); KEEP: A and C come back as the reference
-// leaves them.
-template <bool CYC, bool KEEP>
+// leaves them.  FIELD: the solution goes into the field of out (stored) and
+// not into Dout, with its ghosts and wall rows where out asks for them (the
+// momentum y stages of the single-rank order; by a kernel of its own the
+// stores took 50 us a stage at 256x200x256).
+template <bool CYC, bool KEEP, bool FIELD = false>
 __global__ void __launch_bounds__(EX_W)
 k_ptdma_exact(double *A, const double *B, double *C, const double *Din, double *Dout, int n0, long ss0, long ss1,
-              long lines, int n_row, long rs, int jl) {
+              long lines, int n_row, long rs, int jl, LineOut out) {
     extern __shared__ double lds[];
     const Kept<1> keep{lds, (int)threadIdx.x};
     const long line = (long)blockIdx.x * EX_W + threadIdx.x;
@@ -29,6 +32,12 @@ k_ptdma_exact(double *A, const double *B, double *C, const double *Din, double *
     const long s1 = line / n0, base = (line - s1 * n0) * ss0 + s1 * ss1;
     double *a = A + base, *c = C + base, *d = Dout + base;
     const double *b = B + base, *din = Din + base;
+    const long s0 = line - s1 * n0, fb = out.base + s0 * out.ss0 + s1 * out.ss1;
+    long di = 0, dk = 0;
+    if (FIELD && out.gx > 0) {
+        di = s0 == 0 ? out.gx * out.ss0 : s0 == out.gx - 1 ? -out.gx * out.ss0 : 0;
+        dk = s1 == 0 ? out.gz * out.ss1 : s1 == out.gz - 1 ? -out.gz * out.ss1 : 0;
+    }
     solve<CYC, 1>(
         n_row,
         [&](int j) {
@@ -50,9 +59,15 @@ k_ptdma_exact(double *A, const double *B, double *C, const double *Din, double *
         },
         [&](int j, const Elim<1> &e, const double (&x)[1]) {
             const long o = (long)j * rs;
-            d[o] = x[0];
+            if constexpr (FIELD) part::put_line<double>(out.F, fb + (long)j * out.rs, x[0], di, dk);
+            else d[o] = x[0];
             if constexpr (KEEP) { a[o] = e.a; c[o] = e.c; }
         });
+    if (FIELD && out.gx > 0) {
+        const long lo = fb - out.rs, hi = fb + (long)n_row * out.rs;
+        part::put_line<double>(out.F, lo, out.F[lo], di, dk);
+        part::put_line<double>(out.F, hi, out.F[hi], di, dk);
+    }
 }
 
 // Systems whose rows are contiguous in memory (the x sweep of an (i,j,k)
@@ -191,7 +206,8 @@ k_ptdma_exact_rows(double *A, const double *B, double *C, const double *Din, dou
 }  // namespace
 
 int ptdma_exact_launch(double *A, const double *B, double *C, const double *Din, double *Dout, int n0, long ss0,
-                       int n1, long ss1, int n_row, long rs, bool cyclic, bool keep, hipStream_t st) {
+                       int n1, long ss1, int n_row, long rs, bool cyclic, bool keep, hipStream_t st,
+                       const LineOut &out) {
     if (n0 <= 0 || n1 <= 0) return TCS_OK;
     if (n_row < 2 || n1 > 65535) {
         set_error("ptdma: n_row must be >= 2 and the outer system count <= 65535");
@@ -199,6 +215,11 @@ int ptdma_exact_launch(double *A, const double *B, double *C, const double *Din,
     }
 #define EXACT_PICK(kern) \
     (cyclic ? (keep ? kern<true, true> : kern<true, false>) : (keep ? kern<false, true> : kern<false, false>))
+    const bool field = out.mode == 1;
+    if (out.mode != 0 && (!field || rs == 1 || cyclic || keep)) {
+        set_error("ptdma: field output is stored from non-cyclic strided lines only");
+        return TCS_E_ARG;
+    }
     if (rs == 1) {
         const dim3 grd((unsigned)((n0 + EX_W - 1) / EX_W), (unsigned)n1);
         TCS_LAUNCH(st, cyclic ? "ptdma_rows_cyclic" : "ptdma_rows", EXACT_PICK(k_ptdma_exact_rows), grd, dim3(EX_W),
@@ -207,14 +228,15 @@ int ptdma_exact_launch(double *A, const double *B, double *C, const double *Din,
     }
     const long lines = (long)n0 * n1;
     const int kept = kept_rows<1>(lines, n_row), lds = kept * Kept<1>::ROW_BYTES;
-    const auto kern = EXACT_PICK(k_ptdma_exact);
-    static bool raised[4];  // more than 64 KiB of dynamic LDS (gfx950: 160 KiB per CU)
-    if (!raised[2 * cyclic + keep]) {
+    const auto kern = field ? k_ptdma_exact<false, false, true> : EXACT_PICK(k_ptdma_exact);
+    static bool raised[5];  // more than 64 KiB of dynamic LDS (gfx950: 160 KiB per CU)
+    bool &up = raised[field ? 4 : 2 * cyclic + keep];
+    if (!up) {
         TCS_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, KEPT_LDS));
-        raised[2 * cyclic + keep] = true;
+        up = true;
     }
     TCS_LAUNCH(st, cyclic ? "ptdma_cyclic" : "ptdma", kern, dim3((unsigned)((lines + EX_W - 1) / EX_W)), dim3(EX_W),
-               lds, A, B, C, Din, Dout, n0, ss0, ss1, lines, n_row, rs, n_row - kept);
+               lds, A, B, C, Din, Dout, n0, ss0, ss1, lines, n_row, rs, n_row - kept, out);
 #undef EXACT_PICK
     return TCS_OK;
 }

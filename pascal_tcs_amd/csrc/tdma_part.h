@@ -304,20 +304,6 @@ __device__ __forceinline__ void exchange(RedLDS<T, SX, NR, PM> &red, int line, i
     }
 }
 
-// F[o] = v and its images on the periodic ghost lines di in s0 and dk in s1
-// away (0: none), stored with the value still in registers: read back from the
-// line's own stores afterwards, the images took 50 us of a 110 us solve at
-// 256^3, in the few workgroups that have them.
-template <typename E>
-__device__ __forceinline__ void put_line(E *F, long o, E v, long di, long dk) {
-    F[o] = v;
-    if (di) F[o + di] = v;
-    if (dk) {
-        F[o + dk] = v;
-        if (di) F[o + dk + di] = v;
-    }
-}
-
 // The solution of a part of line (s0, s1): into D at dbase + row*rs
 // (out.mode 0), or into the field of out (modes 1, 2, 3).
 template <typename T, int MM>

@@ -469,17 +469,14 @@ struct ThermalY {
     }
 };
 
-// T(i,j,k) += RHSJ (:518-524)
-// F(i,j,k) = inc (MODE 1) or F(i,j,k) += inc (MODE 2) over interior rows j >= j0
-template <int MODE>
-__global__ void k_interior_out(Grid g, int j0, double *F, const scr_t *__restrict__ inc) {
+// T(i,j,k) += RHSJ (:518-524): F(i,j,k) += inc over the interior
+__global__ void k_add_interior(Grid g, double *F, const scr_t *__restrict__ inc) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
     const int j = blockIdx.y * blockDim.y + threadIdx.y + 1;
     const int k = blockIdx.z + 1;
-    if (i > g.n1m || j > g.n2m || j < j0) return;
+    if (i > g.n1m || j > g.n2m) return;
     const size_t q = g.ix(i, j, k);
-    const double v = inc[g.r3(i, j, k)];
-    const double f = MODE == 1 ? v : F[q] + v;
+    const double f = F[q] + inc[g.r3(i, j, k)];
     F[q] = f;
     if (g.edge(i, 1, j, k, 1)) {
         g.images(F, i, k, q, f);
@@ -487,33 +484,40 @@ __global__ void k_interior_out(Grid g, int j0, double *F, const scr_t *__restric
     }
 }
 
+// y lines in the single-rank order, their solutions into a field
+template <typename S>
+static int exact_store(tcs_ctx *c, S *am, S *ac, S *ap, S *rhs, long n12, int nrows, long n1, const LineOut &out) {
+    if constexpr (sizeof(S) == 8) {
+        return ptdma_exact_launch(am, ac, ap, rhs, rhs, c->n1m, 1, c->n3m, n12, nrows, n1, false, false, c->stream, out);
+    } else {
+        set_error("y sweep: FP32 lines are split");
+        return TCS_E_ARG;
+    }
+}
+
 // y sweep of rows j = j0..j0+nrows-1 (1-based) whose solution ends the
 // stage: stored into (mode 1) or added to (mode 2) the field F's interior.
-// With split lines the solve writes F directly; otherwise a second kernel
-// moves the solution from the scratch.
+// The solve writes F directly, except that the single-rank order adds by a
+// second kernel (its solution comes row after row, each waiting for F).
 int sweep_y_field(tcs_ctx *c, int j0, int nrows, double *F, int mode) {
     const long n1 = c->n1m, n12 = (long)c->n1m * c->n2m;
     const long off = (long)(j0 - 1) * n1;
+    LineOut out;
+    out.F = F;
+    out.mode = mode;
+    out.base = 1 + (long)c->P1 * j0 + (long)c->P1 * c->N2;  // (i,j,k) = (1, j0, 1)
+    out.ss0 = 1;
+    out.ss1 = (long)c->P1 * c->N2;
+    out.rs = c->P1;
+    out.wrap_to(c, nrows);
+    scr_t *am = SCR(c->am) + off, *ac = SCR(c->ac) + off, *ap = SCR(c->ap) + off, *rhs = SCR(c->rhs) + off;
     int P, w1, w2;
-    if (c->tdma_split && ptdma_part_plan(nrows, P, w1, w2)) {
-        LineOut out;
-        out.F = F;
-        out.mode = mode;
-        out.base = 1 + (long)c->P1 * j0 + (long)c->P1 * c->N2;  // (i,j,k) = (1, j0, 1)
-        out.ss0 = 1;
-        out.ss1 = (long)c->P1 * c->N2;
-        out.rs = c->P1;
-        out.wrap_to(c, nrows);
-        return ptdma_part_launch(SCR(c->am) + off, SCR(c->ac) + off, SCR(c->ap) + off, SCR(c->rhs) + off, c->n1m, 1,
-                                 c->n3m, n12, nrows, n1, false, c->stream, out);
-    }
-    TCS_TRY(ptdma_sweep(c, SCR(c->am) + off, SCR(c->ac) + off, SCR(c->ap) + off, SCR(c->rhs) + off, c->n1m, 1,
-                        c->n3m, n12, nrows, n1, false));
-    const dim3 blk = interior_block(), grd = interior_grid(c->n1m, c->n2m, c->n3m);
-    if (mode == 1)
-        TCS_LAUNCH(c->stream, "store_interior", k_interior_out<1>, grd, blk, 0, c->grid(), j0, F, SCR(c->rhs));
-    else
-        TCS_LAUNCH(c->stream, "add_interior", k_interior_out<2>, grd, blk, 0, c->grid(), j0, F, SCR(c->rhs));
+    if (c->tdma_split && ptdma_part_plan(nrows, P, w1, w2))
+        return ptdma_part_launch(am, ac, ap, rhs, c->n1m, 1, c->n3m, n12, nrows, n1, false, c->stream, out);
+    if (mode == 1) return exact_store(c, am, ac, ap, rhs, n12, nrows, n1, out);
+    TCS_TRY(ptdma_sweep(c, am, ac, ap, rhs, c->n1m, 1, c->n3m, n12, nrows, n1, false));
+    TCS_LAUNCH(c->stream, "add_interior", k_add_interior, interior_grid(c->n1m, c->n2m, c->n3m), interior_block(), 0,
+               c->grid(), F, SCR(c->rhs));
     return TCS_OK;
 }
 
@@ -551,8 +555,8 @@ int thermal_solver(tcs_ctx *c, double dt) {
         // the y rows read T around every cell, so the increment goes through
         // the scratch and is added once every line is solved
         TCS_TRY(y_stage_in_solve<ANY_SPLIT>(c, "thermal_y_solve", y, 1, c->n2m, rhs, nullptr, 0));
-        TCS_LAUNCH(c->stream, "add_interior", k_interior_out<2>, interior_grid(c->n1m, c->n2m, c->n3m),
-                   interior_block(), 0, g, 1, T, rhs);
+        TCS_LAUNCH(c->stream, "add_interior", k_add_interior, interior_grid(c->n1m, c->n2m, c->n3m),
+                   interior_block(), 0, g, T, rhs);
         return TCS_OK;
     }
     TCS_TRY(rows3d_launch<false>(c, "thermal_y", y, 1, am, ac, ap, rhs));
