@@ -1144,7 +1144,7 @@ __global__ void __launch_bounds__(256) k_blockLdU_pseudo(BlockLdU cell, Acc acc,
 
 int momentum_blockLdV_pseudo(tcs_ctx *c, double dt, double *Vn) {
     const dim3 blk = interior_block(), grd = cell_grid(c->n1m, c->n2m, c->n3m, LDV_KB, interior_block(), LDV_IB);
-    const BlockLdV cell{c->grid(), c->phys, dt, c->f[TCS_V], c->f[TCS_DW], c->f[TCS_MU], c->f[TCS_INVRHO], c->f[TCS_DV]};
+    const BlockLdV cell{c->cell_grid(), c->phys, dt, c->f[TCS_V], c->f[TCS_DW], c->f[TCS_MU], c->f[TCS_INVRHO], c->f[TCS_DV]};
     TCS_TRY(ensure_twins(c, TWIN_V | TWIN_TAB));
     c->twin_ok &= ~(unsigned)TWIN_V;  // Vn becomes V
     if (!c->wrap) TCS_TRY(copy_shell(c, {TCS_V}));
@@ -1156,7 +1156,7 @@ int momentum_blockLdV_pseudo(tcs_ctx *c, double dt, double *Vn) {
 
 int momentum_blockLdU_pseudo(tcs_ctx *c, double dt, double *Un, double *Wn) {
     const dim3 blk = interior_block(), grd = cell_grid(c->n1m, c->n2m, c->n3m, LDU_KB, interior_block(), LDU_IB);
-    const BlockLdU cell{c->grid(), c->phys, dt, c->f[TCS_U], c->f[TCS_DV], c->f[TCS_DW],
+    const BlockLdU cell{c->cell_grid(), c->phys, dt, c->f[TCS_U], c->f[TCS_DV], c->f[TCS_DW],
                         c->f[TCS_MU], c->f[TCS_INVRHO], c->f[TCS_DU]};
     TCS_TRY(ensure_twins(c, TWIN_U | TWIN_TAB));
     c->twin_ok &= ~(unsigned)(TWIN_U | TWIN_W);  // Un, Wn become U, W

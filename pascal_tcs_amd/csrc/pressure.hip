@@ -918,7 +918,7 @@ int pressure_projection_into(tcs_ctx *c, double dt, double *dPhatn, double *dP0n
     c->twin_ok &= ~(unsigned)(TWIN_U | TWIN_V | TWIN_W | TWIN_P);  // the mixed form's FP32 copies
     const Grid g = c->grid();
     const dim3 blk = interior_block(), grd = cell_grid(c->n1m, c->n2m, c->n3m, PROJ_KB, interior_block(), PROJ_IB);
-    const Projection cell{g, c->phys, dt, c->f[TCS_INVRHO], c->f[TCS_DP], c->f[TCS_DPHAT], c->f[TCS_DP0],
+    const Projection cell{c->cell_grid(), c->phys, dt, c->f[TCS_INVRHO], c->f[TCS_DP], c->f[TCS_DPHAT], c->f[TCS_DP0],
                           c->f[TCS_U], c->f[TCS_V], c->f[TCS_W], c->f[TCS_P]};
     if (!c->wrap) TCS_TRY(copy_shell(c, {TCS_DPHAT, TCS_DP0}));
     else if (!(c->kept >> TCS_DP0 & 1)) TCS_TRY(copy_shell(c, {TCS_DP0}));

@@ -1209,7 +1209,8 @@ struct Wrap {  // tcs_ctx::wrap for a scope
 }  // namespace
 
 // Every ghost-cell update of main's order is made by the kernel that writes
-// the field (tcs_ctx::wrap).
+// the field (tcs_ctx::wrap), on large grids but for the block corrections and
+// the projection (wrap_cells).
 extern "C" int tcs_step(tcs_ctx *c, double dt) {
     CTX_CHECK(c);
     c->cfl_valid = 0;
@@ -1226,13 +1227,22 @@ extern "C" int tcs_step(tcs_ctx *c, double dt) {
     // block corrections with the pseudo-update (U + dU, V + dV, W + dW into
     // the second buffers; the corrections read the old U, V)
     RUN("momentum blockLdV", FORM(c, momentum_blockLdV_pseudo, dt, c->spare[TCS_V]));
+    const bool update = c->wrap_cells() == 2;
+    if (update) RUN("update ghostcell", halo_field(c, TCS_DV));
     RUN("momentum blockLdU", FORM(c, momentum_blockLdU_pseudo, dt, c->spare[TCS_U], c->spare[TCS_W]));
     for (int q : {TCS_U, TCS_V, TCS_W}) std::swap(c->f[q], c->spare[q]);
+    if (update) RUN("update ghostcell", halo(c, {c->f[TCS_U], c->f[TCS_V], c->f[TCS_W]}));
     // the right-hand side is made inside the solve's x transform
     RUN("pressure PoissonSolve", FORM(c, pressure_poisson_rhs, dt));
     RUN("pressure projection", FORM(c, pressure_projection_into, dt, c->spare[TCS_DPHAT], c->spare[TCS_DP0]));
     std::swap(c->f[TCS_DPHAT], c->spare[TCS_DPHAT]);
     std::swap(c->f[TCS_DP0], c->spare[TCS_DP0]);
+    if (update) {
+        RUN("update ghostcell", halo(c, {c->f[TCS_U], c->f[TCS_V], c->f[TCS_W], c->f[TCS_P], c->f[TCS_DPHAT]}));
+        if (c->a32)
+            RUN("update ghostcell", halo(c, {twin(c, c->f[TCS_U]), twin(c, c->f[TCS_V]), twin(c, c->f[TCS_W]),
+                                             twin(c, c->f[TCS_P])}));
+    }
     // the mixed form: the projection wrote the FP32 copies of U, V, W, P
     if (c->a32) c->twin_ok |= TWIN_U | TWIN_V | TWIN_W | TWIN_P;
     return TCS_OK;

@@ -92,7 +92,7 @@ struct Grid {
     int n1m, n2m, n3m;
     int N1, N2, N3;  // full extents n?m+2
     int P1;          // row pitch of the full fields
-    int wrap;        // kernels write the periodic ghosts (tcs_ctx::wrap)
+    int wrap;        // kernels write the periodic ghosts and the wall rows (1), the wall rows (2)
     const double *dx1, *dx2, *dx3, *dmx1, *dmx2, *dmx3;
     const double *rdx1, *rdx2, *rdx3, *rdmx1, *rdmx2, *rdmx3;  // their reciprocals
     // the six tables (dx1, dmx1, dx2, dmx2, dx3, dmx3) back to back rounded to
@@ -114,6 +114,7 @@ struct Grid {
     // the images cost blockLdU 0.5 of 1.8 ms at 512^3.
     template <class E>
     __device__ __forceinline__ void images(E *F, int i, int k, size_t q, E v) const {
+        if (wrap == 2) return;
         const long di = i == 1 ? n1m : i == n1m ? -n1m : 0;
         if (di) F[(long)q + di] = v;
         if (k == 1 || k == n3m) {
@@ -125,7 +126,8 @@ struct Grid {
     // (wrap) whether cells i0..i0+ib-1, j, k0..k0+kb-1 touch the edge of the
     // interior; ib and kb divide n1m and n3m
     __device__ __forceinline__ bool edge(int i0, int ib, int j, int k0, int kb) const {
-        return wrap && (i0 == 1 || i0 + ib > n1m || j == 1 || j == n2m || k0 == 1 || k0 + kb > n3m);
+        return (wrap && (j == 1 || j == n2m)) ||
+               (wrap == 1 && (i0 == 1 || i0 + ib > n1m || k0 == 1 || k0 + kb > n3m));
     }
     // F's wall row next to row j, if there is one, from src's, with its
     // images: the thread of an edge row brings over the wall row of a second
@@ -234,6 +236,13 @@ struct tcs_ctx {
     // called one by one leave the ghosts to tcs_ghostcell_update, as a caller
     // may look at them in between.
     int wrap;
+    // What the block corrections and the projection (one cell a thread, many
+    // fields) write: past 2^23 cells they leave the images to a ghost-cell
+    // update of all their fields, one store per line of memory in a kernel at
+    // its bandwidth costing more than the launch (at 512^3 the images took
+    // 0.22, 0.12 and 0.26 ms, the three launches 0.25; at 256x193x128 edges
+    // cost 3 us a kernel, a launch 6)
+    int wrap_cells() const { return wrap && nint > ((size_t)1 << 23) ? 2 : wrap; }
     // For steps in a row, cleared by every other entry that may write the
     // field or hands out its address, bits 1 << id: dP0's second buffer holds
     // the same shell as dP0; dV's rows 0, 1 and n2m+1 are zero.
@@ -243,6 +252,11 @@ struct tcs_ctx {
     size_t an, aused;
     unsigned twin_ok;
 
+    tcs::Grid cell_grid() const {
+        tcs::Grid g = grid();
+        g.wrap = wrap_cells();
+        return g;
+    }
     tcs::Grid grid() const {
         tcs::Grid g;
         g.n1m = n1m; g.n2m = n2m; g.n3m = n3m;

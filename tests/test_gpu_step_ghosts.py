@@ -22,7 +22,8 @@ def _noise(s, names, seed):
 
 
 @pytest.mark.parametrize("form,split,bound", [(0, 0, 0.0), (0, 1, 0.0), (1, 1, 3e-12), (2, 1, 6e-6)])
-@pytest.mark.parametrize("shape", [(4, 3, 4), (16, 33, 8), (128, 18, 16), (64, 40, 64)])
+@pytest.mark.parametrize("shape", [(4, 3, 4), (16, 33, 8), (128, 18, 16), (64, 40, 64),
+                                   (256, 129, 256)])  # the last past 2^23 cells
 def test_steps_against_routines(shape, form, split, bound):
     from pascal_tcs_amd.solver import TCSSolver
     cfg = small_config(*shape, DeltaT=0.2)
