@@ -762,11 +762,13 @@ __global__ void __launch_bounds__(256) k_dphat_update(DPhatUpdate cell, double *
 
 // ---------------------------------------------------------------- host -----
 // An x transform's workgroups may need more than 64 KiB of LDS (1024 and 2048
-// points; gfx950: 160 KiB per CU): the kernel's limit raised
+// points; gfx950: 160 KiB per CU): the kernel's limit raised, once (a kernel's
+// calls all ask for the same)
 template <class K>
-static int lds_limit(K kernel, size_t bytes) {
-    if (bytes > 65536)
-        TCS_HIP(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+static int lds_limit(K kernel, size_t bytes, bool &raised) {
+    if (bytes <= 65536 || raised) return TCS_OK;
+    TCS_HIP(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+    raised = true;
     return TCS_OK;
 }
 
@@ -791,7 +793,8 @@ static int fft_x_fwd_src_launch(tcs_ctx *c, const char *label, const Src &src, d
         constexpr int N = decltype(len)::value;
         const int TX = XFft<N>::tile(c->n1m);
         const size_t lds = (size_t)fft_lds_len(TX * c->n1m) * 2 * sizeof(double);
-        TCS_TRY(lds_limit(k_fft_x_fwd<N, Src>, lds));
+        static bool raised = false;
+        TCS_TRY(lds_limit(k_fft_x_fwd<N, Src>, lds, raised));
         TCS_LAUNCH(c->stream, label, (k_fft_x_fwd<N, Src>), dim3(c->n3m / TX, c->n2m), dim3(XFft<N>::NT), lds, c->grid(),
                    c->h1p, TX, src, (const double2 *)c->tw1, spec);
         return TCS_OK;
@@ -809,7 +812,8 @@ static int fft_x_inv_launch(tcs_ctx *c, const char *label, const double2 *spec, 
         const int TX = XFft<N>::tile(c->n1m);
         const size_t lds = (size_t)fft_lds_len(TX * c->n1m) * 2 * sizeof(double);
         const auto kernel = sub ? k_fft_x_inv<N, true> : k_fft_x_inv<N, false>;
-        TCS_TRY(lds_limit(kernel, lds));
+        static bool raised[2];
+        TCS_TRY(lds_limit(kernel, lds, raised[sub]));
         TCS_LAUNCH(c->stream, label, kernel, dim3(c->n3m / TX, c->n2m),
                    dim3(XFft<N>::NT), lds, c->grid(), c->h1p, TX, spec, (const double2 *)c->tw1, out, c->linesum,
                    c->scal);

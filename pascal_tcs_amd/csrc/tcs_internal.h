@@ -218,15 +218,6 @@ struct tcs_ctx {
     // (PEND_* bits; tcs::flush_pending runs them as called)
     int pend;
     double pend_dt_ldv, pend_dt_ldu, pend_dt_rhs;
-    // The mixed form (precision 2): every array its stage rows and block
-    // corrections read (T, U, V, W, P and the second buffers of T, U, V, W;
-    // dU, dV, dW; the Mu and invRho tables; the wall tables; the stale
-    // scalars) is carved from one FP64 arena a64 of an elements, and the
-    // FP32 arena a32 holds each one's twin at the same element offset.  The
-    // twins of the increments dU, dV, dW are where the mixed form keeps them
-    // (the FP64 arrays are filled from them on download); the others are
-    // FP32 copies of the FP64 arrays, current while their TWIN_* bit is set
-    // in twin_ok.  Null / 0 in the FP64 forms.
     // Set within tcs_step, which knows that every field a kernel writes whole
     // is followed by its ghost-cell update: the kernels write the periodic
     // ghosts and the wall rows themselves (Grid::edge, images, wall; LineOut::gx)
@@ -247,6 +238,15 @@ struct tcs_ctx {
     // field or hands out its address, bits 1 << id: dP0's second buffer holds
     // the same shell as dP0; dV's rows 0, 1 and n2m+1 are zero.
     unsigned kept;
+    // The mixed form (precision 2): every array its stage rows and block
+    // corrections read (T, U, V, W, P and the second buffers of T, U, V, W;
+    // dU, dV, dW; the Mu and invRho tables; the wall tables; the stale
+    // scalars) is carved from one FP64 arena a64 of an elements, and the
+    // FP32 arena a32 holds each one's twin at the same element offset.  The
+    // twins of the increments dU, dV, dW are where the mixed form keeps them
+    // (the FP64 arrays are filled from them on download); the others are
+    // FP32 copies of the FP64 arrays, current while their TWIN_* bit is set
+    // in twin_ok.  Null / 0 in the FP64 forms.
     double *a64;
     float *a32;
     size_t an, aused;
