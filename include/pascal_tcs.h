@@ -6,8 +6,8 @@
  * mpi_pressure, the 1-D mesh metrics, scratch for the ADI and Poisson
  * solves, and one HIP stream.  Every entry point only enqueues work on that
  * stream and returns; the host waits only where a scalar comes back
- * (tcs_post_div, tcs_post_cfl, tcs_nusselt) or on an explicit download /
- * tcs_sync.  Plain pointers and sizes only; no torch or Fortran types.
+ * (tcs_post_div, tcs_post_cfl, tcs_nusselt), in tcs_adjoint_step and on an
+ * explicit download / tcs_sync.  Plain pointers and sizes only; no torch or Fortran types.
  *
  * Error convention: every entry returns 0 on success, a negative TCS_E_*
  * code otherwise; tcs_last_error() returns a message for the last failure.
@@ -215,7 +215,10 @@ int tcs_nusselt(tcs_ctx *ctx, double Tup, double Tbt, double *nu_bottom, double 
    context's fields as the state before a step and the adjoint fields as
    the gradient with respect to the state after it; it runs the step (the
    fields end as after tcs_step) and leaves the gradient with respect to the
-   state before it, adding the wall arrays' share to their adjoints.
+   state before it, adding the wall arrays' share to their adjoints.  It
+   returns when the stream's work is done (the other adjoint entries only
+   enqueue theirs): device buffers given to tcs_adjoint_copy before it may be
+   written or freed then.
    tcs_adjoint_copy moves an adjoint array from (to_adjoint = 1) or to
    (to_adjoint = 0) a device buffer of its size: kind 0 with a state field
    id, kind 1 with a wall id.  tcs_adjoint_add_nusselt adds weight times

@@ -879,5 +879,9 @@ extern "C" int tcs_adjoint_step(tcs_ctx *c, double dt) {
     c->cfl_valid = 0;
     TCS_TRY(adj::forward_keep(c, c->adj, dt));
     TCS_TRY(adj::backward(c, c->adj, dt));
+    // the step is over when the entry returns: buffers given to
+    // tcs_adjoint_copy before it may be written again, and a device error is
+    // this call's
+    TCS_HIP(hipStreamSynchronize(c->stream));
     return TCS_OK;
 }
