@@ -801,7 +801,6 @@ using namespace tcs;
 extern "C" int tcs_adjoint_zero(tcs_ctx *c) {
     if (!c) return TCS_E_ARG;
     TCS_TRY(flush_pending(c));
-    c->kept = 0;
     TCS_TRY(adjoint_alloc(c));
     AdjWork *w = c->adj;
     adj::Arrays z;
@@ -832,7 +831,6 @@ static double *adjoint_array(tcs_ctx *c, int32_t kind, int32_t id, size_t &n) {
 extern "C" int tcs_adjoint_copy(tcs_ctx *c, int32_t kind, int32_t id, int32_t to_adjoint, double *dev) {
     if (!c || !dev) return TCS_E_ARG;
     TCS_TRY(flush_pending(c));
-    c->kept = 0;
     TCS_TRY(adjoint_alloc(c));
     size_t n = 0;
     double *a = adjoint_array(c, kind, id, n);
@@ -856,7 +854,6 @@ extern "C" int tcs_adjoint_copy(tcs_ctx *c, int32_t kind, int32_t id, int32_t to
 extern "C" int tcs_adjoint_add_nusselt(tcs_ctx *c, double weight, double Tup, double Tbt) {
     if (!c) return TCS_E_ARG;
     TCS_TRY(flush_pending(c));
-    c->kept = 0;
     TCS_TRY(adjoint_alloc(c));
     const Grid g = c->grid();
     const double wgt = weight * c->prm.L2 / (Tbt - Tup) / c->h_dmx2[1] / ((double)c->n1m * (double)c->n3m);
@@ -868,7 +865,6 @@ extern "C" int tcs_adjoint_add_nusselt(tcs_ctx *c, double weight, double Tup, do
 extern "C" int tcs_adjoint_step(tcs_ctx *c, double dt) {
     if (!c) return TCS_E_ARG;
     TCS_TRY(flush_pending(c));
-    c->kept = 0;
     if (c->prm.precision != 0) {
         set_error("tcs_adjoint_step: the adjoint differentiates the plain FP64 step (precision 0)");
         return TCS_E_ARG;

@@ -1058,10 +1058,10 @@ int momentum_solvedV(tcs_ctx *c, double dt) {
     TCS_TRY(z_stage<ANY_SPLIT>(c, "dV_z", "dV_z_solve", z, 2, am, ac, ap, rhs));
     TCS_TRY(x_stage<ANY_SPLIT>(c, "dV_x", "dV_x_solve", DVX{g, c->phys, dt, f[TCS_U], f[TCS_INVRHO], c->stale}, 2, am, ac, ap,
                     rhs));
-    if (!(c->kept >> TCS_DV & 1))
+    // (in a step the split y solve writes dV's zero rows itself)
+    if (!c->wrap || !rows_in_solve<scr_t, ANY_SPLIT>(c, c->n2m))
         TCS_LAUNCH(c->stream, "dV_zero_rows", k_dV_zero_rows<inc_t>, dim3((c->N1 + 63) / 64, c->N3), dim3(64), 0, g,
                    inc(c, TCS_DV));
-    if (c->wrap) c->kept |= 1u << TCS_DV;
     return y_stage<sizeof(scr_t) == 8 ? 8 : 16, true>(c, "dV_y", "dV_y_solve", DVY{g, c->phys, dt, f[TCS_V], f[TCS_MU], f[TCS_INVRHO]}, 2, f[TCS_DV]);
 }
 

@@ -570,10 +570,22 @@ __global__ void k_dp_subtract(Grid g, const double *__restrict__ scal, double *d
 }
 
 // quadratic wall extrapolation (:719-736) of dP or P, with the wall rows'
-// periodic ghosts; F32 (the mixed form, not null): the FP32 copy as well
-__global__ void k_wall_extrap(Grid g, double *F, float *F32) {
+// periodic ghosts; F32 (the mixed form, not null): the FP32 copy as well.
+// The workgroups past the last k copy the cells outside the interior from
+// one buffer to another (a step: of dP0, which no ghost-cell update follows;
+// a launch of their own is 5 us of a step's 260 at 64^3).
+__global__ void k_wall_extrap(Grid g, double *F, float *F32, const double *__restrict__ shell_from,
+                              double *__restrict__ shell_to) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
     const int k = blockIdx.y + 1;
+    if (k > g.n3m) {
+        const size_t row = (size_t)gridDim.x * blockDim.x, n = g.shell_size();
+        for (size_t q = row * (k - 1 - g.n3m) + i - 1; q < n; q += row * (gridDim.y - g.n3m)) {
+            const size_t o = g.shell_cell(q);
+            shell_to[o] = shell_from[o];
+        }
+        return;
+    }
     if (i > g.n1m) return;
     const double *dmx2 = g.dmx2;
     const int n2sub = g.n2m + 1, n2msub = g.n2m;
@@ -835,6 +847,16 @@ static int fft_z_launch(tcs_ctx *c, const char *label, double2 *spec) {
     });
 }
 
+static int wall_extrap(tcs_ctx *c, double *F, float *F32, const double *shell_from = nullptr,
+                       double *shell_to = nullptr) {
+    const Grid g = c->grid();
+    const unsigned gx = (unsigned)((c->n1m + 63) / 64);
+    const size_t rows = shell_from ? (g.shell_size() + gx * 64 - 1) / (gx * 64) : 0;
+    TCS_LAUNCH(c->stream, "wall_extrap", k_wall_extrap, dim3(gx, (unsigned)(c->n3m + std::min<size_t>(rows, 4096))),
+               dim3(64), 0, g, F, F32, shell_from, shell_to);
+    return TCS_OK;
+}
+
 static PressureRHS rhs_cell(tcs_ctx *c, double dt) {
     return PressureRHS{c->grid(),        c->phys,           dt, c->f[TCS_U], c->f[TCS_V], c->f[TCS_W], c->f[TCS_DPHAT],
                        c->f[TCS_INVRHO], c->wall[TCS_VBCUP], c->wall[TCS_VBCBT]};
@@ -886,9 +908,7 @@ static int poisson_after_x(tcs_ctx *c) {
         const dim3 blk = interior_block(), grd = interior_grid(n1m, n2m, n3m);
         TCS_LAUNCH(c->stream, "dp_subtract", k_dp_subtract, grd, blk, 0, g, c->scal, c->f[TCS_DP]);
     }
-    TCS_LAUNCH(c->stream, "wall_extrap", k_wall_extrap, dim3((n1m + 63) / 64, n3m), dim3(64), 0, g, c->f[TCS_DP],
-               (float *)nullptr);
-    return TCS_OK;
+    return wall_extrap(c, c->f[TCS_DP], nullptr);
 }
 
 int pressure_poisson(tcs_ctx *c) {
@@ -913,9 +933,7 @@ int pressure_projection(tcs_ctx *c, double dt) {
                c->f[TCS_P]);
     TCS_LAUNCH(c->stream, "dphat_update", k_dphat_update, grd, blk, 0, DPhatUpdate{g, c->f[TCS_DP], c->f[TCS_DPHAT],
                c->f[TCS_DP0]}, c->f[TCS_DPHAT], c->f[TCS_DP0]);
-    TCS_LAUNCH(c->stream, "wall_extrap", k_wall_extrap, dim3((c->n1m + 63) / 64, c->n3m), dim3(64), 0, g, c->f[TCS_P],
-               twin(c, c->f[TCS_P]));
-    return TCS_OK;
+    return wall_extrap(c, c->f[TCS_P], twin(c, c->f[TCS_P]));
 }
 
 int pressure_projection_into(tcs_ctx *c, double dt, double *dPhatn, double *dP0n) {
@@ -925,8 +943,6 @@ int pressure_projection_into(tcs_ctx *c, double dt, double *dPhatn, double *dP0n
     const Projection cell{c->cell_grid(), c->phys, dt, c->f[TCS_INVRHO], c->f[TCS_DP], c->f[TCS_DPHAT], c->f[TCS_DP0],
                           c->f[TCS_U], c->f[TCS_V], c->f[TCS_W], c->f[TCS_P]};
     if (!c->wrap) TCS_TRY(copy_shell(c, {TCS_DPHAT, TCS_DP0}));
-    else if (!(c->kept >> TCS_DP0 & 1)) TCS_TRY(copy_shell(c, {TCS_DP0}));
-    if (c->wrap) c->kept |= 1u << TCS_DP0;
     const DPhatUpdate hist{g, c->f[TCS_DP], c->f[TCS_DPHAT], c->f[TCS_DP0]};
     if (c->a32) {
         const FieldSet32 tw{{twin(c, c->f[TCS_U]), twin(c, c->f[TCS_V]), twin(c, c->f[TCS_W]), twin(c, c->f[TCS_P])}};
@@ -936,9 +952,7 @@ int pressure_projection_into(tcs_ctx *c, double dt, double *dPhatn, double *dP0n
         TCS_LAUNCH(c->stream, "projection", k_projection_into<false>, grd, blk, 0, cell, hist, c->f[TCS_U], c->f[TCS_V],
                    c->f[TCS_W], c->f[TCS_P], dPhatn, dP0n, FieldSet32{});
     }
-    TCS_LAUNCH(c->stream, "wall_extrap", k_wall_extrap, dim3((c->n1m + 63) / 64, c->n3m), dim3(64), 0, g, c->f[TCS_P],
-               twin(c, c->f[TCS_P]));
-    return TCS_OK;
+    return wall_extrap(c, c->f[TCS_P], twin(c, c->f[TCS_P]), c->wrap ? c->f[TCS_DP0] : nullptr, dP0n);
 }
 
 }  // namespace TCS_FORM

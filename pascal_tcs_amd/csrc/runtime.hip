@@ -135,31 +135,12 @@ __global__ void k_halo(Grid g, Set fs) {
     }
 }
 
-// the cells of a full field outside the interior: the faces i in {0, n1m+1}
-// (all j, k), then j in {0, n2m+1} (interior i, all k), then k in {0, n3m+1}
-// (interior i and j)
 __global__ void k_copy_shell(Grid g, FieldSet src_set, FieldSet dst_set) {
     const double *__restrict__ src = src_set.f[blockIdx.y];  // one pair per grid row
     double *__restrict__ dst = dst_set.f[blockIdx.y];
-    const int N1 = g.N1, N2 = g.N2, N3 = g.N3, n1m = g.n1m, n2m = g.n2m;
-    const size_t fi = (size_t)2 * N2 * N3, fj = (size_t)2 * n1m * N3, fk = (size_t)2 * n1m * n2m;
-    size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    size_t o;
-    if (q < fi) {
-        const int side = (int)(q % 2);
-        const size_t r = q / 2;
-        o = g.ix(side ? N1 - 1 : 0, (int)(r % N2), (int)(r / N2));
-    } else if ((q -= fi) < fj) {
-        const int side = (int)(q % 2);
-        const size_t r = q / 2;
-        o = g.ix((int)(r % n1m) + 1, side ? N2 - 1 : 0, (int)(r / n1m));
-    } else if ((q -= fj) < fk) {
-        const int side = (int)(q % 2);
-        const size_t r = q / 2;
-        o = g.ix((int)(r % n1m) + 1, (int)(r / n1m) + 1, side ? N3 - 1 : 0);
-    } else {
-        return;
-    }
+    const size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (q >= g.shell_size()) return;
+    const size_t o = g.shell_cell(q);
     dst[o] = src[o];
 }
 
@@ -171,7 +152,7 @@ int copy_shell(tcs_ctx *c, std::initializer_list<int> ids) {
         src.f[nf] = c->f[id];
         dst.f[nf++] = c->spare[id];
     }
-    const size_t n = (size_t)2 * c->N2 * c->N3 + (size_t)2 * c->n1m * c->N3 + (size_t)2 * c->n1m * c->n2m;
+    const size_t n = c->grid().shell_size();
     TCS_LAUNCH(c->stream, "copy_shell", k_copy_shell, dim3((unsigned)((n + 255) / 256), (unsigned)nf), dim3(256), 0,
                c->grid(), src, dst);
     return TCS_OK;
@@ -867,7 +848,6 @@ static int check_field(tcs_ctx *c, int id) {
         return TCS_E_ARG;
     }
     TCS_TRY(flush_pending(c));
-    c->kept &= ~(1u << id);
     c->cfl_valid = 0;  // the field may change (upload, halo, a handed-out pointer)
     c->twin_ok &= ~twin_bit(id);  // and with it the mixed form's FP32 copy
     return TCS_OK;
@@ -942,7 +922,6 @@ extern "C" int tcs_field_copy_device(tcs_ctx *c, int32_t id, int32_t to_field, d
 extern "C" int tcs_fields_touched(tcs_ctx *c) {
     if (!c) return TCS_E_ARG;
     TCS_TRY(flush_pending(c));
-    c->kept = 0;
     c->cfl_valid = 0;
     c->twin_ok = 0;
     for (int q : {TCS_DU, TCS_DV, TCS_DW}) TCS_TRY(increment_from_fp64(c, q));
@@ -1017,11 +996,9 @@ extern "C" int tcs_momentum_boundary(tcs_ctx *c, double Uup, double Ubt, double 
 #define CTX_CHECK(c) \
     if (!(c)) { set_error("null context"); return TCS_E_ARG; } \
     TCS_TRY(flush_pending(c));
-// entries that may change fields drop the kept CFL maximum and what a step
-// keeps for the next
+// entries that may change fields drop the kept CFL maximum
 #define CTX_GUARD(c) \
     CTX_CHECK(c) \
-    (c)->kept = 0; \
     (c)->cfl_valid = 0;
 
 #define STAGE(label) ProfStage _stage(c, label)
@@ -1212,8 +1189,7 @@ struct Wrap {  // tcs_ctx::wrap for a scope
 // the field (tcs_ctx::wrap), on large grids but for the block corrections and
 // the projection (wrap_cells).
 extern "C" int tcs_step(tcs_ctx *c, double dt) {
-    CTX_CHECK(c);
-    c->cfl_valid = 0;
+    CTX_GUARD(c);
     STAGE("step");
     const Wrap wrap(c);
     bool swap_T = false;

@@ -270,7 +270,8 @@ int x_stage(tcs_ctx *c, const char *label_rows, const char *label_solve, const R
 // the y lines of rows j = jlo..jlo+nrows-1, right-hand side from the scratch
 // rhs.  The solution is stored into (mode 1) or added to (mode 2) the
 // interior of the field F, or, with F null, written back into rhs.  Rows
-// j < jrow are identity rows (YLineRowsLead) with LEAD.
+// j < jrow are identity rows (YLineRowsLead) with LEAD, which dV's solve asks
+// for: where it writes the wall rows they become zero.
 template <bool ANY, int SX = PT_SX, bool LEAD = false, class Row, typename S>
 int y_stage_in_solve(tcs_ctx *c, const char *label, const Row &row, int jlo, int nrows, S *rhs, double *F,
                      int mode, int jrow = 0) {
@@ -284,6 +285,7 @@ int y_stage_in_solve(tcs_ctx *c, const char *label, const Row &row, int jlo, int
         out.ss1 = (long)c->P1 * c->N2;
         out.rs = c->P1;
         out.wrap_to(c, nrows);
+        out.zero_walls = LEAD;
         if constexpr (sizeof(S) == sizeof(float)) {
             // the mixed form stores its increments into their FP32 twins
             out.G = twin(c, F);

@@ -142,6 +142,26 @@ struct Grid {
             images(F, i, k, q, v);
         }
     }
+    // The cells of a full field outside the interior, numbered: the faces i in
+    // {0, n1m+1} (all j, k), then j in {0, n2m+1} (interior i, all k), then k
+    // in {0, n3m+1} (interior i and j)
+    __host__ __device__ size_t shell_size() const {
+        return (size_t)2 * N2 * N3 + (size_t)2 * n1m * N3 + (size_t)2 * n1m * n2m;
+    }
+    __device__ __forceinline__ size_t shell_cell(size_t q) const {
+        const size_t fi = (size_t)2 * N2 * N3, fj = (size_t)2 * n1m * N3;
+        const int side = (int)(q % 2);  // the faces' sizes are even
+        if (q < fi) {
+            const size_t r = q / 2;
+            return ix(side ? N1 - 1 : 0, (int)(r % N2), (int)(r / N2));
+        }
+        if ((q -= fi) < fj) {
+            const size_t r = q / 2;
+            return ix((int)(r % n1m) + 1, side ? N2 - 1 : 0, (int)(r / n1m));
+        }
+        const size_t r = (q - fj) / 2;
+        return ix((int)(r % n1m) + 1, (int)(r / n1m) + 1, side ? N3 - 1 : 0);
+    }
     __device__ __forceinline__ RelCell ix(Rel i, Rel j, Rel k) const {
         return RelCell{ix(i.v, j.v, k.v), (k.o + 1) * 9 + (j.o + 1) * 3 + (i.o + 1)};
     }
@@ -234,10 +254,6 @@ struct tcs_ctx {
     // 0.22, 0.12 and 0.26 ms, the three launches 0.25; at 256x193x128 edges
     // cost 3 us a kernel, a launch 6)
     int wrap_cells() const { return wrap && nint > ((size_t)1 << 23) ? 2 : wrap; }
-    // For steps in a row, cleared by every other entry that may write the
-    // field or hands out its address, bits 1 << id: dP0's second buffer holds
-    // the same shell as dP0; dV's rows 0, 1 and n2m+1 are zero.
-    unsigned kept;
     // The mixed form (precision 2): every array its stage rows and block
     // corrections read (T, U, V, W, P and the second buffers of T, U, V, W;
     // dU, dV, dW; the Mu and invRho tables; the wall tables; the stale
@@ -338,6 +354,7 @@ struct LineOut {
     // > 0: gx x gz lines of n_row rows, written with their periodic ghosts in
     // s0 and s1 and with the wall rows before and after them (mode 3: Fin's)
     int gx = 0, gz = 0, n_row = 0;
+    bool zero_walls = false;  // (gx > 0) the wall rows become zero (dV's)
     void wrap_to(const tcs_ctx *c, int nr) {
         if (c->wrap) { gx = c->n1m; gz = c->n3m; n_row = nr; }
     }

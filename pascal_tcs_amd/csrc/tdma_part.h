@@ -325,8 +325,8 @@ __device__ __forceinline__ void store(const T (&a)[MM], const T (&c)[MM], const 
             for (int r = 0; r < MM; r++)
                 if (r < m)
                     put_line<float>(out.G, fb + (long)(j0 + r) * out.rs, x_of<T, 1, MM>(a, c, d, 0, r, m, xf, xl), di, dk);
-            if (lo) put_line<float>(out.G, ol, out.G[ol], di, dk);
-            if (hi) put_line<float>(out.G, oh, out.G[oh], di, dk);
+            if (lo) put_line<float>(out.G, ol, out.zero_walls ? 0.0f : out.G[ol], di, dk);
+            if (hi) put_line<float>(out.G, oh, out.zero_walls ? 0.0f : out.G[oh], di, dk);
             return;
         }
     }
@@ -351,7 +351,7 @@ __device__ __forceinline__ void store(const T (&a)[MM], const T (&c)[MM], const 
         for (int w = 0; w < 2; w++)
             if (w ? hi : lo) {
                 const long o = w ? oh : ol;
-                const double v = walls[o];
+                const double v = out.zero_walls ? 0.0 : walls[o];
                 put_line<double>(out.F, o, v, di, dk);
                 if constexpr (sizeof(T) == sizeof(float)) {
                     if (out.G) put_line<float>(out.G, o, (float)v, di, dk);
