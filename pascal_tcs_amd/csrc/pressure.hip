@@ -238,6 +238,7 @@ struct XFft {
     static constexpr int TX = N <= 1024 ? 4 : 2;
     static constexpr int NT = N == 0 || N == 512 ? 256 : N > 512 ? 512 : N == 256 ? 128 : 64;
     static int tile(int n1m) { return N ? TX : n1m > 1024 ? 1 : 4; }
+    static size_t most_lds() { return (size_t)fft_lds_len(N ? TX * N : 4096) * 2 * sizeof(double); }
 };
 
 // x r2c: TX k-lines (k0..k0+TX-1) of row j per workgroup.
@@ -773,17 +774,6 @@ __global__ void __launch_bounds__(256) k_dphat_update(DPhatUpdate cell, double *
 }
 
 // ---------------------------------------------------------------- host -----
-// An x transform's workgroups may need more than 64 KiB of LDS (1024 and 2048
-// points; gfx950: 160 KiB per CU): the kernel's limit raised, once (a kernel's
-// calls all ask for the same)
-template <class K>
-static int lds_limit(K kernel, size_t bytes, bool &raised) {
-    if (bytes <= 65536 || raised) return TCS_OK;
-    TCS_HIP(hipFuncSetAttribute((const void *)kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
-    raised = true;
-    return TCS_OK;
-}
-
 // f(length): the length as a constant where the transforms have it
 template <class F>
 static int with_length(int n, F f) {
@@ -805,8 +795,8 @@ static int fft_x_fwd_src_launch(tcs_ctx *c, const char *label, const Src &src, d
         constexpr int N = decltype(len)::value;
         const int TX = XFft<N>::tile(c->n1m);
         const size_t lds = (size_t)fft_lds_len(TX * c->n1m) * 2 * sizeof(double);
-        static bool raised = false;
-        TCS_TRY(lds_limit(k_fft_x_fwd<N, Src>, lds, raised));
+        static DeviceSet raised;
+        TCS_TRY(lds_limit((const void *)k_fft_x_fwd<N, Src>, XFft<N>::most_lds(), raised));
         TCS_LAUNCH(c->stream, label, (k_fft_x_fwd<N, Src>), dim3(c->n3m / TX, c->n2m), dim3(XFft<N>::NT), lds, c->grid(),
                    c->h1p, TX, src, (const double2 *)c->tw1, spec);
         return TCS_OK;
@@ -824,8 +814,8 @@ static int fft_x_inv_launch(tcs_ctx *c, const char *label, const double2 *spec, 
         const int TX = XFft<N>::tile(c->n1m);
         const size_t lds = (size_t)fft_lds_len(TX * c->n1m) * 2 * sizeof(double);
         const auto kernel = sub ? k_fft_x_inv<N, true> : k_fft_x_inv<N, false>;
-        static bool raised[2];
-        TCS_TRY(lds_limit(kernel, lds, raised[sub]));
+        static DeviceSet raised[2];
+        TCS_TRY(lds_limit((const void *)kernel, XFft<N>::most_lds(), raised[sub]));
         TCS_LAUNCH(c->stream, label, kernel, dim3(c->n3m / TX, c->n2m),
                    dim3(XFft<N>::NT), lds, c->grid(), c->h1p, TX, spec, (const double2 *)c->tw1, out, c->linesum,
                    c->scal);
@@ -886,12 +876,8 @@ static int poisson_after_x(tcs_ctx *c) {
                    n3m, h1p, c->h3p, c->ptab, c->ptab + n2m, c->ptab + 2 * n2m, c->dxk2, c->dzk, spec, P, w1, w2);
     } else {
         const int kept = exact_line::kept_rows<2>(nsys, n2m), lds = kept * exact_line::Kept<2>::ROW_BYTES;
-        static bool lds_raised = false;  // more than 64 KiB of dynamic LDS (gfx950: 160 KiB per CU)
-        if (!lds_raised) {
-            TCS_HIP(hipFuncSetAttribute((const void *)k_poisson_tdma, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                        exact_line::KEPT_LDS));
-            lds_raised = true;
-        }
+        static DeviceSet raised;
+        TCS_TRY(lds_limit((const void *)k_poisson_tdma, exact_line::KEPT_LDS, raised));
         TCS_LAUNCH(c->stream, "poisson_tdma", k_poisson_tdma, dim3((nsys + exact_line::EX_W - 1) / exact_line::EX_W),
                    dim3(exact_line::EX_W), lds, n3m, h1p, n2m, c->h3p, c->ptab, c->ptab + n2m, c->ptab + 2 * n2m,
                    c->dxk2, c->dzk, spec, c->pA, c->pC, n2m - kept);

@@ -98,6 +98,16 @@ struct ProfStage {
     }
 };
 
+int lds_limit(const void *kernel, size_t most, DeviceSet &raised) {
+    if (most <= 65536) return TCS_OK;
+    int dev = 0;
+    TCS_HIP(hipGetDevice(&dev));
+    return once_per_device(raised, dev, [&]() -> int {
+        TCS_HIP(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)most));
+        return TCS_OK;
+    });
+}
+
 // ------------------------------------------------------------ halo --------
 // Single-rank mpi_subdomain_ghostcell_update (src/module_mpi_subdomain.f90:
 // 758-791): the x pass copies planes i=n1m -> 0 and i=1 -> n1sub for every

@@ -11,6 +11,7 @@
 #include <utility>
 
 #include "../../include/pascal_tcs.h"
+#include "device_once.h"
 
 namespace tcs {
 
@@ -318,6 +319,11 @@ __device__ __forceinline__ bool last_arrive(unsigned *count, unsigned n) {
 __device__ __forceinline__ double last_get(const double *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+
+// Dynamic LDS past 64 KiB (gfx950: 160 KiB per CU) needs the kernel's limit
+// raised, on each device: to be called before a launch, with the most that
+// any of the kernel's launches asks for.
+int lds_limit(const void *kernel, size_t most, DeviceSet &raised);
 
 // launch helpers -------------------------------------------------------------
 inline dim3 interior_block() { return dim3(64, 4, 1); }

@@ -229,12 +229,8 @@ int ptdma_exact_launch(double *A, const double *B, double *C, const double *Din,
     const long lines = (long)n0 * n1;
     const int kept = kept_rows<1>(lines, n_row), lds = kept * Kept<1>::ROW_BYTES;
     const auto kern = field ? k_ptdma_exact<false, false, true> : EXACT_PICK(k_ptdma_exact);
-    static bool raised[5];  // more than 64 KiB of dynamic LDS (gfx950: 160 KiB per CU)
-    bool &up = raised[field ? 4 : 2 * cyclic + keep];
-    if (!up) {
-        TCS_HIP(hipFuncSetAttribute((const void *)kern, hipFuncAttributeMaxDynamicSharedMemorySize, KEPT_LDS));
-        up = true;
-    }
+    static DeviceSet raised[5];
+    TCS_TRY(lds_limit((const void *)kern, KEPT_LDS, raised[field ? 4 : 2 * cyclic + keep]));
     TCS_LAUNCH(st, cyclic ? "ptdma_cyclic" : "ptdma", kern, dim3((unsigned)((lines + EX_W - 1) / EX_W)), dim3(EX_W),
                lds, A, B, C, Din, Dout, n0, ss0, ss1, lines, n_row, rs, n_row - kept, out);
 #undef EXACT_PICK

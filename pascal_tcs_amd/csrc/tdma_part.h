@@ -709,13 +709,9 @@ int part_rows_src_launch(hipStream_t st, const char *label, const Src &src, cons
         lsb = std::max(lsb, stage_len(rblock_row0(g + 1, q.P, q.w1, q.w2) - rblock_row0(g, q.P, q.w1, q.w2)));
     const int ls = stage_len(n_row);
     const int lds = (int)sizeof(T) * std::max(XSX * ls, 4 * XSX * lsb);
-    static bool lds_raised = false;  // more than 64 KiB of dynamic LDS (gfx950: 160 KiB per CU)
-    if (!lds_raised) {
-        const int most = std::max(XSX * stage_len(MM * PM), 4 * XSX * stage_len(MM * PM / PT_RBLK));
-        TCS_HIP(hipFuncSetAttribute((const void *)k_ptdma_part_rows_src<T, CYC, Src, XSX, MM, PM>,
-                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(T) * most));
-        lds_raised = true;
-    }
+    static DeviceSet raised;
+    const int most = std::max(XSX * stage_len(MM * PM), 4 * XSX * stage_len(MM * PM / PT_RBLK));
+    TCS_TRY(lds_limit((const void *)k_ptdma_part_rows_src<T, CYC, Src, XSX, MM, PM>, sizeof(T) * most, raised));
     const dim3 blk(XSX * q.P), grd((unsigned)((n0 + XSX - 1) / XSX), (unsigned)n1);
     TCS_LAUNCH(st, label, (k_ptdma_part_rows_src<T, CYC, Src, XSX, MM, PM>), grd, blk, lds, src, D, n0, ss0, ss1, n_row,
                ls, lsb, q.P, q.w1, q.w2);

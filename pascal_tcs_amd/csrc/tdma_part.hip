@@ -191,15 +191,9 @@ static int part_launch(const T *A, const T *B, const T *C, const T *Din, T *D, i
     if (rs == 1) {
         const int ls = stage_len(n_row);
         const int lds = part_lds_bytes<T>(n_row);
-        static bool lds_raised = false;  // allow more than 64 KiB of dynamic LDS (gfx950: 160 KiB per CU)
-        if (!lds_raised) {
-            const int most = part_lds_bytes<T>(PT_MMAX * PT_PMAX);
-            TCS_HIP(hipFuncSetAttribute((const void *)k_ptdma_part_rows<T, false>,
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, most));
-            TCS_HIP(hipFuncSetAttribute((const void *)k_ptdma_part_rows<T, true>,
-                                        hipFuncAttributeMaxDynamicSharedMemorySize, most));
-            lds_raised = true;
-        }
+        static DeviceSet raised[2];
+        TCS_TRY(lds_limit(cyclic ? (const void *)k_ptdma_part_rows<T, true> : (const void *)k_ptdma_part_rows<T, false>,
+                          part_lds_bytes<T>(PT_MMAX * PT_PMAX), raised[cyclic]));
         dim3 blk(PT_SX * P), grd((unsigned)((n0 + PT_SX - 1) / PT_SX), (unsigned)n1);
         if (cyclic)
             TCS_LAUNCH(st, L::rows_cyc, (k_ptdma_part_rows<T, true>), grd, blk, lds, A, B, C, Din, D, n0, ss0, ss1, n_row,
