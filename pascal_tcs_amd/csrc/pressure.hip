@@ -292,6 +292,7 @@ k_fft_x_fwd(Grid g, int h1p, int tx, Src src, const double2 *__restrict__ tw, do
 template <int N>
 struct ZFft {
     static constexpr int NL = N == 0 || N >= 512 ? 1 : 512 / N;
+    static size_t most_lds() { return (size_t)fft_lds_len(N ? NL * N : 4096) * 2 * sizeof(double); }
 };
 template <int SIGN, int NT, int N>
 __global__ void __launch_bounds__(NT)
@@ -831,6 +832,8 @@ static int fft_z_launch(tcs_ctx *c, const char *label, double2 *spec) {
         // the fewest threads that hold a pass's butterflies at FFT_MAXB each
         constexpr int NT = N == 0 ? 256 : N <= 1024 ? 64 : 128;
         const size_t lds = (size_t)fft_lds_len(NL * c->n3m) * 2 * sizeof(double);
+        static DeviceSet raised;
+        TCS_TRY(lds_limit((const void *)k_fft_z<SIGN, NT, N>, ZFft<N>::most_lds(), raised));
         TCS_LAUNCH(c->stream, label, (k_fft_z<SIGN, NT, N>), dim3((c->h1p + NL - 1) / NL, c->n2m), dim3(NT), lds,
                    c->n3m, c->h1p, (const double2 *)c->tw3, spec);
         return TCS_OK;
