@@ -827,16 +827,25 @@ static int fft_x_inv_launch(tcs_ctx *c, const char *label, const double2 *spec, 
 // c2c along z in place
 template <int SIGN>
 static int fft_z_launch(tcs_ctx *c, const char *label, double2 *spec) {
-    return with_length(c->n3m, [&](auto len) {
-        constexpr int N = decltype(len)::value, NL = ZFft<N>::NL;
-        // the fewest threads that hold a pass's butterflies at FFT_MAXB each
-        constexpr int NT = N == 0 ? 256 : N <= 1024 ? 64 : 128;
+    const auto launch = [&](auto len, auto threads) {
+        constexpr int N = decltype(len)::value, NL = ZFft<N>::NL, NT = decltype(threads)::value;
         const size_t lds = (size_t)fft_lds_len(NL * c->n3m) * 2 * sizeof(double);
         static DeviceSet raised;
         TCS_TRY(lds_limit((const void *)k_fft_z<SIGN, NT, N>, ZFft<N>::most_lds(), raised));
         TCS_LAUNCH(c->stream, label, (k_fft_z<SIGN, NT, N>), dim3((c->h1p + NL - 1) / NL, c->n2m), dim3(NT), lds,
                    c->n3m, c->h1p, (const double2 *)c->tw3, spec);
         return TCS_OK;
+    };
+    return with_length(c->n3m, [&](auto len) {
+        // the fewest threads that hold a pass's butterflies at FFT_MAXB each:
+        // lines of 4 to 32 points with the 256 that 4096 points need ran
+        // three waves a workgroup idle (512x512x16: 323 us a transform, 102
+        // with one)
+        constexpr int N = decltype(len)::value;
+        using std::integral_constant;
+        if constexpr (N == 0)
+            if (c->n3m > 1024) return launch(len, integral_constant<int, 256>());
+        return launch(len, integral_constant<int, N == 2048 ? 128 : 64>());
     });
 }
 
