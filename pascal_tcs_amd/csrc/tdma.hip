@@ -92,11 +92,14 @@ k_ptdma_exact_rows(double *A, const double *B, double *C, const double *Din, dou
     const int nch = (n_row + EX_R - 1) / EX_R;
     double *TA = tile[0] + lane * P, *TB = tile[1] + lane * P, *TC = tile[2] + lane * P, *TD = tile[3] + lane * P;
     const int ql = lane / EX_R, qr = lane % EX_R;  // along the lines: line 4q + ql, row qr of the chunk
-    // value (r, lane) of the chunk at row r0 with nr rows
+    // value (r, lane) of the chunk at row r0 with nr rows; the last, shorter one
+    // stays in its lines' order (packing it, or fewer lines, by divisions took
+    // a third of the time: 647 us a line of 1000 rows, 414 now)
     auto spot = [&](int r0, int nr, int r) {
-        if (nl == EX_W && nr == EX_R) return lb + (long)(r * 4 + ql) * ss0 + r0 + qr;
-        const int v = r * nl + lane;
-        return lb + (long)(v / nr) * ss0 + r0 + v % nr;
+        if (nr < EX_R) return lb + (long)lane * ss0 + r0 + r;
+        if (nl == EX_W) return lb + (long)(r * 4 + ql) * ss0 + r0 + qr;
+        const unsigned v = r * nl + lane;
+        return lb + (long)(v / EX_R) * ss0 + r0 + v % EX_R;
     };
     double va[EX_R], vb[EX_R], vc[EX_R], vd[EX_R];
     auto fetch = [&](int ch) {  // a chunk's rows into registers, along the lines
@@ -221,6 +224,15 @@ int ptdma_exact_launch(double *A, const double *B, double *C, const double *Din,
         return TCS_E_ARG;
     }
     if (rs == 1) {
+        // planes of few lines without gaps between them are one plane, so that
+        // workgroups are full (3000 planes of 1 line of 301 rows 493 us, now
+        // 167; of 5 lines 557, 221; above half a workgroup's lines a plane
+        // what is saved may go into a last round of a few workgroups: 2000
+        // planes of 33 lines of 33 rows 92 us, 120 as one)
+        if (2 * n0 <= EX_W && ss1 == (long)n0 * ss0 && (long)n0 * n1 <= INT32_MAX) {
+            n0 *= n1;
+            n1 = 1;
+        }
         const dim3 grd((unsigned)((n0 + EX_W - 1) / EX_W), (unsigned)n1);
         TCS_LAUNCH(st, cyclic ? "ptdma_rows_cyclic" : "ptdma_rows", EXACT_PICK(k_ptdma_exact_rows), grd, dim3(EX_W),
                    0, A, B, C, Din, Dout, n0, ss0, ss1, n_row);
