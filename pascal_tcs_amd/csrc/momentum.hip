@@ -911,7 +911,7 @@ constexpr int LDV_KB = 1, LDU_KB = 4, LDV_IB = 1, LDU_IB = 2;
 
 // blockLdV with the pseudo-update of V: dV(j >= 2) = the new dV and Vn =
 // V + dV; at j = 1 Vn = V + dV * 0 (:178-208)
-template <typename E, class Acc>
+template <typename E, class Acc, bool EDGES>
 __global__ void __launch_bounds__(256) k_blockLdV_pseudo(BlockLdV cell, Acc acc, E *dV, double *__restrict__ Vn) {
     const Grid &g = cell.g;
     const int i0 = (blockIdx.x * blockDim.x + threadIdx.x) * LDV_IB + 1;  // n1m is a multiple of LDV_IB
@@ -941,7 +941,7 @@ __global__ void __launch_bounds__(256) k_blockLdV_pseudo(BlockLdV cell, Acc acc,
         if (j >= 2) dV[q] = o[c];
         Vn[q] = vn[c];
     }
-    if (g.edge(i0, LDV_IB, j, blockIdx.z * LDV_KB + 1, LDV_KB)) {
+    if (EDGES && g.edge(i0, LDV_IB, j, blockIdx.z * LDV_KB + 1, LDV_KB)) {
 #pragma unroll
         for (int c = 0; c < NC; c++) {
             const int i = i0 + c % LDV_IB, k = blockIdx.z * LDV_KB + c / LDV_IB + 1;
@@ -1058,8 +1058,8 @@ int momentum_solvedV(tcs_ctx *c, double dt) {
     TCS_TRY(z_stage<ANY_SPLIT>(c, "dV_z", "dV_z_solve", z, 2, am, ac, ap, rhs));
     TCS_TRY(x_stage<ANY_SPLIT>(c, "dV_x", "dV_x_solve", DVX{g, c->phys, dt, f[TCS_U], f[TCS_INVRHO], c->stale}, 2, am, ac, ap,
                     rhs));
-    // (in a step the split y solve writes dV's zero rows itself)
-    if (!c->wrap || !rows_in_solve<scr_t, ANY_SPLIT>(c, c->n2m))
+    // (on small grids a step's split y solve writes dV's zero rows itself)
+    if (!c->wrap_fields() || !rows_in_solve<scr_t, ANY_SPLIT>(c, c->n2m))
         TCS_LAUNCH(c->stream, "dV_zero_rows", k_dV_zero_rows<inc_t>, dim3((c->N1 + 63) / 64, c->N3), dim3(64), 0, g,
                    inc(c, TCS_DV));
     return y_stage<sizeof(scr_t) == 8 ? 8 : 16, true>(c, "dV_y", "dV_y_solve", DVY{g, c->phys, dt, f[TCS_V], f[TCS_MU], f[TCS_INVRHO]}, 2, f[TCS_DV]);
@@ -1100,7 +1100,7 @@ int momentum_blockLdU(tcs_ctx *c, double dt) {
 
 // blockLdU with the pseudo-update of U and W: dU = the new dU, Un = U + dU,
 // Wn = W + dW (:178-208)
-template <typename E, class Acc>
+template <typename E, class Acc, bool EDGES>
 __global__ void __launch_bounds__(256) k_blockLdU_pseudo(BlockLdU cell, Acc acc, const double *__restrict__ W,
                                                         const E *__restrict__ dW, E *dU,
                                                         double *__restrict__ Un, double *__restrict__ Wn) {
@@ -1129,7 +1129,7 @@ __global__ void __launch_bounds__(256) k_blockLdU_pseudo(BlockLdU cell, Acc acc,
         Un[q] = un[c];
         Wn[q] = wn[c];
     }
-    if (g.edge(i0, LDU_IB, j, blockIdx.z * LDU_KB + 1, LDU_KB)) {
+    if (EDGES && g.edge(i0, LDU_IB, j, blockIdx.z * LDU_KB + 1, LDU_KB)) {
 #pragma unroll
         for (int c = 0; c < NC; c++) {
             const int i = i0 + c % LDU_IB, k = blockIdx.z * LDU_KB + c / LDU_IB + 1;
@@ -1144,25 +1144,29 @@ __global__ void __launch_bounds__(256) k_blockLdU_pseudo(BlockLdU cell, Acc acc,
 
 int momentum_blockLdV_pseudo(tcs_ctx *c, double dt, double *Vn) {
     const dim3 blk = interior_block(), grd = cell_grid(c->n1m, c->n2m, c->n3m, LDV_KB, interior_block(), LDV_IB);
-    const BlockLdV cell{c->cell_grid(), c->phys, dt, c->f[TCS_V], c->f[TCS_DW], c->f[TCS_MU], c->f[TCS_INVRHO], c->f[TCS_DV]};
+    const BlockLdV cell{c->grid(), c->phys, dt, c->f[TCS_V], c->f[TCS_DW], c->f[TCS_MU], c->f[TCS_INVRHO], c->f[TCS_DV]};
     TCS_TRY(ensure_twins(c, TWIN_V | TWIN_TAB));
     c->twin_ok &= ~(unsigned)TWIN_V;  // Vn becomes V
     if (!c->wrap) TCS_TRY(copy_shell(c, {TCS_V}));
     auto acc = cell_access(c);
-    TCS_LAUNCH(c->stream, "blockLdV", (k_blockLdV_pseudo<inc_t, decltype(acc)>), grd, blk, 0, cell, acc,
+    const auto kernel = c->wrap_fields() ? k_blockLdV_pseudo<inc_t, decltype(acc), true>
+                                         : k_blockLdV_pseudo<inc_t, decltype(acc), false>;
+    TCS_LAUNCH(c->stream, "blockLdV", kernel, grd, blk, 0, cell, acc,
                inc(c, TCS_DV), Vn);
     return TCS_OK;
 }
 
 int momentum_blockLdU_pseudo(tcs_ctx *c, double dt, double *Un, double *Wn) {
     const dim3 blk = interior_block(), grd = cell_grid(c->n1m, c->n2m, c->n3m, LDU_KB, interior_block(), LDU_IB);
-    const BlockLdU cell{c->cell_grid(), c->phys, dt, c->f[TCS_U], c->f[TCS_DV], c->f[TCS_DW],
+    const BlockLdU cell{c->grid(), c->phys, dt, c->f[TCS_U], c->f[TCS_DV], c->f[TCS_DW],
                         c->f[TCS_MU], c->f[TCS_INVRHO], c->f[TCS_DU]};
     TCS_TRY(ensure_twins(c, TWIN_U | TWIN_TAB));
     c->twin_ok &= ~(unsigned)(TWIN_U | TWIN_W);  // Un, Wn become U, W
     if (!c->wrap) TCS_TRY(copy_shell(c, {TCS_U, TCS_W}));
     auto acc = cell_access(c);
-    TCS_LAUNCH(c->stream, "blockLdU", (k_blockLdU_pseudo<inc_t, decltype(acc)>), grd, blk, 0, cell, acc,
+    const auto kernel = c->wrap_fields() ? k_blockLdU_pseudo<inc_t, decltype(acc), true>
+                                         : k_blockLdU_pseudo<inc_t, decltype(acc), false>;
+    TCS_LAUNCH(c->stream, "blockLdU", kernel, grd, blk, 0, cell, acc,
                c->f[TCS_W], inc(c, TCS_DW), inc(c, TCS_DU), Un, Wn);
     return TCS_OK;
 }

@@ -560,6 +560,7 @@ k_mean(int n1m, int n2m, int n3m, int h1p, const double2 *__restrict__ spec, con
     if (threadIdx.x == 0) scal[0] = s / (double)n1m / (double)n2m / (double)n3m;
 }
 
+template <bool EDGES>
 __global__ void k_dp_subtract(Grid g, const double *__restrict__ scal, double *dP) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
     const int j = blockIdx.y * blockDim.y + threadIdx.y + 1;
@@ -568,7 +569,7 @@ __global__ void k_dp_subtract(Grid g, const double *__restrict__ scal, double *d
     const size_t q = g.ix(i, j, k);
     const double v = dP[q] - scal[0];
     dP[q] = v;
-    if (g.edge(i, 1, j, k, 1)) g.images(dP, i, k, q, v);
+    if (EDGES && g.edge(i, 1, j, k, 1)) g.images(dP, i, k, q, v);
 }
 
 // quadratic wall extrapolation (:719-736) of dP or P, with the wall rows'
@@ -701,7 +702,7 @@ struct DPhatUpdate {
 // the projection with the new dPhat and dP0 written to second buffers
 // TW (the mixed form): U, V, W, P's FP32 copies (tw[0..3]) of the updated
 // cells written as well
-template <bool TW>
+template <bool TW, bool EDGES>
 __global__ void __launch_bounds__(256) k_projection_into(Projection cell, DPhatUpdate hist, double *U, double *V,
                                                         double *W, double *P, double *__restrict__ dPhatn,
                                                         double *__restrict__ dP0n, FieldSet32 tw) {
@@ -737,7 +738,7 @@ __global__ void __launch_bounds__(256) k_projection_into(Projection cell, DPhatU
             tw.f[3][o] = (float)q[c];
         }
     }
-    if (g.edge(i0, PROJ_IB, j, blockIdx.z * PROJ_KB + 1, PROJ_KB)) {
+    if (EDGES && g.edge(i0, PROJ_IB, j, blockIdx.z * PROJ_KB + 1, PROJ_KB)) {
 #pragma unroll
         for (int c = 0; c < NC; c++) {
             const int i = i0 + c % PROJ_IB, k = blockIdx.z * PROJ_KB + c / PROJ_IB + 1;
@@ -904,9 +905,12 @@ static int poisson_after_x(tcs_ctx *c) {
         TCS_TRY(fft_x_inv_launch(c, "fft_x_inv", spec, c->f[TCS_DP], true));
     } else {
         const dim3 blk = interior_block(), grd = interior_grid(n1m, n2m, n3m);
-        TCS_LAUNCH(c->stream, "dp_subtract", k_dp_subtract, grd, blk, 0, g, c->scal, c->f[TCS_DP]);
+        TCS_LAUNCH(c->stream, "dp_subtract", (c->wrap_fields() ? k_dp_subtract<true> : k_dp_subtract<false>), grd, blk, 0,
+                   g, c->scal, c->f[TCS_DP]);
     }
-    return wall_extrap(c, c->f[TCS_DP], nullptr);
+    TCS_TRY(wall_extrap(c, c->f[TCS_DP], nullptr));
+    if (!SPECTRAL_MEAN && c->wrap && !c->wrap_fields()) return halo(c, c->f[TCS_DP]);
+    return TCS_OK;
 }
 
 int pressure_poisson(tcs_ctx *c) {
@@ -938,16 +942,16 @@ int pressure_projection_into(tcs_ctx *c, double dt, double *dPhatn, double *dP0n
     c->twin_ok &= ~(unsigned)(TWIN_U | TWIN_V | TWIN_W | TWIN_P);  // the mixed form's FP32 copies
     const Grid g = c->grid();
     const dim3 blk = interior_block(), grd = cell_grid(c->n1m, c->n2m, c->n3m, PROJ_KB, interior_block(), PROJ_IB);
-    const Projection cell{c->cell_grid(), c->phys, dt, c->f[TCS_INVRHO], c->f[TCS_DP], c->f[TCS_DPHAT], c->f[TCS_DP0],
+    const Projection cell{g, c->phys, dt, c->f[TCS_INVRHO], c->f[TCS_DP], c->f[TCS_DPHAT], c->f[TCS_DP0],
                           c->f[TCS_U], c->f[TCS_V], c->f[TCS_W], c->f[TCS_P]};
     if (!c->wrap) TCS_TRY(copy_shell(c, {TCS_DPHAT, TCS_DP0}));
     const DPhatUpdate hist{g, c->f[TCS_DP], c->f[TCS_DPHAT], c->f[TCS_DP0]};
     if (c->a32) {
         const FieldSet32 tw{{twin(c, c->f[TCS_U]), twin(c, c->f[TCS_V]), twin(c, c->f[TCS_W]), twin(c, c->f[TCS_P])}};
-        TCS_LAUNCH(c->stream, "projection", k_projection_into<true>, grd, blk, 0, cell, hist, c->f[TCS_U], c->f[TCS_V],
+        TCS_LAUNCH(c->stream, "projection", (c->wrap_fields() ? k_projection_into<true, true> : k_projection_into<true, false>), grd, blk, 0, cell, hist, c->f[TCS_U], c->f[TCS_V],
                    c->f[TCS_W], c->f[TCS_P], dPhatn, dP0n, tw);
     } else {
-        TCS_LAUNCH(c->stream, "projection", k_projection_into<false>, grd, blk, 0, cell, hist, c->f[TCS_U], c->f[TCS_V],
+        TCS_LAUNCH(c->stream, "projection", (c->wrap_fields() ? k_projection_into<false, true> : k_projection_into<false, false>), grd, blk, 0, cell, hist, c->f[TCS_U], c->f[TCS_V],
                    c->f[TCS_W], c->f[TCS_P], dPhatn, dP0n, FieldSet32{});
     }
     return wall_extrap(c, c->f[TCS_P], twin(c, c->f[TCS_P]), c->wrap ? c->f[TCS_DP0] : nullptr, dP0n);

@@ -116,10 +116,16 @@ int lds_limit(const void *kernel, size_t most, DeviceSet &raised) {
 // passes together equal: every ghost cell with i or k on a ghost plane takes
 // the value at (mx(i), j, mz(k)), where mx/mz fold ghost indices onto the
 // periodic interior.  Sources are never ghosts in x or z, so one kernel does
-// it without ordering hazards.
-template <typename E, class Set>
-__global__ void k_halo(Grid g, Set fs) {
-    E *__restrict__ f = fs.f[blockIdx.y];  // one field per grid row
+// it without ordering hazards.  WALLS: the wall rows (interior i and k, and
+// their ghosts) from another buffer, where the field has one.
+template <typename E, class Set, bool WALLS>
+__global__ void k_halo(Grid g, Set fs, FieldSet walls) {
+    E *f = fs.f[blockIdx.y];  // one field per grid row
+    const double *w = WALLS ? walls.f[blockIdx.y] : nullptr;
+    const auto value = [&](int i, int j, int k) -> E {
+        if (WALLS && w && (j == 0 || j == g.N2 - 1)) return (E)w[g.ix(i, j, k)];
+        return f[g.ix(i, j, k)];
+    };
     const int N1 = g.N1, N2 = g.N2, N3 = g.N3;
     const int n1m = g.n1m, n3m = g.n3m;
     // threads over the x-ghost faces (2*N2*N3) then the z-ghost faces (2*N1*N2)
@@ -132,7 +138,7 @@ __global__ void k_halo(Grid g, Set fs) {
         if (k == 0 || k == N3 - 1) return;  // written by the z faces
         const int i = side ? n1m + 1 : 0;
         const int is = side ? 1 : n1m;
-        f[g.ix(i, j, k)] = f[g.ix(is, j, k)];
+        f[g.ix(i, j, k)] = value(is, j, k);
     } else if (q < nx + nz) {
         const size_t r = q - nx;
         const int side = (int)(r % 2);
@@ -141,17 +147,23 @@ __global__ void k_halo(Grid g, Set fs) {
         const int k = side ? n3m + 1 : 0;
         const int ks = side ? 1 : n3m;
         const int is = (i == 0) ? n1m : (i == n1m + 1 ? 1 : i);
-        f[g.ix(i, j, k)] = f[g.ix(is, j, ks)];
+        f[g.ix(i, j, k)] = value(is, j, ks);
+    } else if (WALLS && w && q < nx + nz + (size_t)2 * n1m * n3m) {
+        const size_t r = q - nx - nz, t = r / 2;
+        const int i = (int)(t % n1m) + 1, k = (int)(t / n1m) + 1;
+        const size_t o = g.ix(i, r % 2 ? N2 - 1 : 0, k);
+        f[o] = (E)w[o];
     }
 }
 
-__global__ void k_copy_shell(Grid g, FieldSet src_set, FieldSet dst_set) {
+template <typename E, class DstSet>
+__global__ void k_copy_shell(Grid g, FieldSet src_set, DstSet dst_set) {
     const double *__restrict__ src = src_set.f[blockIdx.y];  // one pair per grid row
-    double *__restrict__ dst = dst_set.f[blockIdx.y];
+    E *__restrict__ dst = dst_set.f[blockIdx.y];
     const size_t q = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (q >= g.shell_size()) return;
     const size_t o = g.shell_cell(q);
-    dst[o] = src[o];
+    dst[o] = (E)src[o];
 }
 
 int copy_shell(tcs_ctx *c, std::initializer_list<int> ids) {
@@ -163,21 +175,21 @@ int copy_shell(tcs_ctx *c, std::initializer_list<int> ids) {
         dst.f[nf++] = c->spare[id];
     }
     const size_t n = c->grid().shell_size();
-    TCS_LAUNCH(c->stream, "copy_shell", k_copy_shell, dim3((unsigned)((n + 255) / 256), (unsigned)nf), dim3(256), 0,
-               c->grid(), src, dst);
+    TCS_LAUNCH(c->stream, "copy_shell", (k_copy_shell<double, FieldSet>), dim3((unsigned)((n + 255) / 256), (unsigned)nf),
+               dim3(256), 0, c->grid(), src, dst);
     return TCS_OK;
 }
 
-int halo(tcs_ctx *c, std::initializer_list<double *> fields) {
-    FieldSet fs{};
-    int nf = 0;
-    for (double *f : fields) {
-        if (nf == FieldSet::MAX) return TCS_E_ARG;
-        fs.f[nf++] = f;
-    }
-    const size_t n = (size_t)2 * c->N2 * c->N3 + (size_t)2 * c->N1 * c->N2;
-    TCS_LAUNCH(c->stream, "halo", (k_halo<double, FieldSet>), dim3((unsigned)((n + 255) / 256), (unsigned)nf),
-               dim3(256), 0, c->grid(), fs);
+int halo(tcs_ctx *c, std::initializer_list<double *> fields, std::initializer_list<const double *> walls) {
+    FieldSet fs{}, ws{};
+    int nf = 0, nw = 0;
+    if (fields.size() > FieldSet::MAX || (walls.size() != 0 && walls.size() != fields.size())) return TCS_E_ARG;
+    for (double *f : fields) fs.f[nf++] = f;
+    for (const double *w : walls) ws.f[nw++] = const_cast<double *>(w);
+    const size_t n = (size_t)2 * c->N2 * c->N3 + (size_t)2 * c->N1 * c->N2 + (nw ? (size_t)2 * c->n1m * c->n3m : 0);
+    const auto kernel = nw ? k_halo<double, FieldSet, true> : k_halo<double, FieldSet, false>;
+    TCS_LAUNCH(c->stream, "halo", kernel, dim3((unsigned)((n + 255) / 256), (unsigned)nf), dim3(256), 0, c->grid(), fs,
+               ws);
     return TCS_OK;
 }
 int halo(tcs_ctx *c, double *f) { return halo(c, {f}); }
@@ -190,8 +202,8 @@ int halo(tcs_ctx *c, std::initializer_list<float *> fields) {
         fs.f[nf++] = f;
     }
     const size_t n = (size_t)2 * c->N2 * c->N3 + (size_t)2 * c->N1 * c->N2;
-    TCS_LAUNCH(c->stream, "halo_f32", (k_halo<float, FieldSet32>), dim3((unsigned)((n + 255) / 256), (unsigned)nf),
-               dim3(256), 0, c->grid(), fs);
+    TCS_LAUNCH(c->stream, "halo_f32", (k_halo<float, FieldSet32, false>), dim3((unsigned)((n + 255) / 256), (unsigned)nf),
+               dim3(256), 0, c->grid(), fs, FieldSet{});
     return TCS_OK;
 }
 
@@ -207,6 +219,22 @@ static unsigned twin_bit(int id) {
     case TCS_MU: case TCS_INVRHO: return TWIN_TAB;
     default: return 0;
     }
+}
+
+// The cells outside the interior of fields into their FP32 twins (the
+// interior's twins written by the kernel that updated it)
+static int shell_to_twins(tcs_ctx *c, std::initializer_list<int> ids) {
+    FieldSet src{};
+    FieldSet32 dst{};
+    int nf = 0;
+    for (int id : ids) {
+        if (nf == FieldSet::MAX || !(dst.f[nf] = twin(c, c->f[id]))) return TCS_E_ARG;
+        src.f[nf++] = c->f[id];
+    }
+    const size_t n = c->grid().shell_size();
+    TCS_LAUNCH(c->stream, "twin_shell", (k_copy_shell<float, FieldSet32>), dim3((unsigned)((n + 255) / 256), (unsigned)nf),
+               dim3(256), 0, c->grid(), src, dst);
+    return TCS_OK;
 }
 
 __global__ void k_to_f32(const double *__restrict__ src, float *__restrict__ dst, size_t n) {
@@ -1196,38 +1224,46 @@ struct Wrap {  // tcs_ctx::wrap for a scope
 }  // namespace
 
 // Every ghost-cell update of main's order is made by the kernel that writes
-// the field (tcs_ctx::wrap), on large grids but for the block corrections and
-// the projection (wrap_cells).
+// the field, or on large grids by a launch after it (tcs_ctx::wrap_fields),
+// the fields written into second buffers with the wall rows of the first.
 extern "C" int tcs_step(tcs_ctx *c, double dt) {
     CTX_GUARD(c);
     STAGE("step");
     const Wrap wrap(c);
     bool swap_T = false;
     RUN("thermal solve", FORM(c, thermal_solver_into, dt, c->spare[TCS_T], &swap_T));
-    if (swap_T) std::swap(c->f[TCS_T], c->spare[TCS_T]);
-    if (c->a32 && swap_T) c->twin_ok |= TWIN_T;  // the mixed form: written by the last thermal sweep
+    const char *H = "update ghostcell";
+    const bool update = !c->wrap_fields();
+    double **f = c->f, **old = c->spare;  // of the fields exchanged
+    if (swap_T) std::swap(f[TCS_T], old[TCS_T]);
+    if (update) RUN(H, swap_T ? halo(c, {f[TCS_T]}, {old[TCS_T]}) : halo(c, f[TCS_T]));
+    if (c->a32 && swap_T) {  // the mixed form: written by the last thermal sweep
+        if (update) RUN(H, shell_to_twins(c, {TCS_T}));
+        c->twin_ok |= TWIN_T;
+    }
     RUN("momentum coeff", FORM(c, momentum_coeffi));
     RUN("momentum solvedU", FORM(c, momentum_solvedU, dt));
+    if (update) RUN(H, halo_field(c, TCS_DU));
     RUN("momentum solvedV", FORM(c, momentum_solvedV, dt));
+    if (update) RUN(H, halo_field(c, TCS_DV));
     RUN("momentum solvedW", FORM(c, momentum_solvedW, dt));
+    if (update) RUN(H, halo_field(c, TCS_DW));
     // block corrections with the pseudo-update (U + dU, V + dV, W + dW into
     // the second buffers; the corrections read the old U, V)
     RUN("momentum blockLdV", FORM(c, momentum_blockLdV_pseudo, dt, c->spare[TCS_V]));
-    const bool update = c->wrap_cells() == 2;
-    if (update) RUN("update ghostcell", halo_field(c, TCS_DV));
+    if (update) RUN(H, halo_field(c, TCS_DV));
     RUN("momentum blockLdU", FORM(c, momentum_blockLdU_pseudo, dt, c->spare[TCS_U], c->spare[TCS_W]));
-    for (int q : {TCS_U, TCS_V, TCS_W}) std::swap(c->f[q], c->spare[q]);
-    if (update) RUN("update ghostcell", halo(c, {c->f[TCS_U], c->f[TCS_V], c->f[TCS_W]}));
+    for (int q : {TCS_U, TCS_V, TCS_W}) std::swap(f[q], old[q]);
+    if (update) RUN(H, halo(c, {f[TCS_U], f[TCS_V], f[TCS_W]}, {old[TCS_U], old[TCS_V], old[TCS_W]}));
     // the right-hand side is made inside the solve's x transform
     RUN("pressure PoissonSolve", FORM(c, pressure_poisson_rhs, dt));
     RUN("pressure projection", FORM(c, pressure_projection_into, dt, c->spare[TCS_DPHAT], c->spare[TCS_DP0]));
-    std::swap(c->f[TCS_DPHAT], c->spare[TCS_DPHAT]);
-    std::swap(c->f[TCS_DP0], c->spare[TCS_DP0]);
+    std::swap(f[TCS_DPHAT], old[TCS_DPHAT]);
+    std::swap(f[TCS_DP0], old[TCS_DP0]);
     if (update) {
-        RUN("update ghostcell", halo(c, {c->f[TCS_U], c->f[TCS_V], c->f[TCS_W], c->f[TCS_P], c->f[TCS_DPHAT]}));
-        if (c->a32)
-            RUN("update ghostcell", halo(c, {twin(c, c->f[TCS_U]), twin(c, c->f[TCS_V]), twin(c, c->f[TCS_W]),
-                                             twin(c, c->f[TCS_P])}));
+        RUN(H, halo(c, {f[TCS_U], f[TCS_V], f[TCS_W], f[TCS_P], f[TCS_DPHAT]},
+                    {nullptr, nullptr, nullptr, nullptr, old[TCS_DPHAT]}));
+        if (c->a32) RUN(H, shell_to_twins(c, {TCS_U, TCS_V, TCS_W, TCS_P}));
     }
     // the mixed form: the projection wrote the FP32 copies of U, V, W, P
     if (c->a32) c->twin_ok |= TWIN_U | TWIN_V | TWIN_W | TWIN_P;

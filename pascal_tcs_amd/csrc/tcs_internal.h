@@ -93,7 +93,7 @@ struct Grid {
     int n1m, n2m, n3m;
     int N1, N2, N3;  // full extents n?m+2
     int P1;          // row pitch of the full fields
-    int wrap;        // kernels write the periodic ghosts and the wall rows (1), the wall rows (2)
+    int wrap;        // kernels that have the code for it write periodic ghosts and wall rows
     const double *dx1, *dx2, *dx3, *dmx1, *dmx2, *dmx3;
     const double *rdx1, *rdx2, *rdx3, *rdmx1, *rdmx2, *rdmx3;  // their reciprocals
     // the six tables (dx1, dmx1, dx2, dmx2, dx3, dmx3) back to back rounded to
@@ -115,7 +115,6 @@ struct Grid {
     // the images cost blockLdU 0.5 of 1.8 ms at 512^3.
     template <class E>
     __device__ __forceinline__ void images(E *F, int i, int k, size_t q, E v) const {
-        if (wrap == 2) return;
         const long di = i == 1 ? n1m : i == n1m ? -n1m : 0;
         if (di) F[(long)q + di] = v;
         if (k == 1 || k == n3m) {
@@ -124,11 +123,10 @@ struct Grid {
             if (di) F[(long)q + dk + di] = v;
         }
     }
-    // (wrap) whether cells i0..i0+ib-1, j, k0..k0+kb-1 touch the edge of the
+    // whether cells i0..i0+ib-1, j, k0..k0+kb-1 touch the edge of the
     // interior; ib and kb divide n1m and n3m
     __device__ __forceinline__ bool edge(int i0, int ib, int j, int k0, int kb) const {
-        return (wrap && (j == 1 || j == n2m)) ||
-               (wrap == 1 && (i0 == 1 || i0 + ib > n1m || k0 == 1 || k0 + kb > n3m));
+        return j == 1 || j == n2m || i0 == 1 || i0 + ib > n1m || k0 == 1 || k0 + kb > n3m;
     }
     // F's wall row next to row j, if there is one, from src's, with its
     // images: the thread of an edge row brings over the wall row of a second
@@ -240,21 +238,23 @@ struct tcs_ctx {
     int pend;
     double pend_dt_ldv, pend_dt_ldu, pend_dt_rhs;
     // Set within tcs_step, which knows that every field a kernel writes whole
-    // is followed by its ghost-cell update: the kernels write the periodic
-    // ghosts and the wall rows themselves (Grid::edge, images, wall; LineOut::gx)
-    // instead of 13 launches that cost 5 us each on a small grid (a step at
-    // 64^3 294 -> 264 us with the reductions' single launches; 256x193x128
-    // 2.07 -> 2.03 ms; 512^3 32.8 -> 32.4 ms).  The routines
-    // called one by one leave the ghosts to tcs_ghostcell_update, as a caller
-    // may look at them in between.
+    // is followed by its ghost-cell update.  The routines called one by one
+    // leave the ghosts to tcs_ghostcell_update, as a caller may look at them
+    // in between.
     int wrap;
-    // What the block corrections and the projection (one cell a thread, many
-    // fields) write: past 2^23 cells they leave the images to a ghost-cell
-    // update of all their fields, one store per line of memory in a kernel at
-    // its bandwidth costing more than the launch (at 512^3 the images took
-    // 0.22, 0.12 and 0.26 ms, the three launches 0.25; at 256x193x128 edges
-    // cost 3 us a kernel, a launch 6)
-    int wrap_cells() const { return wrap && nint > ((size_t)1 << 23) ? 2 : wrap; }
+    // Whether the kernels of a step write the periodic ghosts and the wall
+    // rows of their fields themselves (Grid::edge, images, wall; LineOut::gx).
+    // On a small grid they do, instead of 13 launches that cost 5 us each.
+    // Past 2^23 cells the fields are followed by ghost-cell updates, which
+    // bring the wall rows of a second buffer along, and the kernels are those
+    // without ghost code: the stores of the images, one per line of memory,
+    // and the registers they take in kernels at their bandwidth cost more than
+    // the launches (at 512^3 written by the kernels 32.3 ms a step, 53.0 in
+    // the exact form and 24.7 in the mixed; by launches 32.1, 51.9 and 24.5).
+    // Kernels against launches, plain and mixed: 64^3 211 us against 224 and
+    // 204 against 220; 256x128x128 1.11 ms against 1.12 and 0.85 against 0.87;
+    // 256x128x256 (2^23) 2.16 against 2.15 and 1.56 against 1.57.
+    bool wrap_fields() const { return wrap && nint <= ((size_t)1 << 23); }
     // The mixed form (precision 2): every array its stage rows and block
     // corrections read (T, U, V, W, P and the second buffers of T, U, V, W;
     // dU, dV, dW; the Mu and invRho tables; the wall tables; the stale
@@ -269,11 +269,6 @@ struct tcs_ctx {
     size_t an, aused;
     unsigned twin_ok;
 
-    tcs::Grid cell_grid() const {
-        tcs::Grid g = grid();
-        g.wrap = wrap_cells();
-        return g;
-    }
     tcs::Grid grid() const {
         tcs::Grid g;
         g.n1m = n1m; g.n2m = n2m; g.n3m = n3m;
@@ -362,7 +357,7 @@ struct LineOut {
     int gx = 0, gz = 0, n_row = 0;
     bool zero_walls = false;  // (gx > 0) the wall rows become zero (dV's)
     void wrap_to(const tcs_ctx *c, int nr) {
-        if (c->wrap) { gx = c->n1m; gz = c->n3m; n_row = nr; }
+        if (c->wrap_fields()) { gx = c->n1m; gz = c->n3m; n_row = nr; }
     }
 };
 namespace part {
@@ -462,7 +457,9 @@ struct FieldSet32 {
     float *f[FieldSet::MAX];
 };
 int halo(tcs_ctx *c, double *f);
-int halo(tcs_ctx *c, std::initializer_list<double *> fields);
+// walls (not empty: one for each field, or null): the buffers that the fields'
+// wall rows are brought over from, with their ghosts
+int halo(tcs_ctx *c, std::initializer_list<double *> fields, std::initializer_list<const double *> walls = {});
 // the same ghost-cell update of FP32 fields (the mixed form's increments)
 int halo(tcs_ctx *c, std::initializer_list<float *> fields);
 // The mixed form's FP32 twins of FP64 arrays (tcs_ctx::a32): which are

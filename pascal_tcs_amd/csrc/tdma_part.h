@@ -311,13 +311,39 @@ __device__ __forceinline__ void store(const T (&a)[MM], const T (&c)[MM], const 
                                       int j0, int m, T xf, T xl, T *D, long dbase, long rs, const LineOut &out,
                                       int s0, int s1) {
     const long fb = out.base + (long)s0 * out.ss0 + (long)s1 * out.ss1;
-    long di = 0, dk = 0;
-    if (out.gx > 0) {
-        di = s0 == 0 ? out.gx * out.ss0 : s0 == out.gx - 1 ? -out.gx * out.ss0 : 0;
-        dk = s1 == 0 ? out.gz * out.ss1 : s1 == out.gz - 1 ? -out.gz * out.ss1 : 0;
+    if (out.gx == 0) {  // a loop of its own, with nothing else in it
+        if constexpr (sizeof(T) == sizeof(float)) {
+            if (out.mode == 4) {
+#pragma unroll
+                for (int r = 0; r < MM; r++)
+                    if (r < m) out.G[fb + (long)(j0 + r) * out.rs] = x_of<T, 1, MM>(a, c, d, 0, r, m, xf, xl);
+                return;
+            }
+        }
+        if (out.mode == 0) {
+#pragma unroll
+            for (int r = 0; r < MM; r++)
+                if (r < m) D[dbase + (long)(j0 + r) * rs] = x_of<T, 1, MM>(a, c, d, 0, r, m, xf, xl);
+            return;
+        }
+#pragma unroll
+        for (int r = 0; r < MM; r++) {
+            if (r < m) {
+                const double x = (double)x_of<T, 1, MM>(a, c, d, 0, r, m, xf, xl);
+                const long o = fb + (long)(j0 + r) * out.rs;
+                const double v = out.mode == 1 ? x : (out.mode == 2 ? out.F[o] : out.Fin[o]) + x;
+                out.F[o] = v;
+                if constexpr (sizeof(T) == sizeof(float)) {
+                    if (out.G) out.G[o] = (float)v;  // the mixed form's FP32 copy of the field
+                }
+            }
+        }
+        return;
     }
+    const long di = s0 == 0 ? out.gx * out.ss0 : s0 == out.gx - 1 ? -out.gx * out.ss0 : 0;
+    const long dk = s1 == 0 ? out.gz * out.ss1 : s1 == out.gz - 1 ? -out.gz * out.ss1 : 0;
     // the wall row before the line's first part, after its last
-    const bool lo = out.gx > 0 && j0 == 0, hi = out.gx > 0 && j0 + m == out.n_row;
+    const bool lo = j0 == 0, hi = j0 + m == out.n_row;
     const long ol = fb - out.rs, oh = fb + (long)out.n_row * out.rs;
     if constexpr (sizeof(T) == sizeof(float)) {
         if (out.mode == 4) {  // FP32 lines only: the mixed form's increments
@@ -330,34 +356,28 @@ __device__ __forceinline__ void store(const T (&a)[MM], const T (&c)[MM], const 
             return;
         }
     }
-    if (out.mode == 0) {
 #pragma unroll
-        for (int r = 0; r < MM; r++)
-            if (r < m) D[dbase + (long)(j0 + r) * rs] = x_of<T, 1, MM>(a, c, d, 0, r, m, xf, xl);
-    } else {
-#pragma unroll
-        for (int r = 0; r < MM; r++) {
-            if (r < m) {
-                const double x = (double)x_of<T, 1, MM>(a, c, d, 0, r, m, xf, xl);
-                const long o = fb + (long)(j0 + r) * out.rs;
-                const double v = out.mode == 1 ? x : (out.mode == 2 ? out.F[o] : out.Fin[o]) + x;
-                put_line<double>(out.F, o, v, di, dk);
-                if constexpr (sizeof(T) == sizeof(float)) {
-                    if (out.G) put_line<float>(out.G, o, (float)v, di, dk);  // the mixed form's FP32 copy of the field
-                }
+    for (int r = 0; r < MM; r++) {
+        if (r < m) {
+            const double x = (double)x_of<T, 1, MM>(a, c, d, 0, r, m, xf, xl);
+            const long o = fb + (long)(j0 + r) * out.rs;
+            const double v = out.mode == 1 ? x : (out.mode == 2 ? out.F[o] : out.Fin[o]) + x;
+            put_line<double>(out.F, o, v, di, dk);
+            if constexpr (sizeof(T) == sizeof(float)) {
+                if (out.G) put_line<float>(out.G, o, (float)v, di, dk);
             }
         }
-        const double *walls = out.mode == 3 ? out.Fin : out.F;
-        for (int w = 0; w < 2; w++)
-            if (w ? hi : lo) {
-                const long o = w ? oh : ol;
-                const double v = out.zero_walls ? 0.0 : walls[o];
-                put_line<double>(out.F, o, v, di, dk);
-                if constexpr (sizeof(T) == sizeof(float)) {
-                    if (out.G) put_line<float>(out.G, o, (float)v, di, dk);
-                }
-            }
     }
+    const double *walls = out.mode == 3 ? out.Fin : out.F;
+    for (int w = 0; w < 2; w++)
+        if (w ? hi : lo) {
+            const long o = w ? oh : ol;
+            const double v = out.zero_walls ? 0.0 : walls[o];
+            put_line<double>(out.F, o, v, di, dk);
+            if constexpr (sizeof(T) == sizeof(float)) {
+                if (out.G) put_line<float>(out.G, o, (float)v, di, dk);
+            }
+        }
 }
 
 }  // namespace part

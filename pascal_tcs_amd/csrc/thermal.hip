@@ -470,6 +470,7 @@ struct ThermalY {
 };
 
 // T(i,j,k) += RHSJ (:518-524): F(i,j,k) += inc over the interior
+template <bool EDGES>
 __global__ void k_add_interior(Grid g, double *F, const scr_t *__restrict__ inc) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x + 1;
     const int j = blockIdx.y * blockDim.y + threadIdx.y + 1;
@@ -478,7 +479,7 @@ __global__ void k_add_interior(Grid g, double *F, const scr_t *__restrict__ inc)
     const size_t q = g.ix(i, j, k);
     const double f = F[q] + inc[g.r3(i, j, k)];
     F[q] = f;
-    if (g.edge(i, 1, j, k, 1)) {
+    if (EDGES && g.edge(i, 1, j, k, 1)) {
         g.images(F, i, k, q, f);
         g.wall(F, F, i, j, k);
     }
@@ -516,7 +517,7 @@ int sweep_y_field(tcs_ctx *c, int j0, int nrows, double *F, int mode) {
         return ptdma_part_launch(am, ac, ap, rhs, c->n1m, 1, c->n3m, n12, nrows, n1, false, c->stream, out);
     if (mode == 1) return exact_store(c, am, ac, ap, rhs, n12, nrows, n1, out);
     TCS_TRY(ptdma_sweep(c, am, ac, ap, rhs, c->n1m, 1, c->n3m, n12, nrows, n1, false));
-    TCS_LAUNCH(c->stream, "add_interior", k_add_interior, interior_grid(c->n1m, c->n2m, c->n3m), interior_block(), 0,
+    TCS_LAUNCH(c->stream, "add_interior", (c->wrap_fields() ? k_add_interior<true> : k_add_interior<false>), interior_grid(c->n1m, c->n2m, c->n3m), interior_block(), 0,
                c->grid(), F, SCR(c->rhs));
     return TCS_OK;
 }
@@ -555,7 +556,7 @@ int thermal_solver(tcs_ctx *c, double dt) {
         // the y rows read T around every cell, so the increment goes through
         // the scratch and is added once every line is solved
         TCS_TRY(y_stage_in_solve<ANY_SPLIT>(c, "thermal_y_solve", y, 1, c->n2m, rhs, nullptr, 0));
-        TCS_LAUNCH(c->stream, "add_interior", k_add_interior, interior_grid(c->n1m, c->n2m, c->n3m),
+        TCS_LAUNCH(c->stream, "add_interior", (c->wrap_fields() ? k_add_interior<true> : k_add_interior<false>), interior_grid(c->n1m, c->n2m, c->n3m),
                    interior_block(), 0, g, T, rhs);
         return TCS_OK;
     }
