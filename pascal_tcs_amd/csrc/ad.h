@@ -77,10 +77,12 @@ __device__ __forceinline__ auto pick(bool passed, A a, B b) {
     }
 }
 // x with the wall terms f(x) in wall-term mode WM: 0 computes them, 1 skips
-// them where near is false, 2 leaves them out
+// them where near is false (not in the reverse pass), 2 leaves them out
 template <class S, int WM, class X, class F>
 __device__ __forceinline__ auto with_walls(bool near, const X &x, F f) {
     if constexpr (is_rev<S>()) {
+        // what is recorded must not depend on the cell
+        static_assert(WM != 1, "wall terms of the reverse pass: computed (0) or left out (2)");
         if constexpr (WM == 0) return f(x);
         else return rev_of(x, x.v, 1.0);
     } else if constexpr (WM == 0) {
