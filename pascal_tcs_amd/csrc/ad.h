@@ -102,17 +102,17 @@ struct RawW {
     __device__ __forceinline__ const double *operator()(int, const double *p) const { return p; }
 };
 
+// A value type of the adjoint (neither double nor float).  The stage rows
+// have no branch on j for these: the reverse pass's operations are the same
+// for every cell.
+template <class S>
+constexpr bool is_dual() { return !std::is_same<S, double>::value && !std::is_same<S, float>::value; }
+
 // The mixed form's rows: FP32 arithmetic on the FP32 twins of the arrays
 // they read.  In that form every array a stage row or block correction reads
 // (state, increments, (j, k) tables, wall tables, stale scalars) lives in
 // one FP64 arena and has an FP32 twin at the same element offset of an FP32
 // arena, so the twin of p is f + (p - d).
-// A value type of the adjoint (neither double nor float).  The stage rows
-// have no branch on j for these: the tape of a formula is the same for every
-// cell.
-template <class S>
-constexpr bool is_dual() { return !std::is_same<S, double>::value && !std::is_same<S, float>::value; }
-
 struct F32Ptr {
     const float *p;
     __device__ __forceinline__ float operator[](size_t i) const { return p[i]; }

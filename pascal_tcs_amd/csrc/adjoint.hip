@@ -12,10 +12,10 @@
 //     RHS, pseudo-update): vector-Jacobian products of the cell formulas
 //     (rev.h: one reverse pass a cell);
 //   * each ADI stage x = A^-1 d: lambda = A^-T xbar by the transposed line
-//     solve (the stage's rows, transposed in place along the line, solved by
-//     the single-rank PaScaL_TDMA kernel), row adjoints abar_i = -lambda_i
-//     x_{i-1}, bbar_i = -lambda_i x_i, cbar_i = -lambda_i x_{i+1},
-//     dbar_i = lambda_i, then the rows' vector-Jacobian product;
+//     solve (the stage's rows, stored where the transposed systems have them,
+//     solved as the step solves its lines: split when they are), row adjoints
+//     abar_i = -lambda_i x_{i-1}, bbar_i = -lambda_i x_i, cbar_i = -lambda_i
+//     x_{i+1}, dbar_i = lambda_i, then the rows' vector-Jacobian product;
 //   * the Poisson solve: the same FFT pipeline with every wavenumber's
 //     y-system transposed (the pinned mean mode's row projection after the
 //     solve, the zeroed imaginary parts before it), which is the exact
@@ -869,8 +869,10 @@ extern "C" int tcs_adjoint_step(tcs_ctx *c, double dt) {
         set_error("tcs_adjoint_step: the adjoint differentiates the plain FP64 step (precision 0)");
         return TCS_E_ARG;
     }
-    // the interface's limit on the grid (2^28 values a field)
-    if (c->nfull + FIELD_FRONT + 1 > ((size_t)1 << 28)) return TCS_E_ARG;
+    if (c->nfull + FIELD_FRONT + 1 > ((size_t)1 << 28)) {  // the interface's limit
+        set_error("tcs_adjoint_step: the full fields must hold fewer than 2^28 values");
+        return TCS_E_ARG;
+    }
     TCS_TRY(adjoint_alloc(c));
     c->cfl_valid = 0;
     TCS_TRY(adj::forward_keep(c, c->adj, dt));

@@ -372,7 +372,6 @@ struct DUY {
     }
 };
 
-// interior copy: F(i,j,k) = RHS for j in [j0, n2m]
 // dV(0:n1sub,0:1,0:n3sub) = 0 and dV(:,n2sub,:) = 0 (:907-909)
 template <typename E>
 __global__ void k_dV_zero_rows(Grid g, E *__restrict__ dV) {

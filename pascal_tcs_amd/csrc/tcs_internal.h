@@ -60,7 +60,7 @@ void prof_end(hipStream_t s);
 
 // An index of a cell formula in the adjoint's reverse pass: the index v and
 // its constant offset o in {-1, 0, 1} from the cell's own, which names the
-// input on the tape (rev.h).  RelCell: element q of a field, rel from the
+// input's accumulator (rev.h).  RelCell: element q of a field, rel from the
 // three offsets; RelRow: element q of a (j, k) table.
 struct Rel {
     int v, o;

@@ -2,9 +2,10 @@
 // (PaScaL_TDMA's multi-rank algorithm with one GPU thread per rank), shared
 // by the ADI sweeps (tdma_part.hip) and the Poisson y-solve (pressure.hip).
 //
-// A line of n_row <= 512 rows is split into P parts (P a power of two, rows
-// per part by para_range, PaScaL_TDMA/src/para_range.f90:26-40); the thread
-// of part p holds its m <= PT_MMAX rows in registers.  NR right-hand sides
+// A line is split into P parts (P a power of two, rows per part by
+// para_range, PaScaL_TDMA/src/para_range.f90:26-40), at most 32 for lines of
+// up to 512 rows and in the fast forms 128 for up to 2048; the thread of part
+// p holds its m <= PT_MMAX rows in registers.  NR right-hand sides
 // may share one matrix (the Poisson solve's real and imaginary parts): the
 // matrix recurrences run once, every right-hand side gets exactly the
 // operations a separate solve would give it.
