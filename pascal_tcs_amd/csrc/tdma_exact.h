@@ -16,8 +16,10 @@
 //     as the wavefronts that share a CU leave room for;
 //   * the backward elimination runs twice: once without a store, to find the
 //     two ends of the solution, and once more, the same operations, to
-//     write the solution (112 B an unknown; three passes in place moved
-//     136, 128 when the eliminated coefficients are returned).
+//     write the solution (counted: 111 B an unknown contiguous, 102 to 104
+//     strided at 256x200x256, 49 strided at 128^3, where most rows stay in
+//     LDS; 128 and 124 at 512^3 with the eliminated coefficients returned;
+//     three passes in place moved 136).
 #pragma once
 
 #include <algorithm>
