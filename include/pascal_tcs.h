@@ -51,8 +51,8 @@ typedef struct tcs_params {
                                      ADI lines of up to 2048) split into
                                      parts as PaScaL_TDMA splits them over
                                      ranks (see ptdma_many_solve_part_dev;
-                                     precision 1 and 2 choose the parts by
-                                     the number of lines) */
+                                     precision 1 chooses the parts by the
+                                     number of lines) */
     double Ct, Cmu, Cmt, Cmp;     /* :139-141 */
     double DeltaT;                /* namelist sim_parameter */
     double a10, a11, a12, a13, a14, a15;  /* density polynomial   :117 */

@@ -252,7 +252,7 @@ struct tcs_ctx {
     // the launches (at 512^3 written by the kernels 32.3 ms a step, 53.0 in
     // the exact form and 24.7 in the mixed; by launches 32.1, 51.9 and 24.5).
     // Kernels against launches, plain and mixed: 64^3 211 us against 224 and
-    // 204 against 220; 256x128x128 1.11 ms against 1.12 and 0.85 against 0.87;
+    // 288 against 301; 256x128x128 1.11 ms against 1.12 and 0.85 against 0.87;
     // 256x128x256 (2^23) 2.16 against 2.15 and 1.56 against 1.57.
     bool wrap_fields() const { return wrap && nint <= ((size_t)1 << 23); }
     // The mixed form (precision 2): every array its stage rows and block

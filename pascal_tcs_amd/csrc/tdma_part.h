@@ -43,8 +43,10 @@ inline PartPlan part_plan(int n_row, int mm, int pm) {
 //     makes its part's rows one after the other, which is what a small grid
 //     waits for (64^3: dW z 42 -> 13 us, dU z 24 -> 13, dW x 25 -> 12).  No
 //     part gets fewer than three rows.
-// The lines' errors against 64 bits stay where they were (16x40x32 to
-// 2048x40x16 and 16x1100x16).
+// The errors against 64 bits stay where they were (16x40x32 to 2048x40x16 and
+// 16x1100x16), for FP64 lines: FP32 lines in shorter parts lose digits (the
+// mixed form's U 14 to 22 % further off after two steps at 64^3, 32x128x32 and
+// 16x100x256, P up to 39 %), so they keep the 16-row parts.
 constexpr long PART_FILL = 8L * 64 * 256;
 inline bool part_plan_any(int n_row, long lines, PartPlan &q) {
     if (n_row < 2 || n_row > 4 * PT_MMAX * PT_PMAX) return false;
@@ -383,7 +385,7 @@ __device__ __forceinline__ void store(const T (&a)[MM], const T (&c)[MM], const 
 
 }  // namespace part
 
-// the plan of a stage's lines: part_plan_any's (ANY) or ptdma_part_plan's
+// the plan of a stage's lines: part_plan_any's (ANY, FP64) or ptdma_part_plan's
 template <bool ANY>
 inline bool part_plan_for(int n_row, long lines, PartPlan &q) {
     if constexpr (ANY) return part_plan_any(n_row, lines, q);
@@ -704,17 +706,16 @@ template <bool CYC, int SX, bool ANY, typename T, class Src>
 int ptdma_part_src_launch(hipStream_t st, const char *label, const Src &src, T *D, int n0, int n1, long ss1,
                           int n_row, long rs, const LineOut &out = LineOut()) {
     PartPlan q;
+    constexpr bool CHOOSE = ANY && sizeof(T) == 8;
     if (n0 <= 0 || n1 <= 0) return TCS_OK;
-    if (!part_plan_for<ANY>(n_row, (long)n0 * n1, q) || n1 > 65535) {
+    if (!part_plan_for<CHOOSE>(n_row, (long)n0 * n1, q) || n1 > 65535) {
         set_error("ptdma_part: line length outside the split range or outer line count > 65535");
         return TCS_E_ARG;
     }
-    if constexpr (ANY) {
+    if constexpr (CHOOSE) {
         constexpr int M = PT_MMAX, PP = PT_PMAX;
-        if constexpr (sizeof(T) == 8)
-            if (q.pm == 2 * PP) return part_src_launch<CYC, 8, false, M, 2 * PP>(st, label, src, q, D, n0, n1, ss1, rs, out);
-        if constexpr (sizeof(T) == 8)
-            if (q.pm == 4 * PP) return part_src_launch<CYC, 4, false, M, 4 * PP>(st, label, src, q, D, n0, n1, ss1, rs, out);
+        if (q.pm == 2 * PP) return part_src_launch<CYC, 8, false, M, 2 * PP>(st, label, src, q, D, n0, n1, ss1, rs, out);
+        if (q.pm == 4 * PP) return part_src_launch<CYC, 4, false, M, 4 * PP>(st, label, src, q, D, n0, n1, ss1, rs, out);
         if (q.mm == 8) return part_src_launch<CYC, 16, false, 8, PP>(st, label, src, q, D, n0, n1, ss1, rs, out);
         if (q.mm == 4) return part_src_launch<CYC, 16, false, 4, PP>(st, label, src, q, D, n0, n1, ss1, rs, out);
     }
@@ -742,17 +743,16 @@ template <bool CYC, bool ANY, typename T, class Src>
 int ptdma_part_rows_src_launch(hipStream_t st, const char *label, const Src &src, T *D, int n0, long ss0, int n1,
                                long ss1, int n_row) {
     PartPlan q;
+    constexpr bool CHOOSE = ANY && sizeof(T) == 8;
     if (n0 <= 0 || n1 <= 0) return TCS_OK;
-    if (!part_plan_for<ANY>(n_row, (long)n0 * n1, q) || n1 > 65535) {
+    if (!part_plan_for<CHOOSE>(n_row, (long)n0 * n1, q) || n1 > 65535) {
         set_error("ptdma_part: line length outside the split range or outer line count > 65535");
         return TCS_E_ARG;
     }
     constexpr int M = PT_MMAX, PP = PT_PMAX, X = PT_XSX;
-    if constexpr (ANY) {
-        if constexpr (sizeof(T) == 8)
-            if (q.pm == 2 * PP) return part_rows_src_launch<CYC, X, M, 2 * PP>(st, label, src, q, D, n0, ss0, n1, ss1, n_row);
-        if constexpr (sizeof(T) == 8)
-            if (q.pm == 4 * PP) return part_rows_src_launch<CYC, X, M, 4 * PP>(st, label, src, q, D, n0, ss0, n1, ss1, n_row);
+    if constexpr (CHOOSE) {
+        if (q.pm == 2 * PP) return part_rows_src_launch<CYC, X, M, 2 * PP>(st, label, src, q, D, n0, ss0, n1, ss1, n_row);
+        if (q.pm == 4 * PP) return part_rows_src_launch<CYC, X, M, 4 * PP>(st, label, src, q, D, n0, ss0, n1, ss1, n_row);
         if (q.mm == 8) return part_rows_src_launch<CYC, 8, 8, PP>(st, label, src, q, D, n0, ss0, n1, ss1, n_row);
         if (q.mm == 4) return part_rows_src_launch<CYC, 8, 4, PP>(st, label, src, q, D, n0, ss0, n1, ss1, n_row);
     }
